@@ -19,6 +19,9 @@ SIGNATURES = {
     "nvf_nvfp4_grouped_block_quantize": (_int, [_p, _int, _i64, _i64, _p, _p, _int, _p, _p, _p, _p]),
     "nvf_nvfp4_silu_mul_block_quantize": (_int, [_p, _p, _int, _i64, _i64, _p, _p, _int, _p, _p, _p, _p]),
     "nvf_nvfp4_global_scale": (_int, [_p, _int, _i64, _p, _p]),
+    "nvf_nvfp4_global_scale_workspace_bytes": (_i64, [_i64]),
+    "nvf_nvfp4_global_scale_ws": (_int, [_p, _int, _i64, _p, _p, _i64, _p]),
+    "nvf_grouped_auxiliary_tensors": (_int, [_p, _int, _i64, _i64, _i64, _p, _p, _p]),
     "nvf_preprocess_grouped_matmul_input_sf": (_int, [_p, _int, _i64, _i64, _p, _p, _int, _p, _p]),
     "nvf_mxfp8_block_quantize": (_int, [_p, _int, _i64, _i64, _int, _p, _p, _p]),
     "nvf_cast_f32_to_e2m1": (_int, [_p, _i64, _p, _p]),

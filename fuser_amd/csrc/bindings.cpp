@@ -80,6 +80,13 @@ PYBIND11_MODULE(_C, m) {
         return py::make_tuple(r.first, r.second);
       },
       py::arg("gate"), py::arg("up"), py::arg("input_offsets"), py::arg("output_offsets"), py::arg("global_scale") = py::none());
+  m.def(
+      "grouped_auxiliary_tensors",
+      [](const torch::Tensor& offsets, int64_t rows, int64_t n, int64_t k) {
+        auto r = bq::grouped_auxiliary_tensors(offsets, rows, n, k);
+        return py::make_tuple(r.first, r.second);
+      },
+      py::arg("offsets"), py::arg("rows"), py::arg("n"), py::arg("k"));
   m.def("compute_nvfp4_global_scale", &bq::compute_nvfp4_global_scale, py::arg("tensor"));
 
   // Conventions of the reference's expression nodes around the kernels (csrc/ir/composite_nodes.cpp).

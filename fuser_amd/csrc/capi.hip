@@ -140,11 +140,35 @@ int nvf_nvfp4_silu_mul_block_quantize(const void* gate, const void* up, int in_d
                                         grouped ? groups : 1, out_fp4, out_scales, static_cast<hipStream_t>(stream));
 }
 
-int nvf_nvfp4_global_scale(const void* in, int in_dtype, int64_t numel, float* out_scale, void* stream) {
+static int check_global_scale_args(const void* in, int in_dtype, int64_t numel, const float* out_scale) {
   NVF_REQUIRE(dtype_in(in_dtype), NVF_ERR_INVALID_ARGUMENT, "unknown input dtype %d", in_dtype);
   NVF_REQUIRE(numel >= 0, NVF_ERR_INVALID_ARGUMENT, "negative size %lld", (long long)numel);
   NVF_REQUIRE(out_scale && (in || numel == 0), NVF_ERR_INVALID_ARGUMENT, "NULL buffer");
-  return launch_nvfp4_global_scale(in, in_dtype, numel, out_scale, static_cast<hipStream_t>(stream));
+  return NVF_OK;
+}
+
+int nvf_nvfp4_global_scale(const void* in, int in_dtype, int64_t numel, float* out_scale, void* stream) {
+  if (const int rc = check_global_scale_args(in, in_dtype, numel, out_scale)) return rc;
+  return launch_nvfp4_global_scale(in, in_dtype, numel, out_scale, nullptr, 0, static_cast<hipStream_t>(stream));
+}
+
+int64_t nvf_nvfp4_global_scale_workspace_bytes(int64_t numel) { return nvfp4_global_scale_workspace_bytes(numel); }
+
+int nvf_nvfp4_global_scale_ws(const void* in, int in_dtype, int64_t numel, float* out_scale, void* workspace,
+                              int64_t workspace_bytes, void* stream) {
+  if (const int rc = check_global_scale_args(in, in_dtype, numel, out_scale)) return rc;
+  NVF_REQUIRE(workspace_bytes >= 0 && (workspace || workspace_bytes == 0) && (reinterpret_cast<uintptr_t>(workspace) & 3) == 0,
+              NVF_ERR_INVALID_ARGUMENT, "bad workspace");
+  return launch_nvfp4_global_scale(in, in_dtype, numel, out_scale, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
+}
+
+int nvf_grouped_auxiliary_tensors(const int32_t* offsets, int groups, int64_t rows, int64_t n, int64_t k, int32_t* sf_offsets,
+                                  int32_t* problem_sizes, void* stream) {
+  NVF_REQUIRE(groups >= 0 && rows >= 0 && n >= 0 && k >= 0, NVF_ERR_INVALID_ARGUMENT, "negative size");
+  NVF_REQUIRE(rows <= INT32_MAX && n <= INT32_MAX && k <= INT32_MAX, NVF_ERR_UNSUPPORTED_SHAPE, "dimension exceeds int32");
+  if (groups == 0) return NVF_OK;
+  NVF_REQUIRE(offsets && sf_offsets && problem_sizes, NVF_ERR_INVALID_ARGUMENT, "NULL buffer");
+  return launch_grouped_auxiliary_tensors(offsets, groups, rows, n, k, sf_offsets, problem_sizes, static_cast<hipStream_t>(stream));
 }
 
 int nvf_preprocess_grouped_matmul_input_sf(const void* in, int elem_size, int64_t rows, int64_t cols,

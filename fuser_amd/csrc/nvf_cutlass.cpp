@@ -435,10 +435,27 @@ torch::Tensor compute_nvfp4_global_scale(const torch::Tensor& tensor) {
             "Expected a Float, BFloat16 or Half tensor.");
   c10::DeviceGuard guard(tensor.device());
   torch::Tensor scale = at::empty({}, tensor.options().dtype(at::ScalarType::Float));
-  check_status(nvf_nvfp4_global_scale(tensor.data_ptr(), to_nvf_dtype(t), tensor.numel(), static_cast<float*>(scale.data_ptr()),
-                                      current_stream(tensor)),
+  const int64_t ws_bytes = nvf_nvfp4_global_scale_workspace_bytes(tensor.numel());
+  torch::Tensor workspace;
+  if (ws_bytes > 0) workspace = at::empty({ws_bytes}, tensor.options().dtype(at::ScalarType::Byte));
+  check_status(nvf_nvfp4_global_scale_ws(tensor.data_ptr(), to_nvf_dtype(t), tensor.numel(), static_cast<float*>(scale.data_ptr()),
+                                         ws_bytes > 0 ? workspace.data_ptr() : nullptr, ws_bytes, current_stream(tensor)),
                "compute_nvfp4_global_scale");
   return scale;
+}
+
+std::pair<torch::Tensor, torch::Tensor> grouped_auxiliary_tensors(const torch::Tensor& offsets, int64_t rows, int64_t n, int64_t k) {
+  NVF_CHECK(offsets.is_cuda() && offsets.is_contiguous() && offsets.dim() == 1 && offsets.scalar_type() == at::ScalarType::Int,
+            "Offsets must be contiguous 1-D int32 CUDA tensors.");
+  c10::DeviceGuard guard(offsets.device());
+  const int64_t groups = offsets.size(0);
+  torch::Tensor sf_offsets = at::empty({groups}, offsets.options());
+  torch::Tensor problem_sizes = at::empty({groups, 3}, offsets.options());
+  check_status(nvf_grouped_auxiliary_tensors(static_cast<const int32_t*>(offsets.data_ptr()), static_cast<int>(groups), rows, n, k,
+                                             static_cast<int32_t*>(sf_offsets.data_ptr()),
+                                             static_cast<int32_t*>(problem_sizes.data_ptr()), current_stream(offsets)),
+               "grouped_auxiliary_tensors");
+  return {sf_offsets, problem_sizes};
 }
 
 torch::Tensor preprocess_grouped_matmul_input_sf(const torch::Tensor& input, const torch::Tensor& input_offsets,

@@ -119,6 +119,11 @@ NVF_HOST_API std::pair<torch::Tensor, torch::Tensor> silu_mul_nv_grouped_block_q
 // host round trip.
 NVF_HOST_API torch::Tensor compute_nvfp4_global_scale(const torch::Tensor& tensor);
 
+// (scale slab starts [G], problem sizes [G, 3]) of the groups whose first rows are `offsets`; the last one ends at row `rows`
+// (benchmarks/python/layers_for_inference_benchmark.py:395-424)
+NVF_HOST_API std::pair<torch::Tensor, torch::Tensor> grouped_auxiliary_tensors(const torch::Tensor& offsets, int64_t rows, int64_t n,
+                                                                                int64_t k);
+
 NVF_HOST_API torch::Tensor preprocess_grouped_matmul_input_sf(const torch::Tensor& input,
                                                               const torch::Tensor& input_offsets,
                                                               const torch::Tensor& output_offsets);

@@ -53,8 +53,13 @@ int launch_nvfp4_quantize(const void* in, int in_dtype, int64_t rows, int64_t co
 int launch_nvfp4_silu_mul_quantize(const void* gate, const void* up, int in_dtype, int64_t rows, int64_t cols, const float* gs,
                                    int layout, const int32_t* in_off, const int32_t* out_off, int groups, void* out_fp4,
                                    void* out_sf, hipStream_t stream);
-// out[0] = 448 * 6 / max|in| (1 if the tensor is all zero)
-int launch_nvfp4_global_scale(const void* in, int in_dtype, int64_t n, float* out, hipStream_t stream);
+// out[0] = 448 * 6 / max|in| (1 if the tensor is all zero); workspace: optional (nvfp4_global_scale_workspace_bytes)
+int launch_nvfp4_global_scale(const void* in, int in_dtype, int64_t n, float* out, void* workspace, int64_t workspace_bytes,
+                              hipStream_t stream);
+int64_t nvfp4_global_scale_workspace_bytes(int64_t n);
+// scale slab starts and problem sizes of groups given by their first rows
+int launch_grouped_auxiliary_tensors(const int32_t* offsets, int groups, int64_t rows, int64_t n, int64_t k, int32_t* sf_offsets,
+                                     int32_t* problem_sizes, hipStream_t stream);
 int launch_preprocess_sf(const void* in, int elem_size, int64_t rows, int64_t cols, const int32_t* in_off,
                          const int32_t* out_off, int groups, void* out, hipStream_t stream);
 int launch_mxfp8_quantize(const void* in, int in_dtype, int64_t rows, int64_t cols, int swizzle, void* out_fp8,

@@ -8,6 +8,7 @@
 // half an MXFP8 block); a workgroup is 4 consecutive rows of one segment; details at each kernel.
 #include "nvf_internal.h"
 
+#include <algorithm>
 #include <cfloat>
 
 namespace nvf {
@@ -284,38 +285,6 @@ __device__ __forceinline__ uint32_t abs_bits(float v) { return f32_to_bits(v) & 
 
 __global__ void amax_init_kernel(uint32_t* cell) { *cell = 0u; }
 
-template <typename T>
-__global__ __launch_bounds__(256) void amax_kernel(const T* __restrict__ in, int64_t n, int64_t head, int64_t nvec,
-                                                   uint32_t* __restrict__ cell) {
-  constexpr int VE = 16 / (int)sizeof(T);  // elements per 16-byte load
-  const int64_t tid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  uint32_t m = 0;
-  const u32x4* vec = reinterpret_cast<const u32x4*>(in + head);
-  auto fold = [&](const u32x4 q) {
-    T e[VE];
-    __builtin_memcpy(e, &q, 16);
-#pragma unroll
-    for (int j = 0; j < VE; ++j) m = max(m, abs_bits(e[j]));
-  };
-  int64_t i = tid;
-  for (; i + 3 * stride < nvec; i += 4 * stride) {  // four loads in flight per thread
-    const u32x4 q0 = __builtin_nontemporal_load(vec + i), q1 = __builtin_nontemporal_load(vec + i + stride);
-    const u32x4 q2 = __builtin_nontemporal_load(vec + i + 2 * stride), q3 = __builtin_nontemporal_load(vec + i + 3 * stride);
-    fold(q0);
-    fold(q1);
-    fold(q2);
-    fold(q3);
-  }
-  for (; i < nvec; i += stride) fold(__builtin_nontemporal_load(vec + i));
-  // elements before the first and after the last whole 16-byte vector
-  const int64_t tail0 = head + nvec * VE;
-  for (int64_t t = tid; t < head + (n - tail0); t += stride) m = max(m, abs_bits(in[t < head ? t : tail0 + (t - head)]));
-#pragma unroll
-  for (int d = 32; d >= 1; d >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, d, 64));
-  if ((threadIdx.x & 63) == 0 && m != 0) atomicMax(cell, m);
-}
-
 __device__ __forceinline__ float amax_bits_to_global_scale(uint32_t amax_bits) {
   const float amax = bits_to_f32(amax_bits);
   if (amax != amax) return amax;
@@ -328,43 +297,110 @@ __global__ void amax_to_global_scale_kernel(uint32_t* cell) {
   *reinterpret_cast<float*>(cell) = amax_bits_to_global_scale(*cell);
 }
 
-// small tensors: one workgroup does the whole job in one launch
-template <typename T>
-__global__ __launch_bounds__(1024) void global_scale_small_kernel(const T* __restrict__ in, int64_t n, float* __restrict__ out) {
-  __shared__ uint32_t wave_max[16];
-  uint32_t m = 0;
-  for (int64_t i = threadIdx.x; i < n; i += 1024) m = max(m, abs_bits(in[i]));
+// maximum over the workgroup, valid in thread 0
+template <int THREADS>
+__device__ __forceinline__ uint32_t workgroup_max(uint32_t m) {
+  __shared__ uint32_t wave_max[THREADS / 64];
 #pragma unroll
   for (int d = 32; d >= 1; d >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, d, 64));
   if ((threadIdx.x & 63) == 0) wave_max[threadIdx.x >> 6] = m;
   __syncthreads();
   if (threadIdx.x == 0) {
 #pragma unroll
-    for (int w = 1; w < 16; ++w) m = max(m, wave_max[w]);
-    *out = amax_bits_to_global_scale(m);
+    for (int w = 1; w < THREADS / 64; ++w) m = max(m, wave_max[w]);
+  }
+  return m;
+}
+
+// The thread's maximum over the elements its workgroup (`wg` of `wgs`) owns.  A workgroup reads runs of LOADS * THREADS
+// consecutive 16-byte vectors, so that the chip reads the tensor nearly in order: 940 MB in 133 us (7.1 TB/s), against
+// 168 us where every load of a thread is a whole grid apart.
+template <typename T, int THREADS, int LOADS, bool STREAM>
+__device__ __forceinline__ uint32_t amax_of_part(const T* __restrict__ in, int64_t n, int64_t head, int64_t nvec, int64_t wg, int64_t wgs) {
+  constexpr int VE = 16 / (int)sizeof(T);  // elements per 16-byte load
+  uint32_t m = 0;
+  const u32x4* vec = reinterpret_cast<const u32x4*>(in + head);
+  for (int64_t base = wg * (LOADS * THREADS); base < nvec; base += wgs * (LOADS * THREADS)) {
+    u32x4 q[LOADS];
+#pragma unroll
+    for (int u = 0; u < LOADS; ++u) {
+      const int64_t i = base + u * THREADS + threadIdx.x;
+      q[u] = u32x4{0, 0, 0, 0};
+      if (i < nvec) q[u] = STREAM ? __builtin_nontemporal_load(vec + i) : vec[i];
+    }
+#pragma unroll
+    for (int u = 0; u < LOADS; ++u) {
+      T e[VE];
+      __builtin_memcpy(e, &q[u], 16);
+#pragma unroll
+      for (int j = 0; j < VE; ++j) m = max(m, abs_bits(e[j]));
+    }
+  }
+  // elements before the first and after the last whole 16-byte vector: fewer than 2 * VE
+  const int64_t tail0 = head + nvec * VE, t = threadIdx.x;
+  if (wg == 0 && t < head + (n - tail0)) m = max(m, abs_bits(in[t < head ? t : tail0 + (t - head)]));
+  return m;
+}
+
+// PARTIAL: every workgroup writes the maximum of its part to cell[blockIdx.x]; otherwise all raise the one cell.
+template <typename T, bool STREAM, bool PARTIAL>
+__global__ __launch_bounds__(256) void amax_kernel(const T* __restrict__ in, int64_t n, int64_t head, int64_t nvec,
+                                                   uint32_t* __restrict__ cell) {
+  const uint32_t m = workgroup_max<256>(amax_of_part<T, 256, 4, STREAM>(in, n, head, nvec, blockIdx.x, gridDim.x));
+  if (threadIdx.x == 0) {
+    if constexpr (PARTIAL) cell[blockIdx.x] = m;
+    else atomicMax(cell, m);
   }
 }
 
+// last step: the partial maxima (at most 1024) to the scale
+__global__ __launch_bounds__(1024) void partial_amax_to_global_scale_kernel(const uint32_t* __restrict__ partial, int count,
+                                                                            float* __restrict__ out) {
+  const uint32_t m = workgroup_max<1024>((int)threadIdx.x < count ? partial[threadIdx.x] : 0u);
+  if (threadIdx.x == 0) *out = amax_bits_to_global_scale(m);
+}
+
+// small tensors: one workgroup does the whole job in one launch
 template <typename T>
-int launch_global_scale_typed(const T* in, int64_t n, float* out, hipStream_t stream) {
+__global__ __launch_bounds__(1024) void global_scale_small_kernel(const T* __restrict__ in, int64_t n, int64_t head, int64_t nvec,
+                                                                  float* __restrict__ out) {
+  const uint32_t m = workgroup_max<1024>(amax_of_part<T, 1024, 4, false>(in, n, head, nvec, 0, 1));
+  if (threadIdx.x == 0) *out = amax_bits_to_global_scale(m);
+}
+
+constexpr int64_t kGlobalScaleMaxPartials = 1024;
+constexpr int64_t kGlobalScaleSmall = 65536;  // elements up to which one workgroup does it
+
+template <typename T>
+int launch_global_scale_typed(const T* in, int64_t n, float* out, uint32_t* partial, hipStream_t stream) {
   constexpr int VE = 16 / (int)sizeof(T);
-  if (n <= 65536) {
-    hipLaunchKernelGGL(global_scale_small_kernel<T>, dim3(1), dim3(1024), 0, stream, in, n, out);
+  int64_t head = (int64_t)(((16 - (reinterpret_cast<uintptr_t>(in) & 15)) & 15) / sizeof(T));  // elements up to 16-byte alignment
+  if (head > n) head = n;
+  const int64_t nvec = (n - head) / VE;
+  if (n <= kGlobalScaleSmall) {
+    hipLaunchKernelGGL(global_scale_small_kernel<T>, dim3(1), dim3(1024), 0, stream, in, n, head, nvec, out);
     return check_launch("nvfp4_global_scale");
   }
+  // Tensors beyond what the 256 MB last-level cache holds are read past it (133 us for 940 MB, 152 us with plain loads);
+  // smaller ones may well be in it (32 MB: 6.6 us with plain loads, 8.6 with non-temporal ones).  Two workgroups per
+  // compute unit then keep the reads nearly in order; the small ones want more in flight.
+  const bool stream_loads = n * (int64_t)sizeof(T) > ((int64_t)256 << 20);
+  const int64_t want = ceil_div(nvec, 256 * 4), cap = stream_loads ? 2 * (int64_t)cu_count() : kGlobalScaleMaxPartials;
+  const int64_t wgs = std::min(std::min(want, cap), kGlobalScaleMaxPartials);
+  const dim3 grid((unsigned)wgs);
+  if (partial != nullptr) {
+    if (stream_loads) hipLaunchKernelGGL((amax_kernel<T, true, true>), grid, dim3(256), 0, stream, in, n, head, nvec, partial);
+    else hipLaunchKernelGGL((amax_kernel<T, false, true>), grid, dim3(256), 0, stream, in, n, head, nvec, partial);
+    hipLaunchKernelGGL(partial_amax_to_global_scale_kernel, dim3(1), dim3(1024), 0, stream, partial, (int)wgs, out);
+    return check_launch("nvfp4_global_scale");
+  }
+  // Without room for the partial maxima the workgroups raise the result's own cell: one atomic each, because atomics on
+  // one address take about 10 ns apiece (four per workgroup of a larger grid: 99 us for 32 MB).
   uint32_t* cell = reinterpret_cast<uint32_t*>(out);
   hipLaunchKernelGGL(amax_init_kernel, dim3(1), dim3(1), 0, stream, cell);
-  if (n > 0) {
-    const uintptr_t addr = reinterpret_cast<uintptr_t>(in);
-    int64_t head = (int64_t)(((16 - (addr & 15)) & 15) / sizeof(T));  // elements up to 16-byte alignment
-    if (head > n) head = n;
-    const int64_t nvec = (n - head) / VE;
-    int dev = 0, cus = 256;
-    if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    const int64_t want = ceil_div(nvec > 0 ? nvec : 1, 256 * 4);  // at least 4 loads per thread
-    const int64_t cap = (int64_t)cus * 8;
-    hipLaunchKernelGGL(amax_kernel<T>, dim3((unsigned)(want < cap ? want : cap)), dim3(256), 0, stream, in, n, head, nvec, cell);
-  }
+  const dim3 few((unsigned)std::min(wgs, (int64_t)cu_count()));
+  if (stream_loads) hipLaunchKernelGGL((amax_kernel<T, true, false>), few, dim3(256), 0, stream, in, n, head, nvec, cell);
+  else hipLaunchKernelGGL((amax_kernel<T, false, false>), few, dim3(256), 0, stream, in, n, head, nvec, cell);
   hipLaunchKernelGGL(amax_to_global_scale_kernel, dim3(1), dim3(1), 0, stream, cell);
   return check_launch("nvfp4_global_scale");
 }
@@ -471,6 +507,40 @@ __global__ __launch_bounds__(256) void preprocess_sf_kernel(const E* __restrict_
   out[(int64_t)out_off[g] * padded + swizzle_128x4(r - in_off[g], c, padded)] = in[idx];
 }
 
+// Group sizes and scale slab starts from the groups' first rows, for any number of groups: one workgroup walks them 256
+// at a time with a prefix sum of the slabs (rows rounded up to 128).  Bound by the launch: 2 us on the device, where the
+// chain of tensor operations it stands for (a host-to-device copy that waits for the stream, 12 launches) took 72 us.
+__global__ __launch_bounds__(256) void grouped_auxiliary_kernel(const int32_t* __restrict__ offsets, int groups, int rows, int n, int k,
+                                                                int32_t* __restrict__ sf_offsets, int32_t* __restrict__ problem_sizes) {
+  __shared__ int wave_total[4];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int before = 0;  // slab rows of the groups before this round's
+  for (int base = 0; base < groups; base += 256) {
+    const int g = base + (int)threadIdx.x;
+    int m_g = 0;
+    if (g < groups) m_g = (g + 1 < groups ? offsets[g + 1] : rows) - offsets[g];
+    const int slab = ((m_g + 127) >> 7) << 7;
+    int incl = slab;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int o = __shfl_up(incl, d, 64);
+      if (lane >= d) incl += o;
+    }
+    if (lane == 63) wave_total[wave] = incl;
+    __syncthreads();
+    int lower = before;
+    for (int w = 0; w < wave; ++w) lower += wave_total[w];
+    before += wave_total[0] + wave_total[1] + wave_total[2] + wave_total[3];
+    __syncthreads();  // the totals are overwritten in the next round
+    if (g < groups) {
+      sf_offsets[g] = lower + incl - slab;
+      problem_sizes[3 * g] = m_g;
+      problem_sizes[3 * g + 1] = n;
+      problem_sizes[3 * g + 2] = k;
+    }
+  }
+}
+
 template <int KIND>
 __global__ __launch_bounds__(256) void cast_kernel(const float* __restrict__ in, int64_t n, uint8_t* __restrict__ out) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -520,11 +590,15 @@ int launch_nvfp4_silu_mul_quantize(const void* gate, const void* up, int in_dtyp
   return fail(NVF_ERR_INVALID_ARGUMENT, "silu-mul quantize takes bf16 or f16 inputs, got dtype %d", in_dtype);
 }
 
-int launch_nvfp4_global_scale(const void* in, int in_dtype, int64_t n, float* out, hipStream_t stream) {
+int64_t nvfp4_global_scale_workspace_bytes(int64_t n) { return n <= kGlobalScaleSmall ? 0 : kGlobalScaleMaxPartials * 4; }
+
+int launch_nvfp4_global_scale(const void* in, int in_dtype, int64_t n, float* out, void* workspace, int64_t workspace_bytes,
+                              hipStream_t stream) {
+  uint32_t* partial = workspace_bytes >= kGlobalScaleMaxPartials * 4 ? static_cast<uint32_t*>(workspace) : nullptr;
   switch (in_dtype) {
-    case NVF_F32: return launch_global_scale_typed(static_cast<const float*>(in), n, out, stream);
-    case NVF_BF16: return launch_global_scale_typed(static_cast<const bf16_t*>(in), n, out, stream);
-    case NVF_F16: return launch_global_scale_typed(static_cast<const f16_t*>(in), n, out, stream);
+    case NVF_F32: return launch_global_scale_typed(static_cast<const float*>(in), n, out, partial, stream);
+    case NVF_BF16: return launch_global_scale_typed(static_cast<const bf16_t*>(in), n, out, partial, stream);
+    case NVF_F16: return launch_global_scale_typed(static_cast<const f16_t*>(in), n, out, partial, stream);
   }
   return fail(NVF_ERR_INVALID_ARGUMENT, "unknown input dtype %d", in_dtype);
 }
@@ -563,6 +637,13 @@ int launch_preprocess_sf(const void* in, int elem_size, int64_t rows, int64_t co
       return fail(NVF_ERR_INVALID_ARGUMENT, "element size %d is not 1, 2 or 4", elem_size);
   }
   return check_launch("preprocess_sf_kernel");
+}
+
+int launch_grouped_auxiliary_tensors(const int32_t* offsets, int groups, int64_t rows, int64_t n, int64_t k, int32_t* sf_offsets,
+                                     int32_t* problem_sizes, hipStream_t stream) {
+  hipLaunchKernelGGL(grouped_auxiliary_kernel, dim3(1), dim3(256), 0, stream, offsets, groups, (int)rows, (int)n, (int)k, sf_offsets,
+                     problem_sizes);
+  return check_launch("grouped_auxiliary_kernel");
 }
 
 namespace {

@@ -63,7 +63,11 @@ def compute_auxiliary_tensors(hidden_states, offsets, out_features):
     """-> (blockscale_offsets int32 [G], problem_sizes [G, 3]) from the groups' start rows, as
     ``NVFP4InferenceGroupedLinear.compute_auxiliary_tensors`` derives them
     (layers_for_inference_benchmark.py:395-424): rows per group from neighbouring starts (the last group
-    ends at the last row), scale slabs of whole 128-row tiles laid end to end."""
+    ends at the last row), scale slabs of whole 128-row tiles laid end to end.  One kernel launch for contiguous
+    int32 offsets on the GPU; anything else (CPU tensors, other types, tracing) takes the tensor operations below."""
+    if (type(offsets) is torch.Tensor and offsets.is_cuda and offsets.dtype is torch.int32 and offsets.dim() == 1
+            and offsets.is_contiguous() and not torch.compiler.is_compiling()):
+        return _C.grouped_auxiliary_tensors(offsets, hidden_states.size(0), out_features, hidden_states.size(1))
     total = torch.tensor([hidden_states.size(0)], device=offsets.device, dtype=offsets.dtype)
     rows = torch.diff(torch.cat([offsets, total]))
     problem_sizes = torch.stack(

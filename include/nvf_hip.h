@@ -96,6 +96,14 @@ NVF_API int nvf_nvfp4_silu_mul_block_quantize(const void* gate, const void* up, 
  */
 NVF_API int nvf_nvfp4_global_scale(const void* in, int in_dtype, int64_t numel, float* out_scale, void* stream);
 
+/* nvf_nvfp4_global_scale with scratch memory for the workgroups' partial maxima: two launches and no atomics instead
+ * of three launches.  With fewer than nvf_nvfp4_global_scale_workspace_bytes(numel) bytes (0 for tensors that one
+ * workgroup reads) the call is nvf_nvfp4_global_scale.  workspace: 4-byte aligned, not shared with a call that may run
+ * at the same time. */
+NVF_API int64_t nvf_nvfp4_global_scale_workspace_bytes(int64_t numel);
+NVF_API int nvf_nvfp4_global_scale_ws(const void* in, int in_dtype, int64_t numel, float* out_scale, void* workspace,
+                                      int64_t workspace_bytes, void* stream);
+
 /* runtime/block_quantization_kernels.cu:321-361 bq::preprocessGroupedMatmulInputSf
  * (graph op preprocess_grouped_matmul_input_sf, python/python_direct/ops.cpp:3179-3212).
  * Pure layout: copies a linear [rows, cols] matrix of elem_size-byte elements (1, 2 or 4) into
@@ -103,6 +111,14 @@ NVF_API int nvf_nvfp4_global_scale(const void* in, int in_dtype, int64_t numel, 
 NVF_API int nvf_preprocess_grouped_matmul_input_sf(const void* in, int elem_size, int64_t rows, int64_t cols,
                                                    const int32_t* input_offsets, const int32_t* output_offsets,
                                                    int groups, void* out, void* stream);
+
+/* What the grouped ops need to know about the groups, from their first rows, in one launch
+ * (NVFP4InferenceGroupedLinear.compute_auxiliary_tensors, benchmarks/python/layers_for_inference_benchmark.py:395-424).
+ *   offsets        int32 [groups], the first row of every group; the last group ends at row `rows`
+ *   sf_offsets     int32 [groups]: first row of every group's scale slab, slabs of whole 128-row tiles laid end to end
+ *   problem_sizes  int32 [groups, 3] = (rows of the group, n, k) */
+NVF_API int nvf_grouped_auxiliary_tensors(const int32_t* offsets, int groups, int64_t rows, int64_t n, int64_t k,
+                                          int32_t* sf_offsets, int32_t* problem_sizes, void* stream);
 
 /* runtime/block_quantization_kernels.cu:142-186 bq::block_quantize_to_mxfp8
  * (graph op nv_block_quantize with dtype Float8_e4m3fn).  cols % 32 == 0.

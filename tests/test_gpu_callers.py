@@ -115,3 +115,18 @@ def test_grouped_swiglu_layer_end_to_end(dev):
     mid = torch.nn.functional.silu(gate) * up
     out = proj(mid, dq, dsf, da, hidden)
     assert out.shape == (sum(sizes), hidden) and torch.isfinite(out.float()).all()
+
+
+@pytest.mark.parametrize("groups", [1, 2, 64, 65, 256, 257, 1000])
+def test_auxiliary_tensors_in_one_launch_equal_the_tensor_operations(dev, groups):
+    """One group, whole and partial wavefronts, one more than the workgroup walks at once; empty groups among them."""
+    from fuser_amd import custom_ops
+
+    gen = torch.Generator().manual_seed(groups)
+    sizes = torch.randint(0, 300, (groups,), generator=gen) * torch.randint(0, 2, (groups,), generator=gen)
+    starts = start_offsets(sizes.tolist())
+    hidden = torch.empty(int(sizes.sum()), 64)
+    want = custom_ops.compute_auxiliary_tensors(hidden, starts, 384)
+    got = custom_ops.compute_auxiliary_tensors(hidden.to(dev), starts.to(dev), 384)
+    for g, w in zip(got, want):
+        assert g.dtype == w.dtype and g.shape == w.shape and torch.equal(g.cpu(), w)

@@ -117,3 +117,36 @@ def test_fused_producers_through_the_c_abi(dev):
     with pytest.raises(capi.NvfError):
         capi.check(capi.lib().nvf_nvfp4_silu_mul_block_quantize(gate.data_ptr(), up.data_ptr(), capi.F32, m, k, None, None, 0, None,
                                                                 q.data_ptr(), sf.data_ptr(), None))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("n,offset", [(1, 0), (7, 3), (8191, 1), (65536, 0), (65537, 5), (300001, 7), (4 * 1024 * 1024 + 4099, 3)])
+def test_global_scale_finds_the_largest_value_wherever_it_is(dev, dtype, n, offset):
+    """One workgroup, one part per workgroup and several; buffers that start off a 16-byte boundary; the largest value
+    first, last and in the middle; through the call with and without scratch memory."""
+    from fuser_amd import capi, ops
+
+    buf = torch.rand(n + offset, device=dev).to(dtype)
+    x = buf[offset:]
+    for at in {0, n // 2, n - 1}:
+        keep = x[at].clone()
+        x[at] = -3.0 - at % 7
+        want = torch.tensor(2688.0 / float(3 + at % 7), dtype=torch.float32).item()
+        assert ops.compute_nvfp4_global_scale(x).item() == want
+        scale = torch.empty((), dtype=torch.float32, device=dev)
+        code = {torch.bfloat16: capi.BF16, torch.float16: capi.F16, torch.float32: capi.F32}[dtype]
+        capi.check(capi.lib().nvf_nvfp4_global_scale(x.data_ptr(), code, n, scale.data_ptr(), None))
+        assert scale.item() == want
+        x[at] = keep
+
+
+def test_global_scale_of_a_tensor_larger_than_the_last_level_cache(dev):
+    from fuser_amd import ops
+
+    n = (256 << 20) // 2 + 4097  # bf16: read with non-temporal loads, several parts per workgroup
+    x = torch.zeros(n, dtype=torch.bfloat16, device=dev)
+    for at in (0, n // 3, n - 1):
+        x[at] = 2.0
+        assert ops.compute_nvfp4_global_scale(x).item() == 1344.0
+        x[at] = 0.0
+    assert ops.compute_nvfp4_global_scale(x).item() == 1.0
