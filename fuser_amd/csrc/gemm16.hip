@@ -17,20 +17,13 @@
 //
 // Output layout trick: the MFMA is issued with the B fragment as first operand, so that a lane's
 // accumulator registers hold 4 consecutive N-elements of one output row and are stored as 8 bytes.
+#include "gemm16_device.h"
 #include "nvf_internal.h"
 
 #include <mutex>
 
 namespace nvf {
 namespace {
-
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kMaxGroups = 1024;  // same bound as the reference's <<<1, num_experts>>> set-up kernel
 
@@ -75,22 +68,6 @@ struct Params {
   int ldc = 0;
   __host__ __device__ int out_pitch() const { return ldc ? ldc : n; }
 };
-
-__device__ __forceinline__ uint32_t pack2(float a, float b, bool out_bf16) {
-  if (out_bf16) {
-    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-    bf16x2 v = {(__bf16)a, (__bf16)b};
-    return __builtin_bit_cast(uint32_t, v);
-  }
-  f16x2 v = {(_Float16)a, (_Float16)b};
-  return __builtin_bit_cast(uint32_t, v);
-}
-
-// LDS tile: rows x 64 16-bit elements (128 bytes per row); 16-byte chunk c of row r sits at chunk
-// position c ^ ((r >> 1) & 7): two rows fill the 64 banks once, so the MFMA fragment reads (16
-// consecutive lanes = 16 consecutive rows, one chunk) are conflict-free.
-__device__ __forceinline__ int lds_pos2(int row, int chunk) { return row * 8 + (chunk ^ ((row >> 1) & 7)); }
-__device__ __forceinline__ int lds_pos(int row, int chunk) { return lds_pos2(row, chunk); }
 
 // Block-scaled epilogue (cutlass/nvfp4_scaled_mm_blockscale.cu:87-93: the product is quantized to NVFP4 again along
 // N before it leaves the kernel).  One 32x32 accumulator tile: lane (li, lg) holds row li, columns 8q + 4lg + e in
@@ -410,32 +387,26 @@ int launch_sized(const Params& p, int64_t m_hint, int cus, void* workspace, int6
     // Grouped NVFP4: groups of up to 128 rows (MoE decode, the small experts of a prefill) stream their expert's
     // weights once through the skinny kernel; the launches below then skip them.  The group sizes live on
     // the device, so every kernel is always launched; workgroups without work return at once.
-    if (!dense && p.min_rows == 0 && (p.n & 63) == 0 && (p.k & 127) != 0 && (p.k & 31) == 0 && (int64_t)p.k * 64 < (1ll << 31)) {
-      // K % 128 = 32, 64 or 96: the groups of up to 128 rows on the streaming kernel's variant with a short last chunk
-      // (the form that splits K over the wavefronts), larger groups on the tile kernels
-      int rc = launch_nvfp4_skinny_grouped<4, 2, OUT_BF16, false>(p, 1, 32, stream);
-      if (rc == NVF_OK) rc = launch_nvfp4_skinny_grouped<4, 8, OUT_BF16, false>(p, 33, 128, stream);
-      if (rc != NVF_OK) return rc;
-      Params rest = p;
-      rest.min_rows = 129;
-      return launch_sized<NVFP4, BF16_MMA, OUT_BF16>(rest, m_hint, cus, workspace, workspace_bytes, stream);
-    }
-    if (!dense && p.min_rows == 0 && (p.n & 63) == 0 && (p.k & 127) == 0 && (int64_t)p.k * 64 < (1ll << 31)) {
-      // With a shallow K a split of K over the wavefronts leaves each only a chunk or two: they then own
-      // different weight rows instead (K=2048, N=7168: 549 -> 464 us for 64 tokens x top-8; deeper K: slower),
-      // 64 each where N allows (a group's rows converted once per 4 weight tiles: 512 rows over 256 experts 409 -> 388 us).
-      int rc, tail_done = 0;
-      if (p.k < 4096 && (p.n & 511) == 0) rc = launch_nvfp4_skinny_grouped<4, 2, OUT_BF16, true>(p, 1, 32, stream);
-      else if (p.k < 4096 && (p.n & 255) == 0) rc = launch_nvfp4_skinny_grouped<2, 2, OUT_BF16, true>(p, 1, 32, stream);
-      else rc = launch_nvfp4_skinny_grouped<4, 2, OUT_BF16, false>(p, 1, 32, stream);
-      if (rc != NVF_OK) return rc;
+    if (!dense && p.min_rows == 0) {
+      // The groups of 1..32 rows; and in a call of at most 1024 rows whose 128x128 tiles would leave compute units idle,
+      // each walking all of K on one of them, those of 129 rows and more as well, in slabs of 32 (1024 rows over 8
+      // experts, K = 7168, N = 2048: 118 -> 56 us; 512 rows with Zipf loads: 123 -> 38 us).
+      const bool with_large = m_hint <= 1024 && !is_prefill && tiles(128, 128) <= cus;
+      Gemm16Args small{};
+      small.a = p.a, small.b = p.b, small.sfa = p.sfa, small.sfb = p.sfb, small.alpha = p.alpha, small.out = p.out;
+      small.problem_sizes = p.problem_sizes, small.expert_offsets = p.expert_offsets, small.sf_offsets = p.sf_offsets;
+      small.groups = p.groups, small.m = p.m, small.n = p.n, small.k = p.k, small.dtype = OUT_BF16 ? NVF_BF16 : NVF_F16;
+      int rc = launch_nvfp4_decode(small, with_large, stream), tail_done = 0;
+      if (rc != NVF_OK || m_hint <= 32) return rc;
       // Below the prefill size the groups of 33..128 rows are few: they stream their weights like the smaller ones,
       // found by rank among the groups of their size (a launch with few workgroups when there are few rows in all).  A
       // 128x256 tile of the persistent kernel walks all of K on one compute unit: with 64 or 256 experts, 512..5600
       // rows and K = 4096..14336 the call is 5-40 % slower that way wherever such groups exist and 0-3 % faster where
       // none does; with K < 4096 the tiles win from about 2048 rows on.
-      if (m_hint <= 1024 || (p.k >= 4096 && !is_prefill)) {
+      if ((p.k & 127) != 0 || m_hint <= 1024 || (p.k >= 4096 && !is_prefill)) {
+        // (also where K % 128 = 64: the form with a short last chunk)
         rc = launch_nvfp4_skinny_grouped<4, 8, OUT_BF16, false>(p, 33, 128, stream);
+        if (with_large || m_hint <= 128) return rc;
       } else if ((p.k < 4096 || !is_prefill) && (p.n & 255) == 0 && p.k >= 256) {
         // shallow K: one 128x256 tile of the persistent kernel per weight panel converts a group's rows once per 256
         // weight rows; the streaming kernel whose wavefronts own rows converts them once per wavefront.

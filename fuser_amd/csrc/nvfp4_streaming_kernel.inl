@@ -21,29 +21,6 @@
 //   LDS per slot: NT payload tiles of 16 rows x 64 B, piece p of row r at piece position p ^ ((r >> 2) & 3)
 //   (conflict-free reads), then per operand one 1 KiB scale block per pair of tiles: [tile][col tile][row][16 B].
 // -------------------------------------------------------------------------------------------------
-// LDS-direct load.  lds_byte_addr and base are wave-uniform; lane L's 16 bytes land at lds_byte_addr + 16 * L.
-// Issued from inline assembly: the compiler neither waits for it nor orders LDS reads against it, the
-// kernels do that with explicit s_waitcnt vmcnt(n).
-__device__ __forceinline__ void lds_dma16(uint32_t lds_byte_addr, const uint8_t* base, uint32_t voff) {
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_byte_addr), "v"(voff), "s"(base) : "memory", "m0");
-}
-
-// 32 packed e2m1 values and their two e4m3 block scales -> four MFMA operands of 8 fp16 values
-__device__ __forceinline__ void dequant_frags(const u32x4 q, uint32_t s2, u32x4 out[4]) {
-  const float f0 = __builtin_amdgcn_cvt_f32_fp8((int)s2, 0), f1 = __builtin_amdgcn_cvt_f32_fp8((int)s2, 1);
-  const f16x2 sv[2] = {__builtin_bit_cast(f16x2, __builtin_amdgcn_cvt_pkrtz(f0, f0)),
-                       __builtin_bit_cast(f16x2, __builtin_amdgcn_cvt_pkrtz(f1, f1))};
-#pragma unroll
-  for (int w = 0; w < 4; ++w) {  // dword w = elements 8w..8w+7, scale block w/2
-    const f16x2 h0 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(q[w], 1.0f, 0) * sv[w >> 1];
-    const f16x2 h1 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(q[w], 1.0f, 1) * sv[w >> 1];
-    const f16x2 h2 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(q[w], 1.0f, 2) * sv[w >> 1];
-    const f16x2 h3 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(q[w], 1.0f, 3) * sv[w >> 1];
-    out[w] = u32x4{__builtin_bit_cast(uint32_t, h0), __builtin_bit_cast(uint32_t, h1), __builtin_bit_cast(uint32_t, h2),
-                   __builtin_bit_cast(uint32_t, h3)};
-  }
-}
-
 // GROUPED: one workgroup per (group, block of 16*RT weight rows); it serves groups of rows_lo .. rows_hi rows
 // (at most 16*TT) and returns at once for the others, which other launches take.
 // NSPLIT (grouped only, where the groups supply enough workgroups): the 8 wavefronts own 8 different blocks of
@@ -370,20 +347,6 @@ __global__ __launch_bounds__(W * 64, 2) void nvfp4_skinny_ring_kernel(const Para
       aq = *reinterpret_cast<const u32x4*>(sp + (RT + tt) * 1024 + rd_payload);
       as = *reinterpret_cast<const uint32_t*>(sp + rd_asc[tt] + place * 1024u) >> sc_shift;
       if (is_tail((int)c)) as &= tail_keep();
-    };
-    // e4m3 scales of a lane's two blocks -> fp16 pairs; one dword (8 values of one block) -> one MFMA operand
-    auto scale_pairs = [&](uint32_t s2, f16x2 sv[2]) {
-      const float f0 = __builtin_amdgcn_cvt_f32_fp8((int)s2, 0), f1 = __builtin_amdgcn_cvt_f32_fp8((int)s2, 1);
-      sv[0] = __builtin_bit_cast(f16x2, __builtin_amdgcn_cvt_pkrtz(f0, f0));
-      sv[1] = __builtin_bit_cast(f16x2, __builtin_amdgcn_cvt_pkrtz(f1, f1));
-    };
-    auto dequant_dword = [&](uint32_t qw, f16x2 sv) {
-      const f16x2 h0 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(qw, 1.0f, 0) * sv;
-      const f16x2 h1 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(qw, 1.0f, 1) * sv;
-      const f16x2 h2 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(qw, 1.0f, 2) * sv;
-      const f16x2 h3 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(qw, 1.0f, 3) * sv;
-      return u32x4{__builtin_bit_cast(uint32_t, h0), __builtin_bit_cast(uint32_t, h1), __builtin_bit_cast(uint32_t, h2),
-                   __builtin_bit_cast(uint32_t, h3)};
     };
     // One chunk with TTC activation tiles.  The whole slot is read out into registers at once and refilled with
     // the wavefront's next chunk, which then has a whole chunk's time to land.  The chunk is four 32-deep MFMA
@@ -766,9 +729,7 @@ int launch_nvfp4_skinny_ring_cfg(const Params& p, hipStream_t stream, int slabs 
 template <int RT, int TT, bool OUT_BF16, bool NSPLIT, int W = 8>
 int launch_nvfp4_skinny_grouped(const Params& p0, int rows_lo, int rows_hi, hipStream_t stream) {
   constexpr int SLOT_KIB = RT + TT + (RT + 1) / 2 + (TT + 1) / 2;
-  // One slot per wavefront also where two would fit: measured faster for the groups of up to 32 rows (512 rows
-  // over 256 experts, K=7168: 401 -> 375 us; K=2048: 432 -> 413 us).  Forcing the registers down to two
-  // workgroups per compute unit on top of that costs more than it gains (450 us).
+  // one slot per wavefront, as in the dense launch
   constexpr int DEPTH = 1;
   auto kern = W == 8 && (p0.k & 127) != 0 ? nvfp4_skinny_ring_kernel<RT, TT, OUT_BF16, DEPTH, true, NSPLIT, W == 8, W>
                                           : nvfp4_skinny_ring_kernel<RT, TT, OUT_BF16, DEPTH, true, NSPLIT, false, W>;

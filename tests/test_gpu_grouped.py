@@ -563,3 +563,48 @@ def test_grouped_ops_reject_bad_inputs_on_device(dev):
         nvf_cutlass.grouped_mm(a, b[0], i64, i64, ps, eo)
     out = nvf_cutlass.grouped_mm(a, b, i64, i64, ps, eo)  # all groups empty: nothing computed, still returns [8, 16]
     assert out.shape == (8, 16)
+
+
+@pytest.mark.parametrize("groups,n,k", [
+    (9, 128, 64), (9, 128, 192), (9, 256, 256), (9, 128, 320), (9, 384, 2112), (9, 128, 7168),  # whole and short last steps; fewer steps than wavefronts
+    (128, 1024, 320), (1024, 128, 128),  # items of 128 weight rows; as many groups as a call may have
+    (64, 2048, 4096),                    # weights beyond the last-level cache: read with non-temporal loads
+])
+def test_nvfp4_grouped_mm_decode_kernel(dev, groups, n, k):
+    """Groups of 1..32 rows on both sides of a row tile's border and, in slabs, of 129 rows and more; empty groups; a
+    different alpha per group; poisoned padding of the activation scale slabs.  Every element compared, rows after the last
+    group untouched, run-to-run bit equality."""
+    from fuser_amd import capi, nvf_cutlass
+
+    sizes = [0] * groups
+    for i, t in enumerate([1, 16, 17, 32, 0, 129, 2, 31, 15]):
+        sizes[i * (groups // 9)] = t
+    sizes[groups - 1] = sizes[groups - 1] or 3
+    m = sum(sizes) + 3
+    plan = capi.describe_dispatch("nvfp4_scaled_grouped_mm", m, n, k, groups=groups)
+    assert f"stream={int(k == 4096)},halves={2 if min(groups, m) * (n // 128) >= 1024 else 1}> " in plan and "rows=1..32,129.." in plan, plan
+    gen = torch.Generator().manual_seed(groups + n + k)
+    x = torch.randn(m, k, generator=gen).bfloat16()
+    w = (torch.randn(8, n, k, generator=gen) * 0.05).bfloat16()  # eight different experts, repeated
+    ps, eo, st, ct = _grouped_args(sizes, n, k, dev)
+    so = start_offsets([O.round_up(t, 128) for t in sizes])
+    aq, valid = O.grouped_block_quantize_nvfp4(x, eo, so, None)
+    lin = torch.zeros_like(valid, dtype=torch.bool)
+    for e, t in enumerate(sizes):
+        if t:
+            ones = O.linear_to_swizzled_128_4(torch.ones(t, k // 16, dtype=torch.uint8))
+            lin[int(so[e]) : int(so[e]) + ones.shape[0]] |= ones.bool()
+    asf = torch.where(lin, valid, torch.full_like(valid, 0x7F))  # NaN code wherever no row owns the byte
+    quantized = [O.block_quantize_nvfp4(w[e], gs_of(w[e]), True) for e in range(8)]
+    bq = torch.stack([quantized[e % 8][0] for e in range(groups)])
+    bsf = torch.stack([quantized[e % 8][1] for e in range(groups)])
+    alphas = torch.tensor([(e % 11 + 1) / gs_of(w[e % 8]) for e in range(groups)])
+    ref = O.ref_nvfp4_scaled_grouped_mm(aq, bq, valid, bsf, alphas, ps, eo, so)
+    rows = sum(sizes)
+    args = (fp4(aq.to(dev)), fp4(bq.to(dev)), e4m3(asf.to(dev)), e4m3(bsf.to(dev)), alphas.to(dev), st, ct, ps.to(dev), eo.to(dev), so.to(dev))
+    for dtype in (torch.bfloat16, torch.float16):
+        out = nvf_cutlass.nvfp4_scaled_grouped_mm(*args, dtype)
+        torch.cuda.synchronize()
+        scale = ref[:rows].abs().amax(dim=1, keepdim=True).clamp(min=1e-30)
+        assert ((out[:rows].float().cpu() - ref[:rows]).abs() / scale).max().item() <= GEMM_MAX_REL, dtype
+        assert torch.equal(out[:rows], nvf_cutlass.nvfp4_scaled_grouped_mm(*args, dtype)[:rows])
