@@ -236,9 +236,11 @@ __device__ __forceinline__ void lds_dma16(uint32_t lds_byte_addr, const uint8_t*
 // whose 256x256 tiles would leave compute units idle).  The statement order for TM = 4 is the one the 8192^3
 // measurements were made with.
 // RAGGED_K: K is a multiple of 32 but not of 128.  The last K step of a tile then holds K % 128 elements per row: the
-// lanes whose 16 bytes lie past the end of the row write zeros to their LDS unit instead of loading (the bytes there
-// belong to the next row), and the scale bytes of the blocks past K - padding columns of the scale layout, whose content
-// is not defined - are replaced by 2^0, so that the step adds exact zeros.
+// lanes whose 16 bytes lie past the end of the row load the row's last ones again, and the scale bytes of the blocks past K
+// are replaced by 2^-127 in both operands: what such a lane multiplies is the row's own data (a NaN among them has made the
+// row's results NaN already) times 2^-254, below the smallest fp32 number, so that the step adds exact zeros.  No branch in
+// the K loop: with the lanes' loads predicated and zeros written instead, every load of every step was a block of code of
+// its own (1024 x 5632 x 2880: 31.2 us, against 24.3 for K = 2816; now 29.6 us).
 template <int TM, bool OUT_BF16, bool STREAM_OUT, bool RAGGED_K = false, bool RAGGED_M = false>
 __global__ __launch_bounds__(256, 1) void mxfp8_gemm_256_kernel(const Params p) {
   constexpr int BM = 64 * TM, BN = 256;
@@ -304,9 +306,10 @@ __global__ __launch_bounds__(256, 1) void mxfp8_gemm_256_kernel(const Params p) 
   const uint32_t voff_odd = row_off + (uint32_t)(((lane & 7) ^ ((lane >> 4) | 4)) << 4);
   const uint32_t lds_base = (uint32_t)(uintptr_t)((__attribute__((address_space(3))) void*)lds);
   const uint32_t step8 = 8u * (uint32_t)p.k;  // 8 rows
-  // RAGGED_K: does this lane's chunk of an even / odd load unit exist in the last step?
-  const bool tail_even = (((lane & 7) ^ (lane >> 4)) << 4) < k_tail;
-  const bool tail_odd = (((lane & 7) ^ ((lane >> 4) | 4)) << 4) < k_tail;
+  // RAGGED_K: the row's chunk for a load unit of a step is the lane's or, if that is past the end, the last there is
+  const uint32_t chunk_even = (uint32_t)((lane & 7) ^ (lane >> 4));
+  const uint32_t tail_last = (uint32_t)(k_tail >> 4) - 1u;
+  uint32_t step_even = voff_even, step_odd = voff_odd;  // the lane offsets of the step being issued
 
   // ---- load stream state: the (tile, K step) the next loads are issued for
   // ---- load stream: the loads of step g+2 are issued while step g is computed, so the stream runs
@@ -344,15 +347,15 @@ __global__ __launch_bounds__(256, 1) void mxfp8_gemm_256_kernel(const Params p) 
     const int j = q < 4 * TM ? (q >> 1) : q - 2 * TM;
     const uint32_t l = lds_base + (uint32_t)(buf * BUF_UNITS + (op ? A_UNITS + wave * 512 : wave * (BM * 2))) * 16u + j * 1024u;
     const uint8_t* gp = (op ? lp.b : lp.a) + ((int64_t)l_ks << 7);
-    uint32_t voff = ((j & 1) ? voff_odd : voff_even) + (uint32_t)j * step8;
+    if (RAGGED_K && q == 0) {
+      const uint32_t last = l_ks == nk - 1 ? tail_last : 7u;
+      step_even = row_off + (min(chunk_even, last) << 4);
+      step_odd = row_off + (min(chunk_even ^ 4u, last) << 4);
+    }
+    uint32_t voff = ((j & 1) ? step_odd : step_even) + (uint32_t)j * step8;
     if (RAGGED_M && op == 0) {
       const uint32_t row = min((uint32_t)(wave * (BM / 4) + j * 8) + (uint32_t)(lane >> 3), (uint32_t)(lp.valid - 1));
-      voff = row * (uint32_t)p.k + (((j & 1) ? voff_odd : voff_even) - row_off);
-    }
-    if (RAGGED_K && l_ks == nk - 1) {
-      if ((j & 1) ? tail_odd : tail_even) lds_dma16(l, gp, voff);
-      else *reinterpret_cast<u32x4*>(reinterpret_cast<char*>(lds) + (l - lds_base) + lane * 16) = u32x4{0, 0, 0, 0};
-      return;
+      voff = row * (uint32_t)p.k + (((j & 1) ? step_odd : step_even) - row_off);
     }
     lds_dma16(l, gp, voff);
   };
@@ -428,11 +431,11 @@ __global__ __launch_bounds__(256, 1) void mxfp8_gemm_256_kernel(const Params p) 
   // (tail: the scales are those of a tile's last step, RAGGED_K only)
   auto take_scales = [&](bool tail = false) {
     if (RAGGED_K && tail) {
-      const uint32_t keep = (1u << (k_tail >> 2)) - 1u, fill = 0x7f7f7f7fu & ~keep;  // k_tail / 32 bytes stay
+      const uint32_t keep = (1u << (k_tail >> 2)) - 1u;  // k_tail / 32 bytes stay, the others become 2^-127
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
-        na[c] = (na[c] & keep) | fill;
-        nb[c] = (nb[c] & keep) | fill;
+        na[c] &= keep;
+        nb[c] &= keep;
       }
     }
 #pragma unroll
