@@ -20,6 +20,7 @@
 #include "gemm16_device.h"
 #include "nvf_internal.h"
 
+#include <algorithm>
 #include <mutex>
 
 namespace nvf {
@@ -119,6 +120,7 @@ __global__ __launch_bounds__(256) void zero_fill_kernel(uint32_t* __restrict__ d
 #include "nvfp4_streaming_kernel.inl"
 #include "nvfp4_group_panel_kernel.inl"
 #include "grouped16_kernel.inl"
+#include "grouped16_streaming_kernel.inl"
 
 // -------------------------------------------------------------------------------------------------
 // Launchers of the tile kernels and the dispatch
@@ -382,6 +384,19 @@ int launch_sized(const Params& p, int64_t m_hint, int cus, void* workspace, int6
     if (!dense && m_hint >= 128 * (int64_t)p.groups && tiles(256, 256) >= cus / 2 && (p.n & 255) == 0 && (p.k & 63) == 0 &&
         p.k >= 128 && (int64_t)p.k * 2 * 256 < (1ll << 31))
       return launch_grouped16_fast<BF16_MMA, OUT_BF16>(p, cus, stream);
+    // A decode step: few rows per group on average.  The streaming kernel's partial sums cost more per item the shallower K
+    // and the more rows there are; the 128x128 tiles lose most where they leave compute units idle.  Tile kernel against
+    // streaming kernel, even and Zipf loads, us: 8 experts of 1024 x 1024, 48 rows each 18 / 10 and 20 / 13; 4096 x 4096, 48
+    // rows 84 / 66 and 88 / 77; 64 of 2048 x 7168, 24 rows 336 / 310 and 439 / 377; 32 of 2880 x 2880, 16 rows 120 / 103 and
+    // 121 / 118, 24 rows 120 / 112 and 124 / 130; 8 of 3000 x 1288, 16 rows 25 / 19 and 25 / 20, 48 rows 26 / 27; 64 of
+    // 1024 x 1024, 8 rows 26 / 30.
+    const int64_t first_tiles = p.groups * ceil_div(p.n, 128);
+    int rows_on_average = 0;
+    if (p.k >= 1024 && 4 * first_tiles <= cus) rows_on_average = 48;
+    else if (p.k >= 4096) rows_on_average = first_tiles <= cus ? 48 : 24;
+    else if (p.k >= 2048 || (p.k >= 1024 && 4 * first_tiles <= 3 * (int64_t)cus)) rows_on_average = 16;
+    if (!dense && m_hint <= rows_on_average * (int64_t)p.groups && (m_hint / kStream16Rows + p.groups) * ceil_div(p.n, 32) < (1ll << 31))
+      return launch_grouped16_streaming<BF16_MMA>(p, cus, stream);
   }
   if constexpr (NVFP4) {
     // Grouped NVFP4: groups of up to 128 rows (MoE decode, the small experts of a prefill) stream their expert's

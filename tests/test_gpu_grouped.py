@@ -572,8 +572,8 @@ def test_grouped_ops_reject_bad_inputs_on_device(dev):
 ])
 def test_nvfp4_grouped_mm_decode_kernel(dev, groups, n, k):
     """Groups of 1..32 rows on both sides of a row tile's border and, in slabs, of 129 rows and more; empty groups; a
-    different alpha per group; poisoned padding of the activation scale slabs.  Every element compared, rows after the last
-    group untouched, run-to-run bit equality."""
+    different alpha per group; poisoned padding of the activation scale slabs.  Every element compared, run-to-run bit
+    equality."""
     from fuser_amd import capi, nvf_cutlass
 
     sizes = [0] * groups
@@ -608,3 +608,51 @@ def test_nvfp4_grouped_mm_decode_kernel(dev, groups, n, k):
         scale = ref[:rows].abs().amax(dim=1, keepdim=True).clamp(min=1e-30)
         assert ((out[:rows].float().cpu() - ref[:rows]).abs() / scale).max().item() <= GEMM_MAX_REL, dtype
         assert torch.equal(out[:rows], nvf_cutlass.nvfp4_scaled_grouped_mm(*args, dtype)[:rows])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("groups,n,k", [
+    (16, 8, 1024), (16, 40, 1032), (16, 96, 2040), (16, 1368, 1096),  # short last weight blocks and K steps; 1..3 steps per wavefront
+    (16, 2880, 2880), (1024, 192, 2048),                              # 64 weight rows an item; as many groups as a call may have
+    (64, 1024, 2112),                                                 # weights beyond the last-level cache
+])
+def test_grouped_mm_streaming_kernel(dev, groups, n, k, dtype):
+    """Groups on both sides of a row tile's and a slab's border, empty ones between them; every element compared, rows
+    outside the groups untouched, run-to-run bit equality, non-finite values stay within their row and weight row."""
+    from fuser_amd import capi, nvf_cutlass
+
+    sizes = [0] * groups
+    for i, t in enumerate([1, 16, 0, 17, 64, 2, 65, 33]):
+        sizes[i * (groups // 8)] = t
+    sizes[groups - 1] = 49
+    m, rows = sum(sizes) + 5, sum(sizes)
+    code = capi.BF16 if dtype == torch.bfloat16 else capi.F16
+    plan = capi.describe_dispatch("grouped_mm", m, n, k, groups=groups, dtype=code)
+    want = f"streaming_gemm16_kernel<weight_rows={64 if min(groups, m) * -(-n // 64) >= 512 else 32},stream={int(groups >= 64)}>"
+    assert plan.startswith(want), plan
+    gen = torch.Generator().manual_seed(groups + n + k)
+    x = torch.randn(m, k, generator=gen).to(dtype)
+    w = (torch.randn(8, n, k, generator=gen) * 0.05).to(dtype)  # eight different experts, repeated
+    x[3, k - 1] = float("inf")  # group of 16 rows: row 2
+    w[0, n - 1, k - 1] = float("nan")
+    ps, eo, st, ct = _grouped_args(sizes, n, k, dev)
+    ref = torch.zeros(rows, n)
+    at = 0
+    for e, t in enumerate(sizes):
+        ref[at : at + t] = x[at : at + t].float() @ w[e % 8].float().t()
+        at += t
+    xd, wd = x.to(dev), w.to(dev).repeat(groups // 8, 1, 1)
+    out = nvf_cutlass.grouped_mm(xd, wd, st, ct, ps.to(dev), eo.to(dev))
+    got = out[:rows].float().cpu()
+    finite = ref.isfinite()
+    assert torch.equal(got.isfinite(), finite) and torch.equal(got.isnan(), ref.isnan())
+    got, ref = torch.where(finite, got, 0.0), torch.where(finite, ref, 0.0)
+    scale = ref.abs().amax(dim=1, keepdim=True).clamp(min=1e-30)
+    assert ((got - ref).abs() / scale).max().item() <= GEMM_MAX_REL
+    raw = torch.full((m, n), 7.0, dtype=dtype, device=dev)
+    psd, eod = ps.to(dev), eo.to(dev)
+    capi.check(capi.lib().nvf_grouped_mm(xd.data_ptr(), wd.data_ptr(), raw.data_ptr(), psd.data_ptr(), eod.data_ptr(), groups, m, n, k, code,
+                                         torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    assert bool((raw[rows:] == 7.0).all())
+    assert torch.equal(raw[:rows].view(torch.int16), out[:rows].view(torch.int16))
