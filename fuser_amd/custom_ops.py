@@ -59,14 +59,21 @@ def _(activation, fp4_weight, weight_scaling_factor, weight_global_scale, offset
     return torch.empty(activation.shape[:-1] + (fp4_weight.size(2),), device=activation.device, dtype=torch.bfloat16)
 
 
+def _is_plain(tensor):
+    """Whether a call that torch does not see may take the tensor's memory: no subclass, no vmap or other functional
+    transform's wrapper, nothing that records or replaces the operations (torch.compile, jit.trace, a dispatch mode)."""
+    return (type(tensor) is torch.Tensor and not torch.compiler.is_compiling() and not torch.jit.is_tracing()
+            and not torch._C._len_torch_dispatch_stack() and not torch._C._functorch.is_functorch_wrapped_tensor(tensor))
+
+
 def compute_auxiliary_tensors(hidden_states, offsets, out_features):
     """-> (blockscale_offsets int32 [G], problem_sizes [G, 3]) from the groups' start rows, as
     ``NVFP4InferenceGroupedLinear.compute_auxiliary_tensors`` derives them
     (layers_for_inference_benchmark.py:395-424): rows per group from neighbouring starts (the last group
     ends at the last row), scale slabs of whole 128-row tiles laid end to end.  One kernel launch for contiguous
-    int32 offsets on the GPU; anything else (CPU tensors, other types, tracing) takes the tensor operations below."""
-    if (type(offsets) is torch.Tensor and offsets.is_cuda and offsets.dtype is torch.int32 and offsets.dim() == 1
-            and offsets.is_contiguous() and not torch.compiler.is_compiling()):
+    int32 offsets on the GPU; anything else (CPU tensors, other types, tracing, vmap) takes the tensor operations below."""
+    if (_is_plain(offsets) and offsets.is_cuda and offsets.dtype is torch.int32 and offsets.dim() == 1
+            and offsets.is_contiguous()):
         return _C.grouped_auxiliary_tensors(offsets, hidden_states.size(0), out_features, hidden_states.size(1))
     total = torch.tensor([hidden_states.size(0)], device=offsets.device, dtype=offsets.dtype)
     rows = torch.diff(torch.cat([offsets, total]))

@@ -130,3 +130,23 @@ def test_auxiliary_tensors_in_one_launch_equal_the_tensor_operations(dev, groups
     got = custom_ops.compute_auxiliary_tensors(hidden.to(dev), starts.to(dev), 384)
     for g, w in zip(got, want):
         assert g.dtype == w.dtype and g.shape == w.shape and torch.equal(g.cpu(), w)
+
+
+def test_auxiliary_tensors_under_vmap_and_tracing(dev):
+    """Where torch records or batches the operations, the launch that it does not see is not taken."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+
+    from fuser_amd import custom_ops
+
+    hidden = torch.empty(500, 64, device=dev)
+    starts = torch.tensor([[0, 129, 129, 300], [0, 1, 400, 500]], dtype=torch.int32, device=dev)
+
+    def call(s):
+        return custom_ops.compute_auxiliary_tensors(hidden, s, 384)
+
+    rows = [call(s) for s in starts]
+    for got, *want in zip(torch.vmap(call)(starts), *rows):
+        assert torch.equal(got, torch.stack(want))
+    for traced in (make_fx(call)(starts[0]), torch.jit.trace(call, (starts[0],))):
+        for got, want in zip(traced(starts[1]), rows[1]):
+            assert torch.equal(got, want)
