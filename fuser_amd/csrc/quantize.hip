@@ -10,6 +10,7 @@
 
 #include <algorithm>
 #include <cfloat>
+#include <type_traits>
 
 namespace nvf {
 namespace {
@@ -312,21 +313,29 @@ __device__ __forceinline__ uint32_t workgroup_max(uint32_t m) {
   return m;
 }
 
+// A tensor larger than the last-level cache is read from its end to its start, and the first 96 MB, read last, are left in
+// the cache for the quantizer that starts there: scale and NVFP4 quantization of bf16 40000 x 4096 125.8 -> 122.8 us, f32
+// 30001 x 5120 209.8 -> 206.8, bf16 65536 x 7168 340.3 -> 339.0, the scale alone 133.5 -> 131.8.  208 MB would give the
+// pair 118.1, 204.8 and 337.9 us, but make the scale alone slower (136.5 us).
+constexpr int64_t kGlobalScaleKept = (int64_t)96 << 20;
+
 // The thread's maximum over the elements its workgroup (`wg` of `wgs`) owns.  A workgroup reads runs of LOADS * THREADS
 // consecutive 16-byte vectors, so that the chip reads the tensor nearly in order: 940 MB in 133 us (7.1 TB/s), against
 // 168 us where every load of a thread is a whole grid apart.
+// STREAM: from the tensor's end to its start, past the last-level cache down to the first kGlobalScaleKept bytes.
 template <typename T, int THREADS, int LOADS, bool STREAM>
 __device__ __forceinline__ uint32_t amax_of_part(const T* __restrict__ in, int64_t n, int64_t head, int64_t nvec, int64_t wg, int64_t wgs) {
   constexpr int VE = 16 / (int)sizeof(T);  // elements per 16-byte load
+  constexpr int64_t kRun = LOADS * THREADS;
   uint32_t m = 0;
   const u32x4* vec = reinterpret_cast<const u32x4*>(in + head);
-  for (int64_t base = wg * (LOADS * THREADS); base < nvec; base += wgs * (LOADS * THREADS)) {
+  auto fold_run = [&](int64_t base, auto past_cache) {
     u32x4 q[LOADS];
 #pragma unroll
     for (int u = 0; u < LOADS; ++u) {
       const int64_t i = base + u * THREADS + threadIdx.x;
       q[u] = u32x4{0, 0, 0, 0};
-      if (i < nvec) q[u] = STREAM ? __builtin_nontemporal_load(vec + i) : vec[i];
+      if (i < nvec) q[u] = decltype(past_cache)::value ? __builtin_nontemporal_load(vec + i) : vec[i];
     }
 #pragma unroll
     for (int u = 0; u < LOADS; ++u) {
@@ -335,6 +344,13 @@ __device__ __forceinline__ uint32_t amax_of_part(const T* __restrict__ in, int64
 #pragma unroll
       for (int j = 0; j < VE; ++j) m = max(m, abs_bits(e[j]));
     }
+  };
+  if constexpr (STREAM) {
+    int64_t base = ((nvec + kRun - 1) / kRun - 1 - wg) * kRun;
+    for (; base >= kGlobalScaleKept / 16; base -= wgs * kRun) fold_run(base, std::true_type{});
+    for (; base >= 0; base -= wgs * kRun) fold_run(base, std::false_type{});
+  } else {
+    for (int64_t base = wg * kRun; base < nvec; base += wgs * kRun) fold_run(base, std::false_type{});
   }
   // elements before the first and after the last whole 16-byte vector: fewer than 2 * VE
   const int64_t tail0 = head + nvec * VE, t = threadIdx.x;

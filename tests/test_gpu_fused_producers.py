@@ -150,3 +150,24 @@ def test_global_scale_of_a_tensor_larger_than_the_last_level_cache(dev):
         assert ops.compute_nvfp4_global_scale(x).item() == 1344.0
         x[at] = 0.0
     assert ops.compute_nvfp4_global_scale(x).item() == 1.0
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("offset", [0, 3])
+def test_global_scale_around_the_part_that_stays_in_the_last_level_cache(dev, dtype, offset):
+    """Both sides of the border at 96 MB and of the runs next to it, the first and last runs, a short last run; with and
+    without scratch memory."""
+    from fuser_amd import capi, ops
+
+    size = torch.empty((), dtype=dtype).element_size()
+    n, kept, run = (256 << 20) // size + 16384 // size * 3 + 5, (96 << 20) // size, 16384 // size
+    x = torch.zeros(n + offset, dtype=dtype, device=dev)[offset:]
+    scale = torch.empty((), dtype=torch.float32, device=dev)
+    code = capi.BF16 if dtype == torch.bfloat16 else capi.F32
+    last = (n - 1) // run * run
+    for at in (0, run - 1, run, kept - run, kept - 1, kept, kept + run - 1, kept + run, 300 * run + 7, last - 1, last, n - 1):
+        x[at] = -2.0
+        assert ops.compute_nvfp4_global_scale(x).item() == 1344.0, at
+        capi.check(capi.lib().nvf_nvfp4_global_scale(x.data_ptr(), code, n, scale.data_ptr(), None))
+        assert scale.item() == 1344.0, at
+        x[at] = 0.0
