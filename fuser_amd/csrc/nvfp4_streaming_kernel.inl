@@ -27,7 +27,7 @@
 // 16*RT weight rows and each walks all of K on its own - a long pipeline per wavefront and no reduction -
 // instead of sharing one block and splitting K.
 // RAGGED_K: K % 128 != 0 (a kernel of its own: the tests for the short chunk cost the others 4-8 %).
-// W: wavefronts per workgroup, 8 or (dense, 4 x 8 tiles) 4; two wavefronts per SIMD in both cases, i.e. at most 256
+// W: wavefronts per workgroup, 8 or (4 x 8 tiles) 4; two wavefronts per SIMD in both cases, i.e. at most 256
 // registers, so that two workgroups of 4 fit a compute unit.
 template <int RT, int TT, bool OUT_BF16, int DEPTH, bool GROUPED = false, bool NSPLIT = false, bool RAGGED_K = false, int W = 8>
 __global__ __launch_bounds__(W * 64, 2) void nvfp4_skinny_ring_kernel(const Params p) {
@@ -731,8 +731,8 @@ int launch_nvfp4_skinny_grouped(const Params& p0, int rows_lo, int rows_hi, hipS
   constexpr int SLOT_KIB = RT + TT + (RT + 1) / 2 + (TT + 1) / 2;
   // one slot per wavefront, as in the dense launch
   constexpr int DEPTH = 1;
-  auto kern = W == 8 && (p0.k & 127) != 0 ? nvfp4_skinny_ring_kernel<RT, TT, OUT_BF16, DEPTH, true, NSPLIT, W == 8, W>
-                                          : nvfp4_skinny_ring_kernel<RT, TT, OUT_BF16, DEPTH, true, NSPLIT, false, W>;
+  auto kern = (p0.k & 127) != 0 ? nvfp4_skinny_ring_kernel<RT, TT, OUT_BF16, DEPTH, true, NSPLIT, true, W>
+                                : nvfp4_skinny_ring_kernel<RT, TT, OUT_BF16, DEPTH, true, NSPLIT, false, W>;
   constexpr int red_kib = NSPLIT ? 0 : W * (RT * TT <= 8 ? RT * TT : TT);
   constexpr int ring_kib = W * DEPTH * SLOT_KIB;
   constexpr int lds_bytes = (ring_kib > red_kib ? ring_kib : red_kib) * 1024;
@@ -748,9 +748,9 @@ int launch_nvfp4_skinny_grouped(const Params& p0, int rows_lo, int rows_hi, hipS
   const int64_t wgs = (int64_t)(p.class_slots ? p.class_slots : p.groups) * (p.n / (16 * RT * (NSPLIT ? 8 : 1)));
   // (groups of 33-128 rows, more workgroups than compute units: 4 wavefronts each and two to a compute unit, as in the
   // dense launch; 8 experts x 64 rows, N=14336, K=4096: 111 -> 86 us, 32 x 40 rows, N=7168: 180 -> 142, 64 x 64 rows,
-  // N=2048, K=7168: 187 -> 164)
+  // N=2048, K=7168: 187 -> 164; with a short last chunk, a pass of 32 x 62 rows, N=5760, K=2880: 163 -> 125)
   if constexpr (W == 8 && RT == 4 && TT == 8 && !NSPLIT) {
-    if ((p.k & 127) == 0 && wgs > cu_count()) return launch_nvfp4_skinny_grouped<RT, TT, OUT_BF16, NSPLIT, 4>(p0, rows_lo, rows_hi, stream);
+    if (wgs > cu_count()) return launch_nvfp4_skinny_grouped<RT, TT, OUT_BF16, NSPLIT, 4>(p0, rows_lo, rows_hi, stream);
   }
   if (wgs >= ((int64_t)1 << 31)) return fail(NVF_ERR_UNSUPPORTED_SHAPE, "too many (group, row block) pairs for one launch");
   if (note_launch("nvfp4_skinny_ring_kernel<RT=%d,TT=%d,grouped,nsplit=%d%s> grid=%lld rows=%d..%d", RT, TT, (int)NSPLIT, W == 4 ? ",W=4" : "", (long long)wgs,

@@ -656,3 +656,32 @@ def test_grouped_mm_streaming_kernel(dev, groups, n, k, dtype):
     torch.cuda.synchronize()
     assert bool((raw[rows:] == 7.0).all())
     assert torch.equal(raw[:rows].view(torch.int16), out[:rows].view(torch.int16))
+
+
+@pytest.mark.parametrize("n,k", [(2048, 64), (2048, 192), (2048, 576), (2048, 1088)])
+def test_nvfp4_grouped_mm_four_wavefronts_with_a_short_last_chunk(dev, n, k):
+    """Groups of 33..128 rows, more workgroups than compute units, K % 128 = 64: fewer chunks than wavefronts, as many and
+    more, the short one in the first and in other wavefronts.  Every element compared, run-to-run bit equality."""
+    from fuser_amd import capi, nvf_cutlass
+
+    sizes = [33, 48, 0, 49, 64, 65, 5, 80, 81, 96, 112, 128, 127, 40, 113]
+    m, groups = sum(sizes), len(sizes)
+    plan = capi.describe_dispatch("nvfp4_scaled_grouped_mm", m, n, k, groups=groups)
+    assert f"nvfp4_skinny_ring_kernel<RT=4,TT=8,grouped,nsplit=0,W=4> grid={groups * n // 64} rows=33..128" in plan, plan
+    gen = torch.Generator().manual_seed(k)
+    x = torch.randn(m, k, generator=gen).bfloat16()
+    ps, eo, st, ct = _grouped_args(sizes, n, k, dev)
+    so = start_offsets([O.round_up(t, 128) for t in sizes])
+    aq, asf = O.grouped_block_quantize_nvfp4(x, eo, so, None)
+    w = [(torch.randn(n, k, generator=gen) * 0.05).bfloat16() for _ in range(groups)]
+    quantized = [O.block_quantize_nvfp4(e, gs_of(e), True) for e in w]
+    bq, bsf = (torch.stack([q[i] for q in quantized]) for i in (0, 1))
+    alphas = torch.tensor([(e + 1) / gs_of(w[e]) for e in range(groups)])
+    ref = O.ref_nvfp4_scaled_grouped_mm(aq, bq, asf, bsf, alphas, ps, eo, so)
+    args = (fp4(aq.to(dev)), fp4(bq.to(dev)), e4m3(asf.to(dev)), e4m3(bsf.to(dev)), alphas.to(dev), st, ct, ps.to(dev), eo.to(dev), so.to(dev))
+    for dtype in (torch.bfloat16, torch.float16):
+        out = nvf_cutlass.nvfp4_scaled_grouped_mm(*args, dtype)
+        torch.cuda.synchronize()
+        scale = ref.abs().amax(dim=1, keepdim=True).clamp(min=1e-30)
+        assert ((out.float().cpu() - ref).abs() / scale).max().item() <= GEMM_MAX_REL, dtype
+        assert torch.equal(out, nvf_cutlass.nvfp4_scaled_grouped_mm(*args, dtype))
