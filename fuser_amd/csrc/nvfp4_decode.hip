@@ -282,13 +282,14 @@ __global__ __launch_bounds__(kWaves * 64, 2) void persistent_nvfp4_skinny_ring_k
         }
       }
       // ---- the wavefronts' partial tiles, one row tile at a time, summed by alternate halves of the workgroup
-      const int parts = min(steps, KS);
+      // (those of the first wavefronts also where K = 0 leaves no steps: the result is then zero)
+      const int parts = max(min(steps, KS), 1);
 #pragma unroll
       for (int tt = 0; tt < TILES; ++tt) {
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();  // the previous tile has been summed
         asm volatile("" ::: "memory");
-        if (has_steps) {
+        if (kpart < parts) {
 #pragma unroll
           for (int rt = 0; rt < 4; ++rt) sums[(wave * 4 + rt) * 64 + lane] = acc[rt][tt];
         }

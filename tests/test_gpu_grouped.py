@@ -685,3 +685,28 @@ def test_nvfp4_grouped_mm_four_wavefronts_with_a_short_last_chunk(dev, n, k):
         scale = ref.abs().amax(dim=1, keepdim=True).clamp(min=1e-30)
         assert ((out.float().cpu() - ref).abs() / scale).max().item() <= GEMM_MAX_REL, dtype
         assert torch.equal(out, nvf_cutlass.nvfp4_scaled_grouped_mm(*args, dtype))
+
+
+@pytest.mark.parametrize("sizes,n", [([1, 16, 17, 0, 32, 33, 128, 129, 300], 128), ([3, 20, 31, 0], 32768)])
+def test_nvfp4_grouped_mm_with_empty_k_is_zero(dev, sizes, n):
+    """K = 0 through the C entry (the tensor layer refuses empty operands): every row of every group is an empty sum, i.e.
+    zero, whatever earlier kernels left in LDS; rows outside the groups stay untouched."""
+    from fuser_amd import capi
+
+    m, rows, groups = sum(sizes) + 4, sum(sizes), len(sizes)
+    plan = capi.describe_dispatch("nvfp4_scaled_grouped_mm", m, n, 0, groups=groups)
+    assert f"halves={1 if n == 128 else 2}> " in plan and "rows=1..32,129.." in plan, plan
+    ps, eo, _, _ = _grouped_args(sizes, n, 0, dev)
+    so = start_offsets([O.round_up(t, 128) for t in sizes])
+    psd, eod, sod = ps.to(dev), eo.to(dev), so.to(dev)
+    alphas = torch.full((groups,), 2.0, device=dev)
+    unread = torch.zeros(4096, dtype=torch.uint8, device=dev)  # K = 0: no operand has a byte
+    noise = torch.randn(2048, 2048, device=dev).bfloat16()
+    for dtype, code in ((torch.bfloat16, capi.BF16), (torch.float16, capi.F16)):
+        out = torch.full((m, n), 7.0, dtype=dtype, device=dev)
+        noise @ noise.t()  # something else in LDS
+        capi.check(capi.lib().nvf_nvfp4_scaled_grouped_mm(
+            unread.data_ptr(), unread.data_ptr(), unread.data_ptr(), unread.data_ptr(), alphas.data_ptr(), out.data_ptr(),
+            psd.data_ptr(), eod.data_ptr(), sod.data_ptr(), groups, m, n, 0, code, torch.cuda.current_stream().cuda_stream))
+        torch.cuda.synchronize()
+        assert bool((out[:rows] == 0).all()) and bool((out[rows:] == 7.0).all())
