@@ -18,6 +18,7 @@ It is not imported by ``fuser_amd/__init__.py``: a process that also imports the
 would register the same op name twice.
 """
 import torch
+from torch.utils._device import DeviceContext
 
 from . import _C, ops
 
@@ -61,9 +62,15 @@ def _(activation, fp4_weight, weight_scaling_factor, weight_global_scale, offset
 
 def _is_plain(tensor):
     """Whether a call that torch does not see may take the tensor's memory: no subclass, no vmap or other functional
-    transform's wrapper, nothing that records or replaces the operations (torch.compile, jit.trace, a dispatch mode)."""
-    return (type(tensor) is torch.Tensor and not torch.compiler.is_compiling() and not torch.jit.is_tracing()
-            and not torch._C._len_torch_dispatch_stack() and not torch._C._functorch.is_functorch_wrapped_tensor(tensor))
+    transform's wrapper, nothing that records or replaces the operations (torch.compile, jit.trace, a dispatch or function
+    mode; a default device, which is a function mode too, does neither here)."""
+    try:
+        return (type(tensor) is torch.Tensor and not torch.compiler.is_compiling() and not torch.jit.is_tracing()
+                and not torch._C._len_torch_dispatch_stack() and not torch._C._functorch.is_functorch_wrapped_tensor(tensor)
+                and (not torch._C._len_torch_function_stack() or
+                     all(type(mode) is DeviceContext for mode in torch.overrides._get_current_function_mode_stack())))
+    except AttributeError:  # (a torch whose private names differ: the tensor operations are always right)
+        return False
 
 
 def compute_auxiliary_tensors(hidden_states, offsets, out_features):

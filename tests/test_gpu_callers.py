@@ -150,3 +150,35 @@ def test_auxiliary_tensors_under_vmap_and_tracing(dev):
     for traced in (make_fx(call)(starts[0]), torch.jit.trace(call, (starts[0],))):
         for got, want in zip(traced(starts[1]), rows[1]):
             assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("mode", ["function", "dispatch"])
+def test_auxiliary_tensors_under_recording_modes(dev, mode):
+    """A mode that sees or replaces torch's functions or operators keeps seeing those of this call."""
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    from fuser_amd import custom_ops
+
+    seen = []
+
+    class Functions(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(getattr(func, "__name__", str(func)))
+            return func(*args, **(kwargs or {}))
+
+    class Operators(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    hidden = torch.empty(500, 64, device=dev)
+    starts = torch.tensor([0, 129, 129, 300], dtype=torch.int32, device=dev)
+    want = custom_ops.compute_auxiliary_tensors(hidden, starts, 384)
+    with Functions() if mode == "function" else Operators():
+        got = custom_ops.compute_auxiliary_tensors(hidden, starts, 384)
+    assert any("cat" in name for name in seen) and any("cumsum" in name for name in seen)
+    with torch.device("cpu"):  # a default device records nothing: the launch is still taken
+        assert custom_ops._is_plain(starts)
+    for g, w in zip(got, want):
+        assert torch.equal(g, w)
