@@ -78,9 +78,10 @@ def compute_auxiliary_tensors(hidden_states, offsets, out_features):
     ``NVFP4InferenceGroupedLinear.compute_auxiliary_tensors`` derives them
     (layers_for_inference_benchmark.py:395-424): rows per group from neighbouring starts (the last group
     ends at the last row), scale slabs of whole 128-row tiles laid end to end.  One kernel launch for contiguous
-    int32 offsets on the GPU; anything else (CPU tensors, other types, tracing, vmap) takes the tensor operations below."""
+    int32 offsets on the GPU; anything else (CPU tensors, other types, tracing, vmap, a width that is no plain size) takes
+    the tensor operations below."""
     if (_is_plain(offsets) and offsets.is_cuda and offsets.dtype is torch.int32 and offsets.dim() == 1
-            and offsets.is_contiguous()):
+            and offsets.is_contiguous() and type(out_features) is int and out_features >= 0):
         return _C.grouped_auxiliary_tensors(offsets, hidden_states.size(0), out_features, hidden_states.size(1))
     total = torch.tensor([hidden_states.size(0)], device=offsets.device, dtype=offsets.dtype)
     rows = torch.diff(torch.cat([offsets, total]))

@@ -182,3 +182,16 @@ def test_auxiliary_tensors_under_recording_modes(dev, mode):
         assert custom_ops._is_plain(starts)
     for g, w in zip(got, want):
         assert torch.equal(g, w)
+
+
+@pytest.mark.parametrize("width", [384.0, True, -1, torch.tensor(384)])
+def test_auxiliary_tensors_widths_that_are_no_plain_size(dev, width):
+    """Whatever torch.full_like takes as the value of an int32 tensor, here as on the CPU."""
+    from fuser_amd import custom_ops
+
+    hidden = torch.empty(500, 64)
+    starts = torch.tensor([0, 129, 129, 300], dtype=torch.int32)
+    want = custom_ops.compute_auxiliary_tensors(hidden, starts, width)
+    got = custom_ops.compute_auxiliary_tensors(hidden.to(dev), starts.to(dev), width)
+    for g, w in zip(got, want):
+        assert torch.equal(g.cpu(), w)
