@@ -1,6 +1,7 @@
 // Device-side pieces shared by the kernels whose MFMA operands are 16-bit floats (gemm16.hip and its *_kernel.inl files,
 // nvfp4_decode.hip).
 #pragma once
+#include "lds_direct.h"
 #include "nvf_internal.h"
 
 namespace nvf {
@@ -29,13 +30,6 @@ __device__ __forceinline__ uint32_t pack2(float a, float b, bool out_bf16) {
 // consecutive lanes = 16 consecutive rows, one chunk) are conflict-free.
 __device__ __forceinline__ int lds_pos2(int row, int chunk) { return row * 8 + (chunk ^ ((row >> 1) & 7)); }
 __device__ __forceinline__ int lds_pos(int row, int chunk) { return lds_pos2(row, chunk); }
-
-// LDS-direct load.  lds_byte_addr and base are wave-uniform; lane L's 16 bytes land at lds_byte_addr + 16 * L.
-// Issued from inline assembly: the compiler neither waits for it nor orders LDS reads against it, the
-// kernels do that with explicit s_waitcnt vmcnt(n).
-__device__ __forceinline__ void lds_dma16(uint32_t lds_byte_addr, const uint8_t* base, uint32_t voff) {
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_byte_addr), "v"(voff), "s"(base) : "memory", "m0");
-}
 
 // e4m3 scales of a lane's two blocks -> fp16 pairs; one dword (8 values of one block) -> one MFMA operand
 __device__ __forceinline__ void scale_pairs(uint32_t s2, f16x2 sv[2]) {

@@ -9,6 +9,7 @@
 // The 128x4 scale layout stores, for 32 consecutive rows, 16 bytes per row position holding
 // (rows r, r+32, r+64, r+96) x (4 consecutive K-blocks): one 16-byte load per lane fetches every
 // scale a 128-row wave tile needs for a 128-deep K step.
+#include "lds_direct.h"
 #include "nvf_internal.h"
 
 namespace nvf {
@@ -226,11 +227,6 @@ __global__ __launch_bounds__(256) void mxfp8_gemm_kernel(const Params p) {
 // rows, one chunk) on the 64-bank LDS.
 // -------------------------------------------------------------------------------------------------
 __device__ __forceinline__ int lds_pos2(int row, int chunk) { return row * 8 + (chunk ^ ((row >> 1) & 7)); }
-
-__device__ __forceinline__ void lds_dma16(uint32_t lds_byte_addr, const uint8_t* base, uint32_t voff) {
-  // lds_byte_addr and base are wave-uniform; lane L's 16 bytes land at lds_byte_addr + 16 * L
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_byte_addr), "v"(voff), "s"(base) : "memory", "m0");
-}
 
 // TM = 32-row accumulator tiles of a wavefront along M: 4 -> 256x256 workgroup tile, 2 -> 128x256 (for shapes
 // whose 256x256 tiles would leave compute units idle).  The statement order for TM = 4 is the one the 8192^3

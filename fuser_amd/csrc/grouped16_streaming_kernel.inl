@@ -99,10 +99,6 @@ __global__ __launch_bounds__(kStream16Waves * 64, 2) void streaming_gemm16_kerne
   const uint32_t slot = lds_base + (uint32_t)wave * kSlot;
   const uint32_t piece_even = (uint32_t)((lane & 7) ^ (lane >> 4));  // 8-row blocks 0, 2, ..; the odd ones: ^ 4
   const uint32_t lrow = (uint32_t)(lane >> 3);
-  auto load_weights = [&](uint32_t at, const uint8_t* base, uint32_t voff) {
-    if constexpr (STREAM) asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(at), "v"(voff), "s"(base) : "memory", "m0");
-    else lds_dma16(at, base, voff);
-  };
   auto issue = [&](const Item& it, int c) {
     uint32_t pe = piece_even, po = piece_even ^ 4u;
     if (tail_pieces != 0 && c == steps - 1) {
@@ -114,12 +110,12 @@ __global__ __launch_bounds__(kStream16Waves * 64, 2) void streaming_gemm16_kerne
     if (it.n0 + BN <= p.n) {
       const uint32_t ve = lrow * (uint32_t)kbytes + pe * 16u, vo = lrow * (uint32_t)kbytes + po * 16u;
 #pragma unroll
-      for (int j = 0; j < 2 * WT; ++j) load_weights(slot + j * 1024, b + (int64_t)kbytes * (8 * j), (j & 1) ? vo : ve);
+      for (int j = 0; j < 2 * WT; ++j) lds_dma16<0, STREAM>(slot + j * 1024, b + (int64_t)kbytes * (8 * j), (j & 1) ? vo : ve);
     } else {
       const uint32_t last = (uint32_t)(p.n - it.n0 - 1);
 #pragma unroll
       for (int j = 0; j < 2 * WT; ++j)
-        load_weights(slot + j * 1024, b, __umul24(min(lrow + 8 * j, last), (uint32_t)kbytes) + ((j & 1) ? po : pe) * 16u);
+        lds_dma16<0, STREAM>(slot + j * 1024, b, __umul24(min(lrow + 8 * j, last), (uint32_t)kbytes) + ((j & 1) ? po : pe) * 16u);
     }
 #pragma unroll
     for (int j = 0; j < kStream16Rows / 8; ++j) {

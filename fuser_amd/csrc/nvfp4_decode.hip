@@ -46,20 +46,6 @@ struct DecodeParams {
   int rows_large;  // groups of up to 32 rows and those of rows_large or more are this launch's
 };
 
-// LDS-direct loads of 16 and 4 bytes a lane to lds_byte_addr + OFFSET (the sum is made in m0: a register per address
-// would not fit beside the items')
-template <int OFFSET, bool STREAM = false>
-__device__ __forceinline__ void dma16(uint32_t lds_byte_addr, const uint8_t* base, uint32_t voff) {
-  if constexpr (STREAM)
-    asm volatile("s_add_u32 m0, %0, %3\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(lds_byte_addr), "v"(voff), "s"(base), "i"(OFFSET) : "memory", "m0", "scc");
-  else
-    asm volatile("s_add_u32 m0, %0, %3\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_byte_addr), "v"(voff), "s"(base), "i"(OFFSET) : "memory", "m0", "scc");
-}
-template <int OFFSET>
-__device__ __forceinline__ void dma4(uint32_t lds_byte_addr, const uint8_t* base, uint32_t voff) {
-  asm volatile("s_add_u32 m0, %0, %3\n\tglobal_load_lds_dword %1, %2" ::"s"(lds_byte_addr), "v"(voff), "s"(base), "i"(OFFSET) : "memory", "m0", "scc");
-}
-
 template <bool OUT_BF16, bool STREAM, int RH>
 __global__ __launch_bounds__(kWaves * 64, 2) void persistent_nvfp4_skinny_ring_kernel(const DecodeParams p) {
   extern __shared__ u32x4 lds[];
@@ -161,30 +147,30 @@ __global__ __launch_bounds__(kWaves * 64, 2) void persistent_nvfp4_skinny_ring_k
 
     const uint8_t* b = it.b + (int64_t)c * 128;
     const uint32_t ve = lrow * (uint32_t)kbytes + pe * 16u, vo = lrow * (uint32_t)kbytes + po * 16u;
-    dma16<0, STREAM>(slot, b, ve);
-    dma16<1024, STREAM>(slot, b += rows8, vo);
-    dma16<2048, STREAM>(slot, b += rows8, ve);
-    dma16<3072, STREAM>(slot, b += rows8, vo);
-    dma16<4096, STREAM>(slot, b += rows8, ve);
-    dma16<5120, STREAM>(slot, b += rows8, vo);
-    dma16<6144, STREAM>(slot, b += rows8, ve);
-    dma16<7168, STREAM>(slot, b += rows8, vo);
+    lds_dma16<0, STREAM>(slot, b, ve);
+    lds_dma16<1024, STREAM>(slot, b += rows8, vo);
+    lds_dma16<2048, STREAM>(slot, b += rows8, ve);
+    lds_dma16<3072, STREAM>(slot, b += rows8, vo);
+    lds_dma16<4096, STREAM>(slot, b += rows8, ve);
+    lds_dma16<5120, STREAM>(slot, b += rows8, vo);
+    lds_dma16<6144, STREAM>(slot, b += rows8, ve);
+    lds_dma16<7168, STREAM>(slot, b += rows8, vo);
     const uint8_t* a = it.a + (int64_t)c * 128;
     auto a_off = [&](uint32_t first) { return __umul24(min(lrow + first, (uint32_t)(it.rows - 1)), (uint32_t)kbytes); };
-    dma16<kWeightBytes>(slot, a, a_off(0) + pe * 16u);
-    dma16<kWeightBytes + 1024>(slot, a, a_off(8) + po * 16u);
+    lds_dma16<kWeightBytes>(slot, a, a_off(0) + pe * 16u);
+    lds_dma16<kWeightBytes + 1024>(slot, a, a_off(8) + po * 16u);
     if (it.rows > 16) {
-      dma16<kWeightBytes + 2048>(slot, a, a_off(16) + pe * 16u);
-      dma16<kWeightBytes + 3072>(slot, a, a_off(24) + po * 16u);
+      lds_dma16<kWeightBytes + 2048>(slot, a, a_off(16) + pe * 16u);
+      lds_dma16<kWeightBytes + 3072>(slot, a, a_off(24) + po * 16u);
     }
     const uint8_t* sb = it.sfb + (int64_t)c * 2048;
     const uint8_t* sa = it.sfa + (int64_t)c * 2048;
     const uint32_t off0 = tile[0] * 512u + (uint32_t)(lane & 31) * 16u, off1 = tile[1] * 512u + (uint32_t)(lane & 31) * 16u;
     constexpr int kScales = kWeightBytes + kRowBytes;
-    dma16<kScales>(slot, sb, off0);
-    dma16<kScales + 1024>(slot, sb, off1);
-    dma4<kScales + kWeightScaleBytes>(slot, sa, off0);
-    dma4<kScales + kWeightScaleBytes + 256>(slot, sa, off1);
+    lds_dma16<kScales>(slot, sb, off0);
+    lds_dma16<kScales + 1024>(slot, sb, off1);
+    lds_dma4<kScales + kWeightScaleBytes>(slot, sa, off0);
+    lds_dma4<kScales + kWeightScaleBytes + 256>(slot, sa, off1);
   };
 
   // ---- read side
