@@ -344,6 +344,26 @@ int launch_tile(const Params& p, int grid, hipStream_t stream) {
 // 807 with against 753 without, but evenly loaded experts 639 against 771).
 constexpr int64_t kPrefillRows = 6144;
 
+// Grouped NVFP4, the groups of 129 rows and more: in slabs of 32 rows on the persistent streaming kernel, in calls of at most
+// 1024 rows whose 128x128 tiles (256x256 from 512 rows per group on) would leave compute units idle, each walking all of K on
+// one of them: 1024 rows over 8 experts, K = 7168, N = 2048 118 -> 56 us, 512 rows with Zipf loads 123 -> 38.  Every slab reads
+// the weights again and adds partial sums, so the fuller the chip is with tiles and the shallower K is, the more the tiles
+// gain.  Slabs / tiles, us, 256 rows per group, tiles for 1/2, 3/4, 7/8 and all of the compute units: K = 512 15 / 16, 20 / 17,
+// 23 / 17, 25 / 17; K = 1024 17 / 21, 22 / 22, 25 / 22, 28 / 23; K = 2048 23 / 33, 33 / 34, 37 / 34, 41 / 34; K = 4096 35 / 55,
+// 49 / 56, 56 / 56, 63 / 57; K = 7168 51 / 88, 73 / 89, 84 / 90, 91 / 90.
+// Below 129 rows per group only some groups are that large, and from 512 on the tiles are 256x256: twice as many tiles' worth
+// (8 experts with Zipf loads, 1024 rows, as many tiles as compute units: K = 512 24 / 23, K = 1024 29 / 31; two experts of 512
+// rows: K = 256 25 / 26).  Where two tiles for every group of fewer than 256 rows need a second round, slabs from K = 1024 on
+// (6 groups of 160 rows, N = 4096: K = 512 25 / 21, K = 1024 28 / 29, K = 4096 61 / 77; 3 groups, N = 6144, K = 1024 22 / 28).
+bool nvfp4_large_groups_stream(int64_t groups, int64_t m, int64_t n, int64_t k, int cus) {
+  const int64_t tiles = ceil_div(m, 128) * ceil_div(n, 128);
+  if (m < 129 || m > 1024 || tiles > cus) return false;
+  const bool few_or_large = m < 129 * groups || m >= 512 * groups;
+  if (m >= 129 * groups && m < 256 * groups && k >= 1024 && 2 * groups * ceil_div(n, 128) > cus) return true;
+  const int64_t share = k < 256 ? 4 : k < 512 ? 6 : k < 1024 ? 8 : k < 2048 ? 10 : k < 4096 ? 12 : k < 7168 ? 14 : 16;
+  return 16 * tiles <= (few_or_large ? 2 : 1) * share * cus;
+}
+
 template <bool NVFP4, bool BF16_MMA, bool OUT_BF16>
 int launch_sized(const Params& p, int64_t m_hint, int cus, void* workspace, int64_t workspace_bytes, hipStream_t stream) {
   // Pick the largest tile that still yields about one work item per compute unit.
@@ -399,14 +419,11 @@ int launch_sized(const Params& p, int64_t m_hint, int cus, void* workspace, int6
       return launch_grouped16_streaming<BF16_MMA>(p, cus, stream);
   }
   if constexpr (NVFP4) {
-    // Grouped NVFP4: groups of up to 128 rows (MoE decode, the small experts of a prefill) stream their expert's
-    // weights once through the skinny kernel; the launches below then skip them.  The group sizes live on
-    // the device, so every kernel is always launched; workgroups without work return at once.
+    // Grouped NVFP4: the groups of 1..32 rows and those of 33..128 rows (MoE decode, the small experts of a prefill) have
+    // launches of their own, which stream their experts' weights; the launches below then skip them.  The group sizes live
+    // on the device, so every kernel is always launched; workgroups without work return at once.
     if (!dense && p.min_rows == 0) {
-      // The groups of 1..32 rows; and in a call of at most 1024 rows whose 128x128 tiles would leave compute units idle,
-      // each walking all of K on one of them, those of 129 rows and more as well, in slabs of 32 (1024 rows over 8
-      // experts, K = 7168, N = 2048: 118 -> 56 us; 512 rows with Zipf loads: 123 -> 38 us).
-      const bool with_large = m_hint <= 1024 && !is_prefill && tiles(128, 128) <= cus;
+      const bool with_large = nvfp4_large_groups_stream(p.groups, m_hint, p.n, p.k, cus) && !is_prefill;
       Gemm16Args small{};
       small.a = p.a, small.b = p.b, small.sfa = p.sfa, small.sfb = p.sfb, small.alpha = p.alpha, small.out = p.out;
       small.problem_sizes = p.problem_sizes, small.expert_offsets = p.expert_offsets, small.sf_offsets = p.sf_offsets;

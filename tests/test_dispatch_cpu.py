@@ -223,6 +223,43 @@ def test_nvfp4_grouped_below_the_prefill_size_streams_the_mid_sized_groups(m, n,
     assert "nvfp4_group_panel_kernel" not in got, got
 
 
+@pytest.mark.parametrize("m,n,k,groups,small,large", [
+    # the groups of 129 rows and more: 256 rows per group, tiles for half, 5/8, 3/4, 7/8 and all of the compute units
+    (1024, 2048, 512, 4, "split", "slabs"), (1024, 2176, 512, 4, "split", "tiles"),
+    (1024, 2560, 1024, 4, "split", "slabs"), (1024, 2688, 1024, 4, "split", "tiles"),
+    (1024, 3072, 2048, 4, "split", "slabs"), (1024, 3200, 2048, 4, "split", "tiles"),
+    (1024, 3584, 4096, 4, "split", "slabs"), (1024, 3712, 4096, 4, "split", "tiles"),
+    (1024, 4096, 7168, 4, "split", "slabs"), (1025, 2048, 7168, 8, "split", "tiles"),
+    # fewer rows per group, 512 and more, and tiles in two rounds
+    (1024, 4096, 512, 8, "split", "slabs"), (1024, 3072, 256, 8, "split", "slabs"), (1024, 3200, 256, 8, "split", "tiles"),
+    (1024, 2048, 128, 8, "split", "slabs"), (1024, 2176, 128, 8, "split", "tiles"), (1024, 4096, 512, 2, "split", "slabs"),
+    (960, 4096, 1024, 6, "split", "slabs"), (960, 4096, 960, 6, "split", "tiles"), (480, 5504, 1024, 3, "split", "slabs"), (480, 5376, 1024, 3, "split", "tiles"),
+])
+def test_nvfp4_grouped_small_and_large_groups(m, n, k, groups, small, large):
+    """Which launch takes the groups of 1..32 rows and which those of 129 rows and more (None: there can be none)."""
+    parts = plan("nvfp4_scaled_grouped_mm", m, n, k, groups=groups).split("; ")
+    kernel = {"split": "persistent_nvfp4_skinny_ring_kernel<", "own4": "nvfp4_skinny_ring_kernel<RT=4,TT=2,grouped,nsplit=1>",
+              "own2": "nvfp4_skinny_ring_kernel<RT=2,TT=2,grouped,nsplit=1>"}[small]
+    assert parts[0].startswith(kernel) and "rows=1..32" in parts[0], parts
+    slabs = [p for p in parts if p.startswith("persistent_nvfp4_skinny_ring_kernel<") and p.endswith("129..")]
+    assert len(slabs) == (large == "slabs"), parts
+    if large == "tiles":
+        assert any("min_rows=129" in p for p in parts), parts
+    if large is None:
+        assert len(parts) == 1, parts
+
+
+@pytest.mark.parametrize("m,n,k,groups,rows", [
+    (48 * 8, 1024, 1024, 8, 32), (49 * 8, 1024, 1024, 8, 0), (48 * 8, 4096, 4096, 8, 64), (49 * 8, 4096, 4096, 8, 0),
+    (24 * 64, 2048, 7168, 64, 64), (25 * 64, 2048, 7168, 64, 0), (16 * 32, 2880, 2880, 32, 64), (17 * 32, 2880, 2880, 32, 0),
+    (16 * 8, 3000, 1288, 8, 32), (17 * 8, 3000, 1288, 8, 0), (64, 1024, 1024, 64, 0), (8, 128, 1016, 8, 0),
+])
+def test_grouped_mm_with_few_rows_per_group_streams_the_weights(m, n, k, groups, rows):
+    """Both sides of the lines at 48, 24 and 16 rows per group; `rows`: weight rows of a work item (0: the tile kernel)."""
+    got = plan("grouped_mm", m, n, k, groups=groups)
+    assert got.startswith(f"streaming_gemm16_kernel<weight_rows={rows}," if rows else "gemm16_kernel<") and ";" not in got, got
+
+
 @pytest.mark.parametrize("m,n,k,groups,prefill", [
     (65536, 2048, 7168, 256, True), (6144, 2048, 7168, 256, True), (6000, 2048, 7168, 256, False),
     (1536, 14336, 4096, 8, True),     # a round of 256x256 tiles and 128 rows per group on average
