@@ -364,6 +364,26 @@ bool nvfp4_large_groups_stream(int64_t groups, int64_t m, int64_t n, int64_t k, 
   return 16 * tiles <= (few_or_large ? 2 : 1) * share * cus;
 }
 
+// Grouped NVFP4, the groups of 1..32 rows: on the streaming kernel whose 8 wavefronts own 64 (N % 512 = 0) or 32 weight rows
+// each and walk K alone, instead of the persistent kernel, whose wavefronts split K.  With a shallow K the latter has a step
+// or two per item next to a sum and its barriers; up to K < 4096 it is behind where the other's workgroups are one round of
+// the compute units.  Persistent kernel against this one, us: 256 experts of 4096 x 128, 512 rows with Zipf loads 51 / 23, x 512
+// 53 / 43; 24 rows each: 32 experts of 4096 x 1024 1.26 times as slow, x 2048 equal, 16 of 8192 x 2560 1.27 (32 of 8192 1.07),
+// x 3584 1.12 (1.00), 64 of 2048 x 3584 1.16; for half as many workgroups as compute units 8 of 8192 x 512 1.10, x 1024 1.00,
+// x 2048 0.99, 4096 x 512 (a quarter) 0.84.  From 128 rows per group on such groups are few, and the two are within 7 %.
+// `with_large`: the persistent kernel would take the groups of 129 rows and more along; a launch of it for them alone costs
+// 5-20 % of a call with Zipf loads, which K < 512 outweighs, and up to K = 2048 (where even loads gain 8-20 %) a full round.
+// Below three times 129 rows in all there is hardly such a group.
+bool nvfp4_wavefronts_own_rows(int64_t groups, int64_t m, int64_t n, int64_t k, int cus, bool with_large) {
+  const bool large = with_large && m >= 3 * 129;
+  const int64_t rows = (n & 511) == 0 ? 512 : 256;
+  if ((k & 127) != 0 || n % rows != 0 || m >= 128 * groups) return false;
+  const int64_t wgs = std::min(groups, m) * (n / rows);
+  if (k < 512 || (k < 2048 && !large)) return 2 * wgs >= cus;
+  if (k < 2048) return wgs >= cus && (k < 1024 || wgs < 8 * (int64_t)cus);
+  return k > 2048 && k < 4096 && !large && 8 * wgs >= 7 * (int64_t)cus && wgs <= cus;
+}
+
 template <bool NVFP4, bool BF16_MMA, bool OUT_BF16>
 int launch_sized(const Params& p, int64_t m_hint, int cus, void* workspace, int64_t workspace_bytes, hipStream_t stream) {
   // Pick the largest tile that still yields about one work item per compute unit.
@@ -424,11 +444,15 @@ int launch_sized(const Params& p, int64_t m_hint, int cus, void* workspace, int6
     // on the device, so every kernel is always launched; workgroups without work return at once.
     if (!dense && p.min_rows == 0) {
       const bool with_large = nvfp4_large_groups_stream(p.groups, m_hint, p.n, p.k, cus) && !is_prefill;
+      const bool own_rows = nvfp4_wavefronts_own_rows(p.groups, m_hint, p.n, p.k, cus, with_large);
       Gemm16Args small{};
       small.a = p.a, small.b = p.b, small.sfa = p.sfa, small.sfb = p.sfb, small.alpha = p.alpha, small.out = p.out;
       small.problem_sizes = p.problem_sizes, small.expert_offsets = p.expert_offsets, small.sf_offsets = p.sf_offsets;
       small.groups = p.groups, small.m = p.m, small.n = p.n, small.k = p.k, small.dtype = OUT_BF16 ? NVF_BF16 : NVF_F16;
-      int rc = launch_nvfp4_decode(small, with_large, stream), tail_done = 0;
+      int rc = NVF_OK, tail_done = 0;
+      if (own_rows) rc = (p.n & 511) == 0 ? launch_nvfp4_skinny_grouped<4, 2, OUT_BF16, true>(p, 1, 32, stream)
+                                          : launch_nvfp4_skinny_grouped<2, 2, OUT_BF16, true>(p, 1, 32, stream);
+      if (rc == NVF_OK && (!own_rows || with_large)) rc = launch_nvfp4_decode(small, !own_rows, with_large, stream);
       if (rc != NVF_OK || m_hint <= 32) return rc;
       // Below the prefill size the groups of 33..128 rows are few: they stream their weights like the smaller ones,
       // found by rank among the groups of their size (a launch with few workgroups when there are few rows in all).  A

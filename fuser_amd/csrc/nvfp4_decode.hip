@@ -1,5 +1,5 @@
-// Grouped NVFP4 GEMM, the groups of 1..32 rows (a decode step, the small experts of a prefill): every expert's weights
-// are read once.
+// Grouped NVFP4 GEMM, the groups of 1..32 rows (a decode step, the small experts of a prefill), whose experts' weights are
+// read once; in small calls also those of 129 rows and more, in slabs of 32 rows that each read them.
 //   nvfp4_scaled_grouped_mm   (cutlass/nvfp4_scaled_group_mm.cu:714-788, pointer rule :83-155)
 //
 // Bound by the weight stream, so the kernel is built around keeping it going:
@@ -43,7 +43,7 @@ struct DecodeParams {
   uint16_t* out;
   const int32_t *problem_sizes, *expert_offsets, *sf_offsets;
   int groups, n, k;
-  int rows_large;  // groups of up to 32 rows and those of rows_large or more are this launch's
+  int rows_small, rows_large;  // groups of up to rows_small rows and those of rows_large or more are this launch's
 };
 
 template <bool OUT_BF16, bool STREAM, int RH>
@@ -69,7 +69,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void persistent_nvfp4_skinny_ring_k
     for (int base = 0; base < p.groups; base += kWaves * 64) {
       const int gi = base + tid;
       const int m_g = gi < p.groups ? max(p.problem_sizes[gi * 3], 0) : 0;
-      const int slabs = m_g <= kSlabRows || m_g >= p.rows_large ? (m_g + kSlabRows - 1) / kSlabRows : 0;
+      const int slabs = m_g <= p.rows_small || m_g >= p.rows_large ? (m_g + kSlabRows - 1) / kSlabRows : 0;
       int incl = slabs;
 #pragma unroll
       for (int d = 1; d < 64; d <<= 1) {
@@ -306,7 +306,8 @@ __global__ __launch_bounds__(kWaves * 64, 2) void persistent_nvfp4_skinny_ring_k
 template <bool OUT_BF16, bool STREAM, int RH>
 int launch_decode(const DecodeParams& p, int grid, hipStream_t stream) {
   auto kern = persistent_nvfp4_skinny_ring_kernel<OUT_BF16, STREAM, RH>;
-  if (note_launch("persistent_nvfp4_skinny_ring_kernel<stream=%d,halves=%d> grid=%d rows=1..32%s", (int)STREAM, RH, grid, p.rows_large < INT32_MAX ? ",129.." : ""))
+  const char* const rows = p.rows_small == 0 ? "129.." : p.rows_large < INT32_MAX ? "1..32,129.." : "1..32";
+  if (note_launch("persistent_nvfp4_skinny_ring_kernel<stream=%d,halves=%d> grid=%d rows=%s", (int)STREAM, RH, grid, rows))
     return NVF_OK;
   static std::atomic<uint64_t> configured{0};  // one bit per device
   if (const int rc = allow_dynamic_lds(reinterpret_cast<const void*>(kern), kLdsBytes, configured)) return rc;
@@ -316,7 +317,7 @@ int launch_decode(const DecodeParams& p, int grid, hipStream_t stream) {
 
 }  // namespace
 
-int launch_nvfp4_decode(const Gemm16Args& a, bool large_groups, hipStream_t stream) {
+int launch_nvfp4_decode(const Gemm16Args& a, bool small_groups, bool large_groups, hipStream_t stream) {
   DecodeParams p;
   p.a = static_cast<const uint8_t*>(a.a);
   p.b = static_cast<const uint8_t*>(a.b);
@@ -330,11 +331,12 @@ int launch_nvfp4_decode(const Gemm16Args& a, bool large_groups, hipStream_t stre
   p.groups = a.groups;
   p.n = (int)a.n;
   p.k = (int)a.k;
+  p.rows_small = small_groups ? kSlabRows : 0;
   p.rows_large = large_groups ? 129 : INT32_MAX;
   const int cus = cu_count();
   const int64_t slabs = a.groups + (large_groups ? a.m / kSlabRows : 0);  // at most
   // two halves of 64 weight rows per workgroup, unless such items cannot fill the compute units
-  const bool halves = std::min<int64_t>(a.groups, a.m) * (a.n / 128) >= 4 * (int64_t)cus;
+  const bool halves = small_groups && std::min<int64_t>(a.groups, a.m) * (a.n / 128) >= 4 * (int64_t)cus;
   const int grid = (int)std::min<int64_t>(std::max(cus & ~15, 16), round_up(slabs * (a.n / (halves ? 128 : 64)), 16));
   // weights beyond what the 256 MB last-level cache holds are read past it
   const bool stream_weights = (a.k & 255) == 0 && (double)a.groups * (double)a.n * (double)a.k * (9.0 / 16) > (double)(256 << 20);

@@ -729,9 +729,11 @@ int launch_nvfp4_skinny_ring_cfg(const Params& p, hipStream_t stream, int slabs 
 template <int RT, int TT, bool OUT_BF16, bool NSPLIT, int W = 8>
 int launch_nvfp4_skinny_grouped(const Params& p0, int rows_lo, int rows_hi, hipStream_t stream) {
   constexpr int SLOT_KIB = RT + TT + (RT + 1) / 2 + (TT + 1) / 2;
-  // one slot per wavefront, as in the dense launch
+  // One slot per wavefront also where two would fit: measured faster for the groups of up to 32 rows (512 rows
+  // over 256 experts, K=2048: 432 -> 413 us).
   constexpr int DEPTH = 1;
-  auto kern = (p0.k & 127) != 0 ? nvfp4_skinny_ring_kernel<RT, TT, OUT_BF16, DEPTH, true, NSPLIT, true, W>
+  // (wavefronts that own rows: only where K % 128 = 0)
+  auto kern = (p0.k & 127) != 0 ? nvfp4_skinny_ring_kernel<RT, TT, OUT_BF16, DEPTH, true, NSPLIT, !NSPLIT, W>
                                 : nvfp4_skinny_ring_kernel<RT, TT, OUT_BF16, DEPTH, true, NSPLIT, false, W>;
   constexpr int red_kib = NSPLIT ? 0 : W * (RT * TT <= 8 ? RT * TT : TT);
   constexpr int ring_kib = W * DEPTH * SLOT_KIB;

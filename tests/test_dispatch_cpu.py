@@ -224,6 +224,19 @@ def test_nvfp4_grouped_below_the_prefill_size_streams_the_mid_sized_groups(m, n,
 
 
 @pytest.mark.parametrize("m,n,k,groups,small,large", [
+    # shallow weights: wavefronts that own weight rows, from a workgroup for every second compute unit on
+    (1056, 2048, 384, 32, "own4", "tiles"), (992, 2048, 384, 31, "split", "slabs"), (32, 2048, 512, 32, "own4", None),
+    (31, 2048, 512, 32, "split", None), (1056, 2048, 1920, 32, "own4", "tiles"), (512, 2048, 384, 32, "own4", "slabs"),
+    # ... where there may be large groups to take along, with K from 512 on: from one for every compute unit on
+    (512, 4096, 512, 32, "own4", "slabs"), (512, 4096, 512, 31, "split", "slabs"), (512, 4096, 896, 256, "own4", "slabs"),
+    (512, 2048, 1920, 256, "own4", "slabs"), (512, 4096, 1024, 256, "split", "slabs"), (512, 2048, 2048, 64, "split", "slabs"),
+    (387, 2048, 512, 32, "split", "slabs"), (386, 2048, 512, 32, "own4", "slabs"),
+    # ... and with K beyond 2048 where they are one round of the compute units
+    (1536, 8192, 2048, 16, "split", "tiles"), (1536, 8192, 2176, 16, "own4", "tiles"),
+    (1536, 8192, 2560, 16, "own4", "tiles"), (1536, 8192, 2560, 14, "own4", "tiles"), (1536, 8192, 2560, 13, "split", "tiles"),
+    (1536, 8192, 2560, 17, "split", "tiles"), (1536, 8192, 3968, 16, "own4", "tiles"), (1536, 8192, 4096, 16, "split", "tiles"),
+    (32, 2304, 512, 32, "own2", None), (512, 1408, 512, 256, "split", "slabs"), (512, 4096, 576, 256, "split", "slabs"),
+    (32768, 4096, 1024, 256, "split", "tiles"), (32767, 4096, 1024, 256, "own4", "tiles"),
     # the groups of 129 rows and more: 256 rows per group, tiles for half, 5/8, 3/4, 7/8 and all of the compute units
     (1024, 2048, 512, 4, "split", "slabs"), (1024, 2176, 512, 4, "split", "tiles"),
     (1024, 2560, 1024, 4, "split", "slabs"), (1024, 2688, 1024, 4, "split", "tiles"),

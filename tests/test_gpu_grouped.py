@@ -710,3 +710,43 @@ def test_nvfp4_grouped_mm_with_empty_k_is_zero(dev, sizes, n):
             psd.data_ptr(), eod.data_ptr(), sod.data_ptr(), groups, m, n, 0, code, torch.cuda.current_stream().cuda_stream))
         torch.cuda.synchronize()
         assert bool((out[:rows] == 0).all()) and bool((out[rows:] == 7.0).all())
+
+
+@pytest.mark.parametrize("n,k,rt", [(1024, 128, 4), (1024, 384, 4), (1280, 256, 2)])
+def test_nvfp4_grouped_mm_wavefronts_that_own_weight_rows(dev, n, k, rt):
+    """Shallow weights: the groups of 1..32 rows on the kernel whose wavefronts own 64 or 32 weight rows each, those of 129
+    rows and more in a launch of the persistent kernel for them alone.  Every element compared, rows outside the groups
+    untouched, run-to-run bit equality."""
+    from fuser_amd import capi
+
+    groups = 64
+    sizes = [0] * groups
+    for i, t in enumerate([1, 16, 17, 32, 0, 129, 2, 33, 15, 160, 31]):
+        sizes[i * 6] = t
+    rows, m = sum(sizes), sum(sizes) + 3
+    plan = capi.describe_dispatch("nvfp4_scaled_grouped_mm", m, n, k, groups=groups)
+    assert plan.startswith(f"nvfp4_skinny_ring_kernel<RT={rt},TT=2,grouped,nsplit=1> grid={groups * n // (128 * rt)} rows=1..32; "
+                           "persistent_nvfp4_skinny_ring_kernel<stream=0,halves=1> ") and " rows=129..;" in plan, plan
+    gen = torch.Generator().manual_seed(n + k)
+    x = torch.randn(m, k, generator=gen).bfloat16()
+    ps, eo, _, _ = _grouped_args(sizes, n, k, dev)
+    so = start_offsets([O.round_up(t, 128) for t in sizes])
+    aq, asf = O.grouped_block_quantize_nvfp4(x, eo, so, None)
+    w = [(torch.randn(n, k, generator=gen) * 0.05).bfloat16() for _ in range(8)]
+    quantized = [O.block_quantize_nvfp4(w[e % 8], gs_of(w[e % 8]), True) for e in range(groups)]
+    bq, bsf = (torch.stack([q[i] for q in quantized]) for i in (0, 1))
+    alphas = torch.tensor([(e % 11 + 1) / gs_of(w[e % 8]) for e in range(groups)])
+    ref = O.ref_nvfp4_scaled_grouped_mm(aq, bq, asf, bsf, alphas, ps, eo, so)[:rows]
+    scale = ref.abs().amax(dim=1, keepdim=True).clamp(min=1e-30)
+    on_dev = [t.to(dev) for t in (aq, bq, asf, bsf, alphas, ps, eo, so)]
+    aqd, bqd, asfd, bsfd, ald, psd, eod, sod = [t.data_ptr() for t in on_dev]
+    for dtype, code in ((torch.bfloat16, capi.BF16), (torch.float16, capi.F16)):
+        outs = []
+        for _ in range(2):
+            out = torch.full((m, n), 7.0, dtype=dtype, device=dev)
+            capi.check(capi.lib().nvf_nvfp4_scaled_grouped_mm(aqd, bqd, asfd, bsfd, ald, out.data_ptr(), psd, eod, sod, groups, m, n, k, code,
+                                                              torch.cuda.current_stream().cuda_stream))
+            torch.cuda.synchronize()
+            outs.append(out)
+        assert ((outs[0][:rows].float().cpu() - ref).abs() / scale).max().item() <= GEMM_MAX_REL, dtype
+        assert torch.equal(*outs) and bool((outs[0][rows:] == 7.0).all())
