@@ -1025,3 +1025,43 @@ def test_dense_ops_reject_bad_inputs_on_device(dev):
     with pytest.raises(RuntimeError, match="contiguous"):
         nvf_cutlass.nvfp4_scaled_mm(fp4(torch.zeros(128, 64, dtype=torch.uint8, device=dev)[:, ::2]), a, sa, sa, alpha, torch.bfloat16)
     assert nvf_cutlass.get_sm_version() == 950 and nvf_cutlass.get_multiprocessor_count() == 256
+
+
+@pytest.mark.parametrize("m,n,k", [(512, 4096, 288), (512, 4096, 1088), (600, 4096, 352), (4096, 4096, 4128)])
+def test_mxfp8_gemm_short_last_step_adds_exact_zeros(dev, m, n, k):
+    """K % 128 = 32, 64 or 96 on the persistent kernel: lanes past the row's end multiply the row's last 16 elements again,
+    times 2^-254.  With the largest values there a sum that is zero stays zero, a tiny one stays what it is, and a NaN there
+    stays in its row or column, whatever the scale layout's padding holds."""
+    from fuser_amd import capi
+
+    plan = capi.describe_dispatch("mxfp8_scaled_mm", m, n, k)
+    assert plan.startswith("mxfp8_gemm_256_kernel<") and "ragged_k" in plan and ";" not in plan, plan
+    gen = torch.Generator().manual_seed(m + k)
+    a8, _ = O.block_quantize_mxfp8(torch.randn(m, k, generator=gen).bfloat16())
+    b8, _ = O.block_quantize_mxfp8(torch.randn(n, k, generator=gen).bfloat16())
+    a8, b8 = a8.view(torch.uint8).clone(), b8.view(torch.uint8).clone()
+    sa, sb = torch.full((m, k // 32), 127, dtype=torch.uint8), torch.full((n, k // 32), 127, dtype=torch.uint8)
+    for row in (0, 77, m - 1):  # the products of the first and the last 16 elements cancel: 448 * 448 and -448 * 448
+        a8[row] = 0
+        a8[row, :16] = a8[row, k - 16 :] = 0x7E
+    for row in (1, n - 2):
+        b8[row] = 0
+        b8[row, :16], b8[row, k - 16 :] = 0xFE, 0x7E
+    a8[33] = 0x01  # 2^-9 with scales 2^-100: sums of about 1e-33
+    b8[34] = 0x01
+    sa[33] = sb[34] = 77
+    a8[200, k - 16 :] = b8[300, k - 1] = 0x7F  # NaN
+    ones = [O.linear_to_swizzled_128_4(torch.ones_like(s)) == 0 for s in (sa, sb)]
+    sa_p, sb_p = O.linear_to_swizzled_128_4(sa), O.linear_to_swizzled_128_4(sb)
+    ref = O.ref_mxfp8_scaled_mm(a8, b8, sa_p, sb_p, 1.0)
+    assert (ref[0, 1], ref[77, n - 2], ref[m - 1, 1]) == (0, 0, 0) and 0 < ref[33, 34] < 1e-30
+    sa_p[ones[0]] = sb_p[ones[1]] = 0xFF
+    out = _run_mxfp8(a8, b8, sa_p, sb_p, 1.0, torch.bfloat16, dev).float().cpu()
+    assert torch.equal(out.isnan(), ref.isnan()) and out[200].isnan().all() and out[:, 300].isnan().all()
+    out, ref = torch.nan_to_num(out), torch.nan_to_num(ref)
+    for row in (0, 77, m - 1):
+        for col in (1, n - 2):
+            assert out[row, col] == 0
+    assert abs(out[33, 34] - ref[33, 34]) <= 2.0**-8 * ref[33, 34]  # (one bf16 rounding: the products and their sum are exact)
+    scale = ref.abs().amax(dim=1, keepdim=True).clamp(min=1e-30)
+    assert ((out - ref).abs() / scale).max().item() <= GEMM_MAX_REL

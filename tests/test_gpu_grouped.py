@@ -569,6 +569,7 @@ def test_grouped_ops_reject_bad_inputs_on_device(dev):
     (9, 128, 64), (9, 128, 192), (9, 256, 256), (9, 128, 320), (9, 384, 2112), (9, 128, 7168),  # whole and short last steps; fewer steps than wavefronts
     (128, 1024, 320), (1024, 128, 128),  # items of 128 weight rows; as many groups as a call may have
     (64, 2048, 4096),                    # weights beyond the last-level cache: read with non-temporal loads
+    (64, 1920, 4096), (9, 2048, 320),    # more items of 64 weight rows than workgroups, in cache and past it
 ])
 def test_nvfp4_grouped_mm_decode_kernel(dev, groups, n, k):
     """Groups of 1..32 rows on both sides of a row tile's border and, in slabs, of 129 rows and more; empty groups; a
@@ -583,6 +584,8 @@ def test_nvfp4_grouped_mm_decode_kernel(dev, groups, n, k):
     m = sum(sizes) + 3
     plan = capi.describe_dispatch("nvfp4_scaled_grouped_mm", m, n, k, groups=groups)
     assert f"stream={int(k == 4096)},halves={2 if min(groups, m) * (n // 128) >= 1024 else 1}> " in plan and "rows=1..32,129.." in plan, plan
+    if (groups, n) in ((64, 1920), (9, 2048)):
+        assert "halves=1" in plan and sum(-(-t // 32) for t in sizes if t <= 32 or t >= 129) * (n // 64) > 256 + 32, plan
     gen = torch.Generator().manual_seed(groups + n + k)
     x = torch.randn(m, k, generator=gen).bfloat16()
     w = (torch.randn(8, n, k, generator=gen) * 0.05).bfloat16()  # eight different experts, repeated
@@ -608,6 +611,13 @@ def test_nvfp4_grouped_mm_decode_kernel(dev, groups, n, k):
         scale = ref[:rows].abs().amax(dim=1, keepdim=True).clamp(min=1e-30)
         assert ((out[:rows].float().cpu() - ref[:rows]).abs() / scale).max().item() <= GEMM_MAX_REL, dtype
         assert torch.equal(out[:rows], nvf_cutlass.nvfp4_scaled_grouped_mm(*args, dtype)[:rows])
+        raw = torch.full((m, n), 7.0, dtype=dtype, device=dev)
+        capi.check(capi.lib().nvf_nvfp4_scaled_grouped_mm(
+            args[0].data_ptr(), args[1].data_ptr(), args[2].data_ptr(), args[3].data_ptr(), args[4].data_ptr(), raw.data_ptr(), args[7].data_ptr(),
+            args[8].data_ptr(), args[9].data_ptr(), groups, m, n, k, capi.BF16 if dtype == torch.bfloat16 else capi.F16,
+            torch.cuda.current_stream().cuda_stream))
+        torch.cuda.synchronize()
+        assert torch.equal(raw[:rows], out[:rows]) and bool((raw[rows:] == 7.0).all())
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
