@@ -398,7 +398,7 @@ def main():
                                  "roofline": {"bound": "mfma", "achieved": round(tf, 1), "peak": PEAK_F16_TFLOPS, "unit": "TFLOP/s",
                                               "frac": round(tf / PEAK_F16_TFLOPS, 4),
                                               "traffic": measured_traffic.get(f"nvfp4_grouped_mm_config5_K{k}_N{n}_bytes_per_call"),
-                                              "kernel": "nvfp4_gemm_256_kernel (+ nvfp4_group_panel_kernel, nvfp4_skinny_ring_kernel: the call's launches)",
+                                              "kernel": "nvfp4_gemm_256_kernel (+ nvfp4_group_panel_kernel, persistent_nvfp4_skinny_ring_kernel: the call's launches)",
                                               "algorithmic_bytes": int(g * n * k * 0.5625 + rows * k * 0.5625 + 2 * rows * n)}}
             if not args.no_cpu:
                 ne = 16  # the first 16 experts and their rows

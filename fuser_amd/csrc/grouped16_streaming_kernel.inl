@@ -225,7 +225,8 @@ int launch_grouped16_streaming(const Params& p, int cus, hipStream_t stream) {
   // 32 weight rows an item where items of 64 would not go round the compute units twice
   const bool narrow = std::min<int64_t>(p.groups, p.m) * ceil_div(p.n, 64) < 2 * (int64_t)cus;
   const int grid = (int)std::min<int64_t>(std::max(cus & ~7, 8), round_up(slabs * ceil_div(p.n, narrow ? 32 : 64), 8));
-  // weights beyond what the 256 MB last-level cache holds are read past it
+  // weights beyond what the 256 MB last-level cache holds are read past it (8 experts of 14336 x 4096, 16 rows each: 159 us,
+  // with plain loads 175; 64 of 2048 x 7168, 24 rows 312 / 335)
   const bool past_cache = (p.k & 63) == 0 && 2.0 * p.groups * p.n * p.k > (double)(256 << 20);
   if (narrow) return launch_grouped16_streaming_cfg<BF16, 2, false>(p, grid, stream);
   return past_cache ? launch_grouped16_streaming_cfg<BF16, 4, true>(p, grid, stream) : launch_grouped16_streaming_cfg<BF16, 4, false>(p, grid, stream);

@@ -8,15 +8,16 @@
 //     current one has no more, are under way while it converts and multiplies: the memory pipe does not drain at an item's
 //     end, as it did with a workgroup per item (first loads, 7 chunks, sums, gone).
 //   * A wavefront's step is 256 deep in K: 128 bytes of a weight row, a whole cache line.  Weights that the last-level
-//     cache cannot hold are read with non-temporal loads: 7.0 TB/s, against 6.1 with plain ones (a stream of 1.1 GB
-//     without arithmetic); with 64-byte pieces the non-temporal stream fetches lines twice (5.8), which is also why rows
-//     that do not start on a line (K % 256 != 0) are read with plain loads.
+//     cache cannot hold are read with non-temporal loads: 64 experts of 7168 x 7168, 2 rows each 288 us (6.4 TB/s), with
+//     plain ones 315; 256 of 7168 x 2048 361 / 373.  Where rows do not start on a line (K % 256 != 0) a non-temporal stream
+//     fetches lines twice, and plain loads are used: 256 experts of 7168 x 2688 542 us, with non-temporal ones 575.
 //   * The wavefronts of a half (RH = 2: four) split K and their partial sums are added in order through LDS.
 //     RH = 2 halves the number of sums and barriers per byte and lets both halves read one scale tile (128 weight rows):
-//     N = 7168, K = 2048 193 us against 215.  RH = 1 splits the work finer where there is little of it; there the two
-//     items that share a scale tile run at the same time on one XCD, whose L2 then reads it once.
-//   * 256 experts, 512 rows with Zipf loads (134 active): N = 2048, K = 7168 232 -> 204 us, N = 4096, K = 2048 152 -> 117
-//     us; the stream alone, with conversions and MFMAs left out, takes 161 of 178 us on the small groups.
+//     256 experts of 7168 x 2048, 512 rows with Zipf loads 187 us against 220, of 4096 x 4096 202 / 221, of 2048 x 7168
+//     equal.  RH = 1 splits the work finer where there is little of it; there the two items that share a scale tile run at
+//     the same time on one XCD, whose L2 then reads it once.
+//   * 256 experts, 512 rows with Zipf loads (134 active): N = 2048, K = 7168 232 -> 202 us (6.0 TB/s on the small groups),
+//     N = 4096, K = 2048 160 -> 112 us.
 // LDS of a wavefront: the weight tile of its step (64 rows of 128 bytes, piece c of row r at position c ^ ((r >> 1) & 7)),
 // the activation rows' (32 x 128 bytes, same order) and both operands' scales; loads are LDS-direct, a wavefront reads
 // only what it loaded itself.  Fragments and MFMAs as in the weight-streaming kernel: lane (r, g) holds piece g of row r,

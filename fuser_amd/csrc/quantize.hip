@@ -314,9 +314,9 @@ __device__ __forceinline__ uint32_t workgroup_max(uint32_t m) {
 }
 
 // A tensor larger than the last-level cache is read from its end to its start, and the first 96 MB, read last, are left in
-// the cache for the quantizer that starts there: scale and NVFP4 quantization of bf16 40000 x 4096 125.8 -> 122.8 us, f32
-// 30001 x 5120 209.8 -> 206.8, bf16 65536 x 7168 340.3 -> 339.0, the scale alone 133.5 -> 131.8.  208 MB would give the
-// pair 118.1, 204.8 and 337.9 us, but make the scale alone slower (136.5 us).
+// the cache for the quantizer that starts there: scale and NVFP4 quantization of bf16 40000 x 4096 126.1 -> 123.4 us, 60000 x
+// 2880 133.6 -> 129.4, f32 30001 x 5120 208.7 -> 206.3; no change at bf16 65536 x 7168 (339 us) and for the scale alone.
+// 208 MB would give the first 118.1 us, but make the scale of the largest slower (131.8 -> 136.5 us).
 constexpr int64_t kGlobalScaleKept = (int64_t)96 << 20;
 
 // The thread's maximum over the elements its workgroup (`wg` of `wgs`) owns.  A workgroup reads runs of LOADS * THREADS
