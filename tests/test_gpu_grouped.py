@@ -697,7 +697,7 @@ def test_nvfp4_grouped_mm_four_wavefronts_with_a_short_last_chunk(dev, n, k):
         assert torch.equal(out, nvf_cutlass.nvfp4_scaled_grouped_mm(*args, dtype))
 
 
-@pytest.mark.parametrize("sizes,n", [([1, 16, 17, 0, 32, 33, 128, 129, 300], 128), ([3, 20, 31, 0], 32896)])
+@pytest.mark.parametrize("sizes,n", [([1, 16, 17, 0, 32, 33, 128, 129, 300], 128), ([3, 20, 31, 0], 32896), ([3, 20, 31, 0], 32768)])
 def test_nvfp4_grouped_mm_with_empty_k_is_zero(dev, sizes, n):
     """K = 0 through the C entry (the tensor layer refuses empty operands): every row of every group is an empty sum, i.e.
     zero, whatever earlier kernels left in LDS; rows outside the groups stay untouched."""
@@ -705,7 +705,7 @@ def test_nvfp4_grouped_mm_with_empty_k_is_zero(dev, sizes, n):
 
     m, rows, groups = sum(sizes) + 4, sum(sizes), len(sizes)
     plan = capi.describe_dispatch("nvfp4_scaled_grouped_mm", m, n, 0, groups=groups)
-    assert ("halves=1> " in plan and "rows=1..32,129.." in plan) if n == 128 else "halves=2> " in plan, plan
+    assert {128: "halves=1> grid=64 rows=1..32,129..", 32896: "halves=2> ", 32768: "nsplit=1> "}[n] in plan, plan
     ps, eo, _, _ = _grouped_args(sizes, n, 0, dev)
     so = start_offsets([O.round_up(t, 128) for t in sizes])
     psd, eod, sod = ps.to(dev), eo.to(dev), so.to(dev)
