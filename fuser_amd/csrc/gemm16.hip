@@ -108,6 +108,45 @@ __device__ __forceinline__ void quantize_acc_tile(const f32x16& acc, float alpha
   }
 }
 
+// ... of four neighbouring 16x16 accumulator tiles, i.e. of 16 rows and their four blocks: lane (r, g) holds row r, columns
+// 16 j + 4 g + e in acc[j][e].  Lane (r, g) works out the scale of block g: the exchanges with the lanes 16 and 32 further on
+// hand every lane the other three's maxima of its own block, and their factors back.  q8: the code of block g; h[j]: this
+// lane's payload bytes 2 g, 2 g + 1 of block j.  (All four lanes working out all four scales: 2 us more on a 128x256 tile.)
+__device__ __forceinline__ void quantize_acc_tiles16(const f32x4 (&acc)[4], float alpha, float gs, float decode, uint32_t& q8, uint32_t (&h)[4]) {
+  float x[4][4], m[4];
+  bool nonfinite = false;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    m[j] = -INFINITY;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      x[j][e] = acc[j][e] * alpha;
+      m[j] = fmaxf(m[j], fabsf(x[j][e]));  // NaN ignored, as the quantizer does
+      nonfinite |= !(fabsf(x[j][e]) < INFINITY);
+    }
+  }
+  const int lane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+  const bool odd = (lane & 16) != 0, high = (lane & 32) != 0;
+  auto from = [&](float v, int other) { return __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute((lane ^ other) << 2, __builtin_bit_cast(int, v))); };
+  const float lo = fmaxf(odd ? m[1] : m[0], from(odd ? m[0] : m[1], 16)), hi = fmaxf(odd ? m[3] : m[2], from(odd ? m[2] : m[3], 16));
+  const float own = fmaxf(high ? hi : lo, from(high ? lo : hi, 32));  // of block g = 2 high + odd
+  float r;
+  q8 = nvfp4_block_scale(own, true, gs, decode, true, r);
+  const float other = from(r, 32), r_lo = high ? other : r, r_hi = high ? r : other;  // blocks odd and 2 + odd
+  const float o_lo = from(r_lo, 16), o_hi = from(r_hi, 16);
+  const float f[4] = {odd ? o_lo : r_lo, odd ? r_lo : o_lo, odd ? o_hi : r_hi, odd ? r_hi : o_hi};
+  const bool plain = __builtin_amdgcn_ballot_w64(nonfinite) == 0;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    if (plain) {
+      const uint32_t w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(0u, x[j][0] * f[j], x[j][1] * f[j], 1.0f, 0);
+      h[j] = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, x[j][2] * f[j], x[j][3] * f[j], 1.0f, 1);
+    } else {  // explicit NaN rule of the narrow cast
+      h[j] = f32x2_to_e2m1_byte(x[j][0] * f[j], x[j][1] * f[j]) | f32x2_to_e2m1_byte(x[j][2] * f[j], x[j][3] * f[j]) << 8;
+    }
+  }
+}
+
 // fills n bytes with zero (the padding of the block-scaled result's scale buffer for ragged shapes)
 __global__ __launch_bounds__(256) void zero_fill_kernel(uint32_t* __restrict__ dst, int64_t words) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;

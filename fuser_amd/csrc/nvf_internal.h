@@ -5,6 +5,7 @@
 #include <atomic>
 #include <cstdarg>
 #include <cstdio>
+#include <type_traits>
 
 #include "nvf_hip.h"
 
@@ -190,6 +191,16 @@ __device__ __forceinline__ uint32_t nvfp4_block_scale(float m, bool use_gs, floa
     r = fminf(1.0f / den, 3.402823466e+38f);
   }
   return q8;
+}
+
+// f(integral_constant 0), f(1), .., f(N - 1): a loop that is unrolled by its form, whatever the size of its body, and whose
+// counter is a constant inside
+template <int N, int I = 0, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    static_for<N, I + 1>(f);
+  }
 }
 
 }  // namespace nvf

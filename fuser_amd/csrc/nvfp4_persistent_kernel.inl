@@ -3,9 +3,13 @@
 // NVFP4 fast path: 256x256 (or 128x256) tile, N % 256 == 0, K % 128 == 0 (dense with a 16-bit result: K % 32 == 0),
 // K >= 256; dense with M % 256 (128) == 0,
 // or the whole 256-row tiles of every group of the grouped op; 16-bit or fp32 result.
+//   * Bound by the power limit and by the conversion work next to the MFMAs.  v_mfma_f32_16x16x32_f16: on NVFP4's values
+//     a register-only loop of it runs 2.23 PFLOP/s, of 32x32x16 1.91 (half the accumulator traffic per flop).
+//     8192 x 8192 x 8192 804..827 -> 747..780 us (1.41..1.47 PFLOP/s), 2048 x 14336 x 4096 192 -> 184 us, 1024 x 8192 x 4096
+//     63 -> 60 us against the same kernel with 32x32x16.
 //   * 512 threads: 8 wavefronts as 2 (m) x 4 (n), each with a 128x64 (64x64) accumulator tile, two per SIMD.
 //     A single wavefront issues at most one non-MFMA instruction per ~8 cycles, which is too little for
-//     the conversion work next to 32-cycle MFMAs; with two wavefronts per SIMD one converts while the
+//     the conversion work next to the MFMAs; with two wavefronts per SIMD one converts while the
 //     other's MFMA runs.
 //   * Persistent workgroups walk the tiles in an XCD-aware order; the operand stream (global -> registers
 //     -> fp16 in LDS) runs continuously across tile borders, two 128-deep spans ahead of the MFMAs.
@@ -20,14 +24,13 @@
 //   * Every piece of non-MFMA work is cut into MFMA-slot sized parts (3 conversion instructions, one LDS
 //     access, one global load) and pinned between two MFMAs, because the two wavefronts of a SIMD run
 //     in phase and a long run of other instructions in both would idle the matrix pipe.
-//   * One barrier per step, placed before the last quarter of its MFMAs: by then every wave has written
+//   * One barrier per step, placed before the last rows of its MFMAs: by then every wave has written
 //     its share of the next step and holds this step's last fragments in registers.
 // LDS: two buffers of an A tile and a B tile (stored A0, A1, B0, B1), each tile 256 rows x 128 bytes with 16-byte
 // chunk c of row r at chunk position c ^ ((r >> 1) & 7): conflict-free for the fragment reads.
 // -------------------------------------------------------------------------------------------------
 // TM = 32-row accumulator tiles of a wavefront along M: 4 -> 256x256 workgroup tile, 2 -> 128x256 (dense shapes
-// whose 256x256 tiles would leave compute units idle; 1.5 times the conversion work per MFMA).  The statement
-// order for TM = 4 is the one the 8192^3 measurements were made with.
+// whose 256x256 tiles would leave compute units idle; 1.5 times the conversion work per MFMA).
 // RAGGED_K (16-bit result; grouped: the 256x256 tiles): K % 128 = 32, 64 or 96.  A tile's last span is short: the threads whose 32 elements lie
 // past K fetch their row's first piece instead of the next row's bytes, and their scale load runs past the range of its
 // buffer resource on purpose, which makes it return zero - and a zero scale makes a block count as zero.
@@ -49,9 +52,11 @@ __global__ __launch_bounds__(512) void nvfp4_gemm_256_kernel(const Params p) {
   // buffers and all row tiles through the 16-bit immediate offset of the LDS instructions.
   auto tile_units = [](int buf, int op) { return op ? 2 * A_UNITS + buf * TILE_UNITS : buf * A_UNITS; };
   constexpr int AR = TM / 2;                 // A rows a thread stages per span (rows srow + 128 i)
-  constexpr int NMK = 2 * TM;                // MFMAs per 16-deep sub-step
+  constexpr int NI = 2 * TM, NJ = 4;         // 16-row tiles of a wavefront's accumulator tile, 16-column tiles
+  constexpr int ROWS = 2 * NI;               // rows of NJ MFMAs per 64-deep step: 32 of K times NI tiles, twice
+  constexpr int AHEAD = TM == 4 ? 2 : 3;      // rows that the fragments of A are read ahead
+  constexpr int BARRIER_ROW = ROWS - AHEAD;       // the row of a step before which its barrier stands
   constexpr int NCU = 2 * AR + 4;            // conversion units per step: operand, row, half scale block
-  constexpr int NFU = TM + 2;                // fragment reads per sub-step
   extern __shared__ u32x4 lds[];
   __shared__ int tile_prefix[GROUPED ? kMaxGroups + 1 : 1];
 
@@ -59,7 +64,7 @@ __global__ __launch_bounds__(512) void nvfp4_gemm_256_kernel(const Params p) {
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 2, wn = wave & 3;
-  const int li = lane & 31, lg = lane >> 5;
+  const int r16 = lane & 15, g4 = lane >> 4;
   const int srow = tid >> 2, spiece = tid & 3;  // staging: rows srow and srow+128, 16-byte piece of a 64-byte span
 
   // ---- persistent tile walk: workgroup ids are dealt round-robin to the 8 XCDs, XCD x owns the tile
@@ -227,11 +232,11 @@ __global__ __launch_bounds__(512) void nvfp4_gemm_256_kernel(const Params p) {
   };
 
   // ---- the thread's LDS byte addresses: per operand, one for each half scale block it stages and one for each of the
-  // four 16-deep sub-steps it reads fragments of (the swizzle makes those differ by an exclusive or, not by a sum).
-  // They pass through empty asm statements, so that the compiler keeps exactly these twelve registers and reaches
+  // two 32-deep sub-steps it reads fragments of (the swizzle makes those differ by an exclusive or, not by a sum).
+  // They pass through empty asm statements, so that the compiler keeps exactly these eight registers and reaches
   // buffer, row tile and second staging row through the instructions' immediate offsets.
   uint8_t* const lds_b = reinterpret_cast<uint8_t*>(lds);
-  uint32_t stage_at[2][2], frag_at[2][4];
+  uint32_t stage_at[2][2], frag_at[2][2];
 #pragma unroll
   for (int op = 0; op < 2; ++op) {
 #pragma unroll
@@ -240,8 +245,8 @@ __global__ __launch_bounds__(512) void nvfp4_gemm_256_kernel(const Params p) {
       asm volatile("" : "+v"(stage_at[op][cc]));
     }
 #pragma unroll
-    for (int kk = 0; kk < 4; ++kk) {
-      frag_at[op][kk] = (uint32_t)(tile_units(0, op) + lds_pos2((op ? wn * 64 : wm * (32 * TM)) + li, kk * 2 + lg)) * 16u;
+    for (int kk = 0; kk < 2; ++kk) {
+      frag_at[op][kk] = (uint32_t)(tile_units(0, op) + lds_pos2((op ? wn * 64 : wm * (32 * TM)) + r16, kk * 4 + g4)) * 16u;
       asm volatile("" : "+v"(frag_at[op][kk]));
     }
   }
@@ -277,37 +282,46 @@ __global__ __launch_bounds__(512) void nvfp4_gemm_256_kernel(const Params p) {
     }
   };
 
-  // ---- MFMA fragments of one 16-deep sub-step, loaded in the order of their first use by the MFMA
-  // sequence (a0 b0) (a0 b1) (a1 b0) ...: units 0..NFU-1 = a0, b0, b1, a1, a2, a3
-  struct Frag { u32x4 a[4], b[2]; };
-  auto load_frag_unit = [&](int buf, int kk, int q, Frag& f) {
-    const int op = (q == 1 || q == 2) ? 1 : 0;
-    const int t = op ? q - 1 : (q == 0 ? 0 : q - 2);
-    const u32x4 v = *reinterpret_cast<const u32x4*>(lds_b + frag_at[op][kk] + (buf * (op ? TILE_UNITS : A_UNITS) + t * 256) * 16);
-    if (op) f.b[t] = v; else f.a[t] = v;
+  // ---- MFMA fragments: 16 rows x 32 of K, lane (r16, g4) holds elements 8 g4 .. 8 g4 + 7 of row r16.  A step is ROWS rows of
+  // MFMAs: row m multiplies tile m % NI of A with the NJ tiles of B, 32-deep sub-step m / NI.  A's fragments are read three
+  // rows ahead into four places that take turns, B's for the next sub-step into the other of two sets.
+  u32x4 fa[4], fb[2][NJ];
+  auto load_a_frag = [&](int buf, int m) {  // row m of a step
+    fa[m & 3] = *reinterpret_cast<const u32x4*>(lds_b + frag_at[0][m / NI] + (buf * A_UNITS + (m % NI) * 128) * 16);
+  };
+  auto load_b_frag = [&](int buf, int kk, int j) {
+    fb[kk][j] = *reinterpret_cast<const u32x4*>(lds_b + frag_at[1][kk] + (buf * TILE_UNITS + j * 128) * 16);
   };
 
-  f32x16 acc[TM][2];
+  f32x4 acc[NI][NJ];
   auto zero_acc = [&]() {
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+    for (int i = 0; i < NI; ++i)
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
+      for (int j = 0; j < NJ; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  };
+  // In inline assembly, with the accumulator tied: from the builtin the register allocator makes 32 separate tiles that
+  // trade places in the loop (500 register moves and 110 spills next to its 256 MFMAs).
+  auto mfma16 = [&](f32x4& c, const u32x4& b, const u32x4& a) { asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(c) : "v"(b), "v"(a)); };
+
+  // Keeps the accumulator tiles "used" at this point of the program, so that the MFMAs producing them cannot be moved past
+  // the statement that follows.
+  auto pin_acc = [&]() {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+    for (int i = 0; i < NI; i += 2)
+      asm volatile("" : "+a"(acc[i][0]), "+a"(acc[i][1]), "+a"(acc[i][2]), "+a"(acc[i][3]), "+a"(acc[i + 1][0]), "+a"(acc[i + 1][1]),
+                   "+a"(acc[i + 1][2]), "+a"(acc[i + 1][3]));
+  };
+  // The compiler knows nothing of an MFMA in inline assembly: the wait states between the accumulators' last MFMA and their
+  // first other use, and between their zeroing and the first MFMA, are set here (4 passes and VALU writes need up to 7).
+  auto settle_acc = [&]() {
+    pin_acc();
+    asm volatile("s_nop 15" ::: "memory");
   };
   zero_acc();
-
-  // Keeps the accumulator tiles "used" at this point of the program, so that the MFMAs producing them
-  // cannot be moved past the statement that follows (they have no side effects of their own).
-#define NVF_PIN_ACC()                                                                                        \
-  do {                                                                                                       \
-    asm volatile("" : "+a"(acc[0][0]), "+a"(acc[0][1]), "+a"(acc[1][0]), "+a"(acc[1][1]));                   \
-    if constexpr (TM == 4) asm volatile("" : "+a"(acc[TM - 2][0]), "+a"(acc[TM - 2][1]), "+a"(acc[TM - 1][0]), "+a"(acc[TM - 1][1])); \
-  } while (0)
+  settle_acc();
 
   Raw cur, nxt;  // span whose odd step is converted next / span whose even step is converted next
-  Frag fr[2];
 
   // The stream runs two spans ahead of the MFMAs; with two spans per tile it is a whole tile ahead.
   const int tiles_ahead = nmac == 2 ? 2 : 1;
@@ -330,44 +344,60 @@ __global__ __launch_bounds__(512) void nvfp4_gemm_256_kernel(const Params p) {
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
 #pragma unroll
-  for (int q = 0; q < NFU; ++q) load_frag_unit(0, 0, q, fr[0]);
+  for (int j = 0; j < NJ; ++j) load_b_frag(0, 0, j);
+#pragma unroll
+  for (int m = 0; m < AHEAD; ++m) load_a_frag(0, m);
+
+  // One step: its MFMAs from LDS buffer h; between them the conversion of `src` (parity h ^ 1: the next step) into the
+  // other buffer, the fragment reads and, with `refill`, the loads of the span after the next into it.  The barrier is
+  // three rows before the end: by then every wavefront has written its share of the next step and holds this step's last
+  // fragments in registers.  Everything else is dealt out between the MFMAs in parts of a few instructions.
+  auto step = [&](auto h_c, Raw& src, auto at_barrier, auto refill_c, Raw& refill) {
+    constexpr int h = decltype(h_c)::value;
+    static_for<ROWS>([&](auto m_c) {
+      constexpr int m = decltype(m_c)::value, i = m % NI, kk = m / NI;
+      if constexpr (m == BARRIER_ROW) {
+        pin_acc();
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        at_barrier();
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      static_for<NJ>([&](auto j_c) {
+        constexpr int j = decltype(j_c)::value;
+        if constexpr (m < BARRIER_ROW) {
+          if constexpr (j == 0) load_a_frag(h, m + AHEAD);
+          if constexpr (m < NJ && j == 2) load_b_frag(h, 1, m);
+          constexpr int SLOTS = BARRIER_ROW * NJ, PARTS = 3 * NCU, slot = m * NJ + j;
+          constexpr int first = slot * PARTS / SLOTS, count = (slot + 1) * PARTS / SLOTS - first;
+          static_for<count>([&](auto part_c) {
+            constexpr int part = first + decltype(part_c)::value;
+            convert_phase(src, h ^ 1, unit_of(part / 3), part % 3, h ^ 1);
+          });
+        } else {
+          if constexpr (m == BARRIER_ROW) load_b_frag(h ^ 1, 0, j);
+          if constexpr (m == BARRIER_ROW && j == 3) load_a_frag(h ^ 1, 0);
+          if constexpr (m > BARRIER_ROW && j == 0) load_a_frag(h ^ 1, m - BARRIER_ROW);
+          if constexpr (decltype(refill_c)::value) {
+            constexpr int SLOTS = AHEAD * NJ, slot = (m - BARRIER_ROW) * NJ + j;
+            constexpr int first = slot * 8 / SLOTS, count = (slot + 1) * 8 / SLOTS - first;
+            static_for<count>([&](auto l_c) { issue_load_unit(refill, first + decltype(l_c)::value); });
+            if constexpr (slot == SLOTS - 1) advance_stream();
+          }
+        }
+        mfma16(acc[i][j], fb[kk][j], fa[m & 3]);
+        __builtin_amdgcn_sched_barrier(0);
+      });
+    });
+  };
 
   // The two in-flight spans (`cur`: its odd step is converted next, `nxt`: its even step) normally hand over by a
   // register copy at the end of every span.  With an even number of spans per tile (PAIRS) the loop body is
   // written for two spans with the names swapped in the second, which saves the 24 register-pair moves per span.
   auto span_no_copy = [&](Raw& odd_src, Raw& even_src) {
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-#pragma unroll
-      for (int kk = 0; kk < 4; ++kk) {
-        if (kk == 3) {
-          NVF_PIN_ACC();
-          asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-          __builtin_amdgcn_s_barrier();
-          asm volatile("" ::: "memory");
-        }
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int q = 0; q < NMK; ++q) {
-          const int i = q >> 1, j = q & 1;
-          const int slot_id = kk * NMK + q;
-          if (q < NFU) load_frag_unit(kk < 3 ? h : (h ^ 1), (kk + 1) & 3, q, fr[(kk + 1) & 1]);
-          if (kk < 3) {
-#pragma unroll
-            for (int part = slot_id * NCU / NMK; part < (slot_id + 1) * NCU / NMK; ++part)
-              convert_phase(h ? even_src : odd_src, h ^ 1, unit_of(part / 3), part % 3, h ^ 1);
-          }
-          if (kk == 3 && h == 1) {  // odd_src is dead: it takes the span after even_src
-#pragma unroll
-            for (int l = q * 8 / NMK; l < (q + 1) * 8 / NMK; ++l) issue_load_unit(odd_src, l);
-            if (q == NMK - 1) advance_stream();
-          }
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, fr[kk & 1].b[j]),
-                                                             __builtin_bit_cast(f16x8, fr[kk & 1].a[i]), acc[i][j], 0, 0, 0);
-          __builtin_amdgcn_sched_barrier(0);
-        }
-      }
-    }
+    step(std::integral_constant<int, 0>{}, odd_src, [] {}, std::false_type{}, odd_src);
+    step(std::integral_constant<int, 1>{}, even_src, [] {}, std::true_type{}, odd_src);  // odd_src is dead from the barrier on: it takes the span after even_src
   };
   for (int c_tile = first_tile; c_tile < range_end; c_tile += slots) {
     np = ptrs_or_current(c_tile + tiles_ahead * slots);
@@ -378,77 +408,42 @@ __global__ __launch_bounds__(512) void nvfp4_gemm_256_kernel(const Params p) {
       }
     } else {
       for (int c_mac = 0; c_mac < nmac; ++c_mac) {
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {  // step g = 2*c_mac + h computes from LDS buffer h
-          // h == 0: the odd step of the current span is converted into buffer 1
-          // h == 1: the even step of the next span is converted into buffer 0; then that span becomes the
-          //         current one and the span after it is requested
-#pragma unroll
-          for (int kk = 0; kk < 4; ++kk) {
-            if (kk == 3) {
-              // every wave has written its share of step g+1 and read the last fragments of step g
-              NVF_PIN_ACC();
-              asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-              __builtin_amdgcn_s_barrier();
-              asm volatile("" ::: "memory");
-              if (h == 1) cur = nxt;
-            }
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int q = 0; q < NMK; ++q) {
-              const int i = q >> 1, j = q & 1;
-              const int slot_id = kk * NMK + q;  // 3 * NMK slots for the 3 * NCU conversion parts of the step
-              if (q < NFU) load_frag_unit(kk < 3 ? h : (h ^ 1), (kk + 1) & 3, q, fr[(kk + 1) & 1]);
-              if (kk < 3) {
-#pragma unroll
-                for (int part = slot_id * NCU / NMK; part < (slot_id + 1) * NCU / NMK; ++part)
-                  convert_phase(h ? nxt : cur, h ^ 1, unit_of(part / 3), part % 3, h ^ 1);
-              }
-              if (kk == 3 && h == 1) {
-#pragma unroll
-                for (int l = q * 8 / NMK; l < (q + 1) * 8 / NMK; ++l) issue_load_unit(nxt, l);
-                if (q == NMK - 1) advance_stream();
-              }
-              acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, fr[kk & 1].b[j]),
-                                                                 __builtin_bit_cast(f16x8, fr[kk & 1].a[i]), acc[i][j], 0, 0, 0);
-              __builtin_amdgcn_sched_barrier(0);
-            }
-          }
-        }
+// step 2*c_mac + h computes from LDS buffer h.
+        // h == 0: the odd step of the current span is converted into buffer 1
+        // h == 1: the even step of the next span is converted into buffer 0; then that span becomes the
+        //         current one and the span after it is requested
+        step(std::integral_constant<int, 0>{}, cur, [] {}, std::false_type{}, cur);
+        step(std::integral_constant<int, 1>{}, nxt, [&] { cur = nxt; }, std::true_type{}, nxt);
       }
     }
     // ---- epilogue; the next tile's first step is already in LDS.
-    // acc[i][j][r] = C[m = li][n = (r/4)*8 + lg*4 + r%4] of its 32x32 sub-tile.
+    settle_acc();
+    // acc[i][j][e] = C[m = 16 i + r16][n = 16 j + 4 g4 + e] of the wavefront's tile.
     const Where cw = tile_where(c_tile);
     const float alpha = p.alpha[cw.g];
     if constexpr (OUT_FP4) {
-      // Block-scaled result.  A wavefront's 32 x 64 block i is quantized tile by tile (quantize_acc_tile), its 32 rows
-      // x 32 payload bytes are collected in a private piece of LDS (pitch 48 bytes) and leave as 16 bytes per lane,
-      // two lanes to a row; the four scale codes of a row (its four 16-column blocks are one dword of the 128x4
-      // layout) are kept per i and stored once at the end: 16 bytes per row for the 128 rows of a 256-row tile's
-      // wavefront (they are one whole 128x4 scale tile), 8 bytes for the 64 rows of a 128-row tile's.
+      // Block-scaled result.  A wavefront's 32 x 64 block i is quantized 16 rows at a time, its 32 rows x 32 payload bytes
+      // are collected in a private piece of LDS (pitch 48 bytes) and leave as 16 bytes per lane, two lanes to a row; the
+      // scale codes are collected there in the order of the 128x4 layout and leave at the end: 16 bytes per row for the 128
+      // rows of a 256-row tile's wavefront (they are one whole 128x4 scale tile), 8 bytes for the 64 rows of a 128-row tile's.
       const float gs = p.gnorm[0], decode = 1.0f / gs;
       int elane = lane;
       asm volatile("" : "+v"(elane));
       uint8_t* stage = reinterpret_cast<uint8_t*>(lds + 2 * BUF_UNITS) + wave * 2560;
-      uint8_t* wr = stage + (elane & 31) * 48 + (elane >> 5) * 2;
+      uint8_t* wr = stage + (elane & 15) * 48 + (elane >> 4) * 2;
       const uint8_t* rd = stage + (elane >> 1) * 48 + (elane & 1) * 16;
       const int64_t opitch = p.n >> 1;
       uint8_t* obase = static_cast<uint8_t*>(p.out) + (cw.m0 + wm * (32 * TM) + (elane >> 1)) * opitch + ((cw.n0 + wn * 64) >> 1) + (elane & 1) * 16;
-      uint32_t sfw[TM];
+      uint8_t* const codes = stage + 1536;  // of rows 32 c + q: 16 bytes per q, word c, one byte per block
 #pragma unroll
       for (int i = 0; i < TM; ++i) {
-        sfw[i] = 0;
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          uint32_t h[2], q8[2];
-          quantize_acc_tile(acc[i][j], alpha, gs, decode, true, h, q8);
+        for (int i2 = 0; i2 < 2; ++i2) {
+          uint32_t q8, h[NJ];
+          quantize_acc_tiles16(acc[2 * i + i2], alpha, gs, decode, q8, h);
 #pragma unroll
-          for (int b = 0; b < 2; ++b) {
-            *reinterpret_cast<uint16_t*>(wr + j * 16 + b * 8) = (uint16_t)(h[b] & 0xffffu);
-            *reinterpret_cast<uint16_t*>(wr + j * 16 + b * 8 + 4) = (uint16_t)(h[b] >> 16);
-          }
-          sfw[i] |= (q8[0] | (q8[1] << 8)) << (16 * j);
+          for (int j = 0; j < NJ; ++j) *reinterpret_cast<uint16_t*>(wr + i2 * 768 + j * 8) = (uint16_t)h[j];
+          codes[(i2 * 16 + (elane & 15)) * 16 + i * 4 + (elane >> 4)] = (uint8_t)q8;
         }
         asm volatile("" ::: "memory");  // the read below sees the writes above: one wavefront's LDS accesses stay in order
         const u32x4 v = *reinterpret_cast<const u32x4*>(rd);
@@ -457,38 +452,36 @@ __global__ __launch_bounds__(512) void nvfp4_gemm_256_kernel(const Params p) {
       }
       // (RAGGED_M: the rows past M read as zero, so their scale codes are zero - exactly what the padding rows of the
       // last 128-row scale tile must hold; a 256-row tile with at most 128 rows has no second scale tile to write)
-      if (lg == 0 && (!RAGGED_M || TM == 2 || wm * 128 < cw.valid)) {
+      if (elane < 32 && (!RAGGED_M || TM == 2 || wm * 128 < cw.valid)) {
         const int sf_cols4 = p.n >> 6;  // 512-byte scale tiles per 128 rows (N % 256 == 0: no padding columns)
-        uint8_t* sfp = p.out_sf + ((cw.m0 >> 7) * (int64_t)sf_cols4 + ((cw.n0 + wn * 64) >> 6)) * 512 + li * 16;
-        if constexpr (TM == 4) *reinterpret_cast<u32x4*>(sfp + (int64_t)wm * sf_cols4 * 512) = u32x4{sfw[0], sfw[1], sfw[2], sfw[3]};
-        else *reinterpret_cast<u32x2*>(sfp + wm * 8) = u32x2{sfw[0], sfw[1]};
+        uint8_t* sfp = p.out_sf + ((cw.m0 >> 7) * (int64_t)sf_cols4 + ((cw.n0 + wn * 64) >> 6)) * 512 + elane * 16;
+        if constexpr (TM == 4) *reinterpret_cast<u32x4*>(sfp + (int64_t)wm * sf_cols4 * 512) = *reinterpret_cast<const u32x4*>(codes + elane * 16);
+        else *reinterpret_cast<u32x2*>(sfp + wm * 8) = *reinterpret_cast<const u32x2*>(codes + elane * 16);
       }
     } else if constexpr (OUT_F32) {
       // as below, with 32x16 blocks of fp32 (64-byte row segments)
       int elane = lane;
       asm volatile("" : "+v"(elane));
       uint8_t* stage = reinterpret_cast<uint8_t*>(lds + 2 * BUF_UNITS) + wave * 2560;
-      uint8_t* wr = stage + (elane & 31) * 80 + (elane >> 5) * 16;
+      uint8_t* wr = stage + (elane & 15) * 80 + (elane >> 4) * 16;
       const uint8_t* rd = stage + (elane >> 2) * 80 + (elane & 3) * 16;
       const uint32_t ooff = ((uint32_t)(elane >> 2) * (uint32_t)p.n + (uint32_t)(elane & 3) * 4u) * 4u;
       uint8_t* obase = reinterpret_cast<uint8_t*>(static_cast<float*>(p.out) + (cw.m0 + wm * (32 * TM)) * p.n + cw.n0 + wn * 64);
 #pragma unroll
       for (int i = 0; i < TM; ++i) {
 #pragma unroll
-        for (int jh = 0; jh < 4; ++jh) {  // 16 columns: block j = jh / 2, its rq pair jh % 2
-          const int j = jh >> 1;
+        for (int j = 0; j < NJ; ++j) {  // 16 columns
 #pragma unroll
-          for (int r2 = 0; r2 < 2; ++r2) {
-            const int rq = (jh & 1) * 2 + r2;
-            *reinterpret_cast<f32x4*>(wr + r2 * 32) = f32x4{acc[i][j][rq * 4 + 0] * alpha, acc[i][j][rq * 4 + 1] * alpha,
-                                                            acc[i][j][rq * 4 + 2] * alpha, acc[i][j][rq * 4 + 3] * alpha};
+          for (int i2 = 0; i2 < 2; ++i2) {
+            const f32x4 c = acc[2 * i + i2][j];
+            *reinterpret_cast<f32x4*>(wr + i2 * 1280) = f32x4{c[0] * alpha, c[1] * alpha, c[2] * alpha, c[3] * alpha};
           }
           asm volatile("" ::: "memory");  // one wavefront's LDS accesses stay in order
 #pragma unroll
           for (int t = 0; t < 2; ++t) {
             const f32x4 v = *reinterpret_cast<const f32x4*>(rd + t * 1280);
             if (!RAGGED_M || wm * (32 * TM) + i * 32 + 16 * t + (elane >> 2) < cw.valid)
-              *reinterpret_cast<f32x4*>(obase + ((int64_t)(i * 32 + 16 * t) * p.n + jh * 16) * 4 + ooff) = v;
+              *reinterpret_cast<f32x4*>(obase + ((int64_t)(i * 32 + 16 * t) * p.n + j * 16) * 4 + ooff) = v;
           }
           asm volatile("" ::: "memory");
         }
@@ -504,7 +497,7 @@ __global__ __launch_bounds__(512) void nvfp4_gemm_256_kernel(const Params p) {
       int elane = lane;
       asm volatile("" : "+v"(elane));
       uint8_t* stage = reinterpret_cast<uint8_t*>(lds + 2 * BUF_UNITS) + wave * 2560;
-      uint8_t* wr = stage + (elane & 31) * 80 + (elane >> 5) * 8;
+      uint8_t* wr = stage + (elane & 15) * 80 + (elane >> 4) * 8;
       const uint8_t* rd = stage + (elane >> 2) * 80 + (elane & 3) * 16;
       const int ldc = p.out_pitch();
       const uint32_t ooff = ((uint32_t)(elane >> 2) * (uint32_t)ldc + (uint32_t)(elane & 3) * 8u) * 2u;
@@ -515,11 +508,12 @@ __global__ __launch_bounds__(512) void nvfp4_gemm_256_kernel(const Params p) {
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
 #pragma unroll
-          for (int rq = 0; rq < 4; ++rq) {
+          for (int t = 0; t < 4; ++t) {  // the block's four 16x16 tiles
+            const f32x4 c = acc[2 * i + (t >> 1)][2 * j + (t & 1)];
             u32x2 v;
-            v[0] = pack2(acc[i][j][rq * 4 + 0] * alpha, acc[i][j][rq * 4 + 1] * alpha, OUT_BF16);
-            v[1] = pack2(acc[i][j][rq * 4 + 2] * alpha, acc[i][j][rq * 4 + 3] * alpha, OUT_BF16);
-            *reinterpret_cast<u32x2*>(wr + rq * 16) = v;
+            v[0] = pack2(c[0] * alpha, c[1] * alpha, OUT_BF16);
+            v[1] = pack2(c[2] * alpha, c[3] * alpha, OUT_BF16);
+            *reinterpret_cast<u32x2*>(wr + (t >> 1) * 1280 + (t & 1) * 32) = v;
           }
           asm volatile("" ::: "memory");  // the reads below see the writes above: one wavefront's LDS accesses stay in order
 #pragma unroll
@@ -534,8 +528,8 @@ __global__ __launch_bounds__(512) void nvfp4_gemm_256_kernel(const Params p) {
       }
     }
     zero_acc();
+    settle_acc();
   }
-#undef NVF_PIN_ACC
 }
 
 template <bool OUT_BF16, bool GROUPED, int TM, bool OUT_F32, bool PAIRS, bool OUT_FP4 = false, bool RAGGED_K = false, bool RAGGED_M = false>

@@ -38,3 +38,47 @@ def test_a_write_of_m0_is_a_wait_state_before_the_lds_direct_load_that_uses_it(t
             early += written
         written = name.startswith("s_") and operands.startswith("m0,")
     assert loads > 0 and early == 0, f"{early} of {loads} LDS-direct loads follow the write of m0 at once"
+
+
+def _registers(operand):
+    """The vector registers that an operand names, as (file, number)."""
+    out = []
+    for kind, first, last, single in re.findall(r"\b([va])(?:\[(\d+):(\d+)\]|(\d+)\b)", operand):
+        out += [(kind, n) for n in range(int(first or single), int(last or single) + 1)]
+    return out
+
+
+@pytest.mark.skipif(OBJDUMP is None, reason="llvm-objdump not found")
+def test_mfmas_keep_their_distance_from_vector_instructions(tmp_path):
+    """An MFMA may read a register two wait states after a vector ALU instruction has written it, and other instructions may
+    touch a 16x16 MFMA's result 8 (16-bit operands, K = 32) or 12 (e4m3, K = 128) wait states after its issue: what the
+    compiler keeps between the ones that it knows.  The MFMAs that are written in inline assembly have to keep it by
+    themselves."""
+    import fuser_amd
+
+    settle = {"v_mfma_f32_16x16x32": 8, "v_mfma_scale_f32_16x16x128": 12}
+    mfmas, early = 0, []
+    now, written, results = 0, {}, {}  # registers and when a vector ALU instruction wrote them / an MFMA's result may be used
+    for name, operands in _instructions(Path(fuser_amd.__file__).parent / "libnvf_hip.so", tmp_path):
+        if name == "s_nop":
+            now += int(operands, 0) + 1
+            continue
+        now += 1
+        if name in ("s_endpgm", "s_branch", "s_setpc_b64"):
+            written.clear(), results.clear()
+        elif "mfma" in name:
+            parts = re.split(r",\s*(?![^\[]*\])", operands)
+            mfmas += 1
+            early += [f"{name} {operands}" for part in parts[1:] for r in _registers(part) if now - written.get(r, -9) <= 2]
+            for prefix, states in settle.items():
+                if name.startswith(prefix):
+                    results.update({r: now + states for r in _registers(parts[0])})
+        elif name.startswith(("v_", "ds_", "global_", "buffer_", "scratch_", "flat_")):
+            if results:
+                early += [f"{name} {operands}" for r in _registers(operands) if results.get(r, -9) >= now]
+            if name.startswith("v_"):
+                dest = operands if "swap" in name else re.split(r",\s*(?![^\[]*\])", operands)[0]
+                written.update({r: now for r in _registers(dest)})
+        if now % 64 == 0:
+            results = {r: t for r, t in results.items() if t >= now}
+    assert mfmas > 1000 and not early, f"{len(early)} instructions too early, e.g. {early[:3]}"
