@@ -1,7 +1,8 @@
 // mxfp8_scaled_mm for gfx950 (cutlass/mxfp8_scaled_mm.cu:290-319): C = alpha * A * B^T with e4m3
-// operands and one e8m0 scale per 32 K-elements, on v_mfma_scale_f32_32x32x64_f8f6f4.
+// operands and one e8m0 scale per 32 K-elements, on v_mfma_scale_f32_16x16x128_f8f6f4 (256x256 tiles, weight-streaming kernel)
+// and v_mfma_scale_f32_32x32x64_f8f6f4 (the others).
 //
-// Operand layout of the instruction (fp8 x fp8), measured on hardware:
+// Operand layout of the latter (fp8 x fp8), measured on hardware:
 //   lane l = i + 32*g (i = row of A / column of B, g in {0,1}) supplies 32 bytes:
 //     bytes  0..15 = K [16g,      16g + 16)
 //     bytes 16..31 = K [32 + 16g, 32 + 16g + 16)
@@ -11,6 +12,7 @@
 // scale a 128-row wave tile needs for a 128-deep K step.
 #include "lds_direct.h"
 #include "nvf_internal.h"
+#include "tile256_loop.h"
 
 namespace nvf {
 namespace {
@@ -213,7 +215,271 @@ __global__ __launch_bounds__(256) void mxfp8_gemm_kernel(const Params p) {
 
 
 // -------------------------------------------------------------------------------------------------
-// Fast path: 256x256 or 128x256 tile, M % 256 (128) == N % 256 == K % 128 == 0.
+// Persistent kernels: 256x256 or 128x256 tiles, N % 256 == 0, K % 32 == 0, K >= 256.
+// -------------------------------------------------------------------------------------------------
+
+// The walk over the tiles.  Workgroup ids are dealt round-robin to the 8 XCDs, so XCD x owns the contiguous tile range
+// [x*chunk, (x+1)*chunk) and its workgroups take consecutive tiles of it in each round: with the 8 (m) x 4 (n) blocked tile
+// numbering, the 32 tiles an XCD works on at any time share 8 A panels and 4 B panels in that XCD's L2.
+// RAGGED_M: the last row tile holds fewer than BM rows (kernels of their own: clamping the row of every activation
+// load costs the others time).  Its missing rows load the last row again and are not stored; the scale layout is
+// padded to 128 rows, so only a 256-row tile can ask for a scale tile that does not exist (it takes an existing one).
+template <int BM, bool RAGGED_M>
+struct TileWalk {
+  int tiles_m, tiles_n, first, end, slots, bulk_tiles;
+  bool blocked;
+  __device__ __forceinline__ explicit TileWalk(const Params& p) {
+    tiles_m = RAGGED_M ? (p.m + BM - 1) / BM : p.m / BM;
+    tiles_n = p.n / 256;
+    const int total = tiles_m * tiles_n, chunk = (total + 7) >> 3;
+    const int xcd = blockIdx.x & 7;
+    slots = gridDim.x >> 3;
+    first = xcd * chunk + (blockIdx.x >> 3);
+    end = min((xcd + 1) * chunk, total);
+    // (n-tiles past the last multiple of 4: blocks of 8 (m) x 1..3 (n) after all the others; 8192 x 29440 x 8192, 115
+    // n-tiles: 2.33 -> 2.7 PFLOP/s against the plain m-major order)
+    blocked = (tiles_m & 7) == 0 && tiles_n >= 4;
+    bulk_tiles = tiles_m * (tiles_n & ~3);
+  }
+  __device__ __forceinline__ void coords(int t, int& m0, int& n0) const {
+    int mt, nt;
+    if (blocked && t < bulk_tiles) {
+      const int sb = t >> 5, w = t & 31;
+      mt = (sb % (tiles_m >> 3)) * 8 + (w & 7);
+      nt = (sb / (tiles_m >> 3)) * 4 + (w >> 3);
+    } else if (blocked) {
+      const int u = t - bulk_tiles, bs = 8 * (tiles_n & 3), sb = u / bs, w = u - sb * bs;
+      mt = sb * 8 + (w & 7);
+      nt = (tiles_n & ~3) + (w >> 3);
+    } else {
+      mt = t % tiles_m;
+      nt = t / tiles_m;
+    }
+    m0 = mt * BM;
+    n0 = nt * 256;
+  }
+};
+
+// RAGGED_K: K is a multiple of 32 but not of 128.  The last K step of a tile then holds K % 128 elements per row: the
+// lanes whose 16 bytes lie past the end of the row load the row's last ones again, and the scale bytes of the blocks past K
+// are replaced by 2^-127 in both operands: what such a lane multiplies is the row's own data (a NaN among them has made the
+// row's results NaN already) times 2^-254, below the smallest fp32 number, so that the step adds exact zeros.  No branch in
+// the K loop: with the lanes' loads predicated and zeros written instead, every load of every step was a block of code of
+// its own (1024 x 5632 x 2880: 31.2 us, against 24.3 for K = 2816; now 29.6 us).
+
+// 256x256 tiles, bound by the power limit of the MFMAs: 8192^3 2.93 PFLOP/s, 394 -> 376 us against the 128x256 kernel's K loop
+// with 256 rows (32x32 MFMAs, all of a step's loads in one half of it); 2000 x 8192 x 8192 104 -> 95 us, 8100 x 8192 x 2880
+// 178 -> 163, 2048 x 14336 x 4096 102 -> 100, 16384 x 16384 x 1024 291 -> 279.
+// The K loop is Tile256Loop's.  The scales of a step travel like its operands: 2 KiB of 128x4 tiles (two of A,
+// two of B) by LDS-direct loads, of which every wavefront reads the 16-byte pieces of its rows and keeps its lane group's byte.
+template <bool OUT_BF16, bool STREAM_OUT, bool RAGGED_K, bool RAGGED_M>
+__global__ __launch_bounds__(256, 1) void mxfp8_tile256_kernel(const Params p) {
+  constexpr int BM = 256;
+  constexpr int kScaleBytes = 2048;  // of a step: [operand][128-row tile][row % 32][16]
+  extern __shared__ u32x4 lds[];     // operand tiles | scales of two steps | the epilogue's 18 KiB
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave >> 1, wn = wave & 1;
+  const TileWalk<BM, RAGGED_M> walk(p);
+  if (walk.first >= walk.end) return;
+  const int nk = (p.k + 127) >> 7;
+  const int sf_tiles_k = ((p.k >> 5) + 3) >> 2;  // 512-byte scale tiles per 128-row tile
+  const int k_tail = p.k & 127;                  // elements of the last step (RAGGED_K: 32, 64 or 96)
+
+  // ---- LDS-direct loads of a step.  Load u < 4: 8 rows of A's tiles 0..3 of a wavefront (rows 0..63 of either half of the
+  // tile), u = 4..11: 8 rows of B, u = 12..15: 8 rows of A's tiles 4..7; lane L lands at unit +L, i.e. row +(L>>3), chunk
+  // position L&7, which must hold global chunk (L&7) ^ ((row>>1)&7) = (L&7) ^ ((L>>4) | ((u&1)<<2)).  u = 16: the scales of A
+  // (even wavefronts) or B (odd ones), lanes 0..31 the first 128-row tile's, lanes 32..63 the second's.
+  const uint32_t lds_base = (uint32_t)(uintptr_t)((__attribute__((address_space(3))) void*)lds);
+  const uint32_t chunk_even = (uint32_t)((lane & 7) ^ (lane >> 4)), chunk_odd = chunk_even ^ 4u;
+  const int a_row0 = wm * 128 + wn * 32, b_row0 = wave * 64;  // the wavefront's share (A: and 64 rows further on)
+  const uint32_t a_lds = lds_base + (uint32_t)a_row0 * 128u, b_lds = lds_base + 65536u + (uint32_t)b_row0 * 128u;
+  const uint32_t s_lds = lds_base + kTile256Bytes + (uint32_t)wn * 1024u;
+  uint32_t a_off[8], b_off[8], s_off;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) b_off[j] = (uint32_t)(b_row0 + 8 * j + (lane >> 3)) * (uint32_t)p.k + ((j & 1) ? chunk_odd : chunk_even) * 16u;
+  // RAGGED_K: what takes an offset to the row's last chunk in the last step, where the lane's is past it
+  const uint32_t last_chunk = (uint32_t)(k_tail >> 4) - 1u;
+  const uint32_t tail_even = (min(chunk_even, last_chunk) - chunk_even) * 16u, tail_odd = (min(chunk_odd, last_chunk) - chunk_odd) * 16u;
+  uint32_t sub_even = 0, sub_odd = 0;
+
+  // ---- load stream: the step the next loads are issued for (l_ks of the tile lp), and the tile after it
+  struct TilePtrs { const uint8_t *a, *b, *s; int valid; };
+  auto tile_ptrs = [&](int t) {
+    int m0, n0;
+    walk.coords(t, m0, n0);
+    TilePtrs r;
+    r.a = p.a + (int64_t)m0 * p.k;
+    r.b = p.b + (int64_t)n0 * p.k;
+    r.s = wn ? p.sfb + (int64_t)(n0 >> 7) * sf_tiles_k * 512 : p.sfa + (int64_t)(m0 >> 7) * sf_tiles_k * 512;
+    r.valid = p.m - m0;  // rows of the tile that exist (RAGGED_M: possibly fewer than BM)
+    return r;
+  };
+  TilePtrs lp = tile_ptrs(walk.first), np = lp;
+  int l_ks = 0;
+  uint32_t l_buf = 0, l_sbuf = 0;  // of the step's buffer
+  auto enter_tile = [&]() {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      uint32_t row = (uint32_t)(a_row0 + 64 * (j >> 2) + 8 * (j & 3) + (lane >> 3));
+      if (RAGGED_M) row = min(row, (uint32_t)(lp.valid - 1));
+      a_off[j] = row * (uint32_t)p.k + ((j & 1) ? chunk_odd : chunk_even) * 16u;
+    }
+    s_off = (uint32_t)(lane & 31) * 16u + (lane >= 32 && (!RAGGED_M || wn || lp.valid > 128) ? (uint32_t)sf_tiles_k * 512u : 0u);
+  };
+  enter_tile();
+  auto load = [&](auto u_c) {
+    constexpr int u = decltype(u_c)::value;
+    if constexpr (u == 16) {
+      lds_dma16(s_lds + l_sbuf, lp.s, s_off);
+    } else {
+      constexpr int j = u < 4 ? u : u < 12 ? u - 4 : u - 8;
+      const uint32_t sub = RAGGED_K ? ((j & 1) ? sub_odd : sub_even) : 0u;
+      if constexpr (u >= 4 && u < 12) lds_dma16<j * 1024>(b_lds + l_buf, lp.b, b_off[j] + sub);
+      else lds_dma16<(j >> 2) * 8192 + (j & 3) * 1024>(a_lds + l_buf, lp.a, a_off[j] + sub);
+    }
+  };
+  auto advance = [&]() {
+    l_buf ^= 32768u;
+    l_sbuf ^= (uint32_t)kScaleBytes;
+    lp.a += 128;
+    lp.b += 128;
+    lp.s += 512;
+    ++l_ks;
+    if (RAGGED_K) {
+      sub_even = l_ks == nk - 1 ? tail_even : 0u;
+      sub_odd = l_ks == nk - 1 ? tail_odd : 0u;
+    }
+    if (l_ks == nk) {
+      l_ks = 0;
+      lp = np;
+      if (RAGGED_M) enter_tile();
+    }
+  };
+
+  Tile256Loop<Mma::kMxFp8> loop;
+  loop.init(lds_base, lane, wm, wn);
+
+  // ---- scales of the next step: the lane's rows r (even tiles) and 16 + r (odd ones) of its 128-row tile, whose 16 bytes are
+  // 4 words for the rows 32 apart; byte g of each is the lane group's, and the four are one operand register
+  uint32_t s_rd[2];
+  u32x4 words[2][2];
+  uint32_t next_s[2][2];  // [operand][even, odd tiles]
+  {
+    const uint32_t at = lds_base + kTile256Bytes + (uint32_t)(lane & 15) * 16u;
+    s_rd[0] = at + (uint32_t)wm * 512u;
+    s_rd[1] = at + 1024u + (uint32_t)wn * 512u;
+  }
+  const uint32_t g = (uint32_t)lane >> 4, pick_low = 0x0c0c0400u + g * 0x0101u, pick_high = 0x04000c0cu + g * 0x01010000u;
+  const uint32_t tail_keep = (int)g * 32 < k_tail ? 0xffffffffu : 0u;  // RAGGED_K: the lane group's block exists in the last step
+  uint32_t c_sbuf = 0;  // buffer of the scales to be read
+  auto read_scales = [&]() {
+#pragma unroll
+    for (int op = 0; op < 2; ++op)
+#pragma unroll
+      for (int o = 0; o < 2; ++o) words[op][o] = loop.lds_read(s_rd[op] + c_sbuf + o * 256u);
+    c_sbuf ^= (uint32_t)kScaleBytes;
+  };
+  auto combine_scales = [&](int op, bool tail) {
+#pragma unroll
+    for (int o = 0; o < 2; ++o) {
+      const u32x4 w = words[op][o];
+      next_s[op][o] = __builtin_amdgcn_perm(w[1], w[0], pick_low) | __builtin_amdgcn_perm(w[3], w[2], pick_high);
+      if (RAGGED_K && tail) next_s[op][o] &= tail_keep;
+    }
+  };
+  auto take_scales = [&]() {
+#pragma unroll
+    for (int o = 0; o < 2; ++o) {
+      loop.sa[o] = next_s[0][o];
+      loop.sb[o] = next_s[1][o];
+    }
+    // two wait states between the registers' writing and the first MFMA
+    asm volatile("s_nop 1" : "+v"(loop.sa[0]), "+v"(loop.sa[1]), "+v"(loop.sb[0]), "+v"(loop.sb[1]));
+  };
+
+  // The stream runs two steps ahead of the MFMAs; with two steps per tile it is a whole tile ahead and
+  // already leaves the first tile during this prologue.
+  const int tiles_ahead = nk == 2 ? 2 : 1;
+  np = (walk.first + walk.slots < walk.end) ? tile_ptrs(walk.first + walk.slots) : lp;
+  const TilePtrs first_lp = lp;
+  static_for<17>(load);  // step 0
+  advance();
+  static_for<17>(load);  // step 1
+  advance();
+  loop.template fence<17>();
+  loop.first_fragments();
+  read_scales();
+  combine_scales(0, false);
+  combine_scales(1, false);
+  take_scales();
+
+  const float alpha = p.alpha[0];
+  for (int c_tile = walk.first; c_tile < walk.end; c_tile += walk.slots) {
+    // the tile the stream enters next (past the end of the list: a valid one, loaded and ignored)
+    np = (c_tile + tiles_ahead * walk.slots < walk.end) ? tile_ptrs(c_tile + tiles_ahead * walk.slots) : first_lp;
+    auto step = [&](auto first, int c_ks) {
+      loop.template step<17, decltype(first)::value>(load, [&](auto part) {
+        if constexpr (decltype(part)::value == 0) read_scales();
+        if constexpr (decltype(part)::value == 1) combine_scales(0, c_ks + 2 == nk);
+        if constexpr (decltype(part)::value == 2) combine_scales(1, c_ks + 2 == nk);
+      });
+      take_scales();
+      advance();
+    };
+    step(std::true_type{}, 0);
+    for (int c_ks = 1; c_ks < nk; ++c_ks) step(std::false_type{}, c_ks);
+    loop.settle();
+    // ---- epilogue of this tile; the loads of the next tile's first two steps are already in flight.
+    // A lane holds 8-byte pieces of 16 rows per tile; stored like that, a tile is 8192 sixteen-byte write
+    // requests per compute unit and the L2 takes longer over them than over a whole K step of MFMAs.  Every
+    // 32x64 block of the wavefront's tile is therefore turned round in a private 4.5 KiB of LDS (32 rows of 128
+    // bytes at a pitch of 144 bytes) and leaves in 16-byte pieces, 8 lanes to a row's 128 bytes.  One LDS address
+    // each for writing and reading (the rest are immediate offsets) and one 32-bit lane offset next to a
+    // wave-uniform result address; the lane number passes through an empty asm statement so that they are worked
+    // out here, after the K loop.
+    int m0, n0;
+    walk.coords(c_tile, m0, n0);
+    int elane = lane;
+    asm volatile("" : "+v"(elane));
+    uint8_t* stage = reinterpret_cast<uint8_t*>(lds) + kTile256Bytes + 2 * kScaleBytes + wave * 4608;
+    uint8_t* wr = stage + (elane & 15) * 144 + (elane >> 4) * 8;
+    const uint8_t* rd = stage + (elane >> 3) * 144 + (elane & 7) * 16;
+    const int ldc = p.out_pitch();
+    const uint32_t ooff = ((uint32_t)(elane >> 3) * (uint32_t)ldc + (uint32_t)(elane & 7) * 8u) * 2u;
+    uint8_t* obase = reinterpret_cast<uint8_t*>(static_cast<uint16_t*>(p.out) + (int64_t)(m0 + wm * 128) * ldc + n0 + wn * 128);
+    const int rows_left = p.m - m0 - wm * 128 - (elane >> 3);  // RAGGED_M: rows from this lane's first one to the end
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+#pragma unroll
+      for (int jh = 0; jh < 2; ++jh) {
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {  // the block's 2 x 4 tiles
+          const f32x4 c = loop.acc[2 * i + (t >> 2)][4 * jh + (t & 3)];
+          u32x2 v;
+          v[0] = pack2(c[0] * alpha, c[1] * alpha, OUT_BF16);
+          v[1] = pack2(c[2] * alpha, c[3] * alpha, OUT_BF16);
+          *reinterpret_cast<u32x2*>(wr + (t >> 2) * 2304 + (t & 3) * 32) = v;
+        }
+        asm volatile("" ::: "memory");  // the reads below see the writes above: one wavefront's LDS accesses stay in order
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          const u32x4 v = *reinterpret_cast<const u32x4*>(rd + t * 1152);
+          u32x4* dst = reinterpret_cast<u32x4*>(obase + ((int64_t)(i * 32 + 8 * t) * ldc + jh * 64) * 2 + ooff);
+          if (RAGGED_M && i * 32 + 8 * t >= rows_left) continue;
+          if constexpr (STREAM_OUT) __builtin_nontemporal_store(v, dst);
+          else *dst = v;
+        }
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);  // (the next block's results stay in the accumulators until then)
+      }
+    }
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no LDS-direct load may outlive the workgroup
+}
+
+// 128x256 tiles, for shapes whose 256x256 tiles would leave compute units idle:
 //   * Tiles travel global -> LDS with 16-byte LDS-direct loads (no staging registers) into a double
 //     buffer.  They are issued from inline assembly so that the compiler does not serialise them
 //     against the LDS reads of the other buffer; completion is enforced by the explicit
@@ -228,15 +494,6 @@ __global__ __launch_bounds__(256) void mxfp8_gemm_kernel(const Params p) {
 // -------------------------------------------------------------------------------------------------
 __device__ __forceinline__ int lds_pos2(int row, int chunk) { return row * 8 + (chunk ^ ((row >> 1) & 7)); }
 
-// TM = 32-row accumulator tiles of a wavefront along M: 4 -> 256x256 workgroup tile, 2 -> 128x256 (for shapes
-// whose 256x256 tiles would leave compute units idle).  The statement order for TM = 4 is the one the 8192^3
-// measurements were made with.
-// RAGGED_K: K is a multiple of 32 but not of 128.  The last K step of a tile then holds K % 128 elements per row: the
-// lanes whose 16 bytes lie past the end of the row load the row's last ones again, and the scale bytes of the blocks past K
-// are replaced by 2^-127 in both operands: what such a lane multiplies is the row's own data (a NaN among them has made the
-// row's results NaN already) times 2^-254, below the smallest fp32 number, so that the step adds exact zeros.  No branch in
-// the K loop: with the lanes' loads predicated and zeros written instead, every load of every step was a block of code of
-// its own (1024 x 5632 x 2880: 31.2 us, against 24.3 for K = 2816; now 29.6 us).
 template <int TM, bool OUT_BF16, bool STREAM_OUT, bool RAGGED_K = false, bool RAGGED_M = false>
 __global__ __launch_bounds__(256, 1) void mxfp8_gemm_256_kernel(const Params p) {
   constexpr int BM = 64 * TM, BN = 256;
@@ -254,41 +511,10 @@ __global__ __launch_bounds__(256, 1) void mxfp8_gemm_256_kernel(const Params p) 
   const int wm = wave >> 1, wn = wave & 1;
   const int li = lane & 31, lg = lane >> 5;
 
-  // ---- persistent tile walk.  Workgroup ids are dealt round-robin to the 8 XCDs, so XCD x owns the
-  // contiguous tile range [x*chunk, (x+1)*chunk) and its workgroups take consecutive tiles of it in
-  // each round: with the 8 (m) x 4 (n) blocked tile numbering below, the 32 tiles an XCD works on at
-  // any time share 8 A panels and 4 B panels in that XCD's L2.
-  // RAGGED_M: the last row tile holds fewer than BM rows (a kernel of its own: clamping the row of every activation
-  // load costs the others time).  Its missing rows load the last row again and are not stored; the scale layout is
-  // padded to 128 rows, so only a 256-row tile can ask for a scale tile that does not exist (it takes the last one).
-  const int tiles_m = RAGGED_M ? (p.m + BM - 1) / BM : p.m / BM, tiles_n = p.n / BN;
-  const int total = tiles_m * tiles_n;
-  const int chunk_tiles = (total + 7) >> 3;
-  const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3, slots = gridDim.x >> 3;
-  const int range_end = min((xcd + 1) * chunk_tiles, total);
-  // (n-tiles past the last multiple of 4: blocks of 8 (m) x 1..3 (n) after all the others; 8192 x 29440 x 8192, 115
-  // n-tiles: 2.33 -> 2.7 PFLOP/s against the plain m-major order)
-  const bool blocked = (tiles_m & 7) == 0 && tiles_n >= 4;
-  const int bulk_tiles = tiles_m * (tiles_n & ~3);
-  auto tile_coords = [&](int t, int& m0, int& n0) {
-    int mt, nt;
-    if (blocked && t < bulk_tiles) {
-      const int sb = t >> 5, w = t & 31;
-      mt = (sb % (tiles_m >> 3)) * 8 + (w & 7);
-      nt = (sb / (tiles_m >> 3)) * 4 + (w >> 3);
-    } else if (blocked) {
-      const int u = t - bulk_tiles, bs = 8 * (tiles_n & 3), sb = u / bs, w = u - sb * bs;
-      mt = sb * 8 + (w & 7);
-      nt = (tiles_n & ~3) + (w >> 3);
-    } else {
-      mt = t % tiles_m;
-      nt = t / tiles_m;
-    }
-    m0 = mt * BM;
-    n0 = nt * BN;
-  };
-  const int first_tile = xcd * chunk_tiles + slot;
+  const TileWalk<BM, RAGGED_M> walk(p);
+  const int first_tile = walk.first, range_end = walk.end, slots = walk.slots;
   if (first_tile >= range_end) return;
+  auto tile_coords = [&](int t, int& m0, int& n0) { walk.coords(t, m0, n0); };
 
   const int nk = (p.k + 127) >> 7;
   const int sf_tiles_k = ((p.k >> 5) + 3) >> 2;  // 512-byte scale tiles per 128-row tile
@@ -545,8 +771,11 @@ __global__ __launch_bounds__(256, 1) void mxfp8_gemm_256_kernel(const Params p) 
 
 template <int TM, bool OUT_BF16, bool STREAM_OUT, bool RAGGED_K, bool RAGGED_M = false>
 int launch_fast_cfg(const Params& p, hipStream_t stream) {
-  auto kern = mxfp8_gemm_256_kernel<TM, OUT_BF16, STREAM_OUT, RAGGED_K, RAGGED_M>;
-  constexpr int lds_bytes = 2 * (64 * TM + 256) * 128 + 4 * 4608;  // 128 KiB / 96 KiB of tiles + the epilogue's 18 KiB
+  auto kern = [] {
+    if constexpr (TM == 4) return mxfp8_tile256_kernel<OUT_BF16, STREAM_OUT, RAGGED_K, RAGGED_M>;
+    else return mxfp8_gemm_256_kernel<TM, OUT_BF16, STREAM_OUT, RAGGED_K, RAGGED_M>;
+  }();
+  constexpr int lds_bytes = 2 * (64 * TM + 256) * 128 + (TM == 4 ? 4096 : 0) + 4 * 4608;  // tiles, scales, the epilogue's 18 KiB
   const int64_t tiles = ceil_div(p.m, 64 * TM) * (p.n / 256);
   if (!RAGGED_M && p.m % (64 * TM) != 0) return fail(NVF_ERR_LAUNCH, "mxfp8_gemm_256_kernel: M = %d is no multiple of %d", p.m, 64 * TM);
   const int cus = cu_count() & ~7;  // workgroup ids are dealt round-robin to the 8 XCDs
