@@ -30,6 +30,10 @@ __device__ __forceinline__ uint32_t pack2(float a, float b, bool out_bf16) {
 // consecutive lanes = 16 consecutive rows, one chunk) are conflict-free.
 __device__ __forceinline__ int lds_pos2(int row, int chunk) { return row * 8 + (chunk ^ ((row >> 1) & 7)); }
 __device__ __forceinline__ int lds_pos(int row, int chunk) { return lds_pos2(row, chunk); }
+// ... for tiles that ds_write_b128 fills with 4 neighbouring lanes writing every other chunk of a row: two neighbouring rows
+// differ in the lowest bit of the position as well, so that 8 lanes cover 32 banks, which is what a write is checked for
+// (a read is for 64, and stays conflict-free)
+__device__ __forceinline__ int lds_pos_staged(int row, int chunk) { return lds_pos2(row, chunk ^ (row & 1)); }
 
 // e4m3 scales of a lane's two blocks -> fp16 pairs; one dword (8 values of one block) -> one MFMA operand
 __device__ __forceinline__ void scale_pairs(uint32_t s2, f16x2 sv[2]) {
