@@ -19,7 +19,7 @@
 // accumulator registers hold 4 consecutive N-elements of one output row and are stored as 8 bytes.
 #include "gemm16_device.h"
 #include "nvf_internal.h"
-#include "tile256_loop.h"
+#include "tile_loop.h"
 
 #include <algorithm>
 #include <mutex>

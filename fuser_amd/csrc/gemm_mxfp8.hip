@@ -12,7 +12,7 @@
 // scale a 128-row wave tile needs for a 128-deep K step.
 #include "lds_direct.h"
 #include "nvf_internal.h"
-#include "tile256_loop.h"
+#include "tile_loop.h"
 
 namespace nvf {
 namespace {
@@ -221,16 +221,17 @@ __global__ __launch_bounds__(256) void mxfp8_gemm_kernel(const Params p) {
 // The walk over the tiles.  Workgroup ids are dealt round-robin to the 8 XCDs, so XCD x owns the contiguous tile range
 // [x*chunk, (x+1)*chunk) and its workgroups take consecutive tiles of it in each round: with the 8 (m) x 4 (n) blocked tile
 // numbering, the 32 tiles an XCD works on at any time share 8 A panels and 4 B panels in that XCD's L2.
-// RAGGED_M: the last row tile holds fewer than BM rows (kernels of their own: clamping the row of every activation
-// load costs the others time).  Its missing rows load the last row again and are not stored; the scale layout is
-// padded to 128 rows, so only a 256-row tile can ask for a scale tile that does not exist (it takes an existing one).
-template <int BM, bool RAGGED_M>
+// RAGGED: the last row tile holds fewer than BM rows or the last column tile fewer than BN columns (kernels of their own:
+// clamping the row of every load costs the others time).  The missing rows load the last row again and are not stored; the
+// scale layout is padded to 128 rows, so only a 256-row tile can ask for a scale tile that does not exist (it takes an
+// existing one).
+template <int BM, int BN, bool RAGGED>
 struct TileWalk {
   int tiles_m, tiles_n, first, end, slots, bulk_tiles;
   bool blocked;
   __device__ __forceinline__ explicit TileWalk(const Params& p) {
-    tiles_m = RAGGED_M ? (p.m + BM - 1) / BM : p.m / BM;
-    tiles_n = p.n / 256;
+    tiles_m = RAGGED ? (p.m + BM - 1) / BM : p.m / BM;
+    tiles_n = RAGGED ? (p.n + BN - 1) / BN : p.n / BN;
     const int total = tiles_m * tiles_n, chunk = (total + 7) >> 3;
     const int xcd = blockIdx.x & 7;
     slots = gridDim.x >> 3;
@@ -256,7 +257,7 @@ struct TileWalk {
       nt = t / tiles_m;
     }
     m0 = mt * BM;
-    n0 = nt * 256;
+    n0 = nt * BN;
   }
 };
 
@@ -267,45 +268,60 @@ struct TileWalk {
 // the K loop: with the lanes' loads predicated and zeros written instead, every load of every step was a block of code of
 // its own (1024 x 5632 x 2880: 31.2 us, against 24.3 for K = 2816; now 29.6 us).
 
-// 256x256 tiles, bound by the power limit of the MFMAs: 8192^3 2.93 PFLOP/s, 394 -> 376 us against the 128x256 kernel's K loop
-// with 256 rows (32x32 MFMAs, all of a step's loads in one half of it); 2000 x 8192 x 8192 104 -> 95 us, 8100 x 8192 x 2880
-// 178 -> 163, 2048 x 14336 x 4096 102 -> 100, 16384 x 16384 x 1024 291 -> 279.
-// The K loop is Tile256Loop's.  The scales of a step travel like its operands: 2 KiB of 128x4 tiles (two of A,
-// two of B) by LDS-direct loads, of which every wavefront reads the 16-byte pieces of its rows and keeps its lane group's byte.
-template <bool OUT_BF16, bool STREAM_OUT, bool RAGGED_K, bool RAGGED_M>
-__global__ __launch_bounds__(256, 1) void mxfp8_tile256_kernel(const Params p) {
-  constexpr int BM = 256;
-  constexpr int kScaleBytes = 2048;  // of a step: [operand][128-row tile][row % 32][16]
-  extern __shared__ u32x4 lds[];     // operand tiles | scales of two steps | the epilogue's 18 KiB
+// 256x256 tiles are bound by the power limit of the MFMAs: 8192^3 2.93 PFLOP/s, 394 -> 376 us against a K loop of 32x32 MFMAs
+// with all of a step's loads in one half of it.  The smaller tiles, for shapes whose large ones would leave compute units
+// idle, are bound by LDS (a 128x256 step: 1024 cycles of MFMAs, about 1560 of reads and loads) and, where the operands come
+// from memory, by the loads' latency: three and four buffers.  Weights that change from call to call, before (two buffers) and
+// now, us: 1024 x 4096 x 4096 45 -> 30, 512 x 8192 x 4096 46 -> 23 (128x128), 1979 x 7040 x 8416 157 -> 110, 330 x 9856 x 2688
+// 37 -> 17, 1000 x 5760 x 2880 36 -> 27; 45 shapes of 129..4000 rows 1.30 times as fast in the geometric mean, none more than
+// 3 % slower (999 x 1280 x 9984 39.7 -> 41.0: the columns left over by a cut no longer get a launch of their own).
+// The scales of a step travel like its operands: 2 KiB of 128x4 tiles (two of A, two of B) by LDS-direct loads, of which
+// every wavefront reads the pieces of its rows and keeps its lane group's byte.
+template <int NI, int NJ>
+struct Tiles {
+  static constexpr int BM = 32 * NI, BN = 32 * NJ;
+  static constexpr int NBUF = NI + NJ > 12 ? 2 : NI + NJ > 8 ? 3 : 4;
+  using Loop = TileLoop<Mma::kMxFp8, NI, NJ, NBUF>;
+  static constexpr int kScaleBytes = 2048;                      // of a step: [operand][128-row tile][row % 32][16]
+  static constexpr int kStageRows = NBUF == 3 ? 16 : 32;        // rows that the epilogue turns round at a time
+  static constexpr int kStageBytes = kStageRows * 144;          // ... of a wavefront
+  static constexpr int kLdsBytes = Loop::kTileBytes + NBUF * kScaleBytes + 4 * kStageBytes;
+  static_assert(kLdsBytes <= 160 * 1024, "LDS");
+};
+
+template <int NI, int NJ, bool OUT_BF16, bool STREAM_OUT, bool RAGGED_K, bool RAGGED>
+__global__ __launch_bounds__(256, 1) void mxfp8_tile_kernel(const Params p) {
+  using T = Tiles<NI, NJ>;
+  using Loop = typename T::Loop;
+  constexpr int BM = T::BM, BN = T::BN, NBUF = T::NBUF, kScaleBytes = T::kScaleBytes;
+  extern __shared__ u32x4 lds[];  // operand tiles | scales of NBUF steps | the epilogue's
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 1, wn = wave & 1;
-  const TileWalk<BM, RAGGED_M> walk(p);
+  const TileWalk<BM, BN, RAGGED> walk(p);
   if (walk.first >= walk.end) return;
   const int nk = (p.k + 127) >> 7;
   const int sf_tiles_k = ((p.k >> 5) + 3) >> 2;  // 512-byte scale tiles per 128-row tile
   const int k_tail = p.k & 127;                  // elements of the last step (RAGGED_K: 32, 64 or 96)
 
-  // ---- LDS-direct loads of a step.  Load u < 4: 8 rows of A's tiles 0..3 of a wavefront (rows 0..63 of either half of the
-  // tile), u = 4..11: 8 rows of B, u = 12..15: 8 rows of A's tiles 4..7; lane L lands at unit +L, i.e. row +(L>>3), chunk
-  // position L&7, which must hold global chunk (L&7) ^ ((row>>1)&7) = (L&7) ^ ((L>>4) | ((u&1)<<2)).  u = 16: the scales of A
-  // (even wavefronts) or B (odd ones), lanes 0..31 the first 128-row tile's, lanes 32..63 the second's.
+  // ---- LDS-direct loads of a step.  A load is 8 rows: lane L lands at unit +L, i.e. row +(L>>3), chunk position L&7, which
+  // must hold global chunk (L&7) ^ ((row>>1)&7) = (L&7) ^ ((L>>4) | ((j&1)<<2)) of load j.  The scales: A's by the even
+  // wavefronts, B's by the odd ones, lanes 0..31 the first 128-row tile's, lanes 32..63 the second's (where there is one).
   const uint32_t lds_base = (uint32_t)(uintptr_t)((__attribute__((address_space(3))) void*)lds);
   const uint32_t chunk_even = (uint32_t)((lane & 7) ^ (lane >> 4)), chunk_odd = chunk_even ^ 4u;
-  const int a_row0 = wm * 128 + wn * 32, b_row0 = wave * 64;  // the wavefront's share (A: and 64 rows further on)
-  const uint32_t a_lds = lds_base + (uint32_t)a_row0 * 128u, b_lds = lds_base + 65536u + (uint32_t)b_row0 * 128u;
-  const uint32_t s_lds = lds_base + kTile256Bytes + (uint32_t)wn * 1024u;
-  uint32_t a_off[8], b_off[8], s_off;
-#pragma unroll
-  for (int j = 0; j < 8; ++j) b_off[j] = (uint32_t)(b_row0 + 8 * j + (lane >> 3)) * (uint32_t)p.k + ((j & 1) ? chunk_odd : chunk_even) * 16u;
+  // the wavefront's share: rows of A's first half (the second's: 8 NI rows further on), of B
+  const int a_row0 = wm * (16 * NI) + wn * (4 * NI), b_row0 = wave * (8 * NJ);
+  const uint32_t a_lds = lds_base + (uint32_t)a_row0 * 128u, b_lds = lds_base + NBUF * Loop::kABytes + (uint32_t)b_row0 * 128u;
+  const uint32_t s_lds = lds_base + Loop::kTileBytes + (uint32_t)wn * 1024u;
+  uint32_t a_off[NI], b_off[NJ], s_off;
   // RAGGED_K: what takes an offset to the row's last chunk in the last step, where the lane's is past it
   const uint32_t last_chunk = (uint32_t)(k_tail >> 4) - 1u;
   const uint32_t tail_even = (min(chunk_even, last_chunk) - chunk_even) * 16u, tail_odd = (min(chunk_odd, last_chunk) - chunk_odd) * 16u;
   uint32_t sub_even = 0, sub_odd = 0;
 
   // ---- load stream: the step the next loads are issued for (l_ks of the tile lp), and the tile after it
-  struct TilePtrs { const uint8_t *a, *b, *s; int valid; };
+  struct TilePtrs { const uint8_t *a, *b, *s; int rows, cols; };
   auto tile_ptrs = [&](int t) {
     int m0, n0;
     walk.coords(t, m0, n0);
@@ -313,36 +329,52 @@ __global__ __launch_bounds__(256, 1) void mxfp8_tile256_kernel(const Params p) {
     r.a = p.a + (int64_t)m0 * p.k;
     r.b = p.b + (int64_t)n0 * p.k;
     r.s = wn ? p.sfb + (int64_t)(n0 >> 7) * sf_tiles_k * 512 : p.sfa + (int64_t)(m0 >> 7) * sf_tiles_k * 512;
-    r.valid = p.m - m0;  // rows of the tile that exist (RAGGED_M: possibly fewer than BM)
+    r.rows = p.m - m0;  // rows and columns of the tile that exist (RAGGED: possibly fewer than BM, BN)
+    r.cols = p.n - n0;
     return r;
   };
   TilePtrs lp = tile_ptrs(walk.first), np = lp;
-  int l_ks = 0;
-  uint32_t l_buf = 0, l_sbuf = 0;  // of the step's buffer
+  int l_ks = 0, l_buf = 0;
+  uint32_t l_a = a_lds, l_b = b_lds, l_s = s_lds;  // the step's buffer
   auto enter_tile = [&]() {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      uint32_t row = (uint32_t)(a_row0 + 64 * (j >> 2) + 8 * (j & 3) + (lane >> 3));
-      if (RAGGED_M) row = min(row, (uint32_t)(lp.valid - 1));
-      a_off[j] = row * (uint32_t)p.k + ((j & 1) ? chunk_odd : chunk_even) * 16u;
+    for (int u = 0; u < NI; ++u) {
+      uint32_t row = (uint32_t)(a_row0 + (u < NI / 2 ? 0 : 4 * NI) + 8 * u + (lane >> 3));
+      if (RAGGED) row = min(row, (uint32_t)(lp.rows - 1));
+      a_off[u] = row * (uint32_t)p.k + ((u & 1) ? chunk_odd : chunk_even) * 16u;
     }
-    s_off = (uint32_t)(lane & 31) * 16u + (lane >= 32 && (!RAGGED_M || wn || lp.valid > 128) ? (uint32_t)sf_tiles_k * 512u : 0u);
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      uint32_t row = (uint32_t)(b_row0 + 8 * j + (lane >> 3));
+      if (RAGGED) row = min(row, (uint32_t)(lp.cols - 1));
+      b_off[j] = row * (uint32_t)p.k + ((j & 1) ? chunk_odd : chunk_even) * 16u;
+    }
+    const bool second = (wn ? BN : BM) > 128 && (!RAGGED || (wn ? lp.cols : lp.rows) > 128);
+    s_off = (uint32_t)(lane & 31) * 16u + (lane >= 32 && second ? (uint32_t)sf_tiles_k * 512u : 0u);
   };
   enter_tile();
-  auto load = [&](auto u_c) {
-    constexpr int u = decltype(u_c)::value;
-    if constexpr (u == 16) {
-      lds_dma16(s_lds + l_sbuf, lp.s, s_off);
+  auto load = [&](auto code) {
+    constexpr int u = decltype(code)::value;
+    if constexpr (u == kLoadScales) {
+      lds_dma16(l_s, lp.s, s_off);
     } else {
-      constexpr int j = u < 4 ? u : u < 12 ? u - 4 : u - 8;
-      const uint32_t sub = RAGGED_K ? ((j & 1) ? sub_odd : sub_even) : 0u;
-      if constexpr (u >= 4 && u < 12) lds_dma16<j * 1024>(b_lds + l_buf, lp.b, b_off[j] + sub);
-      else lds_dma16<(j >> 2) * 8192 + (j & 3) * 1024>(a_lds + l_buf, lp.a, a_off[j] + sub);
+      const uint32_t sub = RAGGED_K ? ((u & 1) ? sub_odd : sub_even) : 0u;
+      if constexpr (u >= kLoadB) lds_dma16<(u - kLoadB) * 1024>(l_b, lp.b, b_off[u - kLoadB] + sub);
+      else lds_dma16<(u + (u < NI / 2 ? 0 : NI / 2)) * 1024>(l_a, lp.a, a_off[u] + sub);
     }
   };
+  auto load_step = [&]() {  // in the order of the loop's
+    static_for<NI / 2>(load);
+    static_for<NJ>([&](auto j) { load(std::integral_constant<int, kLoadB + decltype(j)::value>{}); });
+    load(std::integral_constant<int, kLoadScales>{});
+    static_for<NI / 2>([&](auto u) { load(std::integral_constant<int, NI / 2 + decltype(u)::value>{}); });
+  };
   auto advance = [&]() {
-    l_buf ^= 32768u;
-    l_sbuf ^= (uint32_t)kScaleBytes;
+    const int by = l_buf == NBUF - 1 ? 1 - NBUF : 1;
+    l_buf += by;
+    l_a += by * Loop::kABytes;
+    l_b += by * Loop::kBBytes;
+    l_s += by * kScaleBytes;
     lp.a += 128;
     lp.b += 128;
     lp.s += 512;
@@ -354,38 +386,49 @@ __global__ __launch_bounds__(256, 1) void mxfp8_tile256_kernel(const Params p) {
     if (l_ks == nk) {
       l_ks = 0;
       lp = np;
-      if (RAGGED_M) enter_tile();
+      if (RAGGED) enter_tile();
     }
   };
 
-  Tile256Loop<Mma::kMxFp8> loop;
+  Loop loop;
   loop.init(lds_base, lane, wm, wn);
 
   // ---- scales of the next step: the lane's rows r (even tiles) and 16 + r (odd ones) of its 128-row tile, whose 16 bytes are
-  // 4 words for the rows 32 apart; byte g of each is the lane group's, and the four are one operand register
+  // 4 words for the rows 32 apart; byte g of each is the lane group's, and those of a wavefront's tiles are one operand register
   uint32_t s_rd[2];
   u32x4 words[2][2];
   uint32_t next_s[2][2];  // [operand][even, odd tiles]
   {
-    const uint32_t at = lds_base + kTile256Bytes + (uint32_t)(lane & 15) * 16u;
-    s_rd[0] = at + (uint32_t)wm * 512u;
-    s_rd[1] = at + 1024u + (uint32_t)wn * 512u;
+    const uint32_t at = lds_base + Loop::kTileBytes + (uint32_t)(lane & 15) * 16u;
+    s_rd[0] = at + (uint32_t)wm * (NI == 8 ? 512u : 8u);  // (4 tiles: the first or second two words of the one scale tile)
+    s_rd[1] = at + 1024u + (uint32_t)wn * (NJ == 8 ? 512u : 8u);
   }
   const uint32_t g = (uint32_t)lane >> 4, pick_low = 0x0c0c0400u + g * 0x0101u, pick_high = 0x04000c0cu + g * 0x01010000u;
   const uint32_t tail_keep = (int)g * 32 < k_tail ? 0xffffffffu : 0u;  // RAGGED_K: the lane group's block exists in the last step
-  uint32_t c_sbuf = 0;  // buffer of the scales to be read
+  int s_buf = 0;  // of the scales to be read
   auto read_scales = [&]() {
 #pragma unroll
     for (int op = 0; op < 2; ++op)
 #pragma unroll
-      for (int o = 0; o < 2; ++o) words[op][o] = loop.lds_read(s_rd[op] + c_sbuf + o * 256u);
-    c_sbuf ^= (uint32_t)kScaleBytes;
+      for (int o = 0; o < 2; ++o) {
+        if ((op ? NJ : NI) == 8) {
+          words[op][o] = loop.lds_read(s_rd[op] + o * 256u);
+        } else {
+          const u32x2 two = *(__attribute__((address_space(3))) const u32x2*)(uintptr_t)(s_rd[op] + o * 256u);
+          words[op][o] = u32x4{two[0], two[1], 0u, 0u};
+        }
+      }
+    const int by = s_buf == NBUF - 1 ? 1 - NBUF : 1;
+    s_buf += by;
+    s_rd[0] += by * kScaleBytes;
+    s_rd[1] += by * kScaleBytes;
   };
   auto combine_scales = [&](int op, bool tail) {
 #pragma unroll
     for (int o = 0; o < 2; ++o) {
       const u32x4 w = words[op][o];
-      next_s[op][o] = __builtin_amdgcn_perm(w[1], w[0], pick_low) | __builtin_amdgcn_perm(w[3], w[2], pick_high);
+      next_s[op][o] = __builtin_amdgcn_perm(w[1], w[0], pick_low);
+      if ((op ? NJ : NI) == 8) next_s[op][o] |= __builtin_amdgcn_perm(w[3], w[2], pick_high);
       if (RAGGED_K && tail) next_s[op][o] &= tail_keep;
     }
   };
@@ -399,64 +442,72 @@ __global__ __launch_bounds__(256, 1) void mxfp8_tile256_kernel(const Params p) {
     asm volatile("s_nop 1" : "+v"(loop.sa[0]), "+v"(loop.sa[1]), "+v"(loop.sb[0]), "+v"(loop.sb[1]));
   };
 
-  // The stream runs two steps ahead of the MFMAs; with two steps per tile it is a whole tile ahead and
-  // already leaves the first tile during this prologue.
-  const int tiles_ahead = nk == 2 ? 2 : 1;
-  np = (walk.first + walk.slots < walk.end) ? tile_ptrs(walk.first + walk.slots) : lp;
+  // The stream runs NBUF steps ahead of the MFMAs: it enters the tile after the next before the next has begun where a tile
+  // has that few steps.  (c: the tile being computed, in steps of its list; past the end: a valid tile, loaded and ignored)
   const TilePtrs first_lp = lp;
-  static_for<17>(load);  // step 0
-  advance();
-  static_for<17>(load);  // step 1
-  advance();
-  loop.template fence<17>();
+  int stream_tile = walk.first;
+  auto prepare_next = [&]() {
+    stream_tile += walk.slots;
+    np = stream_tile < walk.end ? tile_ptrs(stream_tile) : first_lp;
+  };
+  prepare_next();
+  auto advance_and_prepare = [&]() {
+    advance();
+    if (l_ks == 0) prepare_next();
+  };
+  for (int i = 0; i < NBUF; ++i) {
+    load_step();
+    advance_and_prepare();
+  }
+  loop.fence();
   loop.first_fragments();
   read_scales();
-  combine_scales(0, false);
-  combine_scales(1, false);
+  combine_scales(0, nk == 1);
+  combine_scales(1, nk == 1);
   take_scales();
 
   const float alpha = p.alpha[0];
   for (int c_tile = walk.first; c_tile < walk.end; c_tile += walk.slots) {
-    // the tile the stream enters next (past the end of the list: a valid one, loaded and ignored)
-    np = (c_tile + tiles_ahead * walk.slots < walk.end) ? tile_ptrs(c_tile + tiles_ahead * walk.slots) : first_lp;
     auto step = [&](auto first, int c_ks) {
-      loop.template step<17, decltype(first)::value>(load, [&](auto part) {
+      loop.template step<decltype(first)::value>(load, [&](auto part) {
         if constexpr (decltype(part)::value == 0) read_scales();
         if constexpr (decltype(part)::value == 1) combine_scales(0, c_ks + 2 == nk);
         if constexpr (decltype(part)::value == 2) combine_scales(1, c_ks + 2 == nk);
       });
       take_scales();
-      advance();
+      advance_and_prepare();
     };
     step(std::true_type{}, 0);
     for (int c_ks = 1; c_ks < nk; ++c_ks) step(std::false_type{}, c_ks);
     loop.settle();
-    // ---- epilogue of this tile; the loads of the next tile's first two steps are already in flight.
+    // ---- epilogue of this tile; the loads of the next steps are already in flight.
     // A lane holds 8-byte pieces of 16 rows per tile; stored like that, a tile is 8192 sixteen-byte write
     // requests per compute unit and the L2 takes longer over them than over a whole K step of MFMAs.  Every
-    // 32x64 block of the wavefront's tile is therefore turned round in a private 4.5 KiB of LDS (32 rows of 128
-    // bytes at a pitch of 144 bytes) and leaves in 16-byte pieces, 8 lanes to a row's 128 bytes.  One LDS address
+    // block of 32 (16) rows x 64 columns of the wavefront's tile is therefore turned round in a private piece of LDS (rows of
+    // 128 bytes at a pitch of 144 bytes) and leaves in 16-byte pieces, 8 lanes to a row's 128 bytes.  One LDS address
     // each for writing and reading (the rest are immediate offsets) and one 32-bit lane offset next to a
     // wave-uniform result address; the lane number passes through an empty asm statement so that they are worked
     // out here, after the K loop.
+    constexpr int kRowTiles = T::kStageRows / 16;
     int m0, n0;
     walk.coords(c_tile, m0, n0);
     int elane = lane;
     asm volatile("" : "+v"(elane));
-    uint8_t* stage = reinterpret_cast<uint8_t*>(lds) + kTile256Bytes + 2 * kScaleBytes + wave * 4608;
+    uint8_t* stage = reinterpret_cast<uint8_t*>(lds) + Loop::kTileBytes + NBUF * kScaleBytes + wave * T::kStageBytes;
     uint8_t* wr = stage + (elane & 15) * 144 + (elane >> 4) * 8;
     const uint8_t* rd = stage + (elane >> 3) * 144 + (elane & 7) * 16;
     const int ldc = p.out_pitch();
     const uint32_t ooff = ((uint32_t)(elane >> 3) * (uint32_t)ldc + (uint32_t)(elane & 7) * 8u) * 2u;
-    uint8_t* obase = reinterpret_cast<uint8_t*>(static_cast<uint16_t*>(p.out) + (int64_t)(m0 + wm * 128) * ldc + n0 + wn * 128);
-    const int rows_left = p.m - m0 - wm * 128 - (elane >> 3);  // RAGGED_M: rows from this lane's first one to the end
+    uint8_t* obase = reinterpret_cast<uint8_t*>(static_cast<uint16_t*>(p.out) + (int64_t)(m0 + wm * (16 * NI)) * ldc + n0 + wn * (16 * NJ));
+    // RAGGED: rows and columns from this lane's first ones to the end
+    const int rows_left = p.m - m0 - wm * (16 * NI) - (elane >> 3), cols_left = p.n - n0 - wn * (16 * NJ) - (elane & 7) * 8;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < NI; i += kRowTiles) {
 #pragma unroll
-      for (int jh = 0; jh < 2; ++jh) {
+      for (int jh = 0; jh < NJ / 4; ++jh) {
 #pragma unroll
-        for (int t = 0; t < 8; ++t) {  // the block's 2 x 4 tiles
-          const f32x4 c = loop.acc[2 * i + (t >> 2)][4 * jh + (t & 3)];
+        for (int t = 0; t < 4 * kRowTiles; ++t) {  // the block's tiles
+          const f32x4 c = loop.acc[i + (t >> 2)][4 * jh + (t & 3)];
           u32x2 v;
           v[0] = pack2(c[0] * alpha, c[1] * alpha, OUT_BF16);
           v[1] = pack2(c[2] * alpha, c[3] * alpha, OUT_BF16);
@@ -464,10 +515,10 @@ __global__ __launch_bounds__(256, 1) void mxfp8_tile256_kernel(const Params p) {
         }
         asm volatile("" ::: "memory");  // the reads below see the writes above: one wavefront's LDS accesses stay in order
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
+        for (int t = 0; t < 2 * kRowTiles; ++t) {
           const u32x4 v = *reinterpret_cast<const u32x4*>(rd + t * 1152);
-          u32x4* dst = reinterpret_cast<u32x4*>(obase + ((int64_t)(i * 32 + 8 * t) * ldc + jh * 64) * 2 + ooff);
-          if (RAGGED_M && i * 32 + 8 * t >= rows_left) continue;
+          u32x4* dst = reinterpret_cast<u32x4*>(obase + ((int64_t)(i * 16 + 8 * t) * ldc + jh * 64) * 2 + ooff);
+          if (RAGGED && (i * 16 + 8 * t >= rows_left || jh * 64 >= cols_left)) continue;
           if constexpr (STREAM_OUT) __builtin_nontemporal_store(v, dst);
           else *dst = v;
         }
@@ -479,327 +530,39 @@ __global__ __launch_bounds__(256, 1) void mxfp8_tile256_kernel(const Params p) {
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no LDS-direct load may outlive the workgroup
 }
 
-// 128x256 tiles, for shapes whose 256x256 tiles would leave compute units idle:
-//   * Tiles travel global -> LDS with 16-byte LDS-direct loads (no staging registers) into a double
-//     buffer.  They are issued from inline assembly so that the compiler does not serialise them
-//     against the LDS reads of the other buffer; completion is enforced by the explicit
-//     s_waitcnt vmcnt(0) in front of the one barrier per 128-deep K step.
-//   * MFMA fragments are double-buffered in registers: the LDS reads of the next half step are in
-//     flight under the 16 MFMAs of the current one.
-//   * A load issued in the middle of step ks is consumed after the barrier in the middle of step
-//     ks+1, i.e. it has 32 MFMAs (~2000 cycles) to land.
-// LDS layout per operand tile: 256 rows x 128 bytes; 16-byte chunk c of row r at chunk position
-// c ^ ((r >> 1) & 7): conflict-free for the fragment reads (16 consecutive lanes = 16 consecutive
-// rows, one chunk) on the 64-bank LDS.
-// -------------------------------------------------------------------------------------------------
-__device__ __forceinline__ int lds_pos2(int row, int chunk) { return row * 8 + (chunk ^ ((row >> 1) & 7)); }
-
-template <int TM, bool OUT_BF16, bool STREAM_OUT, bool RAGGED_K = false, bool RAGGED_M = false>
-__global__ __launch_bounds__(256, 1) void mxfp8_gemm_256_kernel(const Params p) {
-  constexpr int BM = 64 * TM, BN = 256;
-  constexpr int A_UNITS = BM * 8;             // 16-byte units of the A tile (BM rows x 8 chunks)
-  constexpr int TILE_UNITS = 2048;            // ... of the B tile
-  constexpr int BUF_UNITS = A_UNITS + TILE_UNITS;
-  constexpr int NM = 4 * TM;                  // MFMAs per half step
-  constexpr int NF = 2 * TM + 8;              // fragment reads (ds_read_b128) per half step
-  constexpr int ND = 2 * TM + 8;              // LDS-direct loads per wavefront and K step
-  extern __shared__ u32x4 lds[];
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave >> 1, wn = wave & 1;
-  const int li = lane & 31, lg = lane >> 5;
-
-  const TileWalk<BM, RAGGED_M> walk(p);
-  const int first_tile = walk.first, range_end = walk.end, slots = walk.slots;
-  if (first_tile >= range_end) return;
-  auto tile_coords = [&](int t, int& m0, int& n0) { walk.coords(t, m0, n0); };
-
-  const int nk = (p.k + 127) >> 7;
-  const int sf_tiles_k = ((p.k >> 5) + 3) >> 2;  // 512-byte scale tiles per 128-row tile
-  const int k_tail = p.k & 127;                  // elements of the last step (RAGGED_K: 32, 64 or 96)
-
-  // ---- LDS-direct load addressing.  Wave w issues 8 loads per operand per K step; load j covers LDS
-  // units [(w*8+j)*64, +64) = rows (w*8+j)*8 .. +7; lane L lands at unit +L, i.e. row +(L>>3), chunk
-  // position L&7, which must hold global chunk (L&7) ^ ((row>>1)&7) = (L&7) ^ ((L>>4) | ((j&1)<<2)).
-  const uint32_t row_off = (uint32_t)(lane >> 3) * (uint32_t)p.k;
-  const uint32_t voff_even = row_off + (uint32_t)(((lane & 7) ^ (lane >> 4)) << 4);
-  const uint32_t voff_odd = row_off + (uint32_t)(((lane & 7) ^ ((lane >> 4) | 4)) << 4);
-  const uint32_t lds_base = (uint32_t)(uintptr_t)((__attribute__((address_space(3))) void*)lds);
-  const uint32_t step8 = 8u * (uint32_t)p.k;  // 8 rows
-  // RAGGED_K: the row's chunk for a load unit of a step is the lane's or, if that is past the end, the last there is
-  const uint32_t chunk_even = (uint32_t)((lane & 7) ^ (lane >> 4));
-  const uint32_t tail_last = (uint32_t)(k_tail >> 4) - 1u;
-  uint32_t step_even = voff_even, step_odd = voff_odd;  // the lane offsets of the step being issued
-
-  // ---- load stream state: the (tile, K step) the next loads are issued for
-  // ---- load stream: the loads of step g+2 are issued while step g is computed, so the stream runs
-  // ahead of the compute loop and crosses into the next tile two steps early.  All of its state is
-  // wave-uniform and it advances without branches (the next tile's base pointers are prepared at the
-  // top of the tile loop), so that the hot loop stays one basic block.
-  struct TilePtrs { const uint8_t *a, *b, *sa, *sb; int valid; };
-  auto tile_ptrs = [&](int t) {
-    int m0, n0;
-    tile_coords(t, m0, n0);
-    TilePtrs r;
-    // (RAGGED_M: the tile's first row; the wavefront's share is part of the lane's clamped row)
-    r.a = p.a + ((int64_t)m0 + (RAGGED_M ? 0 : wave * (BM / 4))) * p.k;
-    r.b = p.b + ((int64_t)n0 + wave * 64) * p.k;
-    r.valid = p.m - m0;  // rows of the tile that exist (RAGGED_M: possibly fewer than BM)
-    // one 16-byte scale load per lane per K step: rows {li, li+32, li+64, li+96} of the wave's 128-row
-    // scale tile x 4 K-blocks
-    int sa_tile = (m0 >> 7) + (TM == 4 ? wm : 0);
-    if (RAGGED_M) sa_tile = min(sa_tile, ((p.m + 127) >> 7) - 1);
-    r.sa = p.sfa + ((int64_t)sa_tile * sf_tiles_k) * 512;
-    r.sb = p.sfb + ((int64_t)((n0 >> 7) + wn) * sf_tiles_k) * 512;
-    return r;
-  };
-  TilePtrs lp = tile_ptrs(first_tile);  // tile the stream is in
-  TilePtrs np = lp;                     // tile it enters next
-  int l_ks = 0, l_count = 0;            // K step inside lp; steps issued so far
-  const uint32_t sc_lane_off = (uint32_t)li * 16u;
-  u32x4 sc_la, sc_lb;  // scales in flight (for step l_count - 1)
-  // Unit q (0..ND-1) of a step's tile loads: 8 rows of one operand.  A and B alternate while A has rows left
-  // (operand q&1, rows (q/2)*8 .. +7 of the wavefront's share), then the rest of B.  Past the end of the
-  // stream the last tile is loaded again (into a buffer nobody reads any more).
-  auto issue_step_unit = [&](int q) {
-    const int buf = l_count & 1;
-    const int op = q < 4 * TM ? (q & 1) : 1;
-    const int j = q < 4 * TM ? (q >> 1) : q - 2 * TM;
-    const uint32_t l = lds_base + (uint32_t)(buf * BUF_UNITS + (op ? A_UNITS + wave * 512 : wave * (BM * 2))) * 16u + j * 1024u;
-    const uint8_t* gp = (op ? lp.b : lp.a) + ((int64_t)l_ks << 7);
-    if (RAGGED_K && q == 0) {
-      const uint32_t last = l_ks == nk - 1 ? tail_last : 7u;
-      step_even = row_off + (min(chunk_even, last) << 4);
-      step_odd = row_off + (min(chunk_even ^ 4u, last) << 4);
-    }
-    uint32_t voff = ((j & 1) ? step_odd : step_even) + (uint32_t)j * step8;
-    if (RAGGED_M && op == 0) {
-      const uint32_t row = min((uint32_t)(wave * (BM / 4) + j * 8) + (uint32_t)(lane >> 3), (uint32_t)(lp.valid - 1));
-      voff = row * (uint32_t)p.k + (((j & 1) ? step_odd : step_even) - row_off);
-    }
-    lds_dma16(l, gp, voff);
-  };
-  // After the 16 units: the step's scale loads, then advance the stream (selects only).
-  auto issue_step_tail = [&]() {
-    sc_la = *reinterpret_cast<const u32x4*>(lp.sa + (int64_t)l_ks * 512 + sc_lane_off);
-    sc_lb = *reinterpret_cast<const u32x4*>(lp.sb + (int64_t)l_ks * 512 + sc_lane_off);
-    ++l_count;
-    const bool wrap = (l_ks + 1 == nk);
-    l_ks = wrap ? 0 : l_ks + 1;
-    lp.a = wrap ? np.a : lp.a;
-    lp.b = wrap ? np.b : lp.b;
-    lp.sa = wrap ? np.sa : lp.sa;
-    lp.sb = wrap ? np.sb : lp.sb;
-    if (RAGGED_M) lp.valid = wrap ? np.valid : lp.valid;
-  };
-  // Fragment storage: [operand: 0 = A, 1 = B][sub-tile][half].  Unit q (0..NF-1) of a half step is one
-  // ds_read_b128: the 2*TM units of A (sub-tile q/2, half q&1), then the 8 units of B.
-  struct Frags { u32x4 h[2][4][2]; };
-  auto load_unit = [&](int buf, int sub, int q, Frags& f) {
-    const int op = q >= 2 * TM ? 1 : 0;
-    const int u = op ? q - 2 * TM : q;
-    const int t = u >> 1, half = u & 1;
-    const u32x4* base = lds + buf * BUF_UNITS + op * A_UNITS;
-    const int row = (op ? wn * 128 : wm * (32 * TM)) + t * 32 + li;
-    f.h[op][t][half] = base[lds_pos2(row, sub * 4 + lg + 2 * half)];
-  };
-  auto frag = [&](const Frags& f, int op, int t) {
-    const u32x4 lo = f.h[op][t][0], hi = f.h[op][t][1];
-    return i32x8{(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
-  };
-
-  f32x16 acc[TM][4];
-  auto zero_acc = [&]() {
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-  };
-  zero_acc();
-
-  // Keeps the 16 accumulator tiles "used" at this point of the program, so that the MFMAs producing
-  // them cannot be moved past the statement that follows (they have no side effects of their own).
-#define NVF_PIN_ACC()                                                                                          \
-  do {                                                                                                         \
-    asm volatile("" : "+a"(acc[0][0]), "+a"(acc[0][1]), "+a"(acc[0][2]), "+a"(acc[0][3]), "+a"(acc[1][0]),     \
-                 "+a"(acc[1][1]), "+a"(acc[1][2]), "+a"(acc[1][3]));                                           \
-    if constexpr (TM == 4)                                                                                     \
-      asm volatile("" : "+a"(acc[TM - 2][0]), "+a"(acc[TM - 2][1]), "+a"(acc[TM - 2][2]), "+a"(acc[TM - 2][3]), \
-                   "+a"(acc[TM - 1][0]), "+a"(acc[TM - 1][1]), "+a"(acc[TM - 1][2]), "+a"(acc[TM - 1][3]));     \
-  } while (0)
-
-  const float alpha = p.alpha[0];
-  const int sh = lg * 8;  // lane group 1 supplies K-blocks 1 and 3 of a step
-
-  Frags f0, f1;      // fragments of the first / second half (K 0..63 / 64..127) of a step
-  u32x4 wa, wb;      // scales of the step being computed, shifted for this lane group
-  u32x4 na, nb;      // scales of the next step
-
-  // The stream runs two steps ahead of the MFMAs; with two steps per tile it is a whole tile ahead and
-  // already leaves the first tile during this prologue.
-  const int tiles_ahead = nk == 2 ? 2 : 1;
-  np = (first_tile + slots < range_end) ? tile_ptrs(first_tile + slots) : lp;
-#pragma unroll
-  for (int q = 0; q < ND; ++q) issue_step_unit(q);  // step 0
-  issue_step_tail();
-  na = sc_la; nb = sc_lb;
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  // scale word of accumulator row tile i: rows {li + 32 c} of a 128-row scale tile are component c of the load;
-  // with 64 rows per wavefront (TM == 2) the wavefront's half of the tile is components 2 wm, 2 wm + 1
-  // (tail: the scales are those of a tile's last step, RAGGED_K only)
-  auto take_scales = [&](bool tail = false) {
-    if (RAGGED_K && tail) {
-      const uint32_t keep = (1u << (k_tail >> 2)) - 1u;  // k_tail / 32 bytes stay, the others become 2^-127
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        na[c] &= keep;
-        nb[c] &= keep;
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < TM; ++i) wa[i] = (TM == 4 ? na[i] : (wm ? na[2 + (i & 1)] : na[i & 1])) >> sh;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) wb[j] = nb[j] >> sh;
-  };
-  take_scales();
-#pragma unroll
-  for (int q = 0; q < ND; ++q) issue_step_unit(q);  // step 1
-  issue_step_tail();
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-#pragma unroll
-  for (int q = 0; q < NF; ++q) load_unit(0, 0, q, f0);
-
-  int g = 0;
-  for (int c_tile = first_tile; c_tile < range_end; c_tile += slots) {
-    // the stream is inside this tile by now; prepare the tile it will enter two steps before the end
-    np = (c_tile + tiles_ahead * slots < range_end) ? tile_ptrs(c_tile + tiles_ahead * slots) : lp;
-    for (int c_ks = 0; c_ks < nk; ++c_ks, ++g) {
-      const int buf = g & 1;
-      // ---- first half: MFMAs on f0, interleaved one-to-one with the LDS reads that fill f1
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int q = 0; q < NM; ++q) {
-        const int i = q >> 2, j = q & 3;
-#pragma unroll
-        for (int u = q * NF / NM; u < (q + 1) * NF / NM; ++u) load_unit(buf, 1, u, f1);
-        acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(frag(f0, 1, j), frag(f0, 0, i), acc[i][j], 0, 0, 0, (int)wb[j], 0, (int)wa[i]);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      NVF_PIN_ACC();
-      // Everything this wave loaded for step g+1 has landed and its reads of buf are complete; after
-      // the barrier that holds for every wave, so buf^1 may be read and buf may be overwritten.
-      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-      __builtin_amdgcn_s_barrier();
-      // The scale words of step g+1 are consumed here and nowhere earlier: their load is covered by the
-      // wait above, and any wait placed before it would also stall on the tile loads just issued.
-      asm volatile("" : "+v"(sc_la), "+v"(sc_lb) : : "memory");
-      na = sc_la; nb = sc_lb;
-      // ---- second half: MFMAs on f1, interleaved with the LDS reads of the next step's f0 (from buf^1;
-      // after the last step they read stale data that is never used) and the loads of step g+2 into buf
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int q = 0; q < NM; ++q) {
-        const int i = q >> 2, j = q & 3;
-#pragma unroll
-        for (int u = q * NF / NM; u < (q + 1) * NF / NM; ++u) load_unit(buf ^ 1, 0, u, f0);
-#pragma unroll
-        for (int u = q * ND / NM; u < (q + 1) * ND / NM; ++u) issue_step_unit(u);
-        if (q == NM - 1) issue_step_tail();  // scalar bookkeeping in the shadow of the MFMAs already queued
-        acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(frag(f1, 1, j), frag(f1, 0, i), acc[i][j], 0, 0, 2, (int)wb[j], 2, (int)wa[i]);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      NVF_PIN_ACC();
-      take_scales(c_ks + 2 == nk);  // the scales of the next step
-    }
-    // ---- epilogue of this tile; the loads of the next tile's first two steps are already in flight.
-    // acc[i][j][r] = C[m = li][n = (r/4)*8 + lg*4 + r%4] of its 32x32 sub-tile.
-    // A lane holds 8-byte pieces of 32 different rows; stored like that, a tile is 8192 sixteen-byte write
-    // requests per compute unit and the L2 takes longer over them than over a whole K step of MFMAs.  Every
-    // 32x64 block of the wavefront's tile is therefore turned round in a private 4.5 KiB of LDS (32 rows of 128
-    // bytes at a pitch of 144 bytes) and leaves in 16-byte pieces, 8 lanes to a row's 128 bytes.  One LDS address
-    // each for writing and reading (the rest are immediate offsets) and one 32-bit lane offset next to a
-    // wave-uniform result address; the lane number passes through an empty asm statement so that they are worked
-    // out here, after the K loop.
-    int m0, n0;
-    tile_coords(c_tile, m0, n0);
-    int elane = lane;
-    asm volatile("" : "+v"(elane));
-    uint8_t* stage = reinterpret_cast<uint8_t*>(lds + 2 * BUF_UNITS) + wave * 4608;
-    uint8_t* wr = stage + (elane & 31) * 144 + (elane >> 5) * 8;
-    const uint8_t* rd = stage + (elane >> 3) * 144 + (elane & 7) * 16;
-    const int ldc = p.out_pitch();
-    const uint32_t ooff = ((uint32_t)(elane >> 3) * (uint32_t)ldc + (uint32_t)(elane & 7) * 8u) * 2u;
-    uint8_t* obase = reinterpret_cast<uint8_t*>(static_cast<uint16_t*>(p.out) + (int64_t)(m0 + wm * (32 * TM)) * ldc + n0 + wn * 128);
-    const int rows_left = p.m - m0 - wm * (32 * TM) - (elane >> 3);  // RAGGED_M: rows from this lane's first one to the end
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-#pragma unroll
-      for (int jh = 0; jh < 2; ++jh) {
-#pragma unroll
-        for (int j2 = 0; j2 < 2; ++j2) {
-#pragma unroll
-          for (int rq = 0; rq < 4; ++rq) {
-            const int j = jh * 2 + j2;
-            u32x2 v;
-            v[0] = pack2(acc[i][j][rq * 4 + 0] * alpha, acc[i][j][rq * 4 + 1] * alpha, OUT_BF16);
-            v[1] = pack2(acc[i][j][rq * 4 + 2] * alpha, acc[i][j][rq * 4 + 3] * alpha, OUT_BF16);
-            *reinterpret_cast<u32x2*>(wr + (j2 * 4 + rq) * 16) = v;
-          }
-        }
-        asm volatile("" ::: "memory");  // the reads below see the writes above: one wavefront's LDS accesses stay in order
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          const u32x4 v = *reinterpret_cast<const u32x4*>(rd + t * 1152);
-          u32x4* dst = reinterpret_cast<u32x4*>(obase + ((int64_t)(i * 32 + 8 * t) * ldc + jh * 64) * 2 + ooff);
-          if (RAGGED_M && i * 32 + 8 * t >= rows_left) continue;
-          if constexpr (STREAM_OUT) __builtin_nontemporal_store(v, dst);
-          else *dst = v;
-        }
-        asm volatile("" ::: "memory");
-      }
-    }
-    zero_acc();
-  }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no LDS-direct load may outlive the workgroup
-#undef NVF_PIN_ACC
-}
-
-template <int TM, bool OUT_BF16, bool STREAM_OUT, bool RAGGED_K, bool RAGGED_M = false>
-int launch_fast_cfg(const Params& p, hipStream_t stream) {
-  auto kern = [] {
-    if constexpr (TM == 4) return mxfp8_tile256_kernel<OUT_BF16, STREAM_OUT, RAGGED_K, RAGGED_M>;
-    else return mxfp8_gemm_256_kernel<TM, OUT_BF16, STREAM_OUT, RAGGED_K, RAGGED_M>;
-  }();
-  constexpr int lds_bytes = 2 * (64 * TM + 256) * 128 + (TM == 4 ? 4096 : 0) + 4 * 4608;  // tiles, scales, the epilogue's 18 KiB
-  const int64_t tiles = ceil_div(p.m, 64 * TM) * (p.n / 256);
-  if (!RAGGED_M && p.m % (64 * TM) != 0) return fail(NVF_ERR_LAUNCH, "mxfp8_gemm_256_kernel: M = %d is no multiple of %d", p.m, 64 * TM);
+template <int NI, int NJ, bool OUT_BF16, bool STREAM_OUT, bool RAGGED_K, bool RAGGED>
+int launch_tiles_cfg(const Params& p, hipStream_t stream) {
+  using T = Tiles<NI, NJ>;
+  auto kern = mxfp8_tile_kernel<NI, NJ, OUT_BF16, STREAM_OUT, RAGGED_K, RAGGED>;
+  const int64_t tiles = ceil_div(p.m, T::BM) * ceil_div(p.n, T::BN);
+  if (!RAGGED && (p.m % T::BM != 0 || p.n % T::BN != 0))
+    return fail(NVF_ERR_LAUNCH, "mxfp8_tile_kernel: %d x %d is no multiple of %d x %d", p.m, p.n, T::BM, T::BN);
   const int cus = cu_count() & ~7;  // workgroup ids are dealt round-robin to the 8 XCDs
   const unsigned grid = (unsigned)(tiles >= cus ? cus : ((tiles + 7) / 8) * 8);
-  if (note_launch("mxfp8_gemm_256_kernel<TM=%d,stream_out=%d%s%s> grid=%u", TM, (int)STREAM_OUT, RAGGED_K ? ",ragged_k" : "",
-                  RAGGED_M ? ",ragged_m" : "", grid))
+  // (TM: 64 rows, TN: 64 columns of the tile each; 256 columns go without saying)
+  if (note_launch("mxfp8_gemm_256_kernel<TM=%d,%sstream_out=%d%s%s%s> grid=%u", NI / 2, NJ == 8 ? "" : "TN=2,", (int)STREAM_OUT, RAGGED_K ? ",ragged_k" : "",
+                  p.m % T::BM ? ",ragged_m" : "", p.n % T::BN ? ",ragged_n" : "", grid))
     return NVF_OK;
   static std::atomic<uint64_t> configured{0};  // one bit per device (and per instantiation of this launcher)
-  if (const int rc = allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds_bytes, configured)) return rc;
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(256), lds_bytes, stream, p);
-  return check_launch("mxfp8_gemm_256_kernel");
+  if (const int rc = allow_dynamic_lds(reinterpret_cast<const void*>(kern), T::kLdsBytes, configured)) return rc;
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(256), T::kLdsBytes, stream, p);
+  return check_launch("mxfp8_tile_kernel");
 }
 
-template <int TM, bool OUT_BF16>
-int launch_fast(const Params& p, hipStream_t stream) {
+template <int NI, int NJ, bool OUT_BF16>
+int launch_tiles(const Params& p, hipStream_t stream) {
   // Operands and result together beyond what the 256 MB last-level cache holds: the result would push the
   // operand panels out of it (and out of the L2s) on its way to memory, so it leaves with non-temporal stores
-  // (8192^3: +5 %, 16384 x 16384 x 2048: +17 %; smaller problems lose 1-5 % that way).
-  const bool stream_out = ((int64_t)p.m + p.n) * p.k + 2 * (int64_t)p.m * p.n > (int64_t)224 << 20;
-  if (p.m % (64 * TM) != 0 && (p.k & 127) != 0)
-    return stream_out ? launch_fast_cfg<TM, OUT_BF16, true, true, true>(p, stream) : launch_fast_cfg<TM, OUT_BF16, false, true, true>(p, stream);
-  if (p.m % (64 * TM) != 0) return stream_out ? launch_fast_cfg<TM, OUT_BF16, true, false, true>(p, stream) : launch_fast_cfg<TM, OUT_BF16, false, false, true>(p, stream);
-  if ((p.k & 127) != 0) return stream_out ? launch_fast_cfg<TM, OUT_BF16, true, true>(p, stream) : launch_fast_cfg<TM, OUT_BF16, false, true>(p, stream);
-  return stream_out ? launch_fast_cfg<TM, OUT_BF16, true, false>(p, stream) : launch_fast_cfg<TM, OUT_BF16, false, false>(p, stream);
+  // (8192^3: +5 %, 16384 x 16384 x 2048: +17 %; smaller problems lose 1-5 % that way).  128x128 tiles are for small ones.
+  const bool ragged = p.m % (32 * NI) != 0 || p.n % (32 * NJ) != 0, ragged_k = (p.k & 127) != 0;
+  if constexpr (NJ == 8) {
+    if (((int64_t)p.m + p.n) * p.k + 2 * (int64_t)p.m * p.n > (int64_t)224 << 20) {
+      if (ragged) return ragged_k ? launch_tiles_cfg<NI, NJ, OUT_BF16, true, true, true>(p, stream) : launch_tiles_cfg<NI, NJ, OUT_BF16, true, false, true>(p, stream);
+      return ragged_k ? launch_tiles_cfg<NI, NJ, OUT_BF16, true, true, false>(p, stream) : launch_tiles_cfg<NI, NJ, OUT_BF16, true, false, false>(p, stream);
+    }
+  }
+  if (ragged) return ragged_k ? launch_tiles_cfg<NI, NJ, OUT_BF16, false, true, true>(p, stream) : launch_tiles_cfg<NI, NJ, OUT_BF16, false, false, true>(p, stream);
+  return ragged_k ? launch_tiles_cfg<NI, NJ, OUT_BF16, false, true, false>(p, stream) : launch_tiles_cfg<NI, NJ, OUT_BF16, false, false, false>(p, stream);
 }
 
 // -------------------------------------------------------------------------------------------------
@@ -1125,39 +888,51 @@ int launch_cfg(const Params& p, hipStream_t stream) {
   return check_launch("mxfp8_gemm_kernel");
 }
 
-// Which kernel a shape gets.  Persistent LDS-direct kernel with 256x256 or 128x256 tiles: a 128-row tile costs about
-// 0.61 of a 256-row tile (half the flops at 82 % of the rate, measured), and the time goes with the rounds of tiles
-// over the compute units; below 48 tiles the tile kernels do as well.
-enum class Plan { kStream, kTiles256, kTiles128, kOther };
+// Which kernel a shape gets: the weight-streaming kernel, the persistent kernel with one of three tiles, or - too few tiles, a
+// shape that neither takes - the tile kernels.
+enum class Plan { kStream, kTiles256, kTiles128, kTiles128x128, kOther };
 // (ns: the estimated duration, where there is an estimate)
 Plan mxfp8_plan(int64_t m, int64_t n, int64_t k, int64_t cus, int64_t* ns = nullptr) {
   if (ns) *ns = INT64_MAX;
   const bool skinny_ok = (k & 31) == 0 && (n & 15) == 0 && k * 64 < (1ll << 31);  // 32-bit lane offsets (a short last chunk is fine)
-  // (the persistent kernel takes any K % 32 == 0: its last step may be short)
-  // (a last row tile with fewer rows: the variant that clamps the rows of its activation loads; the tile counts as a
-  // whole one.  640 x 14336 x 4096: 280 tiles of 128 rows in 2 rounds 60 us, 168 of 256 rows 43 us)
-  const bool fast_shape = (k & 31) == 0 && k >= 256 && (n & 255) == 0 && k * 256 < (1ll << 31);
-  const bool ok256 = fast_shape && ((m & 255) == 0 || m > 128);
-  const bool ok128 = fast_shape && ((m & 127) == 0 || m > 64);
-  const int64_t t256 = ok256 ? ceil_div(m, 256) * (n / 256) : 0, t128 = ok128 ? ceil_div(m, 128) * (n / 256) : 0;
-  const int64_t cost256 = t256 >= 128 ? 100 * ceil_div(t256, cus) : INT64_MAX;
-  const int64_t cost128 = t128 >= 48 ? 61 * ceil_div(t128, cus) : INT64_MAX;
-  const bool fast = cost256 != INT64_MAX || cost128 != INT64_MAX;
-  const int64_t fast_ns = fast ? 5000 + std::min(cost256, cost128) * 113 * ((k + 127) & ~127ll) / 1024 : INT64_MAX;
+  // The persistent kernel takes any K % 32 == 0 (its last step may be short), a last row tile with fewer rows (which counts as a
+  // whole one: 640 x 14336 x 4096 as 280 tiles of 128 rows in 2 rounds 60 us, 168 of 256 rows 43 us) and, where the rows are
+  // ragged too, a last column tile with fewer columns, where the others get a launch of its own for the remaining columns
+  // (1000 x 5760 x 2880: 36 + 5 us cut, 26.5 whole; measured from K = 1024 on).
+  const bool fast_shape = (k & 31) == 0 && k >= 256 && k * 256 < (1ll << 31) && (n & 15) == 0 && (m > 64 || (m & 127) == 0);
+  auto tiles_of = [&](int64_t bm, int64_t bn) { return ceil_div(m, bm) * ceil_div(n, bn); };
+  const bool columns_ok = (n & 255) == 0 || ((m & 127) != 0 && m > 128 && n > 256 && k >= 1024);
+  int64_t t256 = tiles_of(256, 256), t128 = tiles_of(128, 256), t128x128 = tiles_of(128, 128);
+  if (!fast_shape || t256 < 128 || !columns_ok || !((m & 255) == 0 || m > 128)) t256 = 0;
+  // 128x128 tiles: half the work per compute unit in 0.7 of the time, so they win up to a whole round of them, i.e. for half a
+  // round of 128x256 tiles (512 x 8192 x 4096 23.3 against 31.3 us, 1178 x 2816 x 11456 65 / 98, 157 x 14240 x 10752 50 / 71).  Of
+  // the shapes whose N and K are whole multiples of the 128x256 tiles' those with more than two fifths of a round stay on them: the
+  // dispatch of 1024 x 4096 x 4096, 256 x 14336 x 4096 and x 14336 and 1000 x 4096 x 14336 is pinned.
+  const bool whole = (n & 255) == 0 && (k & 127) == 0;
+  if (!fast_shape || m <= 128 || (whole && 5 * t128 >= 2 * cus) || !columns_ok || k < 512 || t128x128 < 16) t128x128 = 0;
+  if (!fast_shape || t128 < 48 || !columns_ok) t128 = 0;
+  // Measured with weights that change from call to call, us per 128-deep step of a round (a round of a few tiles, a full one)
+  // and per call: 256x256 1.08, 1.48 and 7; 128x256 0.75, 0.95 and 5.2; 128x128 0.53, 0.60 and 3.5.
+  auto tile_ns = [&](int64_t tiles, int64_t fixed, int64_t step, int64_t full) {
+    if (tiles == 0) return (int64_t)INT64_MAX;
+    const int64_t steps = (k + 127) >> 7, rounds = ceil_div(tiles, cus);
+    return fixed + steps * (rounds * step + (full - step) * tiles / cus);
+  };
+  const int64_t ns256 = tile_ns(t256, 7000, 1080, 1480), ns128 = tile_ns(t128, 5200, 750, 950), ns128x128 = tile_ns(t128x128, 3500, 530, 600);
+  const int64_t fast_ns = std::min(ns256, std::min(ns128, ns128x128));
+  const bool fast = fast_ns != INT64_MAX;
   if (skinny_ok) {
     const int64_t skinny_ns = mxfp8_skinny_ns(m, n, k, cus);
     if (ns) *ns = skinny_ns;
     if (m <= 32) return Plan::kStream;
     if (fast) {
-      // Skinny or persistent kernel by estimated duration: a round of 128x256 tiles takes 6.9 us per 1024 of K plus
-      // about 5 us (so cost 100 = 11.3 us per 1024 of K), the skinny kernel what its estimate says (its unit is
-      // 0.96 ns).  Measured: 256 x 14336 x 4096 31 (persistent) against 47 us, 512 x 4096 x 7168 51 against 30 us
-      // (skinny), 1024 x 2048 x 14336 97 against 48 us, 1024 x 4096 x 4096 31 against 34 us.
-      // (129..256 rows are three or four slabs of 64, which the estimate puts 15-22 % low against a wide N: 160 and 192 x
-      // 14336 x 4096 run 37 and 40 us streamed, estimated 31, and 31 us on 112 tiles of 128 rows; 256 x 11008 x 4096
-      // 38 against 31 us)
-      const int64_t margin = m > 128 && m <= 256 ? skinny_ns / 5 : 0;
-      if (skinny_ns + margin <= fast_ns) return Plan::kStream;
+      // Skinny or persistent kernel by estimated duration.  Measured: 512 x 4096 x 7168 36.7 (persistent) against 31.8 us,
+      // 700 x 2304 x 5120 22.3 / 23.3, 512 x 4096 x 4096 18.2 / 18.7, 300 x 3072 x 2048 11.4 / 7.1, 1500 x 1408 x 7168 34 / 42.
+      // (With weights that change from call to call the skinny kernel takes, in percent of its estimate, 58-87 for K < 2048,
+      // 75-100 below 3072, 100 around 4096 and 105-150 above, over 45 shapes of 129..4000 rows; from 3072 on the estimate stays as
+      // it is, which the pinned dispatch of 1000 x 4096 x 14336 wants.)
+      const int64_t percent = m <= 128 || k >= 3072 ? 100 : k < 2048 ? 78 : 92;
+      if (skinny_ns * percent / 100 <= fast_ns) return Plan::kStream;
     } else {
       // No persistent kernel for the shape (ragged M or N, or too few tiles): up to 256 rows, i.e. four passes over
       // the weights, the skinny kernel beats the tile kernels (128 x 4096 x 14336: 20 instead of 117 us); with more
@@ -1168,7 +943,7 @@ Plan mxfp8_plan(int64_t m, int64_t n, int64_t k, int64_t cus, int64_t* ns = null
     }
   }
   if (ns) *ns = fast_ns;
-  if (fast) return cost256 <= cost128 ? Plan::kTiles256 : Plan::kTiles128;
+  if (fast) return fast_ns == ns256 ? Plan::kTiles256 : fast_ns == ns128 ? Plan::kTiles128 : Plan::kTiles128x128;
   return Plan::kOther;
 }
 
@@ -1180,10 +955,11 @@ int launch_sized(const Params& p, hipStream_t stream) {
   const Plan whole = mxfp8_plan(p.m, p.n, p.k, cus, &whole_ns);
   // A cut along N or M competes with the kernel the whole shape gets: the tile kernels (no estimate) lose to any cut
   // that works; the weight-streaming kernel loses to a cut whose main part runs on the persistent kernel and is
-  // estimated 5 % faster or more (384 x 29568 x 8192: 291 us on tiles, 256 x 29568 x 8192: 169 us streamed).
+  // estimated 5 % faster or more (384 x 29568 x 8192: 291 us on tiles, 256 x 29568 x 8192: 169 us streamed), and so do tiles
+  // of which the last ones have fewer columns.
   const bool whole_other = whole == Plan::kOther;
-  const int64_t bar = whole_other ? INT64_MAX : whole == Plan::kStream ? whole_ns - whole_ns / 20 : 0;
-  auto is_tiles = [](Plan q) { return q == Plan::kTiles256 || q == Plan::kTiles128; };
+  const int64_t bar = whole_other ? INT64_MAX : whole == Plan::kStream || (p.n & 255) != 0 ? whole_ns - whole_ns / 20 : 0;
+  auto is_tiles = [](Plan q) { return q == Plan::kTiles256 || q == Plan::kTiles128 || q == Plan::kTiles128x128; };
   // N not a multiple of 256 (29568, 1408): the columns up to the last multiple of 256 go to whatever kernel that shape
   // gets, the remaining columns (weight rows) to a launch of their own that writes into the same rows of the result
   // (8192 x 29568 x 8192: 4.1 -> 1.3 ms).
@@ -1237,8 +1013,9 @@ int launch_sized(const Params& p, hipStream_t stream) {
   }
   switch (whole) {
     case Plan::kStream: return launch_skinny<OUT_BF16>(p, stream);
-    case Plan::kTiles256: return launch_fast<4, OUT_BF16>(p, stream);
-    case Plan::kTiles128: return launch_fast<2, OUT_BF16>(p, stream);
+    case Plan::kTiles256: return launch_tiles<8, 8, OUT_BF16>(p, stream);
+    case Plan::kTiles128: return launch_tiles<4, 8, OUT_BF16>(p, stream);
+    case Plan::kTiles128x128: return launch_tiles<4, 4, OUT_BF16>(p, stream);
     case Plan::kOther: break;
   }
   if (tiles(256, 256) >= cus) return launch_cfg<256, 256, OUT_BF16>(p, stream);

@@ -6,7 +6,7 @@
 //   * Persistent workgroups walk the (group, m-tile, n-tile) list derived on the device from
 //     problem_sizes; each XCD owns a contiguous part of the list, whose neighbouring tiles share the
 //     group's weight panel in that XCD's L2.
-//   * The K loop is Tile256Loop's.  Its load stream runs two steps ahead of the MFMAs and continues across tile and
+//   * The K loop is TileLoop's.  Its load stream runs two steps ahead of the MFMAs and continues across tile and
 //     group borders.  Rows past the end of a group load the group's last row again (never another group's memory past
 //     the tensor) and are not stored.
 // -------------------------------------------------------------------------------------------------
@@ -96,22 +96,22 @@ __global__ __launch_bounds__(256, 1) void grouped16_gemm_256_kernel(const Params
     return r;
   };
 
-  // ---- LDS-direct loads of a step.  Load u < 4: 8 rows of A's tiles 0..3 of a wavefront (rows 0..63 of either half of the
-  // tile), u = 4..11: 8 rows of B, u = 12..15: 8 rows of A's tiles 4..7.  Lane L lands at unit +L, i.e. row +(L>>3), chunk
-  // position L&7, which must hold global chunk (L&7) ^ ((row>>1)&7) = (L&7) ^ ((L>>4) | ((u&1)<<2)).
+  // ---- LDS-direct loads of a step.  A load is 8 rows: lane L lands at unit +L, i.e. row +(L>>3), chunk position L&7, which
+  // must hold global chunk (L&7) ^ ((row>>1)&7) = (L&7) ^ ((L>>4) | ((j&1)<<2)) of load j.
+  using Loop = TileLoop<BF16_MMA ? Mma::kBf16 : Mma::kF16, 8, 8, 2>;
   const uint32_t lds_base = (uint32_t)(uintptr_t)((__attribute__((address_space(3))) void*)lds);
   const uint32_t chunk_even = (uint32_t)(((lane & 7) ^ (lane >> 4)) << 4), chunk_odd = chunk_even ^ 64u;
   const int a_row0 = wm * 128 + wn * 32, b_row0 = wave * 64;  // the wavefront's share (A: and 64 rows further on)
   uint32_t a_off[8], b_off[8];
 #pragma unroll
   for (int j = 0; j < 8; ++j) b_off[j] = (uint32_t)(b_row0 + 8 * j + (lane >> 3)) * (uint32_t)kb + ((j & 1) ? chunk_odd : chunk_even);
-  const uint32_t a_lds = lds_base + (uint32_t)a_row0 * 128u, b_lds = lds_base + 65536u + (uint32_t)b_row0 * 128u;
+  const uint32_t a_lds = lds_base + (uint32_t)a_row0 * 128u, b_lds = lds_base + 2 * Loop::kABytes + (uint32_t)b_row0 * 128u;
 
   // ---- load stream: the step the next loads are issued for (l_ks of the tile lp) and the tile after it (np)
   Tile lp = tile_info(first_tile);
   Tile np = lp;
   int l_ks = 0;
-  uint32_t l_buf = 0;  // 0 or 32768
+  uint32_t l_buf = 0;  // 0 or the bytes of a buffer (A's and B's are of one size)
   auto enter_tile = [&]() {
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
@@ -120,17 +120,18 @@ __global__ __launch_bounds__(256, 1) void grouped16_gemm_256_kernel(const Params
     }
   };
   enter_tile();
-  auto load = [&](auto u_c) {
-    constexpr int u = decltype(u_c)::value;
-    if constexpr (u >= 4 && u < 12) {
-      lds_dma16<(u - 4) * 1024>(b_lds + l_buf, lp.b, b_off[u - 4]);
-    } else {
-      constexpr int j = u < 4 ? u : u - 8;
-      lds_dma16<(j >> 2) * 8192 + (j & 3) * 1024>(a_lds + l_buf, lp.a, a_off[j]);
-    }
+  auto load = [&](auto code) {
+    constexpr int u = decltype(code)::value;
+    if constexpr (u >= kLoadB) lds_dma16<(u - kLoadB) * 1024>(b_lds + l_buf, lp.b, b_off[u - kLoadB]);
+    else lds_dma16<(u >> 2) * 8192 + (u & 3) * 1024>(a_lds + l_buf, lp.a, a_off[u]);
+  };
+  auto load_step = [&]() {  // in the order of the loop's
+    static_for<4>(load);
+    static_for<8>([&](auto j) { load(std::integral_constant<int, kLoadB + decltype(j)::value>{}); });
+    static_for<4>([&](auto u) { load(std::integral_constant<int, 4 + decltype(u)::value>{}); });
   };
   auto advance = [&]() {
-    l_buf ^= 32768u;
+    l_buf ^= (uint32_t)Loop::kABytes;
     lp.a += 128;
     lp.b += 128;
     if (++l_ks == nk) {
@@ -140,7 +141,7 @@ __global__ __launch_bounds__(256, 1) void grouped16_gemm_256_kernel(const Params
     }
   };
 
-  Tile256Loop<BF16_MMA ? Mma::kBf16 : Mma::kF16> loop;
+  Loop loop;
   loop.init(lds_base, lane, wm, wn);
   auto& acc = loop.acc;
 
@@ -148,11 +149,11 @@ __global__ __launch_bounds__(256, 1) void grouped16_gemm_256_kernel(const Params
   // already leaves the first tile during this prologue.
   const int tiles_ahead = nk == 2 ? 2 : 1;
   np = (first_tile + slots < range_end) ? tile_info(first_tile + slots) : lp;
-static_for<16>(load);  // step 0
+  load_step();  // step 0
   advance();
-  static_for<16>(load);  // step 1
+  load_step();  // step 1
   advance();
-  loop.template fence<16>();
+  loop.fence();
   loop.first_fragments();
 
   Tile ct = tile_info(first_tile);
@@ -160,10 +161,10 @@ static_for<16>(load);  // step 0
     // prepare the tile the stream enters next (past the end of the list: any valid tile, loaded and ignored)
     const Tile nt_info = (c_tile + slots < range_end) ? tile_info(c_tile + slots) : ct;
     np = (c_tile + tiles_ahead * slots < range_end) ? tile_info(c_tile + tiles_ahead * slots) : ct;
-    loop.template step<16, true>(load, [](auto) {});
+    loop.template step<true>(load, [](auto) {});
     advance();
     for (int c_ks = 1; c_ks < nk; ++c_ks) {
-      loop.template step<16, false>(load, [](auto) {});
+      loop.template step<false>(load, [](auto) {});
       advance();
     }
     loop.settle();
@@ -175,7 +176,7 @@ static_for<16>(load);  // step 0
     // one 32-bit lane offset next to a wave-uniform result address keep the epilogue out of the spill area.
     int elane = lane;
     asm volatile("" : "+v"(elane));
-    uint8_t* stage = reinterpret_cast<uint8_t*>(lds) + kTile256Bytes + wave * 4608;
+    uint8_t* stage = reinterpret_cast<uint8_t*>(lds) + Loop::kTileBytes + wave * 4608;
     uint8_t* wr = stage + (elane & 15) * 144 + (elane >> 4) * 8;
     const uint8_t* rd = stage + (elane >> 3) * 144 + (elane & 7) * 16;
     const uint32_t ooff = ((uint32_t)(elane >> 3) * (uint32_t)p.n + (uint32_t)(elane & 7) * 8u) * 2u;
@@ -215,7 +216,7 @@ static_for<16>(load);  // step 0
 template <bool BF16_MMA, bool OUT_BF16, bool STREAM_OUT>
 int launch_grouped16_fast_cfg(const Params& p, int cus, hipStream_t stream) {
   auto kern = grouped16_gemm_256_kernel<BF16_MMA, OUT_BF16, STREAM_OUT>;
-  constexpr int lds_bytes = kTile256Bytes + 4 * 4608;  // 128 KiB of tiles + the epilogue's 18 KiB
+  constexpr int lds_bytes = TileLoop<Mma::kF16, 8, 8, 2>::kTileBytes + 4 * 4608;  // 128 KiB of tiles + the epilogue's 18 KiB
   if (note_launch("grouped16_gemm_256_kernel<stream_out=%d> grid=%d", (int)STREAM_OUT, cus & ~7)) return NVF_OK;
   static std::atomic<uint64_t> configured{0};  // one bit per device
   if (const int rc = allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds_bytes, configured)) return rc;

@@ -859,6 +859,34 @@ def test_mxfp8_gemm_persistent_256_tile_kernel_full_compare(dev, shape):
     assert torch.equal(out, out2)
 
 
+@pytest.mark.parametrize("shape, tile", [((768, 3072, 512), "TM=2,TN=2"), ((640, 3072, 1088), "TM=2,TN=2"), ((300, 4096, 544), "TM=2,TN=2"),
+                                         ((1153, 1040, 1120), "TM=2,TN=2"), ((200, 8208, 1024), "TM=2,TN=2"), ((2001, 2064, 1024), "TM=2"),
+                                         ((1030, 4112, 1056), "TM=2"), ((2300, 6160, 1024), "TM=4"), ((2200, 8176, 1056), "TM=2")])
+def test_mxfp8_gemm_128x128_tiles_and_a_last_column_tile_with_fewer_columns(dev, shape, tile):
+    """128x128 tiles (four buffers: 4 to 9 steps), and tiles of every size of which the last hold 16 to 240 columns: their
+    missing weight rows load the last one again, their scale tile may not exist, and their columns are not stored.  NaN code in
+    every scale byte of the padding, every element against the oracle, both output types, run-to-run bit equality."""
+    from fuser_amd import capi
+
+    m, n, k = shape
+    plan = capi.describe_dispatch("mxfp8_scaled_mm", m, n, k)
+    assert plan.startswith(f"mxfp8_gemm_256_kernel<{tile},stream_out=") and ("ragged_n" in plan) == (n % (128 if "TN" in tile else 256) != 0) and ";" not in plan, plan
+    gen = torch.Generator().manual_seed(m * 31 + n)
+    (a, sa), (b, sb) = _mxfp8_operand(m, k, gen, 1.0), _mxfp8_operand(n, k, gen, 1.0)
+    ref = O.ref_mxfp8_scaled_mm(a, b, sa, sb, 0.75)
+    sa, sb = sa.clone(), sb.clone()
+    sa[O.linear_to_swizzled_128_4(torch.ones(m, k // 32, dtype=torch.uint8)) == 0] = 0xFF
+    sb[O.linear_to_swizzled_128_4(torch.ones(n, k // 32, dtype=torch.uint8)) == 0] = 0xFF
+    scale = ref.abs().amax(dim=1, keepdim=True).clamp(min=1e-30)
+    for dtype in (torch.bfloat16, torch.float16):
+        if dtype == torch.float16 and ref.abs().max() > 6e4:
+            continue
+        out = _run_mxfp8(a, b, sa, sb, 0.75, dtype, dev)
+        assert out.shape == (m, n)
+        assert ((out.float().cpu() - ref).abs() / scale).max().item() <= GEMM_MAX_REL, (shape, dtype)
+        assert torch.equal(out, _run_mxfp8(a, b, sa, sb, 0.75, dtype, dev))
+
+
 @pytest.mark.parametrize("shape", [(300, 14336, 512), (136, 12288, 512), (80, 28672, 256), (520, 14336, 512), (640, 14336, 1024),
                                    (700, 12288, 256), (2049, 4096, 512), (390, 8192, 1280), (200, 65536, 256), (130, 65536, 256),
                                    (300, 14336, 352), (520, 14336, 288), (700, 12288, 320), (1000, 5632, 2880)])
