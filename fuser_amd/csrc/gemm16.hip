@@ -459,10 +459,10 @@ int launch_sized(const Params& p, int64_t m_hint, int cus, void* workspace, int6
   }
   if constexpr (!NVFP4) {
     // grouped_mm with groups of 128 rows or more on average and tiles for half the compute units: persistent LDS-direct
-    // kernel (at 128..255 rows per group the 128x128 tile kernel used to run: 8 experts, 1536 rows, N=14336, K=4096 373 ->
-    // 272 us; 64 experts, 8192 rows, N=7168, K=2048 571 -> 449 us; below 128 rows per group it stays faster)
-    if (!dense && m_hint >= 128 * (int64_t)p.groups && tiles(256, 256) >= cus / 2 && (p.n & 255) == 0 && (p.k & 63) == 0 &&
-        p.k >= 128 && (int64_t)p.k * 2 * 256 < (1ll << 31))
+    // kernel with 256x256 tiles (at 128..255 rows per group the 128x128 tile kernel used to run: 8 experts, 1536 rows, N=14336,
+    // K=4096 373 -> 272 us; 64 experts, 8192 rows, N=7168, K=2048 571 -> 449 us)
+    const bool lds_direct = !dense && (p.n & 7) == 0 && (p.k & 63) == 0 && (int64_t)p.k * 2 * 256 < (1ll << 31);
+    if (lds_direct && m_hint >= 128 * (int64_t)p.groups && tiles(256, 256) >= cus / 2 && p.k >= ((p.n & 255) == 0 ? 128 : 256))
       return launch_grouped16_fast<BF16_MMA, OUT_BF16>(p, cus, stream);
     // A decode step: few rows per group on average.  The streaming kernel's partial sums cost more per item the shallower K
     // and the more rows there are; the 128x128 tiles lose most where they leave compute units idle.  Tile kernel against
@@ -477,6 +477,11 @@ int launch_sized(const Params& p, int64_t m_hint, int cus, void* workspace, int6
     else if (p.k >= 2048 || (p.k >= 1024 && 4 * first_tiles <= 3 * (int64_t)cus)) rows_on_average = 16;
     if (!dense && m_hint <= rows_on_average * (int64_t)p.groups && (m_hint / kStream16Rows + p.groups) * ceil_div(p.n, 32) < (1ll << 31))
       return launch_grouped16_streaming<BF16_MMA>(p, cus, stream);
+    // ... else the same kernel with 128x128 tiles, except for a wide N with a shallow K: there its tiles end too often for one
+    // workgroup per compute unit, the tile kernels run two (32 experts of 13824 x 2112, 1838 rows 452 / 478 us, 64 of 11840 x
+    // 2560, 1026 rows 733 / 750; 64 of 8000 x 2048, 1254 rows 458 / 399).
+    if (lds_direct && p.k >= 256 && (p.n <= 10240 || p.k >= 3072))
+      return launch_grouped16_small_tiles<BF16_MMA, OUT_BF16>(p, cus, stream);
   }
   if constexpr (NVFP4) {
     // Grouped NVFP4: the groups of 1..32 rows and those of 33..128 rows (MoE decode, the small experts of a prefill) have

@@ -1,29 +1,49 @@
-// Persistent 256x256 kernel for grouped_mm (16-bit operands) of gemm16.hip (included there, inside namespace nvf).
+// Persistent kernel with 256x256 or 128x128 tiles for grouped_mm (16-bit operands) of gemm16.hip (included there, inside namespace nvf).
 // -------------------------------------------------------------------------------------------------
-// grouped_mm fast path (16-bit operands): 256x256 tiles, N % 256 == 0, K % 64 == 0, K >= 128.
+// grouped_mm fast path (16-bit operands): 256x256 tiles, N % 256 == 0, K % 64 == 0.
 // Bound by the power limit of the MFMAs (bf16 8192^3 as one group: 1.50..1.57 PFLOP/s, 810..841 -> 703..735 us against a K loop
 // of 32x32 MFMAs with all of a step's loads in one half of it; 8 experts, 8192 rows, N = 14336, K = 4096 887..907 -> 766..781).
+// 128x128 tiles: groups of fewer rows, or too few 256x256 tiles; any N % 8 == 0.  Bound by the weights' way out of HBM, for which
+// four buffers keep three steps' loads in flight.  Against the 128x128 tile kernel (two workgroups per compute unit, a barrier and
+// a register stage per step): 64 experts of 2048 x 4096, 2048 rows 288 -> 212 us, 16 of 4096 x 4096, 1000 rows 178 -> 127, 8 of
+// 14336 x 4096, 512 rows 220 -> 196, 32 of 2048 x 2048, 2048 rows 86 -> 59, 8 of 2560 x 1600, 474 rows 29 -> 16; 37 shapes of 16 to
+// 2048 rows per group, with the 256x256 tiles', 1.22 times as fast in the geometric mean, none slower.  256x256 tiles with a
+// short last column tile: 8 experts of 6632 x 4096, 16384 rows 1095 -> 687 us.
 //   * Persistent workgroups walk the (group, m-tile, n-tile) list derived on the device from
 //     problem_sizes; each XCD owns a contiguous part of the list, whose neighbouring tiles share the
 //     group's weight panel in that XCD's L2.
-//   * The K loop is TileLoop's.  Its load stream runs two steps ahead of the MFMAs and continues across tile and
-//     group borders.  Rows past the end of a group load the group's last row again (never another group's memory past
-//     the tensor) and are not stored.
+//   * The K loop is TileLoop's.  Its load stream runs NBUF steps ahead of the MFMAs and continues across tile and
+//     group borders.  Rows past the end of a group (and weight rows past N) load the last row again (never another group's
+//     memory past the tensor) and are not stored.
+//   * The groups' rows and places are kept in LDS: a look into global memory at every new tile would wait for all of the
+//     stream's loads.
 // -------------------------------------------------------------------------------------------------
-template <bool BF16_MMA, bool OUT_BF16, bool STREAM_OUT>
-__global__ __launch_bounds__(256, 1) void grouped16_gemm_256_kernel(const Params p) {
-  constexpr int BM = 256, BN = 256;
+template <int NI, int NJ, int NBUF>
+struct Grouped16Tiles {
+  static constexpr int BM = 32 * NI, BN = 32 * NJ;
+  static constexpr int kTileBytes = TileLoop<Mma::kF16, NI, NJ, NBUF>::kTileBytes;
+  static constexpr int kLdsBytes = kTileBytes + 4 * 4608 + (kMaxGroups + 1) * 4 + kMaxGroups * 8;  // tiles, the epilogue's, groups
+  static_assert(kLdsBytes <= 160 * 1024, "LDS");
+};
+
+// STREAM_OUT, STREAM_B: results are stored, weights are read past the last-level cache.  RAGGED_N: N is no multiple of the tile's
+// columns, but of 8.
+template <int NI, int NJ, int NBUF, bool BF16_MMA, bool OUT_BF16, bool STREAM_OUT, bool STREAM_B, bool RAGGED_N>
+__global__ __launch_bounds__(256, 1) void grouped16_tile_kernel(const Params p) {
+  using T = Grouped16Tiles<NI, NJ, NBUF>;
+  constexpr int BM = T::BM, BN = T::BN;
   constexpr int kBand = 4;  // m-tiles that share a weight panel while it is in an XCD's L2 (8: measured no better)
   extern __shared__ u32x4 lds[];
-  __shared__ int tile_prefix[kMaxGroups + 1];
+  u32x2* const group_rows = reinterpret_cast<u32x2*>(reinterpret_cast<char*>(lds) + T::kTileBytes + 4 * 4608);  // {rows, first row}
+  int* const tile_prefix = reinterpret_cast<int*>(group_rows + kMaxGroups);
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 1, wn = wave & 1;
-  const int tiles_n = p.n / BN;
+  const int tiles_n = RAGGED_N ? (p.n + BN - 1) / BN : p.n / BN;
 
-  // ---- work list: prefix sums of 256-row tiles per group (one wavefront, 64 groups per round)
+  // ---- work list: prefix sums of BM-row tiles per group (one wavefront, 64 groups per round)
   if (wave == 0) {
     int running = 0;
     for (int base = 0; base < p.groups; base += 64) {
@@ -32,6 +52,7 @@ __global__ __launch_bounds__(256, 1) void grouped16_gemm_256_kernel(const Params
       if (g < p.groups) {
         const int mg = p.problem_sizes[g * 3];
         cnt = mg > 0 ? (mg + BM - 1) / BM : 0;
+        group_rows[g] = u32x2{(uint32_t)mg, (uint32_t)p.expert_offsets[g]};
       }
       int incl = cnt;
 #pragma unroll
@@ -72,9 +93,9 @@ __global__ __launch_bounds__(256, 1) void grouped16_gemm_256_kernel(const Params
       if (t < tile_prefix[mid] * per_m) hi = mid; else lo = mid;
     }
     const int g = __builtin_amdgcn_readfirstlane(lo);
-    // (loaded through the vector path, which is coherent with this kernel's own stores; made scalar here)
-    const int m_g = __builtin_amdgcn_readfirstlane(p.problem_sizes[g * 3]);
-    const int64_t row_off = __builtin_amdgcn_readfirstlane(p.expert_offsets[g]);
+    const u32x2 rows = group_rows[g];
+    const int m_g = __builtin_amdgcn_readfirstlane((int)rows[0]);
+    const int64_t row_off = __builtin_amdgcn_readfirstlane((int)rows[1]);
     const int tiles_m = (m_g + BM - 1) / BM;
     const int local = __builtin_amdgcn_readfirstlane(t - tile_prefix[g] * per_m);
     // bands of up to kBand m-tiles of near-equal height (9 m-tiles: 5 + 4), n-major inside a band
@@ -98,46 +119,62 @@ __global__ __launch_bounds__(256, 1) void grouped16_gemm_256_kernel(const Params
 
   // ---- LDS-direct loads of a step.  A load is 8 rows: lane L lands at unit +L, i.e. row +(L>>3), chunk position L&7, which
   // must hold global chunk (L&7) ^ ((row>>1)&7) = (L&7) ^ ((L>>4) | ((j&1)<<2)) of load j.
-  using Loop = TileLoop<BF16_MMA ? Mma::kBf16 : Mma::kF16, 8, 8, 2>;
+  using Loop = TileLoop<BF16_MMA ? Mma::kBf16 : Mma::kF16, NI, NJ, NBUF>;
   const uint32_t lds_base = (uint32_t)(uintptr_t)((__attribute__((address_space(3))) void*)lds);
   const uint32_t chunk_even = (uint32_t)(((lane & 7) ^ (lane >> 4)) << 4), chunk_odd = chunk_even ^ 64u;
-  const int a_row0 = wm * 128 + wn * 32, b_row0 = wave * 64;  // the wavefront's share (A: and 64 rows further on)
-  uint32_t a_off[8], b_off[8];
-#pragma unroll
-  for (int j = 0; j < 8; ++j) b_off[j] = (uint32_t)(b_row0 + 8 * j + (lane >> 3)) * (uint32_t)kb + ((j & 1) ? chunk_odd : chunk_even);
-  const uint32_t a_lds = lds_base + (uint32_t)a_row0 * 128u, b_lds = lds_base + 2 * Loop::kABytes + (uint32_t)b_row0 * 128u;
+  // the wavefront's share: rows of A's first half (the second's: 8 NI rows further on), of B
+  const int a_row0 = wm * (16 * NI) + wn * (4 * NI), b_row0 = wave * (8 * NJ);
+  const uint32_t a_lds = lds_base + (uint32_t)a_row0 * 128u, b_lds = lds_base + NBUF * Loop::kABytes + (uint32_t)b_row0 * 128u;
+  uint32_t a_off[NI], b_off[NJ];
 
-  // ---- load stream: the step the next loads are issued for (l_ks of the tile lp) and the tile after it (np)
-  Tile lp = tile_info(first_tile);
-  Tile np = lp;
-  int l_ks = 0;
-  uint32_t l_buf = 0;  // 0 or the bytes of a buffer (A's and B's are of one size)
-  auto enter_tile = [&]() {
+  // ---- load stream: the step the next loads are issued for (l_ks of the tile lp) and the tile after it (np; past the end
+  // of the list: a valid tile, loaded and ignored)
+  const Tile first_info = tile_info(first_tile);
+  Tile lp = first_info, np;
+  int l_ks = 0, l_buf = 0, stream_tile = first_tile;
+  uint32_t l_a = a_lds, l_b = b_lds;  // the step's buffer
+  auto prepare_next = [&]() {
+    stream_tile += slots;
+    np = stream_tile < range_end ? tile_info(stream_tile) : first_info;
+  };
+  prepare_next();
+  auto enter_tile = [&](bool first) {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const uint32_t row = (uint32_t)(a_row0 + 64 * (j >> 2) + 8 * (j & 3) + (lane >> 3));
-      a_off[j] = min(row, (uint32_t)(lp.valid - 1)) * (uint32_t)kb + ((j & 1) ? chunk_odd : chunk_even);
+    for (int u = 0; u < NI; ++u) {
+      const uint32_t row = (uint32_t)(a_row0 + (u < NI / 2 ? 0 : 4 * NI) + 8 * u + (lane >> 3));
+      a_off[u] = min(row, (uint32_t)(lp.valid - 1)) * (uint32_t)kb + ((u & 1) ? chunk_odd : chunk_even);
+    }
+    if (!RAGGED_N && !first) return;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      uint32_t row = (uint32_t)(b_row0 + 8 * j + (lane >> 3));
+      if (RAGGED_N) row = min(row, (uint32_t)(p.n - lp.n0 - 1));
+      b_off[j] = row * (uint32_t)kb + ((j & 1) ? chunk_odd : chunk_even);
     }
   };
-  enter_tile();
+  enter_tile(true);
   auto load = [&](auto code) {
     constexpr int u = decltype(code)::value;
-    if constexpr (u >= kLoadB) lds_dma16<(u - kLoadB) * 1024>(b_lds + l_buf, lp.b, b_off[u - kLoadB]);
-    else lds_dma16<(u >> 2) * 8192 + (u & 3) * 1024>(a_lds + l_buf, lp.a, a_off[u]);
+    if constexpr (u >= kLoadB) lds_dma16<(u - kLoadB) * 1024, STREAM_B>(l_b, lp.b, b_off[u - kLoadB]);
+    else lds_dma16<(u + (u < NI / 2 ? 0 : NI / 2)) * 1024>(l_a, lp.a, a_off[u]);
   };
   auto load_step = [&]() {  // in the order of the loop's
-    static_for<4>(load);
-    static_for<8>([&](auto j) { load(std::integral_constant<int, kLoadB + decltype(j)::value>{}); });
-    static_for<4>([&](auto u) { load(std::integral_constant<int, 4 + decltype(u)::value>{}); });
+    static_for<NI / 2>(load);
+    static_for<NJ>([&](auto j) { load(std::integral_constant<int, kLoadB + decltype(j)::value>{}); });
+    static_for<NI / 2>([&](auto u) { load(std::integral_constant<int, NI / 2 + decltype(u)::value>{}); });
   };
   auto advance = [&]() {
-    l_buf ^= (uint32_t)Loop::kABytes;
+    const int by = l_buf == NBUF - 1 ? 1 - NBUF : 1;
+    l_buf += by;
+    l_a += by * Loop::kABytes;
+    l_b += by * Loop::kBBytes;
     lp.a += 128;
     lp.b += 128;
     if (++l_ks == nk) {
       l_ks = 0;
       lp = np;
-      enter_tile();
+      enter_tile(false);
+      prepare_next();
     }
   };
 
@@ -145,30 +182,23 @@ __global__ __launch_bounds__(256, 1) void grouped16_gemm_256_kernel(const Params
   loop.init(lds_base, lane, wm, wn);
   auto& acc = loop.acc;
 
-  // The stream runs two steps ahead of the MFMAs; with two steps per tile it is a whole tile ahead and
-  // already leaves the first tile during this prologue.
-  const int tiles_ahead = nk == 2 ? 2 : 1;
-  np = (first_tile + slots < range_end) ? tile_info(first_tile + slots) : lp;
-  load_step();  // step 0
-  advance();
-  load_step();  // step 1
-  advance();
+  for (int i = 0; i < NBUF; ++i) {
+    load_step();
+    advance();
+  }
   loop.fence();
   loop.first_fragments();
 
-  Tile ct = tile_info(first_tile);
   for (int c_tile = first_tile; c_tile < range_end; c_tile += slots) {
-    // prepare the tile the stream enters next (past the end of the list: any valid tile, loaded and ignored)
-    const Tile nt_info = (c_tile + slots < range_end) ? tile_info(c_tile + slots) : ct;
-    np = (c_tile + tiles_ahead * slots < range_end) ? tile_info(c_tile + tiles_ahead * slots) : ct;
     loop.template step<true>(load, [](auto) {});
     advance();
     for (int c_ks = 1; c_ks < nk; ++c_ks) {
       loop.template step<false>(load, [](auto) {});
       advance();
     }
+    const Tile ct = tile_info(c_tile);
     loop.settle();
-    // ---- epilogue of this tile; the loads of the next tile's first two steps are already in flight.
+    // ---- epilogue of this tile; the loads of the next steps are already in flight.
     // A lane holds 8-byte pieces of 16 rows per tile; stored like that, a tile is 8192 sixteen-byte write
     // requests per compute unit.  Every 32x64 block of the wavefront's tile is therefore turned round in a
     // private 4.5 KiB of LDS (32 rows of 128 bytes at a pitch of 144 bytes) and leaves in 16-byte pieces, 8 lanes
@@ -180,12 +210,12 @@ __global__ __launch_bounds__(256, 1) void grouped16_gemm_256_kernel(const Params
     uint8_t* wr = stage + (elane & 15) * 144 + (elane >> 4) * 8;
     const uint8_t* rd = stage + (elane >> 3) * 144 + (elane & 7) * 16;
     const uint32_t ooff = ((uint32_t)(elane >> 3) * (uint32_t)p.n + (uint32_t)(elane & 7) * 8u) * 2u;
-    uint8_t* obase = reinterpret_cast<uint8_t*>(static_cast<uint16_t*>(p.out) + (ct.out_row + wm * 128) * (int64_t)p.n + ct.n0 + wn * 128);
-    const int erow = wm * 128 + (elane >> 3);
+    uint8_t* obase = reinterpret_cast<uint8_t*>(static_cast<uint16_t*>(p.out) + (ct.out_row + wm * (16 * NI)) * (int64_t)p.n + ct.n0 + wn * (16 * NJ));
+    const int erow = wm * (16 * NI) + (elane >> 3), cols_left = p.n - ct.n0 - wn * (16 * NJ) - (elane & 7) * 8;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < NI / 2; ++i) {
 #pragma unroll
-      for (int jh = 0; jh < 2; ++jh) {
+      for (int jh = 0; jh < NJ / 4; ++jh) {
 #pragma unroll
         for (int t = 0; t < 8; ++t) {  // the block's 2 x 4 tiles
           const f32x4 c = acc[2 * i + (t >> 2)][4 * jh + (t & 3)];
@@ -199,7 +229,7 @@ __global__ __launch_bounds__(256, 1) void grouped16_gemm_256_kernel(const Params
         for (int t = 0; t < 4; ++t) {
           const int brow = i * 32 + 8 * t;  // first of the 8 rows of this piece, in the wavefront's tile
           const u32x4 v = *reinterpret_cast<const u32x4*>(rd + t * 1152);
-          if (erow + brow < ct.valid) {
+          if (erow + brow < ct.valid && (!RAGGED_N || jh * 64 < cols_left)) {
             u32x4* dst = reinterpret_cast<u32x4*>(obase + ((int64_t)brow * p.n + jh * 64) * 2 + ooff);
             if constexpr (STREAM_OUT) __builtin_nontemporal_store(v, dst);
             else *dst = v;
@@ -208,20 +238,21 @@ __global__ __launch_bounds__(256, 1) void grouped16_gemm_256_kernel(const Params
         asm volatile("" ::: "memory");
       }
     }
-    ct = nt_info;
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no LDS-direct load may outlive the workgroup
 }
 
-template <bool BF16_MMA, bool OUT_BF16, bool STREAM_OUT>
-int launch_grouped16_fast_cfg(const Params& p, int cus, hipStream_t stream) {
-  auto kern = grouped16_gemm_256_kernel<BF16_MMA, OUT_BF16, STREAM_OUT>;
-  constexpr int lds_bytes = TileLoop<Mma::kF16, 8, 8, 2>::kTileBytes + 4 * 4608;  // 128 KiB of tiles + the epilogue's 18 KiB
-  if (note_launch("grouped16_gemm_256_kernel<stream_out=%d> grid=%d", (int)STREAM_OUT, cus & ~7)) return NVF_OK;
+template <int NI, int NJ, int NBUF, bool BF16_MMA, bool OUT_BF16, bool STREAM_OUT, bool STREAM_B, bool RAGGED_N>
+int launch_grouped16_tiles_cfg(const Params& p, int cus, hipStream_t stream) {
+  using T = Grouped16Tiles<NI, NJ, NBUF>;
+  auto kern = grouped16_tile_kernel<NI, NJ, NBUF, BF16_MMA, OUT_BF16, STREAM_OUT, STREAM_B, RAGGED_N>;
+  if (NJ == 8 ? note_launch("grouped16_gemm_256_kernel<stream_out=%d%s> grid=%d", (int)STREAM_OUT, RAGGED_N ? ",ragged_n" : "", cus & ~7)
+              : note_launch("gemm16_kernel<%d,%d,buffers=%d,stream=%d> grid=%d", T::BM, T::BN, NBUF, (int)STREAM_B, cus & ~7))
+    return NVF_OK;
   static std::atomic<uint64_t> configured{0};  // one bit per device
-  if (const int rc = allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds_bytes, configured)) return rc;
-  hipLaunchKernelGGL(kern, dim3((unsigned)(cus & ~7)), dim3(256), lds_bytes, stream, p);
-  return check_launch("grouped16_gemm_256_kernel");
+  if (const int rc = allow_dynamic_lds(reinterpret_cast<const void*>(kern), T::kLdsBytes, configured)) return rc;
+  hipLaunchKernelGGL(kern, dim3((unsigned)(cus & ~7)), dim3(256), T::kLdsBytes, stream, p);
+  return check_launch("grouped16_tile_kernel");
 }
 
 template <bool BF16_MMA, bool OUT_BF16>
@@ -230,6 +261,18 @@ int launch_grouped16_fast(const Params& p, int cus, hipStream_t stream) {
   // non-temporal stores, which keeps it from pushing operand panels out (single 8192-row group, 8192^3: +2.6 %,
   // 16384 x 4096 x 4096: +7 %); smaller problems are better off with plain stores.
   const int64_t bytes = 2 * ((int64_t)p.m * p.k + (int64_t)p.groups * p.n * p.k + (int64_t)p.m * p.n);
-  return bytes > ((int64_t)224 << 20) ? launch_grouped16_fast_cfg<BF16_MMA, OUT_BF16, true>(p, cus, stream)
-                                       : launch_grouped16_fast_cfg<BF16_MMA, OUT_BF16, false>(p, cus, stream);
+  const bool past = bytes > ((int64_t)224 << 20);
+  if ((p.n & 255) != 0)
+    return past ? launch_grouped16_tiles_cfg<8, 8, 2, BF16_MMA, OUT_BF16, true, false, true>(p, cus, stream)
+                : launch_grouped16_tiles_cfg<8, 8, 2, BF16_MMA, OUT_BF16, false, false, true>(p, cus, stream);
+  return past ? launch_grouped16_tiles_cfg<8, 8, 2, BF16_MMA, OUT_BF16, true, false, false>(p, cus, stream)
+              : launch_grouped16_tiles_cfg<8, 8, 2, BF16_MMA, OUT_BF16, false, false, false>(p, cus, stream);
+}
+
+template <bool BF16_MMA, bool OUT_BF16>
+int launch_grouped16_small_tiles(const Params& p, int cus, hipStream_t stream) {
+  // Weights that the last-level cache cannot hold and that hardly more than one row tile per group reads: past it.
+  const bool past = p.m <= 128 * (int64_t)p.groups && 2.0 * p.groups * p.n * p.k > (double)(256 << 20);
+  return past ? launch_grouped16_tiles_cfg<4, 4, 4, BF16_MMA, OUT_BF16, false, true, true>(p, cus, stream)
+              : launch_grouped16_tiles_cfg<4, 4, 4, BF16_MMA, OUT_BF16, false, false, true>(p, cus, stream);
 }

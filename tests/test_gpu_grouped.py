@@ -117,7 +117,7 @@ def test_grouped_mm_group_ends_inside_tiles(dev, n, k):
     assert ((out[:rows].float().cpu() - ref[:rows]).abs() / scale).max().item() <= GEMM_MAX_REL
 
 
-@pytest.mark.parametrize("n,k", [(14336, 192), (8192, 128)])
+@pytest.mark.parametrize("n,k", [(14336, 192), (8192, 128), (8200, 256), (6152, 320)])
 def test_grouped_mm_persistent_kernel_from_128_rows_per_group(dev, n, k):
     """128 to 255 rows per group on average and a wide N: the persistent kernel (most of its 256-row tiles are short,
     one group is empty, two have a single tile of 1 and of 255 rows).  Every element compared, rows after the last
@@ -143,6 +143,40 @@ def test_grouped_mm_persistent_kernel_from_128_rows_per_group(dev, n, k):
         assert (out[rows:] == 7.0).all()
         scale = ref[:rows].abs().amax(dim=1, keepdim=True).clamp(min=1e-30)
         assert ((out[:rows].float().cpu() - ref[:rows]).abs() / scale).max().item() <= GEMM_MAX_REL, tensor_dtype
+
+
+@pytest.mark.parametrize("n,k,groups", [(1024, 256, 10), (1048, 320, 10), (392, 1088, 10), (8, 512, 10), (2048, 1088, 64), (3584, 1024, 40)])
+def test_grouped_mm_tiles_of_128_rows_and_columns(dev, n, k, groups):
+    """128x128 tiles (four buffers, 4 to 17 steps): groups of 127, 128, 129 rows, of one and none, a last column tile of 8 to 120
+    columns, n-tiles dealt to the XCDs and not, fewer tiles than compute units and more, weights within the last-level cache and
+    past it (the last two).  Every element compared, rows after the last group untouched, an infinity stays in its row, run-to-run
+    bit equality, both operand types."""
+    from fuser_amd import capi
+
+    sizes = ([127, 0, 128, 1, 129, 64, 33, 257, 0, 90] * 7)[:groups]
+    m = sum(sizes) + 5
+    plan = capi.describe_dispatch("grouped_mm", m, n, k, groups=len(sizes))
+    assert plan.startswith(f"gemm16_kernel<128,128,buffers=4,stream={int(2 * groups * n * k > 256 << 20)}>"), plan
+    for tensor_dtype, dt in ((torch.bfloat16, capi.BF16), (torch.float16, capi.F16)):
+        gen = torch.Generator().manual_seed(n + k)
+        a = torch.randn(m, k, generator=gen).to(tensor_dtype)
+        b = (torch.randn(len(sizes), n, k, generator=gen) * 0.05).to(tensor_dtype)
+        ps, eo, _, _ = _grouped_args(sizes, n, k, dev)
+        ad, bd, psd, eod = a.to(dev), b.to(dev), ps.to(dev), eo.to(dev)
+        outs = [torch.full((m, n), 7.0, dtype=tensor_dtype, device=dev) for _ in range(3)]
+        for i, out in enumerate(outs):
+            if i == 2:
+                ad[126, 3] = float("inf")  # the first group's last row, which the rows past the group load again
+            capi.check(capi.lib().nvf_grouped_mm(ad.data_ptr(), bd.data_ptr(), out.data_ptr(), psd.data_ptr(), eod.data_ptr(), len(sizes),
+                                                 m, n, k, dt, None))
+        torch.cuda.synchronize()
+        ref = O.ref_grouped_mm(a, b, ps, eo)
+        rows = sum(sizes)
+        assert (outs[0][rows:] == 7.0).all() and torch.equal(outs[0], outs[1])
+        scale = ref[:rows].abs().amax(dim=1, keepdim=True).clamp(min=1e-30)
+        assert ((outs[0][:rows].float().cpu() - ref[:rows]).abs() / scale).max().item() <= GEMM_MAX_REL, tensor_dtype
+        other = torch.arange(m) != 126
+        assert torch.equal(outs[2][other.to(dev)], outs[0][other.to(dev)]) and not torch.isfinite(outs[2][126].float()).any()
 
 
 def _moe_sizes_top2(tokens, experts, seed):
