@@ -369,7 +369,8 @@ __global__ __launch_bounds__(512) void nvfp4_gemm_256_kernel(const Params p) {
         constexpr int j = decltype(j_c)::value;
         if constexpr (m < BARRIER_ROW) {
           if constexpr (j == 0) load_a_frag(h, m + AHEAD);
-          if constexpr (m < NJ && j == 2) load_b_frag(h, 1, m);
+          // (TM == 2: its second sub-step begins at row 4)
+          if constexpr (TM == 4 ? m < NJ && j == 2 : m < NJ / 2 && (j == 1 || j == 2)) load_b_frag(h, 1, TM == 4 ? m : 2 * m + j - 1);
           constexpr int SLOTS = BARRIER_ROW * NJ, PARTS = 3 * NCU, slot = m * NJ + j;
           constexpr int first = slot * PARTS / SLOTS, count = (slot + 1) * PARTS / SLOTS - first;
           static_for<count>([&](auto part_c) {
