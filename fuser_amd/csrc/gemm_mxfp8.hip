@@ -929,9 +929,9 @@ Plan mxfp8_plan(int64_t m, int64_t n, int64_t k, int64_t cus, int64_t* ns = null
       // Skinny or persistent kernel by estimated duration.  Measured: 512 x 4096 x 7168 36.7 (persistent) against 31.8 us,
       // 700 x 2304 x 5120 22.3 / 23.3, 512 x 4096 x 4096 18.2 / 18.7, 300 x 3072 x 2048 11.4 / 7.1, 1500 x 1408 x 7168 34 / 42.
       // (With weights that change from call to call the skinny kernel takes, in percent of its estimate, 58-87 for K < 2048,
-      // 75-100 below 3072, 100 around 4096 and 105-150 above, over 45 shapes of 129..4000 rows; from 3072 on the estimate stays as
-      // it is, which the pinned dispatch of 1000 x 4096 x 14336 wants.)
-      const int64_t percent = m <= 128 || k >= 3072 ? 100 : k < 2048 ? 78 : 92;
+      // 75-100 below 3072, 100 around 4096, 100-130 up to 8000 and 105-200 above, over 45 shapes of 129..4000 rows; against the
+      // larger tiles the estimate stays as it is from K = 3072 on, which the pinned dispatch of 1000 x 4096 x 14336 wants.)
+      const int64_t percent = m <= 128 ? 100 : k < 2048 ? 78 : k < 3072 ? 92 : fast_ns != ns128x128 || k < 4608 ? 100 : k <= 8000 ? 110 : 130;
       if (skinny_ns * percent / 100 <= fast_ns) return Plan::kStream;
     } else {
       // No persistent kernel for the shape (ragged M or N, or too few tiles): up to 256 rows, i.e. four passes over
