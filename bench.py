@@ -358,7 +358,7 @@ def main():
                                     "roofline": {"bound": "mfma", "achieved": round(tf, 1), "peak": PEAK_F16_TFLOPS, "unit": "TFLOP/s",
                                                  "frac": round(tf / PEAK_F16_TFLOPS, 4),
                                                  "traffic": measured_traffic.get("grouped_mm_config4_bytes_per_launch"),
-                                                 "kernel": "grouped16_gemm_256_kernel"},
+                                                 "kernel": "grouped16_tile_kernel"},
                                     "hipblaslt_one_matmul_per_expert_ms": round(ms_v, 4)}
         if not args.no_cpu:
             ha, hb = a.cpu(), b.cpu()
@@ -559,7 +559,7 @@ def main():
         "config": {"workload": "BASELINE config 2: MXFP8 scaled GEMM M=N=K=8192, e8m0 per-32 scales in 128x4 layout, A row-major, B K-major"},
         "roofline": {"bound": "mfma", "achieved": round(tflops, 2), "peak": PEAK_FP8_TFLOPS, "unit": "TFLOP/s",
                      "frac": round(tflops / PEAK_FP8_TFLOPS, 4), "traffic": traffic,
-                     "kernel": "mxfp8_gemm_256_kernel", "flops_per_launch": flops},
+                     "kernel": "mxfp8_tile_kernel", "flops_per_launch": flops},
         "cpu_baseline": cpu,
         "extra": extra,
     }
