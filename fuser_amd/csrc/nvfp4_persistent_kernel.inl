@@ -314,10 +314,12 @@ __global__ __launch_bounds__(512) void nvfp4_gemm_256_kernel(const Params p) {
                    "+a"(acc[i + 1][2]), "+a"(acc[i + 1][3]));
   };
   // The compiler knows nothing of an MFMA in inline assembly: the wait states between the accumulators' last MFMA and their
-  // first other use, and between their zeroing and the first MFMA, are set here (4 passes and VALU writes need up to 7).
+  // first other use, and between their zeroing and the first MFMA, are set here (4 passes and VALU writes need up to 8).  The zeroing
+  // is before the first pin; the uses after the last MFMA depend on the second, which stands behind the wait.
   auto settle_acc = [&]() {
     pin_acc();
     asm volatile("s_nop 15" ::: "memory");
+    pin_acc();
   };
   zero_acc();
   settle_acc();

@@ -121,10 +121,11 @@ struct TileLoop {
 #pragma unroll
       for (int j = 0; j < NJ; j += 4) asm volatile("" : "+a"(acc[i][j]), "+a"(acc[i][j + 1]), "+a"(acc[i][j + 2]), "+a"(acc[i][j + 3]));
   }
-  // between the accumulators' last MFMA and their use (up to 12 wait states)
+  // between the accumulators' last MFMA and their use (up to 12 wait states): the wait comes after the MFMAs, as volatile
+  // statements keep their order, and the uses depend on the pin behind it
   __device__ __forceinline__ void settle() {
-    pin();
     asm volatile("s_nop 15" ::: "memory");
+    pin();
   }
   // The fragments that the first step finds in registers (it reads B's last tile itself); the loads of its step have landed.
   __device__ __forceinline__ void first_fragments() {
