@@ -539,8 +539,7 @@ int launch_tiles_cfg(const Params& p, hipStream_t stream) {
     return fail(NVF_ERR_LAUNCH, "mxfp8_tile_kernel: %d x %d is no multiple of %d x %d", p.m, p.n, T::BM, T::BN);
   const int cus = cu_count() & ~7;  // workgroup ids are dealt round-robin to the 8 XCDs
   const unsigned grid = (unsigned)(tiles >= cus ? cus : ((tiles + 7) / 8) * 8);
-  // (TM: 64 rows, TN: 64 columns of the tile each; 256 columns go without saying)
-  if (note_launch("mxfp8_gemm_256_kernel<TM=%d,%sstream_out=%d%s%s%s> grid=%u", NI / 2, NJ == 8 ? "" : "TN=2,", (int)STREAM_OUT, RAGGED_K ? ",ragged_k" : "",
+  if (note_launch("mxfp8_tile_kernel<%dx%d,stream_out=%d%s%s%s> grid=%u", T::BM, T::BN, (int)STREAM_OUT, RAGGED_K ? ",ragged_k" : "",
                   p.m % T::BM ? ",ragged_m" : "", p.n % T::BN ? ",ragged_n" : "", grid))
     return NVF_OK;
   static std::atomic<uint64_t> configured{0};  // one bit per device (and per instantiation of this launcher)

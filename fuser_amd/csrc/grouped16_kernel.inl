@@ -246,8 +246,8 @@ template <int NI, int NJ, int NBUF, bool BF16_MMA, bool OUT_BF16, bool STREAM_OU
 int launch_grouped16_tiles_cfg(const Params& p, int cus, hipStream_t stream) {
   using T = Grouped16Tiles<NI, NJ, NBUF>;
   auto kern = grouped16_tile_kernel<NI, NJ, NBUF, BF16_MMA, OUT_BF16, STREAM_OUT, STREAM_B, RAGGED_N>;
-  if (NJ == 8 ? note_launch("grouped16_gemm_256_kernel<stream_out=%d%s> grid=%d", (int)STREAM_OUT, RAGGED_N ? ",ragged_n" : "", cus & ~7)
-              : note_launch("gemm16_kernel<%d,%d,buffers=%d,stream=%d> grid=%d", T::BM, T::BN, NBUF, (int)STREAM_B, cus & ~7))
+  if (note_launch("grouped16_tile_kernel<%dx%d,stream_out=%d,stream_weights=%d%s> grid=%d", T::BM, T::BN, (int)STREAM_OUT, (int)STREAM_B,
+                  p.n % T::BN ? ",ragged_n" : "", cus & ~7))
     return NVF_OK;
   static std::atomic<uint64_t> configured{0};  // one bit per device
   if (const int rc = allow_dynamic_lds(reinterpret_cast<const void*>(kern), T::kLdsBytes, configured)) return rc;

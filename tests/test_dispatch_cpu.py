@@ -1,6 +1,9 @@
 """Which kernel every BASELINE shape is dispatched to, pinned without a GPU through the dry run of
 nvf_describe_dispatch (it walks the same launcher code as the real call and stops in front of each launch).
 A tuning constant that silently reroutes one of the benchmark's shapes fails here."""
+import re
+from pathlib import Path
+
 import pytest
 
 from fuser_amd import capi
@@ -17,8 +20,8 @@ def test_config1_small_nvfp4_gemm_streams_the_weights():
 
 
 def test_config2_mxfp8_8192_cubed_takes_the_persistent_256x256_kernel():
-    assert plan("mxfp8_scaled_mm", 8192, 8192, 8192) == "mxfp8_gemm_256_kernel<TM=4,stream_out=1> grid=256"
-    assert plan("mxfp8_scaled_mm", 8192, 8192, 8192, dtype=F16) == "mxfp8_gemm_256_kernel<TM=4,stream_out=1> grid=256"
+    assert plan("mxfp8_scaled_mm", 8192, 8192, 8192) == "mxfp8_tile_kernel<256x256,stream_out=1> grid=256"
+    assert plan("mxfp8_scaled_mm", 8192, 8192, 8192, dtype=F16) == "mxfp8_tile_kernel<256x256,stream_out=1> grid=256"
 
 
 @pytest.mark.parametrize("m,n,k,kernel", [
@@ -70,16 +73,16 @@ def test_deep_k_with_a_workspace_splits_k_only_where_it_wins():
     (128, 4096, 4096, "mxfp8_skinny_kernel<RT=4,TT=2> grid=64x4"),
     (128, 14336, 4096, "mxfp8_skinny_kernel<RT=4,TT=4,W=4> grid=224x2"),
     (128, 4096, 14336, "mxfp8_skinny_kernel<RT=4,TT=2> grid=64x4"),
-    (2048, 4096, 4096, "mxfp8_gemm_256_kernel<TM=2,stream_out=0> grid=256"),
-    (2048, 14336, 4096, "mxfp8_gemm_256_kernel<TM=4,stream_out=0> grid=256"),
+    (2048, 4096, 4096, "mxfp8_tile_kernel<128x256,stream_out=0> grid=256"),
+    (2048, 14336, 4096, "mxfp8_tile_kernel<256x256,stream_out=0> grid=256"),
     # streaming or persistent kernel by estimated duration
-    (256, 14336, 4096, "mxfp8_gemm_256_kernel<TM=2,stream_out=0> grid=112"),
-    (256, 14336, 14336, "mxfp8_gemm_256_kernel<TM=2,stream_out=0> grid=112"),
+    (256, 14336, 4096, "mxfp8_tile_kernel<128x256,stream_out=0> grid=112"),
+    (256, 14336, 14336, "mxfp8_tile_kernel<128x256,stream_out=0> grid=112"),
     (512, 4096, 7168, "mxfp8_skinny_kernel<RT=4,TT=4,W=4> grid=64x8"),
     (512, 4096, 14336, "mxfp8_skinny_kernel<RT=4,TT=4> grid=64x8"),
     (1024, 2048, 14336, "mxfp8_skinny_kernel<RT=4,TT=4> grid=32x16"),
-    (1024, 4096, 4096, "mxfp8_gemm_256_kernel<TM=2,stream_out=0> grid=128"),
-    (1024, 8192, 4096, "mxfp8_gemm_256_kernel<TM=2,stream_out=0> grid=256"),
+    (1024, 4096, 4096, "mxfp8_tile_kernel<128x256,stream_out=0> grid=128"),
+    (1024, 8192, 4096, "mxfp8_tile_kernel<128x256,stream_out=0> grid=256"),
 ])
 def test_mxfp8_llm_and_mid_sized_shapes(m, n, k, kernel):
     assert plan("mxfp8_scaled_mm", m, n, k).startswith(kernel), plan("mxfp8_scaled_mm", m, n, k)
@@ -147,30 +150,31 @@ def test_nvfp4_dense_m_not_a_multiple_of_the_tile_height_takes_the_persistent_ke
 def test_mxfp8_dense_m_not_a_multiple_of_the_tile_height_takes_the_persistent_kernel_with_a_short_last_row_tile():
     op = "mxfp8_scaled_mm"
     # a prefill of any token count: one launch, the last row tile with fewer rows
-    for m, n, k, tm, grid in ((4000, 4096, 4096, 4, 256), (8100, 8192, 8192, 4, 256), (320, 14336, 4096, 2, 168), (640, 14336, 4096, 4, 168),
-                              (96, 28672, 4096, 2, 112), (384, 28672, 4096, 4, 224)):
+    for m, n, k, rows, grid in ((4000, 4096, 4096, 256, 256), (8100, 8192, 8192, 256, 256), (320, 14336, 4096, 128, 168), (640, 14336, 4096, 256, 168),
+                                (96, 28672, 4096, 128, 112), (384, 28672, 4096, 256, 224)):
         got = plan(op, m, n, k)
-        assert got.startswith(f"mxfp8_gemm_256_kernel<TM={tm},") and "ragged_m" in got and f"grid={grid}" in got and ";" not in got, (m, n, k, got)
+        assert got.startswith(f"mxfp8_tile_kernel<{rows}x256,") and "ragged_m" in got and f"grid={grid}" in got and ";" not in got, (m, n, k, got)
     # where the weight-streaming kernel is estimated faster it takes all rows, and multiples of the tile height are as before
     got = plan(op, 1000, 4096, 14336)
     assert "skinny" in got and ";" not in got, got
     assert "ragged_m" not in plan(op, 4096, 4096, 4096) and "skinny" in plan(op, 300, 4096, 4096)
     # K % 128 != 0 as well: the variant with a short last K step and a short last row tile
     got = plan(op, 4000, 4096, 2880)
-    assert got.startswith("mxfp8_gemm_256_kernel<TM=4,") and "ragged_k,ragged_m" in got and ";" not in got, got
+    assert got.startswith("mxfp8_tile_kernel<256x256,") and "ragged_k,ragged_m" in got and ";" not in got, got
 
 
 @pytest.mark.parametrize("op", ["nvfp4_scaled_mm", "mxfp8_scaled_mm"])
 def test_dense_n_not_a_multiple_of_256_is_cut_into_a_main_part_and_the_remaining_columns(op):
     got = plan(op, 8192, 29568, 8192).split("; ")
-    assert len(got) == 2 and "gemm_256_kernel<" in got[0] and "TM=4" in got[0] and "grid=256" in got[0] and "skinny" in got[1], got
+    tiles = "nvfp4_gemm_256_kernel<grouped=0,TM=4," if op == "nvfp4_scaled_mm" else "mxfp8_tile_kernel<256x256,"
+    assert len(got) == 2 and got[0].startswith(tiles) and "grid=256" in got[0] and "skinny" in got[1], got
     # few rows: the weight-streaming kernel takes any N % 16 == 0 in one launch (MXFP8 from 65 rows on: one round of
     # 128x256 tiles with 100 rows each for the columns up to the last multiple of 256 is estimated faster)
     got = plan(op, 100 if op == "nvfp4_scaled_mm" else 48, 29568, 4096).split("; ")
     assert len(got) == 1 and "skinny" in got[0], got
     if op == "mxfp8_scaled_mm":
         got = plan(op, 100, 29568, 4096).split("; ")
-        assert len(got) == 2 and got[0].startswith("mxfp8_gemm_256_kernel<TM=2,") and "ragged_m" in got[0] and "skinny" in got[1], got
+        assert len(got) == 2 and got[0].startswith("mxfp8_tile_kernel<128x256,") and "ragged_m" in got[0] and "skinny" in got[1], got
 
 
 def test_nvfp4_8192_cubed_takes_the_persistent_256x256_kernel():
@@ -179,12 +183,12 @@ def test_nvfp4_8192_cubed_takes_the_persistent_256x256_kernel():
 
 def test_config4_bf16_grouped_takes_the_persistent_kernel_in_one_launch():
     got = plan("grouped_mm", 8192, 14336, 4096, groups=8)
-    assert got.startswith("grouped16_gemm_256_kernel<") and ";" not in got, got
-    # from 128 rows per group on average, where its 256x256 tiles cover half the compute units; the tile kernels below
-    assert plan("grouped_mm", 1024, 14336, 4096, groups=8).startswith("grouped16_gemm_256_kernel<")
-    assert plan("grouped_mm", 8192, 2048, 7168, groups=64).startswith("grouped16_gemm_256_kernel<")
-    assert plan("grouped_mm", 1000, 14336, 4096, groups=8).startswith("gemm16_kernel<")
-    assert plan("grouped_mm", 1024, 4096, 14336, groups=8).startswith("gemm16_kernel<")  # 64 tiles of 256x256 only
+    assert got.startswith("grouped16_tile_kernel<256x256,") and ";" not in got, got
+    # 256x256 tiles from 128 rows per group on average, where they cover half the compute units; 128x128 below
+    assert plan("grouped_mm", 1024, 14336, 4096, groups=8).startswith("grouped16_tile_kernel<256x256,")
+    assert plan("grouped_mm", 8192, 2048, 7168, groups=64).startswith("grouped16_tile_kernel<256x256,")
+    assert plan("grouped_mm", 1000, 14336, 4096, groups=8).startswith("grouped16_tile_kernel<128x128,stream_out=0,")
+    assert plan("grouped_mm", 1024, 4096, 14336, groups=8).startswith("grouped16_tile_kernel<128x128,stream_out=0,")  # 64 tiles of 256x256 only
 
 
 @pytest.mark.parametrize("n,k", [(2048, 7168), (7168, 2048)])
@@ -268,9 +272,11 @@ def test_nvfp4_grouped_small_and_large_groups(m, n, k, groups, small, large):
     (16 * 8, 3000, 1288, 8, 32), (17 * 8, 3000, 1288, 8, 0), (64, 1024, 1024, 64, 0), (8, 128, 1016, 8, 0),
 ])
 def test_grouped_mm_with_few_rows_per_group_streams_the_weights(m, n, k, groups, rows):
-    """Both sides of the lines at 48, 24 and 16 rows per group; `rows`: weight rows of a work item (0: the tile kernel)."""
+    """Both sides of the lines at 48, 24 and 16 rows per group; `rows`: weight rows of a work item (0: tiles, by a kernel of
+    its own where K % 64 != 0)."""
     got = plan("grouped_mm", m, n, k, groups=groups)
-    assert got.startswith(f"streaming_gemm16_kernel<weight_rows={rows}," if rows else "gemm16_kernel<") and ";" not in got, got
+    tiles = "grouped16_tile_kernel<128x128," if k % 64 == 0 else "gemm16_kernel<128,128>"
+    assert got.startswith(f"streaming_gemm16_kernel<weight_rows={rows}," if rows else tiles) and ";" not in got, got
 
 
 @pytest.mark.parametrize("m,n,k,groups,prefill", [
@@ -321,16 +327,16 @@ def test_blockscale_is_one_launch_and_ragged_shapes_add_only_the_fill_kernel():
     assert len(dump) == 2 and "fp4_blockscale" in dump[0] and "f32=1" in dump[1], dump
 
 
-KNOWN_KERNELS = ("nvfp4_skinny_ring_kernel<", "nvfp4_gemm_256_kernel<", "nvfp4_tile_kernel<", "nvfp4_group_panel_kernel<",
-                 "gemm16_kernel<", "grouped16_gemm_256_kernel<", "mxfp8_gemm_256_kernel<", "mxfp8_skinny_kernel<", "mxfp8_gemm_kernel<",
-                 "zero_fill_kernel", "nvfp4_act_convert_kernel", "nvfp4_skinny_f16a_kernel<", "splitk_reduce_kernel")
+# the kernels that there are, by the sources
+KERNELS = {name for path in (Path(__file__).parents[1] / "fuser_amd" / "csrc").glob("*.*") if path.suffix in (".hip", ".inl")
+           for name in re.findall(r"__global__[^;{]*?void (\w+)\(", path.read_text())}
 
 
 def _assert_known(got):
     assert got, "empty plan"
     assert "grid=0" not in got, got
-    for part in got.split("; "):
-        assert any(k in part for k in KNOWN_KERNELS), got
+    for part in re.split("; | [+] ", got):
+        assert re.match(r"\w+", part).group() in KERNELS, got
 
 
 def test_sweep_of_other_shapes_reaches_a_kernel_on_every_branch():

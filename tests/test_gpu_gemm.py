@@ -417,7 +417,7 @@ def test_mxfp8_gemm_k_not_a_multiple_of_128_on_the_persistent_kernel(dev, shape)
     sa8_p[O.linear_to_swizzled_128_4(torch.ones(m, k // 32, dtype=torch.uint8)) == 0] = 0xFF
     sb8_p[O.linear_to_swizzled_128_4(torch.ones(n, k // 32, dtype=torch.uint8)) == 0] = 0xFF
     plan = capi.describe_dispatch("mxfp8_scaled_mm", m, n, k)
-    assert "mxfp8_gemm_256_kernel" in plan and "ragged_k" in plan, plan
+    assert "mxfp8_tile_kernel<" in plan and "ragged_k" in plan, plan
     for dtype in (torch.bfloat16, torch.float16):
         if dtype == torch.float16 and ref.abs().max() > 6e4:
             continue
@@ -859,9 +859,9 @@ def test_mxfp8_gemm_persistent_256_tile_kernel_full_compare(dev, shape):
     assert torch.equal(out, out2)
 
 
-@pytest.mark.parametrize("shape, tile", [((768, 3072, 512), "TM=2,TN=2"), ((640, 3072, 1088), "TM=2,TN=2"), ((300, 4096, 544), "TM=2,TN=2"),
-                                         ((1153, 1040, 1120), "TM=2,TN=2"), ((200, 8208, 1024), "TM=2,TN=2"), ((2001, 2064, 1024), "TM=2"),
-                                         ((1030, 4112, 1056), "TM=2"), ((2300, 6160, 1024), "TM=4"), ((2200, 8176, 1056), "TM=2")])
+@pytest.mark.parametrize("shape, tile", [((768, 3072, 512), "128x128"), ((640, 3072, 1088), "128x128"), ((300, 4096, 544), "128x128"),
+                                         ((1153, 1040, 1120), "128x128"), ((200, 8208, 1024), "128x128"), ((2001, 2064, 1024), "128x256"),
+                                         ((1030, 4112, 1056), "128x256"), ((2300, 6160, 1024), "256x256"), ((2200, 8176, 1056), "128x256")])
 def test_mxfp8_gemm_128x128_tiles_and_a_last_column_tile_with_fewer_columns(dev, shape, tile):
     """128x128 tiles (four buffers: 4 to 9 steps), and tiles of every size of which the last hold 16 to 240 columns: their
     missing weight rows load the last one again, their scale tile may not exist, and their columns are not stored.  NaN code in
@@ -870,7 +870,7 @@ def test_mxfp8_gemm_128x128_tiles_and_a_last_column_tile_with_fewer_columns(dev,
 
     m, n, k = shape
     plan = capi.describe_dispatch("mxfp8_scaled_mm", m, n, k)
-    assert plan.startswith(f"mxfp8_gemm_256_kernel<{tile},stream_out=") and ("ragged_n" in plan) == (n % (128 if "TN" in tile else 256) != 0) and ";" not in plan, plan
+    assert plan.startswith(f"mxfp8_tile_kernel<{tile},stream_out=") and ("ragged_n" in plan) == (n % int(tile[4:]) != 0) and ";" not in plan, plan
     gen = torch.Generator().manual_seed(m * 31 + n)
     (a, sa), (b, sb) = _mxfp8_operand(m, k, gen, 1.0), _mxfp8_operand(n, k, gen, 1.0)
     ref = O.ref_mxfp8_scaled_mm(a, b, sa, sb, 0.75)
@@ -903,7 +903,7 @@ def test_mxfp8_gemm_last_row_tile_with_fewer_rows_on_the_persistent_kernel(dev, 
 
     m, n, k = shape
     plan = capi.describe_dispatch("mxfp8_scaled_mm", m, n, k)
-    assert plan.startswith("mxfp8_gemm_256_kernel<") and "ragged_m" in plan and ";" not in plan, plan
+    assert plan.startswith("mxfp8_tile_kernel<") and "ragged_m" in plan and ";" not in plan, plan
     gen = torch.Generator().manual_seed(m * 31 + n)
     a, sa = _mxfp8_operand(m, k, gen, 1.0)
     b, sb = _mxfp8_operand(n, k, gen, 1.0)
@@ -1063,7 +1063,7 @@ def test_mxfp8_gemm_short_last_step_adds_exact_zeros(dev, m, n, k):
     from fuser_amd import capi
 
     plan = capi.describe_dispatch("mxfp8_scaled_mm", m, n, k)
-    assert plan.startswith("mxfp8_gemm_256_kernel<") and "ragged_k" in plan and ";" not in plan, plan
+    assert plan.startswith("mxfp8_tile_kernel<") and "ragged_k" in plan and ";" not in plan, plan
     gen = torch.Generator().manual_seed(m + k)
     a8, _ = O.block_quantize_mxfp8(torch.randn(m, k, generator=gen).bfloat16())
     b8, _ = O.block_quantize_mxfp8(torch.randn(n, k, generator=gen).bfloat16())

@@ -105,7 +105,7 @@ def test_grouped_mm_group_ends_inside_tiles(dev, n, k):
     b = (torch.randn(len(sizes), n, k, generator=gen) * 0.05).bfloat16()
     ps, eo, _, _ = _grouped_args(sizes, n, k, dev)
     ad, bd, psd, eod = a.to(dev), b.to(dev), ps.to(dev), eo.to(dev)
-    assert capi.describe_dispatch("grouped_mm", m, n, k, groups=len(sizes)).startswith("grouped16_gemm_256_kernel")
+    assert capi.describe_dispatch("grouped_mm", m, n, k, groups=len(sizes)).startswith("grouped16_tile_kernel<256x256,")
     out = torch.full((m, n), 7.0, dtype=torch.bfloat16, device=dev)
     capi.check(capi.lib().nvf_grouped_mm(ad.data_ptr(), bd.data_ptr(), out.data_ptr(), psd.data_ptr(), eod.data_ptr(), len(sizes),
                                          m, n, k, capi.BF16, None))
@@ -127,7 +127,7 @@ def test_grouped_mm_persistent_kernel_from_128_rows_per_group(dev, n, k):
     sizes = [130, 0, 255, 1, 200, 128, 300, 129, 90, 257]
     m = sum(sizes) + 5
     assert 128 * len(sizes) <= m < 256 * len(sizes)
-    assert capi.describe_dispatch("grouped_mm", m, n, k, groups=len(sizes)).startswith("grouped16_gemm_256_kernel")
+    assert capi.describe_dispatch("grouped_mm", m, n, k, groups=len(sizes)).startswith("grouped16_tile_kernel<256x256,")
     for tensor_dtype, dt in ((torch.bfloat16, capi.BF16), (torch.float16, capi.F16)):
         gen = torch.Generator().manual_seed(n + k)
         a = torch.randn(m, k, generator=gen).to(tensor_dtype)
@@ -156,7 +156,7 @@ def test_grouped_mm_tiles_of_128_rows_and_columns(dev, n, k, groups):
     sizes = ([127, 0, 128, 1, 129, 64, 33, 257, 0, 90] * 7)[:groups]
     m = sum(sizes) + 5
     plan = capi.describe_dispatch("grouped_mm", m, n, k, groups=len(sizes))
-    assert plan.startswith(f"gemm16_kernel<128,128,buffers=4,stream={int(2 * groups * n * k > 256 << 20)}>"), plan
+    assert plan.startswith(f"grouped16_tile_kernel<128x128,stream_out=0,stream_weights={int(2 * groups * n * k > 256 << 20)}{',ragged_n' if n % 128 else ''}>"), plan
     for tensor_dtype, dt in ((torch.bfloat16, capi.BF16), (torch.float16, capi.F16)):
         gen = torch.Generator().manual_seed(n + k)
         a = torch.randn(m, k, generator=gen).to(tensor_dtype)
