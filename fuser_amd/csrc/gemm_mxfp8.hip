@@ -904,20 +904,19 @@ Plan mxfp8_plan(int64_t m, int64_t n, int64_t k, int64_t cus, int64_t* ns = null
   int64_t t256 = tiles_of(256, 256), t128 = tiles_of(128, 256), t128x128 = tiles_of(128, 128);
   if (!fast_shape || t256 < 128 || !columns_ok || !((m & 255) == 0 || m > 128)) t256 = 0;
   // 128x128 tiles: half the work per compute unit in 0.7 of the time, so they win up to a whole round of them, i.e. for half a
-  // round of 128x256 tiles (512 x 8192 x 4096 23.3 against 31.3 us, 1178 x 2816 x 11456 65 / 98, 157 x 14240 x 10752 50 / 71).  Of
-  // the shapes whose N and K are whole multiples of the 128x256 tiles' those with more than two fifths of a round stay on them: the
-  // dispatch of 1024 x 4096 x 4096, 256 x 14336 x 4096 and x 14336 and 1000 x 4096 x 14336 is pinned.
-  const bool whole = (n & 255) == 0 && (k & 127) == 0;
-  if (!fast_shape || m <= 128 || (whole && 5 * t128 >= 2 * cus) || !columns_ok || k < 512 || t128x128 < 16) t128x128 = 0;
+  // round of 128x256 tiles (512 x 8192 x 4096 24.1 against 31.3 us, 1024 x 4096 x 4096 23.3 / 29.6, 256 x 14336 x 4096 24.2 / 31.8,
+  // 1000 x 4096 x 14336 72.6 / 99.5 and 110 streamed, 160 x 14336 x 4096 22.2 / 30.0 and 36 streamed, 948 x 3840 x 2560 15.4 / 21.5).
+  if (!fast_shape || m <= 128 || !columns_ok || k < 512 || t128x128 < 16) t128x128 = 0;
   if (!fast_shape || t128 < 48 || !columns_ok) t128 = 0;
   // Measured with weights that change from call to call, us per 128-deep step of a round (a round of a few tiles, a full one)
-  // and per call: 256x256 1.08, 1.48 and 7; 128x256 0.75, 0.95 and 5.2; 128x128 0.53, 0.60 and 3.5.
-  auto tile_ns = [&](int64_t tiles, int64_t fixed, int64_t step, int64_t full) {
+  // and per call: 256x256 1.08, 1.48 and 7; 128x256 0.75, 0.95 and 5.2; 128x128 0.53, 0.60 and 3.1, and 0.4 per round besides
+  // (K = 768, 1280 x 4096 in two rounds 11.5, as one of 128x256 tiles 10.6; 4096 x 3072 x 512 in three 12.6, 13.6 as two).
+  auto tile_ns = [&](int64_t tiles, int64_t fixed, int64_t round, int64_t step, int64_t full) {
     if (tiles == 0) return (int64_t)INT64_MAX;
     const int64_t steps = (k + 127) >> 7, rounds = ceil_div(tiles, cus);
-    return fixed + steps * (rounds * step + (full - step) * tiles / cus);
+    return fixed + rounds * round + steps * (rounds * step + (full - step) * tiles / cus);
   };
-  const int64_t ns256 = tile_ns(t256, 7000, 1080, 1480), ns128 = tile_ns(t128, 5200, 750, 950), ns128x128 = tile_ns(t128x128, 3500, 530, 600);
+  const int64_t ns256 = tile_ns(t256, 7000, 0, 1080, 1480), ns128 = tile_ns(t128, 5200, 0, 750, 950), ns128x128 = tile_ns(t128x128, 3100, 400, 530, 600);
   const int64_t fast_ns = std::min(ns256, std::min(ns128, ns128x128));
   const bool fast = fast_ns != INT64_MAX;
   if (skinny_ok) {

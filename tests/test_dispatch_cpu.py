@@ -76,12 +76,21 @@ def test_deep_k_with_a_workspace_splits_k_only_where_it_wins():
     (2048, 4096, 4096, "mxfp8_tile_kernel<128x256,stream_out=0> grid=256"),
     (2048, 14336, 4096, "mxfp8_tile_kernel<256x256,stream_out=0> grid=256"),
     # streaming or persistent kernel by estimated duration
-    (256, 14336, 4096, "mxfp8_tile_kernel<128x256,stream_out=0> grid=112"),
-    (256, 14336, 14336, "mxfp8_tile_kernel<128x256,stream_out=0> grid=112"),
+    (256, 14336, 4096, "mxfp8_tile_kernel<128x128,stream_out=0> grid=224"),
+    (256, 14336, 14336, "mxfp8_tile_kernel<128x128,stream_out=0> grid=224"),
+    (160, 14336, 4096, "mxfp8_tile_kernel<128x128,stream_out=0,ragged_m> grid=224"),
+    (192, 14336, 4096, "mxfp8_tile_kernel<128x128,stream_out=0,ragged_m> grid=224"),
+    (512, 8192, 4096, "mxfp8_tile_kernel<128x128,stream_out=0> grid=256"),
+    (948, 3840, 2560, "mxfp8_tile_kernel<128x128,stream_out=0,ragged_m> grid=240"),
+    (1000, 4096, 14336, "mxfp8_tile_kernel<128x128,stream_out=0,ragged_m> grid=256"),
+    # a shallow K: more rounds of 128x128 tiles than of larger ones only where they are filled better
+    (4096, 3072, 512, "mxfp8_tile_kernel<128x128,stream_out=0> grid=256"),
+    (1280, 4096, 768, "mxfp8_tile_kernel<128x256,stream_out=0> grid=160"),
+    (640, 14336, 1024, "mxfp8_tile_kernel<256x256,stream_out=0,ragged_m> grid=168"),
     (512, 4096, 7168, "mxfp8_skinny_kernel<RT=4,TT=4,W=4> grid=64x8"),
     (512, 4096, 14336, "mxfp8_skinny_kernel<RT=4,TT=4> grid=64x8"),
     (1024, 2048, 14336, "mxfp8_skinny_kernel<RT=4,TT=4> grid=32x16"),
-    (1024, 4096, 4096, "mxfp8_tile_kernel<128x256,stream_out=0> grid=128"),
+    (1024, 4096, 4096, "mxfp8_tile_kernel<128x128,stream_out=0> grid=256"),
     (1024, 8192, 4096, "mxfp8_tile_kernel<128x256,stream_out=0> grid=256"),
 ])
 def test_mxfp8_llm_and_mid_sized_shapes(m, n, k, kernel):
@@ -155,7 +164,7 @@ def test_mxfp8_dense_m_not_a_multiple_of_the_tile_height_takes_the_persistent_ke
         got = plan(op, m, n, k)
         assert got.startswith(f"mxfp8_tile_kernel<{rows}x256,") and "ragged_m" in got and f"grid={grid}" in got and ";" not in got, (m, n, k, got)
     # where the weight-streaming kernel is estimated faster it takes all rows, and multiples of the tile height are as before
-    got = plan(op, 1000, 4096, 14336)
+    got = plan(op, 999, 1280, 9984)
     assert "skinny" in got and ";" not in got, got
     assert "ragged_m" not in plan(op, 4096, 4096, 4096) and "skinny" in plan(op, 300, 4096, 4096)
     # K % 128 != 0 as well: the variant with a short last K step and a short last row tile
