@@ -845,11 +845,20 @@ int64_t mxfp8_skinny_best(int64_t m, int64_t n, int64_t k, int64_t cus, int* sla
   if (w_out) *w_out = w;
   return best;
 }
-// estimated duration of the form that mxfp8_skinny_best picks, in ns
+// Estimated duration of the form that mxfp8_skinny_best picks, in ns: what plans and cuts compare with the other kernels.
+// From 129 rows on it is scaled to what the kernel takes when the weights change from call to call (150 shapes of 129..3000
+// rows; measured / unscaled, median: K <= 1536 0.8, 2048 0.9, 4096 1.0, 7168 1.07, 8192..11008 1.2, 14336 1.2).  Workgroups go
+// to the XCDs in turn: with a number of them per slab that is no multiple of 4 the slabs that share weight rows lie in
+// different XCDs, each of which reads those rows again (256 x 2880 x 8192 22.9 us, 256 x 2560 x 7168 14; measured / unscaled
+// 1.25..1.5 times as much as else at that K, 512 x 2880 x 2880 22.0 against 16.4 on 128x128 tiles).  With the scaled
+// estimate the kernel picked is within 1 % of the fastest in the geometric mean over 336 shapes, 9 % at worst.
 int64_t mxfp8_skinny_ns(int64_t m, int64_t n, int64_t k, int64_t cus) {
   int slab, rt, w;
   if (mxfp8_skinny_best(m, n, k, cus, &slab, &rt, &w) == INT64_MAX) return INT64_MAX;
-  return mxfp8_skinny_cost(m, n, k, slab, rt, cus, true, w) * 963 / 1000;
+  const int64_t ns = mxfp8_skinny_cost(m, n, k, slab, rt, cus, true, w) * 963 / 1000;
+  if (m <= 128) return ns;  // (its constants were fitted there, with weights that stay)
+  const int64_t percent = std::min<int64_t>({std::max<int64_t>(77, 50 + 20 * k / 1024), 80 + 5 * k / 1024, 125});
+  return ns * percent / 100 * (n / (16 * rt) % 4 ? 5 : 4) / 4;
 }
 
 template <bool OUT_BF16>
@@ -926,11 +935,7 @@ Plan mxfp8_plan(int64_t m, int64_t n, int64_t k, int64_t cus, int64_t* ns = null
     if (fast) {
       // Skinny or persistent kernel by estimated duration.  Measured: 512 x 4096 x 7168 36.7 (persistent) against 31.8 us,
       // 700 x 2304 x 5120 22.3 / 23.3, 512 x 4096 x 4096 18.2 / 18.7, 300 x 3072 x 2048 11.4 / 7.1, 1500 x 1408 x 7168 34 / 42.
-      // (With weights that change from call to call the skinny kernel takes, in percent of its estimate, 58-87 for K < 2048,
-      // 75-100 below 3072, 100 around 4096, 100-130 up to 8000 and 105-200 above, over 45 shapes of 129..4000 rows; against the
-      // larger tiles the estimate stays as it is from K = 3072 on, which the pinned dispatch of 1000 x 4096 x 14336 wants.)
-      const int64_t percent = m <= 128 ? 100 : k < 2048 ? 78 : k < 3072 ? 92 : fast_ns != ns128x128 || k < 4608 ? 100 : k <= 8000 ? 110 : 130;
-      if (skinny_ns * percent / 100 <= fast_ns) return Plan::kStream;
+      if (skinny_ns <= fast_ns) return Plan::kStream;
     } else {
       // No persistent kernel for the shape (ragged M or N, or too few tiles): up to 256 rows, i.e. four passes over
       // the weights, the skinny kernel beats the tile kernels (128 x 4096 x 14336: 20 instead of 117 us); with more

@@ -83,6 +83,13 @@ def test_deep_k_with_a_workspace_splits_k_only_where_it_wins():
     (512, 8192, 4096, "mxfp8_tile_kernel<128x128,stream_out=0> grid=256"),
     (948, 3840, 2560, "mxfp8_tile_kernel<128x128,stream_out=0,ragged_m> grid=240"),
     (1000, 4096, 14336, "mxfp8_tile_kernel<128x128,stream_out=0,ragged_m> grid=256"),
+    # streaming or tiles around the line: by K, and by how many workgroups a slab has (5760: 90, no multiple of 4)
+    (224, 7168, 3584, "mxfp8_skinny_kernel<RT=4,TT=4,W=4> grid=112x4"),
+    (224, 8192, 11008, "mxfp8_skinny_kernel<RT=4,TT=4> grid=128x4"),
+    (256, 8192, 8192, "mxfp8_skinny_kernel<RT=4,TT=4> grid=128x4"),
+    (384, 4096, 2880, "mxfp8_tile_kernel<128x128,stream_out=0,ragged_k> grid=96"),
+    (192, 5760, 8192, "mxfp8_tile_kernel<128x128,stream_out=0,ragged_m> grid=96"),
+    (192, 6144, 8192, "mxfp8_skinny_kernel<RT=4,TT=4> grid=96x3"),
     # a shallow K: more rounds of 128x128 tiles than of larger ones only where they are filled better
     (4096, 3072, 512, "mxfp8_tile_kernel<128x128,stream_out=0> grid=256"),
     (1280, 4096, 768, "mxfp8_tile_kernel<128x256,stream_out=0> grid=160"),
