@@ -904,12 +904,13 @@ Plan mxfp8_plan(int64_t m, int64_t n, int64_t k, int64_t cus, int64_t* ns = null
   if (ns) *ns = INT64_MAX;
   const bool skinny_ok = (k & 31) == 0 && (n & 15) == 0 && k * 64 < (1ll << 31);  // 32-bit lane offsets (a short last chunk is fine)
   // The persistent kernel takes any K % 32 == 0 (its last step may be short), a last row tile with fewer rows (which counts as a
-  // whole one: 640 x 14336 x 4096 as 280 tiles of 128 rows in 2 rounds 60 us, 168 of 256 rows 43 us) and, where the rows are
-  // ragged too, a last column tile with fewer columns, where the others get a launch of its own for the remaining columns
-  // (1000 x 5760 x 2880: 36 + 5 us cut, 26.5 whole; measured from K = 1024 on).
+  // whole one: 640 x 14336 x 4096 as 280 tiles of 128 rows in 2 rounds 60 us, 168 of 256 rows 43 us) and, measured from K = 1024
+  // on, a last column tile with fewer columns (against a launch of its own for the remaining columns, us: 2048 x 6208 x 1408
+  // 22.4 / 36.6, 640 rows of it 10.8 / 27.6, 2048 x 5760 x 2880 41.2 / 49.1, 768 x 2064 x 4096 19.0 / 34.5 streamed, 4096 x 11040
+  // x 4096 155 / 159, 8192 x 29568 x 8192 1422 / 1450).
   const bool fast_shape = (k & 31) == 0 && k >= 256 && k * 256 < (1ll << 31) && (n & 15) == 0 && (m > 64 || (m & 127) == 0);
   auto tiles_of = [&](int64_t bm, int64_t bn) { return ceil_div(m, bm) * ceil_div(n, bn); };
-  const bool columns_ok = (n & 255) == 0 || ((m & 127) != 0 && m > 128 && n > 256 && k >= 1024);
+  const bool columns_ok = (n & 255) == 0 || (m > 128 && n > 256 && k >= 1024);
   int64_t t256 = tiles_of(256, 256), t128 = tiles_of(128, 256), t128x128 = tiles_of(128, 128);
   if (!fast_shape || t256 < 128 || !columns_ok || !((m & 255) == 0 || m > 128)) t256 = 0;
   // 128x128 tiles: half the work per compute unit in 0.7 of the time, so they win up to a whole round of them, i.e. for half a

@@ -181,9 +181,12 @@ def test_mxfp8_dense_m_not_a_multiple_of_the_tile_height_takes_the_persistent_ke
 
 @pytest.mark.parametrize("op", ["nvfp4_scaled_mm", "mxfp8_scaled_mm"])
 def test_dense_n_not_a_multiple_of_256_is_cut_into_a_main_part_and_the_remaining_columns(op):
-    got = plan(op, 8192, 29568, 8192).split("; ")
-    tiles = "nvfp4_gemm_256_kernel<grouped=0,TM=4," if op == "nvfp4_scaled_mm" else "mxfp8_tile_kernel<256x256,"
-    assert len(got) == 2 and got[0].startswith(tiles) and "grid=256" in got[0] and "skinny" in got[1], got
+    if op == "nvfp4_scaled_mm":
+        got = plan(op, 8192, 29568, 8192).split("; ")
+        assert len(got) == 2 and got[0].startswith("nvfp4_gemm_256_kernel<grouped=0,TM=4,") and "grid=256" in got[0] and "skinny" in got[1], got
+    else:  # (from K = 1024 on MXFP8's last column tile has fewer columns instead)
+        got = plan(op, 8192, 29568, 896).split("; ")
+        assert len(got) == 2 and got[0].startswith("mxfp8_tile_kernel<256x256,") and "grid=256" in got[0] and "ragged_n" not in got[0], got
     # few rows: the weight-streaming kernel takes any N % 16 == 0 in one launch (MXFP8 from 65 rows on: one round of
     # 128x256 tiles with 100 rows each for the columns up to the last multiple of 256 is estimated faster)
     got = plan(op, 100 if op == "nvfp4_scaled_mm" else 48, 29568, 4096).split("; ")
@@ -191,6 +194,17 @@ def test_dense_n_not_a_multiple_of_256_is_cut_into_a_main_part_and_the_remaining
     if op == "mxfp8_scaled_mm":
         got = plan(op, 100, 29568, 4096).split("; ")
         assert len(got) == 2 and got[0].startswith("mxfp8_tile_kernel<128x256,") and "ragged_m" in got[0] and "skinny" in got[1], got
+
+
+@pytest.mark.parametrize("m", [1024, 1000])
+def test_mxfp8_dense_n_not_a_multiple_of_256_in_one_launch_with_a_short_last_column_tile(m):
+    """Whatever the rows are: whole multiples of the tile's and not."""
+    for n, k, tile in ((5760, 2880, "128x256"), (6208, 1408, "128x256"), (2880, 2880, "128x128"), (1408, 4096, "128x128")):
+        got = plan("mxfp8_scaled_mm", m, n, k)
+        assert got.startswith(f"mxfp8_tile_kernel<{tile},") and ("ragged_n" in got) == (n % int(tile[4:]) != 0) and ";" not in got, got
+    for rows, n, k in ((8 * m, 29568, 8192), (4 * m, 11040, 4096), (2 * m, 5760, 2880)):
+        got = plan("mxfp8_scaled_mm", rows, n, k)
+        assert got.startswith("mxfp8_tile_kernel<256x256,") and "ragged_n" in got and ";" not in got, got
 
 
 def test_nvfp4_8192_cubed_takes_the_persistent_256x256_kernel():

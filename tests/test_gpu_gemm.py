@@ -369,8 +369,9 @@ def test_dense_gemms_with_n_not_a_multiple_of_256(dev, shape):
     """N > 256 and not a multiple of 256: the columns up to the last multiple of 256 go to the persistent kernel, the
     remaining 32..224 columns to a launch of their own (tile kernel or weight-streaming kernel) that writes into the same
     rows of the result at the full row pitch; the second shape is cut along M as well (K % 128 != 0), the last three
-    have a short last row tile in the main part (100 rows: MXFP8 only, NVFP4 streams; the last: both ops).  Both ops,
-    both output types, every element against the oracle (a launch writing at the wrong pitch would show), run-to-run
+    have a short last row tile in the main part (100 rows: MXFP8 only, NVFP4 streams; the last: both ops).  MXFP8's
+    fourth shape: one launch of 128x128 tiles (from K = 1024 on its last column tile may be short, the cut is taken where it saves
+    a round: the fifth and the last).  Both ops, both output types, every element against the oracle (a launch writing at the wrong pitch would show), run-to-run
     bit equality."""
     from fuser_amd import capi
 
@@ -397,7 +398,8 @@ def test_dense_gemms_with_n_not_a_multiple_of_256(dev, shape):
         assert out.shape == (m, n)
         assert ((out.float().cpu() - ref).abs() / scale).max().item() <= GEMM_MAX_REL, (shape, dtype, plans[-1])
         assert torch.equal(out, _run_mxfp8(a8, b8, sa8, sb8, 0.75, dtype, dev))
-    assert any("; " in p for p in plans), plans
+    assert ("; " in plans[1]) == (shape != (640, 4224, 2048)), plans
+    assert ("; " in plans[0]) == (shape not in ((640, 4224, 2048), (100, 16512, 512), (200, 12352, 512))), plans
 
 
 @pytest.mark.parametrize("shape", [(2048, 2048, 2880), (512, 4096, 288), (1024, 2048, 416), (1024, 1536, 352), (4096, 5120, 2880)])
@@ -428,7 +430,7 @@ def test_mxfp8_gemm_k_not_a_multiple_of_128_on_the_persistent_kernel(dev, shape)
 
 
 @pytest.mark.parametrize("shape", [(16, 4096, 2880), (128, 5760, 2880), (300, 4096, 2880), (64, 512, 96), (7, 256, 32), (100, 1024, 4192),
-                                   (33, 2048, 160), (2048, 5760, 2880)])
+                                   (33, 2048, 160), (120, 20608, 1056)])
 def test_mxfp8_gemm_k_not_a_multiple_of_128_on_the_streaming_kernel(dev, shape):
     """The same on the weight-streaming kernel (decode sizes, ragged M, and - last shape - the columns that the persistent
     kernel leaves over): the last 128-deep chunk of a row is short.  NaN codes in all scale padding."""
@@ -861,10 +863,12 @@ def test_mxfp8_gemm_persistent_256_tile_kernel_full_compare(dev, shape):
 
 @pytest.mark.parametrize("shape, tile", [((768, 3072, 512), "128x128"), ((640, 3072, 1088), "128x128"), ((300, 4096, 544), "128x128"),
                                          ((1153, 1040, 1120), "128x128"), ((200, 8208, 1024), "128x128"), ((2001, 2064, 1024), "128x256"),
-                                         ((1030, 4112, 1056), "128x256"), ((2300, 6160, 1024), "256x256"), ((2200, 8176, 1056), "128x256")])
+                                         ((1030, 4112, 1056), "128x256"), ((2300, 6160, 1024), "256x256"), ((2200, 8176, 1056), "128x256"),
+                                         ((640, 2576, 1024), "128x128"), ((1024, 5760, 1056), "128x256"), ((2048, 5760, 2880), "256x256"),
+                                         ((2304, 6160, 1024), "256x256")])
 def test_mxfp8_gemm_128x128_tiles_and_a_last_column_tile_with_fewer_columns(dev, shape, tile):
-    """128x128 tiles (four buffers: 4 to 9 steps), and tiles of every size of which the last hold 16 to 240 columns: their
-    missing weight rows load the last one again, their scale tile may not exist, and their columns are not stored.  NaN code in
+    """128x128 tiles (four buffers: 4 to 9 steps), and tiles of every size of which the last hold 16 to 240 columns, with rows
+    that are whole multiples of the tile's and not: their missing weight rows load the last one again, their scale tile may not exist, and their columns are not stored.  NaN code in
     every scale byte of the padding, every element against the oracle, both output types, run-to-run bit equality."""
     from fuser_amd import capi
 
