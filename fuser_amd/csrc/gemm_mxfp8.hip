@@ -919,14 +919,15 @@ Plan mxfp8_plan(int64_t m, int64_t n, int64_t k, int64_t cus, int64_t* ns = null
   if (!fast_shape || m <= 128 || !columns_ok || k < 512 || t128x128 < 16) t128x128 = 0;
   if (!fast_shape || t128 < 48 || !columns_ok) t128 = 0;
   // Measured with weights that change from call to call, us per 128-deep step of a round (a round of a few tiles, a full one)
-  // and per call: 256x256 1.08, 1.48 and 7; 128x256 0.75, 0.95 and 5.2; 128x128 0.53, 0.60 and 3.1, and 0.4 per round besides
-  // (K = 768, 1280 x 4096 in two rounds 11.5, as one of 128x256 tiles 10.6; 4096 x 3072 x 512 in three 12.6, 13.6 as two).
+  // and per call: 256x256 1.08, 1.48 and 7; 128x256 0.75, 0.95 and 5.2; 128x128 0.53, 0.60 and 2.8, and 0.7 per round besides
+  // (300 x 14336 x 512 in two rounds 10.0, as one of 128x256 tiles 9.2; 1280 x 4096 x 768 11.5 / 10.6; but 4096 x 3072 x 512 in
+  // three 12.6, as two of 128x256 tiles 13.6).
   auto tile_ns = [&](int64_t tiles, int64_t fixed, int64_t round, int64_t step, int64_t full) {
     if (tiles == 0) return (int64_t)INT64_MAX;
     const int64_t steps = (k + 127) >> 7, rounds = ceil_div(tiles, cus);
     return fixed + rounds * round + steps * (rounds * step + (full - step) * tiles / cus);
   };
-  const int64_t ns256 = tile_ns(t256, 7000, 0, 1080, 1480), ns128 = tile_ns(t128, 5200, 0, 750, 950), ns128x128 = tile_ns(t128x128, 3100, 400, 530, 600);
+  const int64_t ns256 = tile_ns(t256, 7000, 0, 1080, 1480), ns128 = tile_ns(t128, 5200, 0, 750, 950), ns128x128 = tile_ns(t128x128, 2800, 700, 530, 600);
   const int64_t fast_ns = std::min(ns256, std::min(ns128, ns128x128));
   const bool fast = fast_ns != INT64_MAX;
   if (skinny_ok) {

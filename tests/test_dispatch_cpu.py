@@ -93,6 +93,8 @@ def test_deep_k_with_a_workspace_splits_k_only_where_it_wins():
     # a shallow K: more rounds of 128x128 tiles than of larger ones only where they are filled better
     (4096, 3072, 512, "mxfp8_tile_kernel<128x128,stream_out=0> grid=256"),
     (1280, 4096, 768, "mxfp8_tile_kernel<128x256,stream_out=0> grid=160"),
+    (300, 14336, 512, "mxfp8_tile_kernel<128x256,stream_out=0,ragged_m> grid=168"),
+    (512, 16384, 640, "mxfp8_tile_kernel<128x256,stream_out=0> grid=256"),
     (640, 14336, 1024, "mxfp8_tile_kernel<256x256,stream_out=0,ragged_m> grid=168"),
     (512, 4096, 7168, "mxfp8_skinny_kernel<RT=4,TT=4,W=4> grid=64x8"),
     (512, 4096, 14336, "mxfp8_skinny_kernel<RT=4,TT=4> grid=64x8"),
