@@ -91,11 +91,11 @@ def test_grouped_mm_persistent_256_tile_kernel_full_compare(dev, tensor_dtype, k
     assert ((out[:rows].float().cpu() - ref[:rows]).abs() / scale).max().item() <= GEMM_MAX_REL
 
 
-@pytest.mark.parametrize("n,k", [(2048, 192), (2304, 128), (4096, 320), (2304, 1024)])
+@pytest.mark.parametrize("n,k", [(2048, 192), (2304, 128), (4096, 320), (2304, 1024), (16384, 320), (16392, 320), (2312, 1024)])
 def test_grouped_mm_group_ends_inside_tiles(dev, n, k):
     """Persistent 256-row-tile kernel: groups that end 128, 129, 1, 100 and 127 rows into a tile, groups smaller than
-    half a tile, N with 8 | N/256 (n-tiles dealt to the XCDs) and without, two to 16 K steps.  Every element
-    compared, rows after the last group untouched."""
+    half a tile, N with 8 | N/256 (n-tiles dealt to the XCDs) and without, a last column tile of 8 columns, results within the
+    last-level cache and past it (N = 16384 on), two to 16 K steps.  Every element compared, rows after the last group untouched."""
     from fuser_amd import capi
 
     sizes = [384, 128, 129, 895, 100, 2048 + 127, 256, 0, 257]
@@ -105,7 +105,8 @@ def test_grouped_mm_group_ends_inside_tiles(dev, n, k):
     b = (torch.randn(len(sizes), n, k, generator=gen) * 0.05).bfloat16()
     ps, eo, _, _ = _grouped_args(sizes, n, k, dev)
     ad, bd, psd, eod = a.to(dev), b.to(dev), ps.to(dev), eo.to(dev)
-    assert capi.describe_dispatch("grouped_mm", m, n, k, groups=len(sizes)).startswith("grouped16_tile_kernel<256x256,")
+    form = f"grouped16_tile_kernel<256x256,stream_out={int(n >= 16384)},stream_weights=0{',ragged_n' if n % 256 else ''}> "
+    assert capi.describe_dispatch("grouped_mm", m, n, k, groups=len(sizes)).startswith(form)
     out = torch.full((m, n), 7.0, dtype=torch.bfloat16, device=dev)
     capi.check(capi.lib().nvf_grouped_mm(ad.data_ptr(), bd.data_ptr(), out.data_ptr(), psd.data_ptr(), eod.data_ptr(), len(sizes),
                                          m, n, k, capi.BF16, None))
