@@ -465,11 +465,13 @@ int launch_sized(const Params& p, int64_t m_hint, int cus, void* workspace, int6
     if (lds_direct && m_hint >= 128 * (int64_t)p.groups && tiles(256, 256) >= cus / 2 && p.k >= ((p.n & 255) == 0 ? 128 : 256))
       return launch_grouped16_fast<BF16_MMA, OUT_BF16>(p, cus, stream);
     // A decode step: few rows per group on average.  The streaming kernel's partial sums cost more per item the shallower K
-    // and the more rows there are; the 128x128 tiles lose most where they leave compute units idle.  Tile kernel against
-    // streaming kernel, even and Zipf loads, us: 8 experts of 1024 x 1024, 48 rows each 18 / 10 and 20 / 13; 4096 x 4096, 48
-    // rows 84 / 66 and 88 / 77; 64 of 2048 x 7168, 24 rows 336 / 310 and 439 / 377; 32 of 2880 x 2880, 16 rows 120 / 103 and
-    // 121 / 118, 24 rows 120 / 112 and 124 / 130; 8 of 3000 x 1288, 16 rows 25 / 19 and 25 / 20, 48 rows 26 / 27; 64 of
-    // 1024 x 1024, 8 rows 26 / 30.
+    // and the more rows there are; the 128x128 tiles lose most where they leave compute units idle.  128x128 tiles (the kernel
+    // below; where K % 64 != 0, the tile kernel) against streaming kernel, even and Zipf loads, us: 8 experts of 1024 x 1024, 48
+    // rows each 10.9 / 8.4 and 11.2 / 13.2; 4096 x 4096, 48 rows 65 / 64 and 80 / 70; 64 of 2048 x 7168, 16 rows 296 / 286 and
+    // 343 / 316, 24 rows 303 / 312 and 350 / 360; 8 of 14336 x 4096, 24 rows 194 / 171 and 182 / 182; 8 of 4096 x 14336, 24 rows
+    // 152 / 161 and 168 / 207, 48 rows 178 / 177 and 271 / 240; 32 of 2880 x 2880, 16 rows 90 / 96 and 104 / 101, 24 rows 91 / 114
+    // and 105 / 119; 16 of 4096 x 2048, 16 rows 63 / 58 and 64 / 60; 8 of 3000 x 1288, 16 rows 25 / 19 and 25 / 20, 48 rows
+    // 26 / 27; 64 of 1024 x 1024, 8 rows 28 / 33 and 28 / 36.
     const int64_t first_tiles = p.groups * ceil_div(p.n, 128);
     int rows_on_average = 0;
     if (p.k >= 1024 && 4 * first_tiles <= cus) rows_on_average = 48;
@@ -477,10 +479,19 @@ int launch_sized(const Params& p, int64_t m_hint, int cus, void* workspace, int6
     else if (p.k >= 2048 || (p.k >= 1024 && 4 * first_tiles <= 3 * (int64_t)cus)) rows_on_average = 16;
     if (!dense && m_hint <= rows_on_average * (int64_t)p.groups && (m_hint / kStream16Rows + p.groups) * ceil_div(p.n, 32) < (1ll << 31))
       return launch_grouped16_streaming<BF16_MMA>(p, cus, stream);
-    // ... else the same kernel with 128x128 tiles, except for a wide N with a shallow K: there its tiles end too often for one
-    // workgroup per compute unit, the tile kernels run two (32 experts of 13824 x 2112, 1838 rows 452 / 478 us, 64 of 11840 x
-    // 2560, 1026 rows 733 / 750; 64 of 8000 x 2048, 1254 rows 458 / 399).
-    if (lds_direct && p.k >= 256 && (p.n <= 10240 || p.k >= 3072))
+    // ... else the same kernel with 128x128 tiles, with two exceptions.  A shallow K with more tiles than compute units and so
+    // few rows that there is one tile per weight panel and group: the tile kernel runs two workgroups per compute unit (tile
+    // kernel / this one, us: 64 experts of 1024 x 1024, 8 rows each 27.3 / 29.5, of 1024 x 512 17.4 / 19.0; 16 of 4096 x 512 17.1 /
+    // 18.3; 32 of 4096 x 256, 32 rows 20.6 / 22.5, 64 rows 23.7 / 24.1; 64 of 1024 x 1024, 16 rows: even loads 27.9 / 30.3, Zipf,
+    // where some groups have two tiles, 47 / 39).  And a wide N with N / 128 no multiple of 8: each XCD then owns a piece of the
+    // list instead of the same share of every group, and skewed groups make the pieces uneven (Zipf, 32 experts of 13824 x 2112, 57
+    // rows 457 / 488, 16 of them, 24 rows 197 / 214, 64 of 11840 x 2560, 57 rows 943 / 1039; even loads 190 / 165 for 16 of 13824 x
+    // 2112, 32 rows; narrower ones, Zipf: 64 of 8000 x 2048, 20 rows 461 / 406, 57 rows 543 / 529; dealt lists, Zipf: 8 of 14336 x
+    // 2048, 100 rows 144 / 129, 32 of 12288 x 2880 538 / 484, 64 of 14336 x 1024 484 / 436).
+    const bool two_per_cu = first_tiles > cus && (p.k < 512 ? m_hint <= 32 * (int64_t)p.groups
+                                                            : p.k <= 1024 && first_tiles <= 2 * (int64_t)cus && m_hint <= 8 * (int64_t)p.groups);
+    const bool uneven = (ceil_div(p.n, 128) & 7) != 0 && p.n > 10240 && p.k < 3072;
+    if (lds_direct && p.k >= 256 && !two_per_cu && !uneven)
       return launch_grouped16_small_tiles<BF16_MMA, OUT_BF16>(p, cus, stream);
   }
   if constexpr (NVFP4) {

@@ -304,11 +304,26 @@ def test_nvfp4_grouped_small_and_large_groups(m, n, k, groups, small, large):
     (16 * 8, 3000, 1288, 8, 32), (17 * 8, 3000, 1288, 8, 0), (64, 1024, 1024, 64, 0), (8, 128, 1016, 8, 0),
 ])
 def test_grouped_mm_with_few_rows_per_group_streams_the_weights(m, n, k, groups, rows):
-    """Both sides of the lines at 48, 24 and 16 rows per group; `rows`: weight rows of a work item (0: tiles, by a kernel of
-    its own where K % 64 != 0)."""
+    """Both sides of the lines at 48, 24 and 16 rows per group; `rows`: weight rows of a work item (0: tiles, by the tile
+    kernel where K % 64 != 0 and, with one row per group and a shallow K, for two tiles per compute unit)."""
     got = plan("grouped_mm", m, n, k, groups=groups)
-    tiles = "grouped16_tile_kernel<128x128," if k % 64 == 0 else "gemm16_kernel<128,128>"
+    tiles = "grouped16_tile_kernel<128x128," if k % 64 == 0 and m > groups else "gemm16_kernel<128,128>"
     assert got.startswith(f"streaming_gemm16_kernel<weight_rows={rows}," if rows else tiles) and ";" not in got, got
+
+
+@pytest.mark.parametrize("m,n,k,groups,tiles128", [
+    # a shallow K, more tiles than compute units: two workgroups of the tile kernel per compute unit, up to 8 rows per group and
+    # two tiles per compute unit, below K = 512 up to 32 rows and any number of tiles
+    (8 * 64, 1024, 1024, 64, False), (9 * 64, 1024, 1024, 64, True), (8 * 64, 1024, 1088, 64, True), (8 * 64, 1032, 1024, 64, True),
+    (8 * 16, 4096, 512, 16, False), (8 * 16, 2048, 512, 16, True), (32 * 32, 4096, 256, 32, False), (33 * 32, 4096, 256, 32, True),
+    (32 * 32, 4096, 512, 32, True), (32 * 32, 1024, 256, 32, True),
+    # a wide N, N / 128 no multiple of 8, K < 3072
+    (1824, 13824, 2112, 32, False), (1824, 14336, 2112, 32, True), (1824, 13824, 3072, 32, True), (1824, 10368, 2112, 32, False),
+    (1824, 10240, 2112, 32, True), (3648, 8000, 2048, 64, True), (800, 28672, 1024, 8, True),
+])
+def test_grouped_mm_tiles_of_128_rows_or_the_tile_kernel(m, n, k, groups, tiles128):
+    got = plan("grouped_mm", m, n, k, groups=groups)
+    assert got.startswith("grouped16_tile_kernel<128x128," if tiles128 else "gemm16_kernel<128,128>") and ";" not in got, got
 
 
 @pytest.mark.parametrize("m,n,k,groups,prefill", [
