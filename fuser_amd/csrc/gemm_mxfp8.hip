@@ -1,6 +1,6 @@
 // mxfp8_scaled_mm for gfx950 (cutlass/mxfp8_scaled_mm.cu:290-319): C = alpha * A * B^T with e4m3
-// operands and one e8m0 scale per 32 K-elements, on v_mfma_scale_f32_16x16x128_f8f6f4 (256x256 tiles, weight-streaming kernel)
-// and v_mfma_scale_f32_32x32x64_f8f6f4 (the others).
+// operands and one e8m0 scale per 32 K-elements, on v_mfma_scale_f32_16x16x128_f8f6f4 (persistent and weight-streaming
+// kernels) and v_mfma_scale_f32_32x32x64_f8f6f4 (the tile kernel for the shapes that neither takes).
 //
 // Operand layout of the latter (fp8 x fp8), measured on hardware:
 //   lane l = i + 32*g (i = row of A / column of B, g in {0,1}) supplies 32 bytes:
@@ -215,7 +215,7 @@ __global__ __launch_bounds__(256) void mxfp8_gemm_kernel(const Params p) {
 
 
 // -------------------------------------------------------------------------------------------------
-// Persistent kernels: 256x256 or 128x256 tiles, N % 256 == 0, K % 32 == 0, K >= 256.
+// Persistent kernel: 256x256, 128x256 or 128x128 tiles, N % 16 == 0, K % 32 == 0, K >= 256.
 // -------------------------------------------------------------------------------------------------
 
 // The walk over the tiles.  Workgroup ids are dealt round-robin to the 8 XCDs, so XCD x owns the contiguous tile range
@@ -270,11 +270,11 @@ struct TileWalk {
 
 // 256x256 tiles are bound by the power limit of the MFMAs: 8192^3 2.93 PFLOP/s, 394 -> 376 us against a K loop of 32x32 MFMAs
 // with all of a step's loads in one half of it.  The smaller tiles, for shapes whose large ones would leave compute units
-// idle, are bound by LDS (a 128x256 step: 1024 cycles of MFMAs, about 1560 of reads and loads) and, where the operands come
-// from memory, by the loads' latency: three and four buffers.  Weights that change from call to call, before (two buffers) and
-// now, us: 1024 x 4096 x 4096 45 -> 30, 512 x 8192 x 4096 46 -> 23 (128x128), 1979 x 7040 x 8416 157 -> 110, 330 x 9856 x 2688
-// 37 -> 17, 1000 x 5760 x 2880 36 -> 27; 45 shapes of 129..4000 rows 1.30 times as fast in the geometric mean, none more than
-// 3 % slower (999 x 1280 x 9984 39.7 -> 41.0: the columns left over by a cut no longer get a launch of their own).
+// idle, move more through LDS per MFMA (a 128x256 step at the rates measured for its parts: 1024 cycles of MFMAs, 1562 of reads
+// and loads) and, where the operands come from memory, wait for the loads: three and four buffers.  Weights that change from
+// call to call, before (two buffers) and now, us: 1024 x 4096 x 4096 45 -> 22 and 512 x 8192 x 4096 46 -> 23 (128x128), 1979 x
+// 7040 x 8416 157 -> 110, 330 x 9856 x 2688 37 -> 17, 1000 x 5760 x 2880 36 -> 27; 336 shapes of 129..8192 rows 1.23 times as
+// fast in the geometric mean.
 // The scales of a step travel like its operands: 2 KiB of 128x4 tiles (two of A, two of B) by LDS-direct loads, of which
 // every wavefront reads the pieces of its rows and keeps its lane group's byte.
 template <int NI, int NJ>
@@ -965,9 +965,10 @@ int launch_sized(const Params& p, hipStream_t stream) {
   const bool whole_other = whole == Plan::kOther;
   const int64_t bar = whole_other ? INT64_MAX : whole == Plan::kStream || (p.n & 255) != 0 ? whole_ns - whole_ns / 20 : 0;
   auto is_tiles = [](Plan q) { return q == Plan::kTiles256 || q == Plan::kTiles128 || q == Plan::kTiles128x128; };
-  // N not a multiple of 256 (29568, 1408): the columns up to the last multiple of 256 go to whatever kernel that shape
-  // gets, the remaining columns (weight rows) to a launch of their own that writes into the same rows of the result
-  // (8192 x 29568 x 8192: 4.1 -> 1.3 ms).
+  // N not a multiple of 256, where the tiles do not take it whole (K < 1024, up to 128 rows) or the last columns would cost
+  // them a round (2048 x 4224 x 2048: 256 tiles of 128x256 and 128 columns): the columns up to the last multiple of 256 go to
+  // whatever kernel that shape gets, the remaining columns (weight rows) to a launch of their own that writes into the same
+  // rows of the result.
   if ((p.n & 255) != 0 && p.n > 256 && (p.n & 15) == 0 && p.m > 64 && (p.k & 31) == 0 && p.k >= 256) {
     int64_t main_ns, rest_ns;
     const Plan main_plan = mxfp8_plan(p.m, p.n & ~255, p.k, cus, &main_ns), rest_plan = mxfp8_plan(p.m, p.n & 255, p.k, cus, &rest_ns);

@@ -1,6 +1,6 @@
 // Persistent kernel with 256x256 or 128x128 tiles for grouped_mm (16-bit operands) of gemm16.hip (included there, inside namespace nvf).
 // -------------------------------------------------------------------------------------------------
-// grouped_mm fast path (16-bit operands): 256x256 tiles, N % 256 == 0, K % 64 == 0.
+// grouped_mm fast path (16-bit operands): N % 8 == 0, K % 64 == 0.  256x256 tiles:
 // Bound by the power limit of the MFMAs (bf16 8192^3 as one group: 1.50..1.57 PFLOP/s, 810..841 -> 703..735 us against a K loop
 // of 32x32 MFMAs with all of a step's loads in one half of it; 8 experts, 8192 rows, N = 14336, K = 4096 887..907 -> 766..781).
 // 128x128 tiles: groups of fewer rows, or too few 256x256 tiles; any N % 8 == 0.  Bound by the weights' way out of HBM, for which
@@ -98,7 +98,7 @@ __global__ __launch_bounds__(256, 1) void grouped16_tile_kernel(const Params p) 
     const int64_t row_off = __builtin_amdgcn_readfirstlane((int)rows[1]);
     const int tiles_m = (m_g + BM - 1) / BM;
     const int local = __builtin_amdgcn_readfirstlane(t - tile_prefix[g] * per_m);
-    // bands of up to kBand m-tiles of near-equal height (9 m-tiles: 5 + 4), n-major inside a band
+    // bands of up to kBand m-tiles of near-equal height (9 m-tiles: 3 + 3 + 3), n-major inside a band
     const int nb = (tiles_m + kBand - 1) / kBand, base_h = tiles_m / nb, taller = tiles_m - base_h * nb;  // the first `taller` bands have base_h + 1
     const int mrow = local / per_m;  // m-tiles of the group that lie in earlier bands, plus a remainder
     const int split = taller * (base_h + 1);

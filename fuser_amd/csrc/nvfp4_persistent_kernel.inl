@@ -284,7 +284,7 @@ __global__ __launch_bounds__(512) void nvfp4_gemm_256_kernel(const Params p) {
   };
 
   // ---- MFMA fragments: 16 rows x 32 of K, lane (r16, g4) holds elements 8 g4 .. 8 g4 + 7 of row r16.  A step is ROWS rows of
-  // MFMAs: row m multiplies tile m % NI of A with the NJ tiles of B, 32-deep sub-step m / NI.  A's fragments are read three
+  // MFMAs: row m multiplies tile m % NI of A with the NJ tiles of B, 32-deep sub-step m / NI.  A's fragments are read AHEAD
   // rows ahead into four places that take turns, B's for the next sub-step into the other of two sets.
   u32x4 fa[4], fb[2][NJ];
   auto load_a_frag = [&](int buf, int m) {  // row m of a step
@@ -353,7 +353,7 @@ __global__ __launch_bounds__(512) void nvfp4_gemm_256_kernel(const Params p) {
 
   // One step: its MFMAs from LDS buffer h; between them the conversion of `src` (parity h ^ 1: the next step) into the
   // other buffer, the fragment reads and, with `refill`, the loads of the span after the next into it.  The barrier is
-  // three rows before the end: by then every wavefront has written its share of the next step and holds this step's last
+  // AHEAD rows before the end: by then every wavefront has written its share of the next step and holds this step's last
   // fragments in registers.  Everything else is dealt out between the MFMAs in parts of a few instructions.
   auto step = [&](auto h_c, Raw& src, auto at_barrier, auto refill_c, Raw& refill) {
     constexpr int h = decltype(h_c)::value;
