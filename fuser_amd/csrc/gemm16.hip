@@ -232,8 +232,9 @@ DensePlan nvfp4_dense_plan(int64_t m, int64_t n, int64_t k, int cus) {
     if (m <= 128 || (m <= 256 && !(persistent_ok && k >= 2048))) {
       stream = true;  // at most two passes over the weights (256 x 14336 x 4096: 38 instead of 58 us on tiles)
     } else if (persistent_ok && k >= 2048) {
-      // by estimated duration (measured: 512 x 4096 x 14336 115 -> 57 us, 384 x 8192 x 7168 82 -> 57 us,
-      // 640 x 14336 x 14336 381 -> 268 us; 1024 x 8192 x 4096 stays on 128x256 tiles: 64 against 76 us)
+      // by estimated duration (tiles / streaming kernel, us: 512 x 4096 x 14336 180 / 57, 384 x 8192 x 7168 92 / 53,
+      // 640 x 14336 x 14336 295 / 251, 1024 x 8192 x 4096 60 / 66, 384 x 28672 x 4096 91 / 97; over 130 shapes of 160..3000 rows
+      // the pick is within 2 % of the fastest in the geometric mean, the tiles take 0.9 of their estimate)
       stream = stream_ns <= rest_ns;
     } else {
       // Ragged shapes, which only the tile kernels take otherwise: with a deep K and a small N the streaming kernel
