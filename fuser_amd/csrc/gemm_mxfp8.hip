@@ -849,8 +849,8 @@ int64_t mxfp8_skinny_best(int64_t m, int64_t n, int64_t k, int64_t cus, int* sla
 // From 129 rows on it is scaled to what the kernel takes when the weights change from call to call (150 shapes of 129..3000
 // rows; measured / unscaled, median: K <= 1536 0.8, 2048 0.9, 4096 1.0, 7168 1.07, 8192..11008 1.2, 14336 1.2).  Workgroups go
 // to the XCDs in turn: with a number of them per slab that is no multiple of 4 the slabs that share weight rows lie in
-// different XCDs, each of which reads those rows again (256 x 2880 x 8192 22.9 us, 256 x 2560 x 7168 14; measured / unscaled
-// 1.25..1.5 times as much as else at that K, 512 x 2880 x 2880 22.0 against 16.4 on 128x128 tiles).  With the scaled
+// different XCDs, each of which reads those rows again (measured / unscaled 1.54 for 256 x 2880 x 8192, 1.30 for
+// 192 x 2560 x 8192; 1.31 for 640 x 2880 x 2880, 1.04 for 384 x 2560 x 2880).  With the scaled
 // estimate the kernel picked is within 1 % of the fastest in the geometric mean over 336 shapes, 9 % at worst.
 int64_t mxfp8_skinny_ns(int64_t m, int64_t n, int64_t k, int64_t cus) {
   int slab, rt, w;
