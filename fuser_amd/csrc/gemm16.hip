@@ -27,50 +27,6 @@
 namespace nvf {
 namespace {
 
-constexpr int kMaxGroups = 1024;  // same bound as the reference's <<<1, num_experts>>> set-up kernel
-
-struct Params {
-  const uint8_t* a;
-  const uint8_t* b;
-  const uint8_t* sfa;
-  const uint8_t* sfb;
-  const float* alpha;
-  void* out;
-  const int32_t* problem_sizes;   // nullptr => dense
-  const int32_t* expert_offsets;
-  const int32_t* sf_offsets;
-  int groups;
-  int m, n, k;
-  // split of K over workgroups (dense NVFP4 tile kernel only): work item w = tile w / splits, K spans
-  // [ (w % splits) * spans_per_split, ... ); fp32 partial tiles go to partial[split][m][n]
-  float* partial = nullptr;
-  int splits = 1;
-  int spans_per_split = 0;
-  // NVFP4 tile kernel, grouped: 1 = rows [0, rows & ~255) of every group are computed by the 256x256 kernel,
-  // take only the rows after them
-  int skip_whole_256 = 0;
-  // skinny kernel: first activation row this launch computes (its slabs of 16*TT rows follow in blockIdx.y order)
-  int m_base = 0;
-  // grouped skinny kernel: the group sizes it serves; the tile kernel skips groups of fewer than min_rows rows
-  int rows_lo = 0, rows_hi = 0, min_rows = 0;
-  // grouped skinny kernel: 0 = one block of workgroups per group (those of other sizes return at once); otherwise the
-  // launch has class_slots blocks and block i looks for the i-th group of rows_lo..rows_hi rows
-  int class_slots = 0;
-  int tail_done = 0;  // grouped NVFP4 dispatch: the ends of the large groups have been computed by an earlier launch
-  // block-scaled result (nvfp4_scaled_mm_blockscale): out = packed e2m1 [m, n/2], out_sf = e4m3 scales in the 128x4
-  // layout of [roundUp(m,128), roundUp(n/16,4)], gnorm = the result's global (encode) scale on the device
-  uint8_t* out_sf = nullptr;
-  const float* gnorm = nullptr;
-  // dense weight-streaming kernel: 0 = 16-bit result, 1 = the block-scaled result above, 2 = the fp32 product itself
-  int stream_result = 0;
-  // ... with stream_result 1: the kernel also zeroes the padding rows and columns of the scale buffer's last 128x4 tiles
-  int stream_zero_pad = 0;
-  // dense NVFP4 with a 16-bit result: elements between rows of the result; 0: n (a launch that computes some of the
-  // columns sets it)
-  int ldc = 0;
-  __host__ __device__ int out_pitch() const { return ldc ? ldc : n; }
-};
-
 // Block-scaled epilogue (cutlass/nvfp4_scaled_mm_blockscale.cu:87-93: the product is quantized to NVFP4 again along
 // N before it leaves the kernel).  One 32x32 accumulator tile: lane (li, lg) holds row li, columns 8q + 4lg + e in
 // register 4q + e, so each of the row's two 16-column blocks is shared by the lanes (li, 0) and (li, 1): amax over
@@ -109,45 +65,6 @@ __device__ __forceinline__ void quantize_acc_tile(const f32x16& acc, float alpha
   }
 }
 
-// ... of four neighbouring 16x16 accumulator tiles, i.e. of 16 rows and their four blocks: lane (r, g) holds row r, columns
-// 16 j + 4 g + e in acc[j][e].  Lane (r, g) works out the scale of block g: the exchanges with the lanes 16 and 32 further on
-// hand every lane the other three's maxima of its own block, and their factors back.  q8: the code of block g; h[j]: this
-// lane's payload bytes 2 g, 2 g + 1 of block j.  (All four lanes working out all four scales: 2 us more on a 128x256 tile.)
-__device__ __forceinline__ void quantize_acc_tiles16(const f32x4 (&acc)[4], float alpha, float gs, float decode, uint32_t& q8, uint32_t (&h)[4]) {
-  float x[4][4], m[4];
-  bool nonfinite = false;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    m[j] = -INFINITY;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      x[j][e] = acc[j][e] * alpha;
-      m[j] = fmaxf(m[j], fabsf(x[j][e]));  // NaN ignored, as the quantizer does
-      nonfinite |= !(fabsf(x[j][e]) < INFINITY);
-    }
-  }
-  const int lane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
-  const bool odd = (lane & 16) != 0, high = (lane & 32) != 0;
-  auto from = [&](float v, int other) { return __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute((lane ^ other) << 2, __builtin_bit_cast(int, v))); };
-  const float lo = fmaxf(odd ? m[1] : m[0], from(odd ? m[0] : m[1], 16)), hi = fmaxf(odd ? m[3] : m[2], from(odd ? m[2] : m[3], 16));
-  const float own = fmaxf(high ? hi : lo, from(high ? lo : hi, 32));  // of block g = 2 high + odd
-  float r;
-  q8 = nvfp4_block_scale(own, true, gs, decode, true, r);
-  const float other = from(r, 32), r_lo = high ? other : r, r_hi = high ? r : other;  // blocks odd and 2 + odd
-  const float o_lo = from(r_lo, 16), o_hi = from(r_hi, 16);
-  const float f[4] = {odd ? o_lo : r_lo, odd ? r_lo : o_lo, odd ? o_hi : r_hi, odd ? r_hi : o_hi};
-  const bool plain = __builtin_amdgcn_ballot_w64(nonfinite) == 0;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    if (plain) {
-      const uint32_t w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(0u, x[j][0] * f[j], x[j][1] * f[j], 1.0f, 0);
-      h[j] = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, x[j][2] * f[j], x[j][3] * f[j], 1.0f, 1);
-    } else {  // explicit NaN rule of the narrow cast
-      h[j] = f32x2_to_e2m1_byte(x[j][0] * f[j], x[j][1] * f[j]) | f32x2_to_e2m1_byte(x[j][2] * f[j], x[j][3] * f[j]) << 8;
-    }
-  }
-}
-
 // fills n bytes with zero (the padding of the block-scaled result's scale buffer for ragged shapes)
 __global__ __launch_bounds__(256) void zero_fill_kernel(uint32_t* __restrict__ dst, int64_t words) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -156,7 +73,6 @@ __global__ __launch_bounds__(256) void zero_fill_kernel(uint32_t* __restrict__ d
 
 // The kernels, one file each (this translation unit includes them: they share the helpers above and the launchers below)
 #include "gemm16_tile_kernels.inl"
-#include "nvfp4_persistent_kernel.inl"
 #include "nvfp4_streaming_kernel.inl"
 #include "nvfp4_group_panel_kernel.inl"
 #include "grouped16_kernel.inl"
@@ -165,6 +81,11 @@ __global__ __launch_bounds__(256) void zero_fill_kernel(uint32_t* __restrict__ d
 // -------------------------------------------------------------------------------------------------
 // Launchers of the tile kernels and the dispatch
 // -------------------------------------------------------------------------------------------------
+template <bool OUT_BF16, bool GROUPED, int TM = 4, bool OUT_F32 = false, bool OUT_FP4 = false>
+int launch_nvfp4_fast(const Params& p, int cus, hipStream_t stream) {
+  return launch_nvfp4_persistent(p, OUT_F32 ? Nvfp4Out::kF32 : OUT_FP4 ? Nvfp4Out::kFp4 : OUT_BF16 ? Nvfp4Out::kBf16 : Nvfp4Out::kF16, GROUPED, TM, cus, stream);
+}
+
 template <int BM, int BN, bool BF16_MMA, bool OUT_BF16>
 int launch_cfg(const Params& p, int grid, hipStream_t stream) {
   auto kern = gemm16_kernel<BM, BN, BF16_MMA, OUT_BF16>;

@@ -183,14 +183,6 @@ __global__ __launch_bounds__(256) void gemm16_kernel(const Params p) {
   }
 }
 
-// Grouped NVFP4: the rows of a group of m_g rows that the 256x256 kernel computes: its whole 256-row tiles, and a
-// last tile of more than 128 rows (its missing rows read as zero through the buffer range and are not stored).
-// The tile kernel takes the rows from there on; a value >= m_g means none are left.
-__device__ __forceinline__ int rows_in_256_tiles(int m_g) {
-  const int whole = m_g & ~255;
-  return m_g - whole > 128 ? whole + 256 : whole;
-}
-
 // -------------------------------------------------------------------------------------------------
 // NVFP4 tile kernel for every shape the specialised NVFP4 kernels below do not take (ragged sizes, groups,
 // fp32 result).  Same persistent walk over (group, m-tile, n-tile) items, LDS layout and MFMA loop as the
