@@ -795,3 +795,39 @@ def test_nvfp4_grouped_mm_wavefronts_that_own_weight_rows(dev, n, k, rt):
             outs.append(out)
         assert ((outs[0][:rows].float().cpu() - ref).abs() / scale).max().item() <= GEMM_MAX_REL, dtype
         assert torch.equal(*outs) and bool((outs[0][rows:] == 7.0).all())
+
+
+@pytest.mark.parametrize("last,extra,k", [(60, [], 576), (66, [], 576), (60, [130], 1024), (66, [130], 1024), (60, [], 64)])
+def test_nvfp4_grouped_mm_mid_sized_groups_in_slabs_or_in_a_launch_of_their_own(dev, last, extra, k):
+    """Calls of at most 1024 rows: with N = 2048 the groups of 33..128 rows are taken along with the small ones up to 24 slabs of
+    32 rows and have a launch of their own from 25 on.  Both sides of the line, groups at the edges of the slabs, K % 256 != 0, rows
+    outside the groups.  Every element compared; the same bits from call to call."""
+    from fuser_amd import capi
+
+    sizes = [33, 1, 64, 65, 0, 96, 97, 32, 128, 40, 5, 50, last, *extra]  # 24 slabs with last = 60, 25 with 66
+    slabs = sum(-(-s // 32) for s in sizes if 33 <= s <= 128)
+    assert slabs == (24 if last == 60 else 25)
+    n, groups, rows = 2048, len(sizes), sum(sizes)
+    m = rows + 3
+    gen = torch.Generator().manual_seed(k + last)
+    x = torch.randn(m, k, generator=gen).bfloat16()
+    ps, eo, _, _ = _grouped_args(sizes, n, k, dev)
+    so = start_offsets([O.round_up(t, 128) for t in sizes])
+    aq, asf = O.grouped_block_quantize_nvfp4(x, eo, so, None)
+    w = [(torch.randn(n, k, generator=gen) * 0.05).bfloat16() for _ in range(groups)]
+    quantized = [O.block_quantize_nvfp4(e, gs_of(e), True) for e in w]
+    bq, bsf = (torch.stack([q[i] for q in quantized]) for i in (0, 1))
+    alphas = torch.tensor([(e + 1) / gs_of(w[e]) for e in range(groups)])
+    ref = O.ref_nvfp4_scaled_grouped_mm(aq, bq, asf, bsf, alphas, ps, eo, so)[:rows]
+    held = [t.to(dev) for t in (aq, bq, asf, bsf, alphas, ps, eo, so)]
+    for dtype, code in ((torch.bfloat16, capi.BF16), (torch.float16, capi.F16)):
+        outs = []
+        for _ in range(2):
+            out = torch.full((m, n), 7.0, dtype=dtype, device=dev)
+            capi.check(capi.lib().nvf_nvfp4_scaled_grouped_mm(*[t.data_ptr() for t in held[:5]], out.data_ptr(), *[t.data_ptr() for t in held[5:]],
+                                                              groups, m, n, k, code, torch.cuda.current_stream().cuda_stream))
+            torch.cuda.synchronize()
+            outs.append(out)
+        assert bool((outs[0][rows:] == 7.0).all()) and torch.equal(outs[0], outs[1])
+        scale = ref.abs().amax(dim=1, keepdim=True).clamp(min=1e-30)
+        assert ((outs[0][:rows].float().cpu() - ref).abs() / scale).max().item() <= GEMM_MAX_REL, dtype
