@@ -346,15 +346,22 @@ bool nvfp4_wavefronts_own_rows(int64_t groups, int64_t m, int64_t n, int64_t k, 
   return k > 2048 && k < 4096 && !large && 8 * wgs >= 7 * (int64_t)cus && wgs <= cus;
 }
 
-// Grouped NVFP4, calls of at most 1024 rows: up to how many slabs of 32 rows the groups of 33..128 rows may make for the
-// persistent streaming kernel to take them along with the groups of 1..32 rows.  A launch of their own takes at least as long as
-// a workgroup walks all of K (K = 7168: 34 us), however few they are; each slab reads the weights again.  Both kernels count the
-// slabs on the device, and one of them does the work.  Own launch / slabs, us, the whole call: 512 rows over 256 experts with
-// Zipf loads (2 such groups), K = 7168, N = 2048 202 / 179; 256 over 32, 4096 x 4096 74 / 68; 300 over 8, K = 14336, N = 4096 (8
-// slabs) 120 / 94.  Line: items (slab x 64 weight rows) for three times the compute units.  N = 2048: 15 slabs 15.4 / 12.1
-// (K = 2048), 30 35 / 52 (K = 7168); N = 4096, K = 4096: 10 slabs 53 / 52, 14 102 / 106, 32 42 / 61; N = 7168: 4 192 / 193, 30
-// 40 / 56; N = 14336: 2 70 / 67, 5 82 / 89.
-int nvfp4_mid_slabs(int64_t m, int64_t n, int cus) { return m > 1024 ? 0 : (int)std::min<int64_t>(3 * (int64_t)cus * 64 / n, kMaxMidSlabs); }
+// Grouped NVFP4, calls of at most 1024 rows: the groups of 33..128 rows in slabs of 32 rows on the persistent streaming kernel, which
+// takes the groups of 1..32 rows, and no launch of their own.  That one takes 2 us with no such group, and with any as long as a
+// workgroup walks all of K; every slab reads the weights again.  Decided by the call's sizes alone, for what its groups could
+// be at worst (two slabs for every 33 rows): were it decided by the groups' sizes, where both kernels can see them, a group's
+// bits would depend on the others' (they sum K in different orders).
+// Few rows per group: up to four items (slab x 64 weight rows) per compute unit.  Own launch / slabs, us, Zipf loads: 512 rows
+// over 256 experts, N = 2048, K = 7168 221 / 190, over 64 125 / 94, 128 experts, N = 1024, K = 4096, 1024 rows 78 / 60, 16 of
+// 4096 x 4096, 256 rows 46 / 36; even ones, where no group is so large: 256 of 2048 x 7168, 512 rows 288 / 285, 16 of 2048 x 2048, 384
+// rows 17 / 15.  Beyond four Zipf loads gain 2 % (512 rows, N = 7168, K = 2048 203 / 199).  What it costs where all rows are in
+// groups of 36: up to three items 1.5 times (108 rows over 64, N = 4096, K = 14336 30 / 44), at four 1.7.
+// From 24 rows per group on most groups may be such ones: up to one item.  Even loads, one item: 4 groups of 34 rows, N = 2048,
+// K = 7168 18.0 / 15.4, 2 of 64, 4096 x 4096 14.9 / 10.0, 16 of 34, N = 512, K = 4096 13.3 / 13.6; two items: 8 of 34, N = 2048,
+// K = 7168 21.7 / 26.3, 4 of 40, 4096 x 4096 15.6 / 18.6, 2 of 34, N = 7168, K = 2048 10.4 / 11.9.
+bool nvfp4_mid_groups_as_slabs(int64_t groups, int64_t m, int64_t n, int cus) {
+  return m > 32 && m <= 1024 && 2 * (m / 33) * (n / 64) <= (m <= 24 * groups ? 4 : 1) * (int64_t)cus;
+}
 
 template <bool NVFP4, bool BF16_MMA, bool OUT_BF16>
 int launch_sized(const Params& p, int64_t m_hint, int cus, void* workspace, int64_t workspace_bytes, hipStream_t stream) {
@@ -437,22 +444,21 @@ int launch_sized(const Params& p, int64_t m_hint, int cus, void* workspace, int6
       small.a = p.a, small.b = p.b, small.sfa = p.sfa, small.sfb = p.sfb, small.alpha = p.alpha, small.out = p.out;
       small.problem_sizes = p.problem_sizes, small.expert_offsets = p.expert_offsets, small.sf_offsets = p.sf_offsets;
       small.groups = p.groups, small.m = p.m, small.n = p.n, small.k = p.k, small.dtype = OUT_BF16 ? NVF_BF16 : NVF_F16;
-      const int mid_slabs = own_rows ? 0 : nvfp4_mid_slabs(m_hint, p.n, cus);
+      const bool mid_along = !own_rows && nvfp4_mid_groups_as_slabs(p.groups, m_hint, p.n, cus);
       int rc = NVF_OK, tail_done = 0;
       if (own_rows) rc = (p.n & 511) == 0 ? launch_nvfp4_skinny_grouped<4, 2, OUT_BF16, true>(p, 1, 32, stream)
                                           : launch_nvfp4_skinny_grouped<2, 2, OUT_BF16, true>(p, 1, 32, stream);
-      if (rc == NVF_OK && (!own_rows || with_large)) rc = launch_nvfp4_decode(small, !own_rows, mid_slabs, with_large, stream);
+      if (rc == NVF_OK && (!own_rows || with_large)) rc = launch_nvfp4_decode(small, own_rows ? 0 : mid_along ? 128 : 32, with_large, stream);
       if (rc != NVF_OK || m_hint <= 32) return rc;
       // Below the prefill size the groups of 33..128 rows are few: they stream their weights like the smaller ones,
-      // found by rank among the groups of their size (a launch with few workgroups when there are few rows in all).  A
+      // found by rank among the groups of their size (a launch with few workgroups when there are few rows in all), unless the
+      // launch above has taken them along.  A
       // 128x256 tile of the persistent kernel walks all of K on one compute unit: with 64 or 256 experts, 512..5600
       // rows and K = 4096..14336 the call is 5-40 % slower that way wherever such groups exist and 0-3 % faster where
       // none does; with K < 4096 the tiles win from about 2048 rows on.
       if ((p.k & 127) != 0 || m_hint <= 1024 || (p.k >= 4096 && !is_prefill)) {
         // (also where K % 128 = 64: the form with a short last chunk)
-        Params mid = p;
-        mid.mid_slabs = mid_slabs;
-        rc = launch_nvfp4_skinny_grouped<4, 8, OUT_BF16, false>(mid, 33, 128, stream);
+        if (!mid_along) rc = launch_nvfp4_skinny_grouped<4, 8, OUT_BF16, false>(p, 33, 128, stream);
         if (with_large || m_hint <= 128) return rc;
       } else if ((p.k < 4096 || !is_prefill) && (p.n & 255) == 0 && p.k >= 256) {
         // shallow K: one 128x256 tile of the persistent kernel per weight panel converts a group's rows once per 256

@@ -34,7 +34,6 @@ struct Params {
   // grouped skinny kernel: 0 = one block of workgroups per group (those of other sizes return at once); otherwise the
   // launch has class_slots blocks and block i looks for the i-th group of rows_lo..rows_hi rows
   int class_slots = 0;
-  int mid_slabs = 0;  // ... and, if its groups make no more than this many slabs of 32 rows, has been done by another launch (0: never)
   int tail_done = 0;  // grouped NVFP4 dispatch: the ends of the large groups have been computed by an earlier launch
   // block-scaled result (nvfp4_scaled_mm_blockscale): out = packed e2m1 [m, n/2], out_sf = e4m3 scales in the 128x4
   // layout of [roundUp(m,128), roundUp(n/16,4)], gnorm = the result's global (encode) scale on the device

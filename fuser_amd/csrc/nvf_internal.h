@@ -92,10 +92,9 @@ struct Gemm16Args {
 };
 constexpr int kDtypeFp4BlockScaled = 100;  // internal result type code of launch_gemm16, next to nvf_dtype
 int launch_gemm16(int op, const Gemm16Args& args, hipStream_t stream);
-// grouped NVFP4 (nvfp4_decode.hip): the groups of 1..32 rows, those of 129 rows and more (in calls of at most 1024 rows), or both;
-// with the former those of 33..128 rows too if they are at most mid_slabs slabs of 32 rows
-constexpr int kMaxMidSlabs = 64;
-int launch_nvfp4_decode(const Gemm16Args& args, bool small_groups, int mid_slabs, bool large_groups, hipStream_t stream);
+// grouped NVFP4 (nvfp4_decode.hip), the groups of 1..rows_small rows (0, 32 or 128; from 33 on in calls of at most 1024 rows), those of
+// 129 rows and more (in calls of at most 1024 rows), or both
+int launch_nvfp4_decode(const Gemm16Args& args, int rows_small, bool large_groups, hipStream_t stream);
 // scratch bytes with which the dense NVFP4 GEMM of this shape runs faster (0: none needed)
 int64_t nvfp4_gemm_workspace_bytes(int64_t m, int64_t n, int64_t k);
 // the library's own scratch array (one per device, no allocation): its size and its address on the current device

@@ -35,7 +35,7 @@ constexpr int kMaxEntries = 1024 + 32;  // (group, slab) pairs: every group has 
 constexpr int kWeightBytes = 64 * 128, kRowBytes = kSlabRows * 128, kWeightScaleBytes = 4 * 512, kRowScaleBytes = 4 * 128;
 constexpr int kSlotBytes = kWeightBytes + kRowBytes + kWeightScaleBytes + kRowScaleBytes;
 constexpr int kSumBytes = kWaves * 4 * 1024;  // one partial 16x16 tile per weight tile, wavefront
-constexpr int kLdsBytes = kWaves * kSlotBytes + kSumBytes + (kMaxEntries + kMaxMidSlabs) * 8;
+constexpr int kLdsBytes = kWaves * kSlotBytes + kSumBytes + kMaxEntries * 8;
 static_assert(kLdsBytes <= 160 * 1024, "LDS");
 
 struct DecodeParams {
@@ -45,7 +45,6 @@ struct DecodeParams {
   const int32_t *problem_sizes, *expert_offsets, *sf_offsets;
   int groups, n, k;
   int rows_small, rows_large;  // groups of up to rows_small rows and those of rows_large or more are this launch's
-  int mid_slabs;               // ... and those in between, if there are no more slabs of them than this
 };
 
 template <bool OUT_BF16, bool STREAM, int RH>
@@ -63,20 +62,16 @@ __global__ __launch_bounds__(kWaves * 64, 2) void persistent_nvfp4_skinny_ring_k
   const int steps = (p.k + 255) >> 8;
   const int tail_pieces = (p.k & 255) >> 5;  // 32-element pieces of a row in a short last step (0: it is whole)
 
-  // ---- the list of (group, slab) pairs: {first row, rows | slab << 6 | group << 16}; behind it, in a list of their own, those of
-  // the groups of 33..128 rows, if they are few
-  u32x2* const mid_entries = entries + kMaxEntries;
-  int entry_count, mid_count;
+  // ---- the list of (group, slab) pairs: {first row, rows | slab << 6 | group << 16}
+  int entry_count;
   {
     int* const wave_total = reinterpret_cast<int*>(lds);
-    int before = 0;  // (both lists' counts in one number: low and high 16 bits)
+    int before = 0;
     for (int base = 0; base < p.groups; base += kWaves * 64) {
       const int gi = base + tid;
       const int m_g = gi < p.groups ? max(p.problem_sizes[gi * 3], 0) : 0;
       const int slabs = m_g <= p.rows_small || m_g >= p.rows_large ? (m_g + kSlabRows - 1) / kSlabRows : 0;
-      const int mids = p.mid_slabs != 0 && m_g > p.rows_small && m_g <= 128 ? (m_g + kSlabRows - 1) / kSlabRows : 0;
-      const int own = min(slabs, 8191) | mids << 16;
-      int incl = own;
+      int incl = slabs;
 #pragma unroll
       for (int d = 1; d < 64; d <<= 1) {
         const int o = __shfl_up(incl, d, 64);
@@ -84,29 +79,25 @@ __global__ __launch_bounds__(kWaves * 64, 2) void persistent_nvfp4_skinny_ring_k
       }
       if (lane == 63) wave_total[wave] = incl;
       __syncthreads();
-      int at = before + incl - own;
+      int at = before + incl - slabs;
       for (int w = 0; w < kWaves; ++w) {
         if (w < wave) at += wave_total[w];
         before += wave_total[w];
       }
       __syncthreads();
-      if (own != 0) {
+      if (slabs > 0) {
         const uint32_t row0 = (uint32_t)p.expert_offsets[gi];
-        u32x2* const list = mids != 0 ? mid_entries : entries;
-        const int first = mids != 0 ? at >> 16 : at & 0xffff, limit = mids != 0 ? kMaxMidSlabs : kMaxEntries;
-        for (int s = 0; s < slabs + mids && first + s < limit; ++s)
-          list[first + s] = u32x2{row0 + s * kSlabRows, (uint32_t)min(m_g - s * kSlabRows, kSlabRows) | (uint32_t)s << 6 | (uint32_t)gi << 16};
+        for (int s = 0; s < slabs && at + s < kMaxEntries; ++s)
+          entries[at + s] = u32x2{row0 + s * kSlabRows, (uint32_t)min(m_g - s * kSlabRows, kSlabRows) | (uint32_t)s << 6 | (uint32_t)gi << 16};
       }
     }
-    entry_count = __builtin_amdgcn_readfirstlane(min(before & 0xffff, kMaxEntries));
-    mid_count = __builtin_amdgcn_readfirstlane(before >> 16);
-    if (mid_count > p.mid_slabs) mid_count = 0;
+    entry_count = __builtin_amdgcn_readfirstlane(min(before, kMaxEntries));
     __syncthreads();
   }
   constexpr int KS = kWaves / RH;  // wavefronts that split K
   const int half = wave / KS, kpart = wave % KS;
   const int blocks = p.n / (64 * RH);
-  const int total = (entry_count + mid_count) * blocks;
+  const int total = entry_count * blocks;
 
   struct Item {
     const uint8_t *a, *b, *sfa, *sfb;
@@ -120,7 +111,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void persistent_nvfp4_skinny_ring_k
       if ((t | 15) < total) t = (t & ~15) + 2 * (j & 7) + (j >> 3);
     }
     const int e = t / blocks, block = t - e * blocks;
-    const u32x2 v = e < entry_count ? entries[e] : mid_entries[e - entry_count];
+    const u32x2 v = entries[e];
     Item it;
     it.row0 = __builtin_amdgcn_readfirstlane((int)v[0]);
     const int packed = __builtin_amdgcn_readfirstlane((int)v[1]);
@@ -317,7 +308,8 @@ template <bool OUT_BF16, bool STREAM, int RH>
 int launch_decode(const DecodeParams& p, int grid, hipStream_t stream) {
   auto kern = persistent_nvfp4_skinny_ring_kernel<OUT_BF16, STREAM, RH>;
   const char* const rows = p.rows_small == 0 ? "129.." : p.rows_large < INT32_MAX ? "1..32,129.." : "1..32";
-  if (note_launch("persistent_nvfp4_skinny_ring_kernel<stream=%d,halves=%d> grid=%d rows=%s", (int)STREAM, RH, grid, rows))
+  const char* const mid = p.rows_small > kSlabRows ? "mid_groups=1," : "";  // and those in between
+  if (note_launch("persistent_nvfp4_skinny_ring_kernel<%sstream=%d,halves=%d> grid=%d rows=%s", mid, (int)STREAM, RH, grid, rows))
     return NVF_OK;
   static std::atomic<uint64_t> configured{0};  // one bit per device
   if (const int rc = allow_dynamic_lds(reinterpret_cast<const void*>(kern), kLdsBytes, configured)) return rc;
@@ -327,7 +319,7 @@ int launch_decode(const DecodeParams& p, int grid, hipStream_t stream) {
 
 }  // namespace
 
-int launch_nvfp4_decode(const Gemm16Args& a, bool small_groups, int mid_slabs, bool large_groups, hipStream_t stream) {
+int launch_nvfp4_decode(const Gemm16Args& a, int rows_small, bool large_groups, hipStream_t stream) {
   DecodeParams p;
   p.a = static_cast<const uint8_t*>(a.a);
   p.b = static_cast<const uint8_t*>(a.b);
@@ -341,13 +333,12 @@ int launch_nvfp4_decode(const Gemm16Args& a, bool small_groups, int mid_slabs, b
   p.groups = a.groups;
   p.n = (int)a.n;
   p.k = (int)a.k;
-  p.rows_small = small_groups ? kSlabRows : 0;
-  p.mid_slabs = small_groups ? mid_slabs : 0;
+  p.rows_small = rows_small;
   p.rows_large = large_groups ? 129 : INT32_MAX;
   const int cus = cu_count();
-  const int64_t slabs = a.groups + (p.mid_slabs != 0 || large_groups ? a.m / kSlabRows : 0);  // at most
+  const int64_t slabs = a.groups + (rows_small > kSlabRows || large_groups ? a.m / kSlabRows : 0);  // at most
   // two halves of 64 weight rows per workgroup, unless such items cannot fill the compute units
-  const bool halves = small_groups && std::min<int64_t>(a.groups, a.m) * (a.n / 128) >= 4 * (int64_t)cus;
+  const bool halves = rows_small != 0 && std::min<int64_t>(a.groups, a.m) * (a.n / 128) >= 4 * (int64_t)cus;
   const int grid = (int)std::min<int64_t>(std::max(cus & ~15, 16), round_up(slabs * (a.n / (halves ? 128 : 64)), 16));
   // weights beyond what the 256 MB last-level cache holds are read past it
   const bool stream_weights = (a.k & 255) == 0 && (double)a.groups * (double)a.n * (double)a.k * (9.0 / 16) > (double)(256 << 20);

@@ -89,8 +89,8 @@ __global__ __launch_bounds__(W * 64, 2) void nvfp4_skinny_ring_kernel(const Para
       // the block-th group of the size class, in group order: every wavefront counts the groups, 256 at a time (four
       // loads in flight: a workgroup that finds no group of its own is gone after one round trip to the L2)
       grp = -1;
-      int before = 0, slabs = 0;  // (slabs: of 32 rows, 2..4 a group, where the launch may have nothing to do)
-      for (int base = 0; base < p.groups && (grp < 0 || p.mid_slabs != 0); base += 256) {
+      int before = 0;
+      for (int base = 0; base < p.groups && grp < 0; base += 256) {
         int mg[4];
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
@@ -106,11 +106,9 @@ __global__ __launch_bounds__(W * 64, 2) void nvfp4_skinny_ring_kernel(const Para
             grp = base + u * 64 + __builtin_ctzll(in_class);
           }
           before += count;
-          slabs += 2 * count + __builtin_popcountll(__builtin_amdgcn_ballot_w64(mg[u] > 64 && mg[u] <= p.rows_hi)) +
-                   __builtin_popcountll(__builtin_amdgcn_ballot_w64(mg[u] > 96 && mg[u] <= p.rows_hi));
         }
       }
-      if (grp < 0 || slabs <= p.mid_slabs) return;
+      if (grp < 0) return;
     }
     n0 = ((blockIdx.x - block * nblocks) * (NSPLIT ? W : 1) + (NSPLIT ? wave : 0)) * (16 * RT);
     m_loc = __builtin_amdgcn_readfirstlane(p.problem_sizes[grp * 3]);

@@ -236,14 +236,14 @@ def test_config5_nvfp4_grouped(n, k):
 
 
 @pytest.mark.parametrize("m,n,k,groups,streams,slots", [
-    (512, 2048, 7168, 256, True, 15),     # a decode step: 64 tokens x top-8 (the benchmark's decode-sized call)
-    (512, 7168, 2048, 256, True, 15),     # few rows in all: also against shallow weights
+    (561, 2048, 7168, 256, True, 17),     # few rows in all, but more than the launch for the smaller groups takes along
+    (512, 7168, 2048, 256, True, 15),     # also against shallow weights
     (4096, 2048, 7168, 256, True, 124),   # a short prefill against deep weights
     (4096, 4096, 14336, 64, True, 64),
     (4096, 7168, 2048, 256, False, 0),    # shallow weights from 1025 rows on: 128x256 tiles of the persistent kernel
     (3072, 7168, 2048, 32, False, 0),     # 96 rows per group and one round of 256x256 tiles: no prefill yet
     (1536, 14336, 4096, 64, True, 46),
-    (132, 2048, 7168, 256, True, 4),      # 128 workgroups: 8 wavefronts each
+    (192, 2048, 7168, 4, True, 4),        # 128 workgroups: 8 wavefronts each
 ])
 def test_nvfp4_grouped_below_the_prefill_size_streams_the_mid_sized_groups(m, n, k, groups, streams, slots):
     got = plan("nvfp4_scaled_grouped_mm", m, n, k, groups=groups)
@@ -257,6 +257,24 @@ def test_nvfp4_grouped_below_the_prefill_size_streams_the_mid_sized_groups(m, n,
     else:
         assert mid[0].startswith("nvfp4_gemm_256_kernel<grouped=1,TM=2"), got
     assert "nvfp4_group_panel_kernel" not in got, got
+
+
+@pytest.mark.parametrize("m,n,k,groups,along", [
+    # the benchmark's decode-sized call (64 tokens x top-8); up to four items of 32 x 64 per compute unit if every 33 rows were
+    # a group
+    (512, 2048, 7168, 256, True), (527, 2048, 7168, 256, True), (528, 2048, 7168, 256, True), (561, 2048, 7168, 256, False),
+    (512, 7168, 2048, 256, False), (164, 7168, 2048, 256, True), (165, 7168, 2048, 256, False),
+    (1024, 1024, 4096, 256, True), (1024, 1152, 4096, 256, False), (1025, 128, 4096, 256, False),
+    # from 24 rows per group on average on up to one
+    (192, 4096, 4096, 8, True), (193, 4096, 4096, 8, False), (98, 4096, 4096, 4, True), (99, 4096, 4096, 4, False),
+    (1024, 256, 4096, 32, True), (1024, 384, 4096, 32, False), (34, 14336, 4096, 1, False), (34, 8192, 4096, 1, True),
+    # small groups on the kernel whose wavefronts own weight rows; too few rows for such a group
+    (512, 2048, 384, 32, False), (32, 2048, 7168, 256, False), (33, 2048, 7168, 256, True),
+])
+def test_nvfp4_grouped_mid_sized_groups_along_with_the_small_ones(m, n, k, groups, along):
+    parts = plan("nvfp4_scaled_grouped_mm", m, n, k, groups=groups).split("; ")
+    assert parts[0].startswith("persistent_nvfp4_skinny_ring_kernel<mid_groups=1,") == along, parts
+    assert sum("rows=33..128" in p for p in parts) == (not along and m > 32), parts
 
 
 @pytest.mark.parametrize("m,n,k,groups,small,large", [

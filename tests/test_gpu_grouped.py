@@ -458,12 +458,13 @@ def test_nvfp4_grouped_mm_mid_sized_groups_of_a_prefill(dev, n, k):
 
 
 @pytest.mark.parametrize("n,k,few_rows", [(256, 4096, False), (128, 4224, False), (256, 512, False), (256, 512, True), (128, 4096, True),
-                                          (1024, 4096, False), (2048, 512, True)])
+                                          (128, 4160, False), (1024, 4096, False), (2048, 512, True)])
 def test_nvfp4_grouped_mm_mid_sized_groups_below_the_prefill_size(dev, n, k, few_rows):
     """300 experts, most of them with 0..3 rows, a few with 33..128 at indices on both sides of the borders at which
     the streaming kernel counts the groups of a size class (63 | 64, 255 | 256, the last one), two large ones.  Up to
-    1024 rows in all, or below 6144 with K >= 4096, the mid-sized groups stream their weights from a launch with one
-    block of workgroups per group of 33 rows that the call could hold (the block finds its group by rank); otherwise
+    1024 rows in all, or below 6144 with K >= 4096 or K % 128 != 0, the mid-sized groups stream their weights from a launch with one
+    block of workgroups per group of 33 rows that the call could hold (the block finds its group by rank), or, in the few
+    rows of 128 x 4096, as slabs in the small groups' launch; otherwise
     they run as 128x256 tiles of the persistent kernel.  The last two shapes give that launch more workgroups than compute
     units: workgroups of 4 wavefronts, two to a compute unit.  A different alpha per group, poisoned padding of the activation
     scale slabs; every element compared, rows after the last group untouched, run-to-run bit equality."""
@@ -482,8 +483,11 @@ def test_nvfp4_grouped_mm_mid_sized_groups_below_the_prefill_size(dev, n, k, few
     assert (m <= 1024) == few_rows and m < 6144
     got = capi.describe_dispatch("nvfp4_scaled_grouped_mm", m, n, k, groups=g)
     mid = [part for part in got.split("; ") if "rows=33..128" in part]
-    assert len(mid) == 1 and mid[0].startswith("nvfp4_skinny_ring_kernel<" if few_rows or k >= 4096 else "nvfp4_gemm_256_kernel<grouped=1,TM=2"), got
-    assert (",W=4>" in mid[0]) == (n >= 1024), got
+    if few_rows and n == 128:
+        assert len(mid) == 0 and "<mid_groups=1," in got, got
+    else:
+        assert len(mid) == 1 and mid[0].startswith("nvfp4_skinny_ring_kernel<" if few_rows or k >= 4096 else "nvfp4_gemm_256_kernel<grouped=1,TM=2"), got
+        assert (",W=4>" in mid[0]) == (n >= 1024), got
     gen = torch.Generator().manual_seed(n + k + few_rows)
     x = torch.randn(m, k, generator=gen).bfloat16()
     w = (torch.randn(8, n, k, generator=gen) * 0.05).bfloat16()  # eight different experts, repeated
@@ -797,27 +801,38 @@ def test_nvfp4_grouped_mm_wavefronts_that_own_weight_rows(dev, n, k, rt):
         assert torch.equal(*outs) and bool((outs[0][rows:] == 7.0).all())
 
 
-@pytest.mark.parametrize("last,extra,k", [(60, [], 576), (66, [], 576), (60, [130], 1024), (66, [130], 1024), (60, [], 64)])
-def test_nvfp4_grouped_mm_mid_sized_groups_in_slabs_or_in_a_launch_of_their_own(dev, last, extra, k):
-    """Calls of at most 1024 rows: with N = 2048 the groups of 33..128 rows are taken along with the small ones up to 24 slabs of
-    32 rows and have a launch of their own from 25 on.  Both sides of the line, groups at the edges of the slabs, K % 256 != 0, rows
-    outside the groups.  Every element compared; the same bits from call to call."""
+@pytest.mark.parametrize("groups,n,k,loads,plan_has", [
+    (14, 256, 576, [60], "<mid_groups=1,stream=0,halves=1> "),        # a short last step; sizes on both sides of every slab's border
+    (14, 256, 1024, [60, 130], "<mid_groups=1,stream=0,halves=1> "),  # with a group of 129 rows and more
+    (14, 256, 64, [60], "<mid_groups=1,stream=0,halves=1> "),         # a step for one wavefront
+    (256, 512, 2880, [60, 130], "<mid_groups=1,stream=0,halves=2> "), # items of 128 weight rows
+    (64, 1024, 7168, [], "<mid_groups=1,stream=0,halves=1> "),        # several steps per wavefront, as many items as workgroups and more
+    (256, 512, 4096, [60], "<mid_groups=1,stream=1,halves=2> "),      # weights past the last-level cache
+    (600, 128, 256, [60, 40], "<mid_groups=1,stream=0,halves=1> "),   # the list of slabs in two rounds of 512 groups
+    (14, 512, 576, [60], "rows=33..128"),                             # more items than the rule takes: a launch of their own
+    (14, 512, 1024, [60, 130], "rows=33..128"),
+])
+def test_nvfp4_grouped_mm_mid_sized_groups_in_slabs_or_in_a_launch_of_their_own(dev, groups, n, k, loads, plan_has):
+    """Calls of at most 1024 rows: by the call's sizes the groups of 33..128 rows are taken along with the small ones in slabs of 32
+    rows, or have a launch of their own.  Groups at the edges of the slabs, empty ones between them, with more than 512
+    groups on both sides of index 512; rows outside the groups.  Every element compared; the same bits from call to call."""
     from fuser_amd import capi
 
-    sizes = [33, 1, 64, 65, 0, 96, 97, 32, 128, 40, 5, 50, last, *extra]  # 24 slabs with last = 60, 25 with 66
-    slabs = sum(-(-s // 32) for s in sizes if 33 <= s <= 128)
-    assert slabs == (24 if last == 60 else 25)
-    n, groups, rows = 2048, len(sizes), sum(sizes)
-    m = rows + 3
-    gen = torch.Generator().manual_seed(k + last)
+    sizes = [0] * groups
+    spread = [33, 1, 64, 65, 0, 96, 97, 32, 128, 40, 5, 50, *loads] if groups < 600 else [33, 1, 64, 97, *loads]
+    for i, t in enumerate(spread):
+        sizes[i * (groups // 14) if groups < 600 else [0, 1, 510, 511, 512, 599][i]] = t
+    rows, m = sum(sizes), sum(sizes) + 3
+    assert plan_has in capi.describe_dispatch("nvfp4_scaled_grouped_mm", m, n, k, groups=groups)
+    gen = torch.Generator().manual_seed(k + n)
     x = torch.randn(m, k, generator=gen).bfloat16()
     ps, eo, _, _ = _grouped_args(sizes, n, k, dev)
     so = start_offsets([O.round_up(t, 128) for t in sizes])
     aq, asf = O.grouped_block_quantize_nvfp4(x, eo, so, None)
-    w = [(torch.randn(n, k, generator=gen) * 0.05).bfloat16() for _ in range(groups)]
+    w = [(torch.randn(n, k, generator=gen) * 0.05).bfloat16() for _ in range(9)]  # nine different experts, repeated
     quantized = [O.block_quantize_nvfp4(e, gs_of(e), True) for e in w]
-    bq, bsf = (torch.stack([q[i] for q in quantized]) for i in (0, 1))
-    alphas = torch.tensor([(e + 1) / gs_of(w[e]) for e in range(groups)])
+    bq, bsf = (torch.stack([quantized[e % 9][i] for e in range(groups)]) for i in (0, 1))
+    alphas = torch.tensor([(e % 11 + 1) / gs_of(w[e % 9]) for e in range(groups)])
     ref = O.ref_nvfp4_scaled_grouped_mm(aq, bq, asf, bsf, alphas, ps, eo, so)[:rows]
     held = [t.to(dev) for t in (aq, bq, asf, bsf, alphas, ps, eo, so)]
     for dtype, code in ((torch.bfloat16, capi.BF16), (torch.float16, capi.F16)):
@@ -831,3 +846,38 @@ def test_nvfp4_grouped_mm_mid_sized_groups_in_slabs_or_in_a_launch_of_their_own(
         assert bool((outs[0][rows:] == 7.0).all()) and torch.equal(outs[0], outs[1])
         scale = ref.abs().amax(dim=1, keepdim=True).clamp(min=1e-30)
         assert ((outs[0][:rows].float().cpu() - ref).abs() / scale).max().item() <= GEMM_MAX_REL, dtype
+
+
+@pytest.mark.parametrize("n,k,groups,m,sizes,more", [
+    (2048, 7168, 64, 600, [60, 100, 33, 1, 32], [40] * 9),
+    (2048, 2880, 64, 600, [60, 100, 33, 1, 32], [40] * 9),    # a short last chunk
+    (2048, 7168, 64, 512, [60, 100, 33, 1, 32], [40] * 7),    # as slabs with the small groups
+    (2048, 2048, 8, 820, [100, 97, 65], [100] * 5),
+    (2048, 2560, 64, 600, [60, 100, 33, 1, 32], [40] * 9),
+    (4096, 2048, 8, 300, [60, 40, 33], [33] * 5),
+])
+def test_nvfp4_grouped_mm_rows_do_not_depend_on_the_other_groups(dev, n, k, groups, m, sizes, more):
+    """Two calls of the same m, n, k and number of groups, whose first groups are the same rows: these rows' results are the same
+    bits, whether the other groups are empty or many of 33..128 rows.  Scales over 2^-3..2^3, so that sums in another order round differently (about one f16 result in 10^4)."""
+    from fuser_amd import capi
+
+    gen = torch.Generator(device=dev).manual_seed(k)
+    def codes(lo, hi, *shape):
+        return torch.randint(lo, hi, shape, generator=gen, device=dev, dtype=torch.uint8)
+    cols = O.round_up(k // 16, 4)
+    a, b = codes(0, 256, m, k // 2), codes(0, 256, groups, n, k // 2)
+    asf, bsf = codes(0x20, 0x50, m + 128 * groups, cols), codes(0x20, 0x50, groups, n, cols)
+    alphas = torch.full((groups,), 1e-3, device=dev)
+    outs = []
+    for rest in ([], more):
+        loads = sizes + rest + [0] * (groups - len(sizes) - len(rest))
+        assert sum(loads) <= m
+        ps, eo, _, _ = _grouped_args(loads, n, k, dev)
+        held = [t.to(dev) for t in (ps, eo, start_offsets([O.round_up(t, 128) for t in loads]))]
+        out = torch.empty(m, n, dtype=torch.float16, device=dev)
+        capi.check(capi.lib().nvf_nvfp4_scaled_grouped_mm(*[t.data_ptr() for t in (a, b, asf, bsf, alphas, out, *held)], groups, m, n, k, capi.F16,
+                                                          torch.cuda.current_stream().cuda_stream))
+        torch.cuda.synchronize()
+        outs.append(out[: sum(sizes)])
+    assert outs[0].isfinite().all() and outs[0].float().abs().mean() > 0.01
+    assert torch.equal(*outs)
