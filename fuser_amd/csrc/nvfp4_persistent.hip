@@ -202,8 +202,20 @@ __global__ __launch_bounds__(64 * W, 2) void nvfp4_gemm_256_kernel(const Params 
     st_a += 64, st_b += 64, st_sa += 1024, st_sb += 1024;
     if (++st_step == nsteps) {
       st_step = 0;
-      if (st_tile + slots < range_end) st_tile += slots;  // (past the last tile: its first steps again, which nobody reads)
-      enter_tile(st_tile);
+      if (st_tile + slots < range_end) {
+        enter_tile(st_tile += slots);
+      } else {
+        // Past the last tile nobody reads what is loaded.  From here on every load is of one row's 64 bytes (its own piece by each
+        // lane, so that tail_back stays inside the row) and one row's scales, of this tile, which is not looked up again.  (All rows
+        // of its first steps again: 2048 x 4096 x 256 10.9 -> 10.4 us, x 512 14.0 -> 13.2; 16 groups of 128 rows, N = 2048, K = 512
+        // 18.0 -> 16.6 a call.)
+        st_a -= 64 * nsteps, st_b -= 64 * nsteps, st_sa -= 1024 * nsteps, st_sb -= 1024 * nsteps;
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) b_off[j] = (uint32_t)lpiece * 16u;
+#pragma unroll
+        for (int t = 0; t < NT; ++t) a_off[t] = (uint32_t)lpiece * 16u;
+        sa_off = sb_off = 0;
+      }
     }
   };
 

@@ -484,11 +484,11 @@ def test_nvfp4_gemm_k_not_a_multiple_of_128_on_the_streaming_kernel(dev, shape):
 
 
 @pytest.mark.parametrize("shape", [(2048, 4096, 4160), (2048, 4096, 2976), (4096, 5120, 2880), (4096, 4096, 1504), (2048, 5760, 2880),
-                                   (2100, 4096, 2880)])
+                                   (1920, 4096, 288), (8192, 2048, 288), (2100, 4096, 2880)])
 def test_nvfp4_gemm_k_not_a_multiple_of_128_on_the_persistent_kernel(dev, shape):
     """K % 128 = 32, 64 or 96 on the persistent kernel (128x256 and 256x256 tiles, an odd and an even number of spans;
-    the last two shapes are cut along N and along M as well): a tile's last span is short.  NaN codes in all scale
-    padding; every element against the oracle, both output types, run-to-run bit equality."""
+    fewer spans than the loads run ahead, with the loads past the only tile among them; the fifth and the last shape are cut
+    along N and along M as well): a tile's last span is short.  NaN codes in all scale padding; every element against the oracle, both output types, run-to-run bit equality."""
     from fuser_amd import capi
 
     m, n, k = shape
