@@ -455,14 +455,30 @@ __global__ __launch_bounds__(64 * W, 2) void nvfp4_gemm_256_kernel(const Params 
         asm volatile("" ::: "memory");
       }
     } else if constexpr (OUT == Nvfp4Out::kF32) {
-      float* const obase = static_cast<float*>(p.out) + (cw.m0 + (elane & 15)) * p.n + n_w + 4 * (elane >> 4);
+      // 16 rows of 128 bytes at a time, 16-byte chunk c of row y at position c ^ (y & 7), so that whole lines leave.  (Straight
+      // from the accumulators, 16 rows' 16 bytes to 16 lanes: a block-scaled call with this dump 512 x 14336 x 4096 114.7 ->
+      // 105.2 us, 8192 x 8192 x 256 123.6 -> 116.0.)
+      uint8_t* const wr = stage + (elane & 15) * 128;
+      const int wr_chunk = (elane >> 4) ^ (elane & 7);
+      const int erow = elane >> 3;
+      const uint8_t* const rd = stage + erow * 128 + ((elane & 7) ^ erow) * 16;
+      const uint32_t ooff = ((uint32_t)erow * (uint32_t)p.n + (uint32_t)(elane & 7) * 4u) * 4u;
+      uint8_t* const obase = reinterpret_cast<uint8_t*>(static_cast<float*>(p.out) + cw.m0 * p.n + n_w);
 #pragma unroll
-      for (int i = 0; i < NIC; ++i)
+      for (int i = 0; i < NIC; ++i) {
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
           const f32x4 c = acc[i][j];
-          if (16 * i + (elane & 15) < cw.valid) *reinterpret_cast<f32x4*>(obase + (int64_t)(16 * i) * p.n + 16 * j) = f32x4{c[0] * alpha, c[1] * alpha, c[2] * alpha, c[3] * alpha};
+          *reinterpret_cast<f32x4*>(wr + (wr_chunk ^ (4 * j)) * 16) = f32x4{c[0] * alpha, c[1] * alpha, c[2] * alpha, c[3] * alpha};
         }
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          const f32x4 v = *reinterpret_cast<const f32x4*>(rd + t * 1024);
+          if (16 * i + 8 * t + erow < cw.valid) *reinterpret_cast<f32x4*>(obase + (int64_t)(16 * i + 8 * t) * p.n * 4 + ooff) = v;
+        }
+        asm volatile("" ::: "memory");
+      }
     } else {
       // Block-scaled result, 32 rows x 32 columns at a time: lane (r, g4) works out the scale of row r of block g4 & 1 of row
       // tile g4 >> 1.  The rows' 16 payload bytes are collected in LDS and leave 16 bytes per lane, a row's two codes as one
