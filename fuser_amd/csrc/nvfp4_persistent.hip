@@ -480,30 +480,45 @@ __global__ __launch_bounds__(64 * W, 2) void nvfp4_gemm_256_kernel(const Params 
         asm volatile("" ::: "memory");
       }
     } else {
-      // Block-scaled result, 32 rows x 32 columns at a time: lane (r, g4) works out the scale of row r of block g4 & 1 of row
-      // tile g4 >> 1.  The rows' 16 payload bytes are collected in LDS and leave 16 bytes per lane, a row's two codes as one
-      // 16-bit store.  Rows past M: the padding rows of the last 128-row scale tile get code zero; a 256-row tile with at most
-      // 128 rows has no second scale tile to write.
+      // Block-scaled result.  All wavefronts' parts of the tile are collected in A's second half buffer, rows of 128 payload
+      // bytes with 16-byte chunk c of row y at position c ^ (y & 7), and leave as whole rows; the codes behind the slots in the
+      // order of the 128x4 layout, where a tile's are 2 KiB in a row for every 128 rows.  Lane (r, g4) works out the scale of row r
+      // of block g4 & 1 of row tile g4 >> 1.  Rows past M: the padding rows of the last 128-row scale tile get code zero; a
+      // 256-row tile with at most 128 rows has no second scale tile to write.  (Each wavefront its 16 bytes of 32 rows and their two
+      // codes at a time, without the barriers: 2048 x 4096 x 256 10.6 -> 10.4 us, 8192 x 8192 x 256 52.6 -> 51.1, x 1024 116 -> 114.)
       const float gs = p.gnorm[0], decode = 1.0f / gs;
       const int er = elane & 15, eg = elane >> 4;
-      uint8_t* const obase = static_cast<uint8_t*>(p.out) + (cw.m0 + elane) * (p.n >> 1) + (n_w >> 1);
-      uint8_t* const sfp = p.out_sf + ((cw.m0 >> 7) * (int64_t)(p.n >> 6) + (n_w >> 6)) * 512 + ((n_w >> 5) & 1) * 2;
-      const int sf_rows = (cw.valid + 127) & ~127;
+      uint8_t* const rows = reinterpret_cast<uint8_t*>(lds) + L::kHalf;
+      uint8_t* const codes = reinterpret_cast<uint8_t*>(lds) + L::kBytes;
+      uint8_t* const wr = rows + er * 128 + ((wave ^ (er & 7)) * 16) + eg * 2;
+      uint8_t* const wc = codes + (wave >> 1) * 512 + er * 16 + (wave & 1) * 2 + (eg & 1);
 #pragma unroll
       for (int i = 0; i < NIC; i += 2) {
         const f32x4 c[4] = {acc[i][0], acc[i][1], acc[i + 1][0], acc[i + 1][1]};
         uint32_t q8, h[4];
         quantize_acc_tiles16(c, alpha, gs, decode, q8, h);
 #pragma unroll
-        for (int t = 0; t < 4; ++t) *reinterpret_cast<uint16_t*>(stage + ((t >> 1) * 16 + er) * 16 + (t & 1) * 8 + eg * 2) = (uint16_t)h[t];
-        const uint32_t other = (uint32_t)__builtin_amdgcn_ds_bpermute((elane ^ 16) << 2, (int)q8);
-        asm volatile("" ::: "memory");
-        if (elane < 32 && 16 * i + elane < cw.valid) *reinterpret_cast<u32x4*>(obase + (int64_t)(16 * i) * (p.n >> 1)) = *reinterpret_cast<const u32x4*>(stage + elane * 16);
-        const int row = 16 * (i + (eg >> 1)) + er;
-        if ((eg & 1) == 0 && row < sf_rows)
-          *reinterpret_cast<uint16_t*>(sfp + (int64_t)(row >> 7) * (p.n >> 6) * 512 + (row & 31) * 16 + ((row >> 5) & 3) * 4) = row < cw.valid ? (uint16_t)(q8 | other << 8) : (uint16_t)0;
-        asm volatile("" ::: "memory");
+        for (int t = 0; t < 4; ++t) *reinterpret_cast<uint16_t*>(wr + (i + (t >> 1)) * 2048 + (t & 1) * 8) = (uint16_t)h[t];
+        const int row = 16 * (i + (eg >> 1));
+        wc[(row >> 7) * 2048 + (row & 16) * 16 + ((row >> 5) & 3) * 4] = row + er < cw.valid ? (uint8_t)q8 : (uint8_t)0;
       }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      const int erow = elane >> 3;
+      const uint8_t* const rd = rows + erow * 128 + ((elane & 7) ^ erow) * 16;
+      uint8_t* const obase = static_cast<uint8_t*>(p.out) + (cw.m0 + erow) * (p.n >> 1) + (cw.n0 >> 1) + (elane & 7) * 16;
+#pragma unroll
+      for (int t = 0; t < NIC / 4; ++t) {
+        const int row = (wave * (NIC / 4) + t) * 8;
+        if (row + erow < cw.valid) *reinterpret_cast<u32x4*>(obase + (int64_t)row * (p.n >> 1)) = *reinterpret_cast<const u32x4*>(rd + row * 128);
+      }
+      if (wave < NIC / 4 && (wave >> 1) * 128 < cw.valid)
+        *reinterpret_cast<u32x4*>(p.out_sf + (((cw.m0 >> 7) + (wave >> 1)) * (p.n >> 6) + (cw.n0 >> 6)) * 512 + (wave & 1) * 1024 + elane * 16) =
+            *reinterpret_cast<const u32x4*>(codes + wave * 1024 + elane * 16);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // read out: the next tile's operands may be written
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
     }
     };
     // (a group's tile may hold few rows: the MFMAs of row tiles that do not exist are left out)
@@ -522,7 +537,7 @@ __global__ __launch_bounds__(64 * W, 2) void nvfp4_gemm_256_kernel(const Params 
 template <Nvfp4Out OUT, bool GROUPED, int TM, bool RAGGED_K>
 int launch_cfg(const Params& p, int cus, hipStream_t stream) {
   auto kern = nvfp4_gemm_256_kernel<OUT, GROUPED, TM, RAGGED_K>;
-  constexpr int lds_bytes = PersistentLds<4 * TM, TM == 4 ? 2 : 4>::kBytes;
+  constexpr int lds_bytes = PersistentLds<4 * TM, TM == 4 ? 2 : 4>::kBytes + (OUT == Nvfp4Out::kFp4 ? 1024 * TM : 0);  // (its scale codes: 16 bytes a row)
   static_assert(lds_bytes + (GROUPED ? (kMaxGroups + 1) * 4 : 4) <= 160 * 1024, "LDS");
   // grouped: an upper bound (128-row tiles: one per weight panel and group of at least rows_lo rows)
   const bool ragged_m = !GROUPED && p.m % (64 * TM) != 0;
