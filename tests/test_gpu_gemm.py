@@ -512,9 +512,8 @@ def test_nvfp4_gemm_k_not_a_multiple_of_128_on_the_persistent_kernel(dev, shape)
 @pytest.mark.parametrize("shape", [(300, 14336, 512), (264, 12288, 256), (520, 14336, 512), (640, 14336, 384), (700, 12288, 256),
                                    (2049, 4096, 512), (390, 28672, 384), (200, 49152, 2048)])
 def test_nvfp4_gemm_last_row_tile_with_fewer_rows_on_the_persistent_kernel(dev, shape):
-    """M no multiple of the tile height, N % 256 == K % 128 == 0 and enough tiles: the persistent kernel's variant whose
-    last row tile reads the rows past M as zero (the range of its buffer ends with the last row) and does not store
-    them.  128-row tiles with 44 and 8 rows in the last one, 256-row tiles with 8 rows (the scale tile of the tile's
+    """M no multiple of the tile height, N % 256 == K % 128 == 0 and enough tiles: the persistent kernel's last row tile reads
+    copies of the last row in the place of the rows past M and does not store them.  128-row tiles with 44 and 8 rows in the last one, 256-row tiles with 8 rows (the scale tile of the tile's
     second half does not exist and is not read), 128 (M % 256 == 128), 188, 1 and 134 rows, and a single 256-row tile row
     with 200 rows; 2 to 16 spans.
     NaN code in all scale padding, both output types, every element against the oracle, run-to-run bit equality; through

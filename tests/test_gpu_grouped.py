@@ -324,10 +324,10 @@ def test_nvfp4_grouped_mm_fewer_rows_in_all_than_the_smallest_mid_sized_group(de
                                        ([219, 130, 300, 0, 1, 257, 129, 500], 12288, 256), ([90, 40, 700, 64, 33, 1400, 128, 160, 8, 500], 22528, 256)])
 def test_nvfp4_grouped_mm_whole_tiles_and_group_ends(dev, sizes, n, k):
     """A prefill-sized call (6144 rows or more; the last two cases: fewer rows against weights so wide that the 256-row
-    tiles of the large groups fill a round with 128 rows per group, or two rounds), N % 256 == 0 (the last two cases with K % 128 = 64: a short last span): the whole 256-row tiles of every group, and a last tile of
-    more than 128 rows, run on the persistent 256x256 kernel (the rows past such a group read as zero payload
-    with whatever the scale padding holds - it is poisoned here - and are not stored), the other group ends
-    on the 128x128 tile kernel.  Groups with no whole tile, only whole tiles, one row past a tile, 255 of 256
+    tiles of the large groups fill a round with 128 rows per group, or two rounds), N % 256 == 0 (the last two cases with K % 128 =
+    64: a short last span): the whole 256-row tiles of every group, and a last tile of more than 128 rows, run on the persistent
+    256x256 kernel (the rows past such a group are read as copies of its last one, with whatever the scale padding holds - it is
+    poisoned here - and are not stored), the other group ends on the 128x128 tile kernel.  Groups with no whole tile, only whole tiles, one row past a tile, 255 of 256
     rows, empty groups; two, three and five spans per tile; the third case has more than 320 tiles, i.e. two
     per workgroup for some; the [3700, 2248, 130, 400] case ends with a 144-row tile whose 256 rows would reach past the
     activation tensor.  The last two cases add groups of every
@@ -367,15 +367,14 @@ def test_nvfp4_grouped_mm_whole_tiles_and_group_ends(dev, sizes, n, k):
         assert ((out[:rows].float().cpu() - ref[:rows]).abs() / scale).max().item() <= GEMM_MAX_REL, (sizes, dtype)
 
 
-@pytest.mark.parametrize("n,k", [(128, 128), (384, 384), (256, 1152), (128, 2048), (256, 4096), (512, 5120), (256, 320), (512, 2880), (128, 192)])
+@pytest.mark.parametrize("n,k", [(128, 128), (384, 384), (256, 1152), (128, 2048), (256, 4096), (512, 5120), (256, 320), (512, 2880), (128, 192), (384, 320)])
 def test_nvfp4_grouped_mm_small_groups_stream_their_weights(dev, n, k):
-    """Groups of 1..32 and of 33..128 rows each run on the weight-streaming kernel (one workgroup
-    per group and 64 weight rows), larger groups on the tile kernels, which skip the small ones; the last three
-    shapes have K % 128 = 64 (a short last chunk).  Sizes on
+    """Groups of 1..32 rows, and those of 129 rows and more in slabs, on the persistent streaming kernel; those of 33..128 rows
+    as slabs there too (N = 128 and 256) or on the weight-streaming kernel, one workgroup of 8 wavefronts that split K per group and 64
+    weight rows (N = 384 and 512); the last four shapes have K % 128 = 64 (a short last chunk or step).  Sizes on
     both sides of every class border, empty groups, a different alpha per group, poisoned padding of the
-    activation scale slabs, one to forty 128-deep chunks (wavefronts without work); N % 256 == 0 with K < 4096
-    takes the variant whose wavefronts own different weight rows, the rest the one that splits K; every
-    element compared, rows after the last group untouched, run-to-run bit equality."""
+    activation scale slabs, one to forty 128-deep chunks (wavefronts without work); every element compared, rows after the last group
+    untouched, run-to-run bit equality."""
     from fuser_amd import nvf_cutlass
 
     sizes = [0, 1, 16, 17, 32, 33, 64, 65, 128, 129, 300, 0, 2, 100]
@@ -403,7 +402,9 @@ def test_nvfp4_grouped_mm_small_groups_stream_their_weights(dev, n, k):
     rows = sum(sizes)
     args = (fp4(aq.to(dev)), fp4(bq.to(dev)), e4m3(asf.to(dev)), e4m3(bsf.to(dev)), alphas.to(dev), st, ct, ps.to(dev), eo.to(dev), so.to(dev))
     from fuser_amd import capi
-    assert "nvfp4_skinny_ring_kernel<" in capi.describe_dispatch("nvfp4_scaled_grouped_mm", m, n, k, g)
+    plan = capi.describe_dispatch("nvfp4_scaled_grouped_mm", m, n, k, g)
+    assert plan.startswith("persistent_nvfp4_skinny_ring_kernel<mid_groups=1," if n <= 256 else "persistent_nvfp4_skinny_ring_kernel<stream="), plan
+    assert ("; nvfp4_skinny_ring_kernel<RT=4,TT=8,grouped,nsplit=0> " in plan) == (n > 256) and plan.count(";") == (n > 256), plan
     for dtype in (torch.bfloat16, torch.float16):
         out = nvf_cutlass.nvfp4_scaled_grouped_mm(*args, dtype)
         torch.cuda.synchronize()
@@ -736,15 +737,15 @@ def test_nvfp4_grouped_mm_four_wavefronts_with_a_short_last_chunk(dev, n, k):
         assert torch.equal(out, nvf_cutlass.nvfp4_scaled_grouped_mm(*args, dtype))
 
 
-@pytest.mark.parametrize("sizes,n", [([1, 16, 17, 0, 32, 33, 128, 129, 300], 128), ([3, 20, 31, 0], 32896), ([3, 20, 31, 0], 32768)])
+@pytest.mark.parametrize("sizes,n", [([1, 16, 17, 0, 32, 33, 128, 129, 300], 128), ([1, 16, 17, 0, 32, 33, 128, 129, 300], 640), ([3, 20, 31, 0], 32896), ([3, 20, 31, 0], 32768)])
 def test_nvfp4_grouped_mm_with_empty_k_is_zero(dev, sizes, n):
-    """K = 0 through the C entry (the tensor layer refuses empty operands): every row of every group is an empty sum, i.e.
-    zero, whatever earlier kernels left in LDS; rows outside the groups stay untouched."""
+    """K = 0 through the C entry (the tensor layer refuses empty operands), the groups of 33..128 rows as slabs and in a launch of
+    their own: every row of every group is an empty sum, i.e. zero, whatever earlier kernels left in LDS; rows outside the groups stay untouched."""
     from fuser_amd import capi
 
     m, rows, groups = sum(sizes) + 4, sum(sizes), len(sizes)
     plan = capi.describe_dispatch("nvfp4_scaled_grouped_mm", m, n, 0, groups=groups)
-    assert {128: "halves=1> grid=64 rows=1..32,129..", 32896: "halves=2> ", 32768: "nsplit=1> "}[n] in plan, plan
+    assert {128: "halves=1> grid=64 rows=1..32,129..", 640: "nvfp4_skinny_ring_kernel<RT=4,TT=8,grouped,nsplit=0> grid=90 rows=33..128", 32896: "halves=2> ", 32768: "nsplit=1> "}[n] in plan, plan
     ps, eo, _, _ = _grouped_args(sizes, n, 0, dev)
     so = start_offsets([O.round_up(t, 128) for t in sizes])
     psd, eod, sod = ps.to(dev), eo.to(dev), so.to(dev)
