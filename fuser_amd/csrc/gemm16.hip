@@ -115,6 +115,10 @@ int launch_nvfp4_tile(const Params& p, int grid, hipStream_t stream) {
 // K): a round of 128-row tiles costs 58 (half the flops at 86 % of the rate); the tile kernels run their 128x128 tiles
 // two to a compute unit: 68 per such round, 45 for a last round of one tile per compute unit, and 22..47 when there
 // is no more than that in all (all measured: M = 128..1024, N = 2048..14336, K = 4096 and 14336).
+// The persistent kernel's costs are those of its form with both operands staged in LDS.  The present one takes 0.76..0.9 of
+// them from K = 4096 on (768 x 14336 x 4096 77 of 102 us, 512 x 14336 x 4096 51 of 62, 2048 x 14336 x 4096 170 of 198, 1024 x 8192 x
+// 14336 177 of 201), as much at K = 1024 (8192 x 8192 106 of 102).  The lines are where they were: near them calls still
+// stream that the tiles may do faster.
 // the streaming kernel's cost estimate is in ns within 0.8 (K = 2048) .. 1.1 (K = 14336)
 // (the form with 4 wavefronts: its discount in the cost holds among the streaming forms; against the tiles it made 26 of
 // 91 changed picks slower, at K = 2048 and 7168, and 43 faster, so there only 4 % of it stay, for 3072 <= K < 6144:
@@ -133,7 +137,8 @@ struct DensePlan {
 DensePlan nvfp4_dense_plan(int64_t m, int64_t n, int64_t k, int cus) {
   const bool stream_ok = (k & 31) == 0 && (n & 15) == 0 && k * 64 < (1ll << 31);  // 32-bit lane offsets (a short last chunk is fine)
   // (a short last span is fine; so is, with whole spans, a last row tile with fewer rows, which counts as a whole one:
-  // 384 x 28672 x 4096 as 224 tiles of 256 rows in one round instead of 336 of 128 rows in two)
+  // 384 x 28672 x 4096 as 224 tiles of 256 rows in one round instead of 336 of 128 rows in two.  The kernel would take both at
+  // once too: not measured against the cuts that such calls get now)
   const bool persistent_shape = (n & 255) == 0 && (k & 31) == 0 && k >= 256;
   const bool ok256 = persistent_shape && ((m & 255) == 0 || ((k & 127) == 0 && m > 128));
   const bool persistent_ok = persistent_shape && ((m & 127) == 0 || ((k & 127) == 0 && m > 128));
@@ -153,9 +158,9 @@ DensePlan nvfp4_dense_plan(int64_t m, int64_t n, int64_t k, int cus) {
     if (m <= 128 || (m <= 256 && !(persistent_ok && k >= 2048))) {
       stream = true;  // at most two passes over the weights (256 x 14336 x 4096: 38 instead of 58 us on tiles)
     } else if (persistent_ok && k >= 2048) {
-      // by estimated duration (tiles / streaming kernel, us: 512 x 4096 x 14336 180 / 57, 384 x 8192 x 7168 92 / 53,
+      // by estimated duration (the tiles' form that the costs were fitted to / streaming kernel, us: 512 x 4096 x 14336 180 / 57, 384 x 8192 x 7168 92 / 53,
       // 640 x 14336 x 14336 295 / 251, 1024 x 8192 x 4096 60 / 66, 384 x 28672 x 4096 91 / 97; over 130 shapes of 160..3000 rows
-      // the pick is within 2 % of the fastest in the geometric mean, the tiles take 0.9 of their estimate)
+      // the pick was within 2 % of the fastest in the geometric mean)
       stream = stream_ns <= rest_ns;
     } else {
       // Ragged shapes, which only the tile kernels take otherwise: with a deep K and a small N the streaming kernel

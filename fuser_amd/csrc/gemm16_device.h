@@ -76,12 +76,7 @@ __device__ __forceinline__ uint32_t pack2(float a, float b, bool out_bf16) {
 // LDS tile: rows x 64 16-bit elements (128 bytes per row); 16-byte chunk c of row r sits at chunk
 // position c ^ ((r >> 1) & 7): two rows fill the 64 banks once, so the MFMA fragment reads (16
 // consecutive lanes = 16 consecutive rows, one chunk) are conflict-free.
-__device__ __forceinline__ int lds_pos2(int row, int chunk) { return row * 8 + (chunk ^ ((row >> 1) & 7)); }
-__device__ __forceinline__ int lds_pos(int row, int chunk) { return lds_pos2(row, chunk); }
-// ... for tiles that ds_write_b128 fills with 4 neighbouring lanes writing every other chunk of a row: two neighbouring rows
-// differ in the lowest bit of the position as well, so that 8 lanes cover 32 banks, which is what a write is checked for
-// (a read is for 64, and stays conflict-free)
-__device__ __forceinline__ int lds_pos_staged(int row, int chunk) { return lds_pos2(row, chunk ^ (row & 1)); }
+__device__ __forceinline__ int lds_pos(int row, int chunk) { return row * 8 + (chunk ^ ((row >> 1) & 7)); }
 
 // e4m3 scales of a lane's two blocks -> fp16 pairs; one dword (8 values of one block) -> one MFMA operand
 __device__ __forceinline__ void scale_pairs(uint32_t s2, f16x2 sv[2]) {
@@ -107,7 +102,7 @@ __device__ __forceinline__ void dequant_frags(const u32x4 q, uint32_t s2, u32x4 
 }
 
 // Grouped NVFP4: the rows of a group of m_g rows that the 256x256 kernel computes: its whole 256-row tiles, and a
-// last tile of more than 128 rows (its missing rows read as zero through the buffer range and are not stored).
+// last tile of more than 128 rows (its missing rows are read as copies of the last one and are not stored).
 // The tile kernel takes the rows from there on; a value >= m_g means none are left.
 __device__ __forceinline__ int rows_in_256_tiles(int m_g) {
   const int whole = m_g & ~255;

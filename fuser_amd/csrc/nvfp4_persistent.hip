@@ -24,7 +24,7 @@
 //
 // Bound by the card's power limit on full chips (8192^3: 693 us on N(0,1) data, 560 on zeros; with the staged operands 726 and
 // 634), by instruction issue next to the MFMAs on small ones.  2048 x 14336 x 4096 175.6 -> 165.6 us, 512 x 14336 x 4096 56.1 ->
-// 49.3, 1000 x 5760 x 2816 40.4 -> 33.7.
+// 49.3.
 #include "gemm16_device.h"
 #include "nvf_internal.h"
 
@@ -545,9 +545,8 @@ int launch_cfg(const Params& p, int cus, hipStream_t stream) {
   const int64_t tiles = tiles_m * (p.n / 256);
   const unsigned grid = (unsigned)(tiles >= cus ? (cus & ~7) : ((tiles + 7) / 8) * 8);
   if (grid == 0) return NVF_OK;  // fewer rows in the whole call than the smallest group this launch serves: no work
-  // (pairs: an even number of steps)
-  if (note_launch("nvfp4_gemm_256_kernel<grouped=%d,TM=%d,f32=%d,pairs=%d%s%s%s> grid=%u rows=%d..%d min_rows=%d", (int)GROUPED, TM,
-                  (int)(OUT == Nvfp4Out::kF32), (int)((((p.k + 127) >> 7) & 1) == 0), OUT == Nvfp4Out::kFp4 ? ",fp4_blockscale" : "", ragged_m ? ",ragged_m" : "",
+  if (note_launch("nvfp4_gemm_256_kernel<grouped=%d,TM=%d,f32=%d%s%s%s> grid=%u rows=%d..%d min_rows=%d", (int)GROUPED, TM,
+                  (int)(OUT == Nvfp4Out::kF32), OUT == Nvfp4Out::kFp4 ? ",fp4_blockscale" : "", ragged_m ? ",ragged_m" : "",
                   RAGGED_K ? ",ragged_k" : "", grid, p.rows_lo, p.rows_hi, p.min_rows))
     return NVF_OK;
   static std::atomic<uint64_t> configured{0};  // one bit per device

@@ -142,9 +142,9 @@ def test_mxfp8_streaming_form_with_four_wavefronts_where_it_saves_a_round():
     (640, 8192, 4096, "nvfp4_skinny_ring_kernel<RT=4,TT=8,W=4> grid=128x5"),
     (1024, 4096, 14336, "nvfp4_skinny_ring_kernel<RT=4,TT=8,W=4> grid=64x8"),
     (256, 14336, 4096, "nvfp4_skinny_ring_kernel<RT=4,TT=8,W=4> grid=224x2"),
-    (1024, 8192, 4096, "nvfp4_gemm_256_kernel<grouped=0,TM=2,f32=0,pairs=1> grid=256"),
-    (512, 14336, 4096, "nvfp4_gemm_256_kernel<grouped=0,TM=2,f32=0,pairs=1> grid=224"),
-    (768, 14336, 4096, "nvfp4_gemm_256_kernel<grouped=0,TM=4,f32=0,pairs=1> grid=168"),
+    (1024, 8192, 4096, "nvfp4_gemm_256_kernel<grouped=0,TM=2,f32=0> grid=256"),
+    (512, 14336, 4096, "nvfp4_gemm_256_kernel<grouped=0,TM=2,f32=0> grid=224"),
+    (768, 14336, 4096, "nvfp4_gemm_256_kernel<grouped=0,TM=4,f32=0> grid=168"),
 ])
 def test_nvfp4_mid_sized_shapes(m, n, k, kernel):
     assert plan("nvfp4_scaled_mm", m, n, k).startswith(kernel), plan("nvfp4_scaled_mm", m, n, k)
@@ -210,7 +210,7 @@ def test_mxfp8_dense_n_not_a_multiple_of_256_in_one_launch_with_a_short_last_col
 
 
 def test_nvfp4_8192_cubed_takes_the_persistent_256x256_kernel():
-    assert plan("nvfp4_scaled_mm", 8192, 8192, 8192).startswith("nvfp4_gemm_256_kernel<grouped=0,TM=4,f32=0,pairs=1> grid=256")
+    assert plan("nvfp4_scaled_mm", 8192, 8192, 8192).startswith("nvfp4_gemm_256_kernel<grouped=0,TM=4,f32=0> grid=256")
 
 
 def test_config4_bf16_grouped_takes_the_persistent_kernel_in_one_launch():
