@@ -171,9 +171,10 @@ __global__ __launch_bounds__(64 * W, 2) void nvfp4_gemm_256_kernel(const Params 
   int st_tile = first_tile, st_step = 0;
   const uint8_t *st_a, *st_b, *st_sa, *st_sb;
   auto enter_tile = [&](int t) {
-    const Where w = tile_where(t);
+    const bool past = t >= range_end;
+    const Where w = past ? Where{0, 0, 0, 0, 1} : tile_where(t);
     st_a = p.a + w.m0 * kbytes;
-    const int64_t sa_slab = GROUPED ? (int64_t)__builtin_amdgcn_readfirstlane(p.sf_offsets[w.g]) * sf_padded : 0;
+    const int64_t sa_slab = GROUPED && !past ? (int64_t)__builtin_amdgcn_readfirstlane(p.sf_offsets[w.g]) * sf_padded : 0;
     // (rows past the last one are fetched as copies of it, and scales of a row group past the last as its)
     const int a0 = min(w.gm0 + AR * wave, (w.gm0 + w.valid - 1) & ~(AR - 1));
     st_sa = p.sfa + sa_slab + swizzle_128x4(a0, 0, sf_padded);
@@ -202,20 +203,17 @@ __global__ __launch_bounds__(64 * W, 2) void nvfp4_gemm_256_kernel(const Params 
     st_a += 64, st_b += 64, st_sa += 1024, st_sb += 1024;
     if (++st_step == nsteps) {
       st_step = 0;
-      if (st_tile + slots < range_end) {
-        enter_tile(st_tile += slots);
-      } else {
+      st_tile += slots;
+      if (st_tile >= range_end) {
         // Past the last tile nobody reads what is loaded.  From here on every load is of one row's 64 bytes (its own piece by each
-        // lane, so that tail_back stays inside the row) and one row's scales, of this tile, which is not looked up again.  (All rows
-        // of its first steps again: 2048 x 4096 x 256 10.9 -> 10.4 us, x 512 14.0 -> 13.2; 16 groups of 128 rows, N = 2048, K = 512
-        // 18.0 -> 16.6 a call.)
-        st_a -= 64 * nsteps, st_b -= 64 * nsteps, st_sa -= 1024 * nsteps, st_sb -= 1024 * nsteps;
+        // lane, so that tail_back stays inside the row) and one row's scales, of the first tile of all, which needs no look at the
+        // list.  (All rows of the last tile's first steps again: 2048 x 4096 x 256 10.9 -> 10.4 us, x 512 14.0 -> 13.2; 16 groups of
+        // 128 rows, N = 2048, K = 512 18.0 -> 16.6 a call.  In assembly: assigned, the offsets are copied at every step.)
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) b_off[j] = (uint32_t)lpiece * 16u;
-#pragma unroll
-        for (int t = 0; t < NT; ++t) a_off[t] = (uint32_t)lpiece * 16u;
-        sa_off = sb_off = 0;
+        for (int j = 0; j < NJ; ++j) asm volatile("v_mov_b32 %0, %1" : "+v"(b_off[j]) : "v"((uint32_t)lpiece * 16u));
+        asm volatile("v_mov_b32 %0, 0\n\tv_mov_b32 %1, 0" : "+v"(sa_off), "+v"(sb_off));
       }
+      enter_tile(st_tile);
     }
   };
 
