@@ -351,8 +351,8 @@ bool nvfp4_wavefronts_own_rows(int64_t groups, int64_t m, int64_t n, int64_t k, 
   return k > 2048 && k < 4096 && !large && 8 * wgs >= 7 * (int64_t)cus && wgs <= cus;
 }
 
-// Grouped NVFP4, calls of at most 1024 rows: the groups of 33..128 rows in slabs of 32 rows on the persistent streaming kernel, which
-// takes the groups of 1..32 rows, and no launch of their own.  That one takes 2 us with no such group, and with any as long as a
+// Grouped NVFP4, calls of at most 1024 rows (as many slabs as that kernel's list holds): the groups of 33..128 rows in slabs of 32
+// rows on the persistent streaming kernel, which takes the groups of 1..32 rows, and no launch of their own.  That one takes 2 us with no such group, and with any as long as a
 // workgroup walks all of K; every slab reads the weights again.  Decided by the call's sizes alone, for what its groups could
 // be at worst (two slabs for every 33 rows): were it decided by the groups' sizes, where both kernels can see them, a group's
 // bits would depend on the others' (they sum K in different orders).
