@@ -856,6 +856,8 @@ def test_nvfp4_grouped_mm_mid_sized_groups_in_slabs_or_in_a_launch_of_their_own(
     (2048, 2048, 8, 820, [100, 97, 65], [100] * 5),
     (2048, 2560, 64, 600, [60, 100, 33, 1, 32], [40] * 9),
     (4096, 2048, 8, 300, [60, 40, 33], [33] * 5),
+    (1024, 4096, 64, 2000, [60, 100, 33, 1, 32, 300, 129], [40] * 20),                     # more rows; a prefill
+    (512, 1088, 64, 6400, [60, 100, 81, 33, 1, 32, 300, 200, 385], [70] * 20 + [500] * 5),
 ])
 def test_nvfp4_grouped_mm_rows_do_not_depend_on_the_other_groups(dev, n, k, groups, m, sizes, more):
     """Two calls of the same m, n, k and number of groups, whose first groups are the same rows: these rows' results are the same
